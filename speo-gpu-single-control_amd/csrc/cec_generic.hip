@@ -13,21 +13,15 @@
 #include <mutex>
 
 #include "cec_generic.h"
+#include "eval_f64.h"
 
 namespace speo {
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
+typedef double doublex2 __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr double kPi = 3.1415926535897932384626433832795029;
-constexpr double kE = 2.7182818284590452353602874713526625;
-constexpr int kAS = 65;  // LDS row stride (doubles) of a 64-wide A chunk
-
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
 __device__ __forceinline__ double wave_prod(double v) {
     for (int off = 32; off > 0; off >>= 1) v *= __shfl_xor(v, off, 64);
     return v;
@@ -39,10 +33,10 @@ struct Seg {
     const double *z;
     const int *perm;
     int start, len;
-    double rate;
+    double rate, par;
     __device__ __forceinline__ double y(int i) const {
         int j = start + i;
-        if (perm) j = perm[j] - 1;
+        if (perm) j = gld(perm + j) - 1;
         return rate * z[j];
     }
 };
@@ -50,11 +44,11 @@ struct Seg {
 __device__ __forceinline__ double grie_of_rosen(double a, double b) {
     const double t1 = a * a - b, t2 = a - 1.0;
     const double t = 100.0 * t1 * t1 + t2 * t2;
-    return (t * t) / 4000.0 - cos(t) + 1.0;
+    return (t * t) / 4000.0 - cos64(t) + 1.0;
 }
 
 __device__ __forceinline__ double scaffer6(double r2) {
-    double t1 = sin(sqrt(r2));
+    double t1 = sin64(sqrt(r2));
     t1 = t1 * t1;
     const double t2 = 1.0 + 0.001 * r2;
     return 0.5 + (t1 - 0.5) / (t2 * t2);
@@ -63,120 +57,63 @@ __device__ __forceinline__ double scaffer6(double r2) {
 // The objective of one segment (FP64, CEC2014.cc forms), every lane of the
 // wave taking coordinates lane, lane + 64, ...; the wave's value is
 // returned on every lane.
-__device__ double seg_value(int obj, const Seg &s, int lane) {
+__device__ __forceinline__ double seg_value(int obj, const Seg &s, int lane) {
     const int n = s.len;
     double a = 0.0, b = 0.0;
     switch (obj) {
-    case SPEO_OBJ_ELLIPTIC:  // :481-497
-        for (int i = lane; i < n; i += 64) {
-            const double y = s.y(i);
-            a += pow(10.0, 6.0 * i / (n - 1)) * y * y;
-        }
-        return wave_sum(a);
-    case SPEO_OBJ_BENT_CIGAR:  // :499-516
-        for (int i = lane; i < n; i += 64) {
-            const double y = s.y(i);
-            a += (i == 0 ? 1.0 : 1.0e6) * y * y;
-        }
-        return wave_sum(a);
-    case SPEO_OBJ_DISCUS:  // :518-530
-        for (int i = lane; i < n; i += 64) {
-            const double y = s.y(i);
-            a += (i == 0 ? 1.0e6 : 1.0) * y * y;
-        }
-        return wave_sum(a);
     case SPEO_OBJ_ROSENBROCK:  // :552-568, fixed shift 1
         for (int i = lane; i < n - 1; i += 64) {
             const double y0 = s.y(i) + 1.0, y1 = s.y(i + 1) + 1.0;
             const double t1 = y0 * y0 - y1, t2 = y0 - 1.0;
             a += 100.0 * t1 * t1 + t2 * t2;
         }
-        return wave_sum(a);
-    case SPEO_OBJ_ACKLEY:  // :590-612
-        for (int i = lane; i < n; i += 64) {
-            const double y = s.y(i);
-            a += y * y;
-            b += cos(2.0 * kPi * y);
-        }
-        a = wave_sum(a);
-        b = wave_sum(b);
-        return kE - 20.0 * exp(-0.2 * sqrt(a / (double)n)) + 20.0 - exp(b / (double)n);
+        return wave_sum64(a);
     case SPEO_OBJ_WEIERSTRASS: {  // :615-644, a = 0.5, b = 3, k_max = 20
         // a^k and b^k as running products: 2^-k and 3^k (< 2^53) are exact in
         // FP64, so these are the values pow(a, k), pow(b, k) return
         for (int i = lane; i < n; i += 64) {
             const double y = s.y(i);
             double t = 0.0, ak = 1.0, bk = 1.0;
-            for (int k = 0; k <= 20; ++k, ak *= 0.5, bk *= 3.0) t += ak * cos(2.0 * kPi * bk * (y + 0.5));
+#pragma unroll 3
+            for (int k = 0; k <= 20; ++k, ak *= 0.5, bk *= 3.0) t += ak * cos64(2.0 * kPi64 * bk * (y + 0.5));
             a += t;
         }
-        double c = 0.0, ak = 1.0, bk = 1.0;
-        for (int k = 0; k <= 20; ++k, ak *= 0.5, bk *= 3.0) c += ak * cos(2.0 * kPi * bk * 0.5);
-        return wave_sum(a) - n * c;
+        // the constant at y = 0: sum_k 2^-k cos(3^k pi) = -(2 - 2^-20)
+        return wave_sum64(a) + n * (2.0 - 0x1p-20);
     }
     case SPEO_OBJ_GRIEWANK: {  // :646-666
         double p = 1.0;
         for (int i = lane; i < n; i += 64) {
             const double y = s.y(i);
             a += y * y;
-            p *= cos(y / sqrt(1.0 + i));
+            p *= cos64(y / sqrt(1.0 + i));
         }
-        return 1.0 + wave_sum(a) / 4000.0 - wave_prod(p);
+        return 1.0 + wave_sum64(a) / 4000.0 - wave_prod(p);
     }
-    case SPEO_OBJ_RASTRIGIN:  // :668-683
-        for (int i = lane; i < n; i += 64) {
-            const double y = s.y(i);
-            a += (y * y - 10.0 * cos(2.0 * kPi * y) + 10.0);
-        }
-        return wave_sum(a);
-    case SPEO_OBJ_SCHWEFEL:  // :705-738
-        for (int i = lane; i < n; i += 64) {
-            const double v = s.y(i) + 4.209687462275036e+002;
-            if (v > 500.0) {
-                const double m = 500.0 - fmod(v, 500.0);
-                a -= m * sin(sqrt(m));
-                const double t = (v - 500.0) / 100.0;
-                a += t * t / n;
-            } else if (v < -500.0) {
-                const double m = 500.0 - fmod(fabs(v), 500.0);
-                a += m * sin(sqrt(m));
-                const double t = (v + 500.0) / 100.0;
-                a += t * t / n;
-            } else {
-                a -= v * sin(sqrt(fabs(v)));
-            }
-        }
-        return wave_sum(a) + 4.189828872724338e+002 * n;
     case SPEO_OBJ_KATSUURA: {  // :739-765
-        const double e = 10.0 / pow(1.0 * n, 1.2);
+        // |v - floor(v + 1/2)| and |v - rint(v)| differ at halves only, where
+        // both are 1/2; 2^j and its inverse as running products are exact.
+        // A lane's factors are multiplied before their common power
+        // par = 10 / n^1.2 is taken (at most 16 of them, each <= 1 + n / 2: no
+        // overflow).
         double p = 1.0;
         for (int i = lane; i < n; i += 64) {
             const double y = s.y(i);
-            double t = 0.0;
-            for (int j = 1; j <= 32; ++j) {
-                const double sc = ldexp(1.0, j), v = sc * y;
-                t += fabs(v - floor(v + 0.5)) / sc;
+            double t = 0.0, sc = 2.0, inv = 0.5;
+#pragma unroll 4
+            for (int j = 1; j <= 32; ++j, sc *= 2.0, inv *= 0.5) {
+                const double v = sc * y;
+                t = fma(fabs(v - rint(v)), inv, t);
             }
-            p *= pow(1.0 + (i + 1) * t, e);
+            p *= 1.0 + (i + 1) * t;
         }
         const double c = 10.0 / n / n;
-        return wave_prod(p) * c - c;
+        return wave_prod(exp(s.par * log(p))) * c - c;
     }
-    case SPEO_OBJ_HAPPYCAT:  // :907-929
-    case SPEO_OBJ_HGBAT:     // :931-953
-        for (int i = lane; i < n; i += 64) {
-            const double u = s.y(i) - 1.0;
-            a += u * u;
-            b += u;
-        }
-        a = wave_sum(a);
-        b = wave_sum(b);
-        if (obj == SPEO_OBJ_HAPPYCAT) return pow(fabs(a - n), 0.25) + (0.5 * a + b) / n + 0.5;
-        return pow(fabs(a * a - b * b), 0.5) + (0.5 * a + b) / n + 0.5;
     case SPEO_OBJ_GRIE_ROSEN:  // :842-868, fixed shift 1, wrap-around pair
         for (int i = lane; i < n; i += 64)
             a += grie_of_rosen(s.y(i) + 1.0, s.y(i + 1 < n ? i + 1 : 0) + 1.0);
-        return wave_sum(a);
+        return wave_sum64(a);
     case SPEO_OBJ_ESCAFFER6:  // :870-905, wrap-around pair; one coordinate alone
         if (n == 1) {
             const double y = s.y(0);
@@ -186,182 +123,216 @@ __device__ double seg_value(int obj, const Seg &s, int lane) {
             const double y0 = s.y(i), y1 = s.y(i + 1 < n ? i + 1 : 0);
             a += scaffer6(y0 * y0 + y1 * y1);
         }
-        return wave_sum(a);
-    default:
-        return __builtin_nan("");
+        return wave_sum64(a);
+    default:  // the objectives of two coordinate sums (1..8)
+        if (obj < SPEO_OBJ_ELLIPTIC || obj > SPEO_OBJ_SCHWEFEL) return __builtin_nan("");
+        for (int i = lane; i < n; i += 64) add_terms64(obj, i, n, s.y(i), a, b);
+        return finish_objective64(obj, wave_sum64(a), wave_sum64(b), n);
     }
-}
-
-__device__ __forceinline__ double shift_at(const GenComp &c, int k) {
-    return c.o64 ? c.o64[k] : (double)c.o32[k];
-}
-__device__ __forceinline__ double rot_at(const GenComp &c, int dim, int col, int k) {
-    return c.M64 ? c.M64[(size_t)col * dim + k] : (double)c.B32[(size_t)k * c.ldb + col];
 }
 
 }  // namespace
 
-// LDS: Z tile [16][ldz] doubles (ldz = round_up(dim, 16) + 1), an A chunk
-// [16][65], and per component the rows' fit and squared distance.
-static size_t generic_lds_bytes(int dim) {
-    const size_t ldz = (size_t)round_up(dim, 16) + 1;
-    return sizeof(double) * (kGenRows * ldz + kGenRows * kAS + 2 * kMaxComp * kGenRows);
-}
+// LDS: 16 rows of round_up(dim, 8) + 2 doubles, the shifted rows and then z in
+// the same place, and each row's component values.  (The stride is 4 banks past a multiple of 16, so the 16
+// rows of a 16-byte operand read start in different banks.)
+static int generic_ld(int dim) { return round_up(dim, 8) + 2; }
+static size_t generic_lds_bytes(int dim) { return sizeof(double) * (size_t)kGenRows * (generic_ld(dim) + 2 * kMaxComp); }
 
-// NQ: 16-column tiles of Z per wave (dim <= 64 NQ).
-template <int NQ>
-__global__ __launch_bounds__(256) void k_eval_generic(GenLaunch p) {
+// A block of 16 waves takes 16 rows through every component: wave r shifts
+// row r into LDS (and sums its squared distance), the waves share the
+// 16-column tiles of z (NQ per wave, dim <= 256 NQ) on v_mfma_f64_16x16x4f64
+// with the accumulators in registers, z replaces the rows in LDS, and wave r
+// evaluates row r.  K runs in steps of 8 as two MFMA steps whose lanes take
+// k = 8 s + 2 lk and + 1, so that a lane's part of M is one 16-byte load; eight
+// of them are in flight before the first is used.
+//
+// What bounds it: at D = 100 the objective phase (FP64 vector work, one row
+// per wave) and the latency of the phases, at D >= 250 the FP64 matrix pipe (64
+// cycles per step of 4).  Measured, FP64 values of 2048 rows x 250, three
+// components: 770 us with a block per row (M read again for every row), 45 us
+// here; a five-component CEC2014 composition on 4096 rows x 100: 164 us with
+// four waves per block (four rows per wave one after another, 8-byte strided
+// loads of M, library cosines), 41 us here.  Up to 256 columns two blocks fit a
+// compute unit (64 registers); spilled registers cost more than the occupancy
+// gives (15 us per component and block at 128 registers with 40 spilled).
+template <int NQ, bool ARRAYS>
+__global__ __launch_bounds__(kGenThreads) __attribute__((amdgpu_waves_per_eu(NQ == 1 && !ARRAYS ? 8 : 4))) void k_eval_generic(GenLaunch p) {
     extern __shared__ __align__(16) char lds_raw[];
-    const int dim = p.P.dim;
-    const int ldz = round_up(dim, 16) + 1;
-    double *Zs = reinterpret_cast<double *>(lds_raw);
-    double *As = Zs + kGenRows * ldz;
-    double *gv = As + kGenRows * kAS;  // [comp][row] fit
-    double *dv = gv + kMaxComp * kGenRows;  // [comp][row] |x - o_c|^2
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int dim = p.dim, nc = p.ncomp;
+    const int ld = round_up(dim, 8) + 2;
+    double *As = reinterpret_cast<double *>(lds_raw);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lk = lane >> 4;
     const int row0 = blockIdx.x * kGenRows;
-    const int nrows = min(kGenRows, p.n - row0);
-    auto xrow = [&](int r) -> const float * {
-        const int i = row0 + r;
-        const int li = p.rows ? p.rows[i] - p.row_base : i;
-        return p.X + (size_t)li * p.ld;
-    };
-    const int T = (dim + 15) >> 4;  // 16-column tiles of Z; wave w owns w, w + 4, ...
+    const int row = row0 + wave;           // this wave's row
+    const bool mine = row < p.n;
+    const float *x = p.X;
+    if (mine) x += (size_t)(p.rows ? p.rows[row] - p.row_base : row) * p.ld;
+    double *z = As + wave * ld;
+    const int T = (dim + 15) >> 4;
 
-    for (int ci = 0; ci < p.P.ncomp; ++ci) {
-        const GenComp &C = p.P.comp[ci];
+    double *part = As + kGenRows * ld + wave * 2 * kMaxComp;  // per component: fit, squared distance
+    for (int ci = 0; ci < nc; ++ci) {
+        const GenComp &C = p.P->comp[ci];
+        const float *o32 = p.o32 + (size_t)ci * p.stride, *B32 = p.B32 + (size_t)ci * p.stride * dim;
+        const int *perm = ARRAYS ? (p.perm ? p.perm + (size_t)ci * p.stride : nullptr) : C.perm;
+        const double rate = C.rate;
+        double d = 0.0;
+        if (mine) {
+            for (int k = lane; k < round_up(dim, 8); k += 64) {
+                double v = 0.0;
+                if (k < dim) v = (double)gld(x + k) - (ARRAYS ? (double)gld(o32 + k) : gld(C.o64 + k));
+                z[k] = v * rate;
+                d = fma(v, v, d);
+            }
+        }
         if (C.rotate) {
+            __syncthreads();
             doublex4 acc[NQ];
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) acc[q] = doublex4{0.0, 0.0, 0.0, 0.0};
-            for (int k0 = 0; k0 < dim; k0 += 64) {
-                __syncthreads();
-                for (int e = tid; e < kGenRows * 64; e += 256) {
-                    const int r = e >> 6, k = k0 + (e & 63);
-                    double v = 0.0;
-                    if (r < nrows && k < dim) v = ((double)xrow(r)[k] - shift_at(C, k)) * C.rate;
-                    As[r * kAS + (e & 63)] = v;
-                }
-                __syncthreads();
-                const int ksteps = (min(64, dim - k0) + 3) >> 2;
-                for (int ks = 0; ks < ksteps; ++ks) {
-                    const int k = k0 + 4 * ks + lk;
-                    const double a = As[lr * kAS + 4 * ks + lk];
-#pragma unroll
-                    for (int q = 0; q < NQ; ++q) {
-                        const int t = wave + 4 * q;
-                        if (t < T) {
-                            const int col = 16 * t + lr;
-                            const double b = (k < dim && col < dim) ? rot_at(C, dim, col, k) : 0.0;
-                            acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[q], 0, 0, 0);
-                        }
+            for (int q = 0; q < NQ; ++q) {
+                acc[q] = doublex4{0.0, 0.0, 0.0, 0.0};
+                __builtin_amdgcn_sched_barrier(0);
+                const int t = wave + (kGenThreads / 64) * q;
+                if (t >= T) continue;
+                const double *a = As + lr * ld + 2 * lk;
+                const int steps = ARRAYS ? dim >> 3 : (dim + 7) >> 3;
+                const int col = min(16 * t + lr, dim - 1);  // (columns past the last are not stored)
+                const double *m = C.M64f + ((size_t)t * ((dim + 7) >> 3) * 64 + lane) * 2;
+                const float *bc = B32 + col;
+                auto load = [&](int s) __attribute__((always_inline)) {
+                    if constexpr (ARRAYS) {
+                        const float *q0 = bc + (size_t)(8 * s + 2 * lk) * dim;
+                        return doublex2{(double)gld(q0), (double)gld(q0 + dim)};
+                    } else {
+                        return gld(reinterpret_cast<const doublex2 *>(m + (size_t)s * 128));
                     }
+                };
+                auto step = [&](int s, doublex2 b) __attribute__((always_inline)) {
+                    const doublex2 av = *reinterpret_cast<const doublex2 *>(a + 8 * s);
+                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, b.x, acc[q], 0, 0, 0);
+                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, b.y, acc[q], 0, 0, 0);
+                };
+                constexpr int NB = 4;
+                int s = 0;
+                for (; s + NB <= steps; s += NB) {
+                    doublex2 b[NB];
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) b[u] = load(s + u);
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) step(s + u, b[u]);
+                }
+                for (; s < steps; ++s) step(s, load(s));
+                if (ARRAYS && (dim & 7)) {  // the caller's M^T ends inside the step (the rows in LDS are zero there)
+                    const int k = 8 * s + 2 * lk;
+                    doublex2 b = {0.0, 0.0};
+                    if (k < dim) b.x = (double)gld(bc + (size_t)k * dim);
+                    if (k + 1 < dim) b.y = (double)gld(bc + (size_t)(k + 1) * dim);
+                    step(s, b);
                 }
             }
+            __syncthreads();
             // accumulator element i of lane l of v_mfma_f64_16x16x4f64: row
             // l / 16 + 4 i, column l % 16
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const int t = wave + 4 * q, col = 16 * t + lr;
-                if (t < T && col < dim)
+                const int col = 16 * (wave + (kGenThreads / 64) * q) + lr;
+                if (col < dim)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) Zs[(lk + 4 * i) * ldz + col] = acc[q][i];
+                    for (int i = 0; i < 4; ++i) As[(lk + 4 * i) * ld + col] = acc[q][i];
             }
-        } else {
             __syncthreads();
-            for (int e = tid; e < kGenRows * dim; e += 256) {
-                const int r = e / dim, k = e - r * dim;
-                Zs[r * ldz + k] = r < nrows ? ((double)xrow(r)[k] - shift_at(C, k)) * C.rate : 0.0;
-            }
         }
-        __syncthreads();
-        for (int r = wave; r < nrows; r += 4) {
-            const double *z = Zs + r * ldz;
-            double g = 0.0;
-            int start = 0;
-            for (int s = 0; s < C.nseg; ++s) {
-                const Seg sv{z, C.perm, start, C.seg[s].len, C.seg[s].rate};
-                g += seg_value(C.seg[s].obj, sv, lane);
-                start += C.seg[s].len;
-            }
-            double d = 0.0;
-            if (p.P.ncomp > 1) {
-                const float *x = xrow(r);
-                for (int j = lane; j < dim; j += 64) {
-                    const double v = (double)x[j] - shift_at(C, j);
-                    d += v * v;
-                }
-                d = wave_sum(d);
-            }
-            if (lane == 0) {
-                gv[ci * kGenRows + r] = C.lambda * g + C.bias;
-                dv[ci * kGenRows + r] = d;
-            }
+        if (!mine) continue;
+        // (from here to the next component's shift a wave touches its own row only)
+        double g = 0.0;
+        int start = 0;
+        for (int s = 0; s < C.nseg; ++s) {
+            const Seg sv{z, perm, start, C.seg[s].len, C.seg[s].rate, C.seg[s].par};
+            g += seg_value(C.seg[s].obj, sv, lane);
+            start += C.seg[s].len;
+        }
+        d = wave_sum64(d);
+        if (lane == 0) {
+            part[2 * ci] = C.lambda * g + C.bias;
+            part[2 * ci + 1] = d;
         }
     }
-    __syncthreads();
-    if (tid < nrows) {
-        const int nc = p.P.ncomp;
-        double f;
-        if (nc == 1) {
-            f = gv[tid];
-        } else {
-            // cf_cal (CEC2014.cc:1481-1519)
-            double w[kMaxComp], wmax = 0.0, wsum = 0.0;
-            for (int c = 0; c < nc; ++c) {
-                const double d = dv[c * kGenRows + tid];
-                const double sg = p.P.sigma32 ? (double)p.P.sigma32[c] : p.P.comp[c].sigma;
-                w[c] = d != 0.0 ? pow(1.0 / d, 0.5) * exp(-d / 2.0 / dim / (sg * sg)) : 1.0e99;
-                wmax = fmax(wmax, w[c]);
-            }
-            for (int c = 0; c < nc; ++c) wsum += w[c];
-            if (wmax == 0.0) {
-                for (int c = 0; c < nc; ++c) w[c] = 1.0;
-                wsum = nc;
-            }
-            f = 0.0;
-            for (int c = 0; c < nc; ++c) f += w[c] / wsum * gv[c * kGenRows + tid];
-        }
-        f += p.out_bias;
-        if (p.f32) p.f32[row0 + tid] = (float)f;
-        if (p.f64) p.f64[row0 + tid] = f;
+    if (!mine) return;
+    double f;
+    if (nc == 1) {
+        f = part[0];
+    } else {
+        const int c = min(lane, nc - 1);
+        f = combine64(nc, dim, part[2 * c], part[2 * c + 1],
+                      p.sigma32 ? (double)p.sigma32[c] : p.P->comp[c].sigma, lane);
     }
+    f += p.out_bias;
+    if (lane == 0) {
+        if (p.f32) p.f32[row] = (float)f;
+        if (p.f64) p.f64[row] = f;
+    }
+}
+
+__global__ void k_gen_fragments(const double *M64, int dim, double *out) {
+    const int t = blockIdx.x, S = (dim + 7) >> 3;
+    for (int e = threadIdx.x; e < S * 128; e += blockDim.x) {
+        const int s = e >> 7, l = (e >> 1) & 63;
+        const int col = 16 * t + (l & 15), k = 8 * s + 2 * (l >> 4) + (e & 1);
+        out[(size_t)t * S * 128 + e] = col < dim && k < dim ? M64[(size_t)col * dim + k] : 0.0;
+    }
+}
+
+int gen_fragments(const double *M64, int dim, double *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_gen_fragments, dim3((dim + 15) / 16), dim3(256), 0, s, M64, dim, out);
+    return check_launch("k_gen_fragments");
+}
+
+template <int NQ, bool ARRAYS>
+static int launch_generic(const GenLaunch &p, hipStream_t s) {
+    static_assert(NQ == 1 || 256 * NQ == kGenMaxDim, "column tiles of a wave");
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval_generic<NQ, ARRAYS>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)generic_lds_bytes(256 * NQ));
+    });
+    const dim3 grid((p.n + kGenRows - 1) / kGenRows);
+    hipLaunchKernelGGL((k_eval_generic<NQ, ARRAYS>), grid, dim3(kGenThreads), generic_lds_bytes(p.dim), s, p);
+    return check_launch("k_eval_generic");
+}
+
+int check_gen_problem(const GenProblem &g, bool arrays) {
+    if (g.dim < 1 || g.dim > kGenMaxDim || g.ncomp < 1 || g.ncomp > kMaxComp)
+        return set_error(SPEO_ERR_UNSUPPORTED, "generic evaluation: dim must be in [1, 1024]");
+    for (int c = 0; c < g.ncomp; ++c) {
+        const GenComp &C = g.comp[c];
+        int total = 0;
+        for (int q = 0; q < C.nseg; ++q) total += C.seg[q].len;
+        if (C.nseg < 1 || C.nseg > kGenMaxSeg || total != g.dim)
+            return set_error(SPEO_ERR_ARG, "generic evaluation: segments do not cover the dimension");
+        if (!arrays && !C.o64) return set_error(SPEO_ERR_ARG, "generic evaluation: missing shift");
+        if (!arrays && C.rotate && !C.M64f)
+            return set_error(SPEO_ERR_ARG, "generic evaluation: missing rotation");
+    }
+    return SPEO_OK;
 }
 
 int eval_generic(const GenLaunch &p, hipStream_t s) {
     if (p.n <= 0) return SPEO_OK;
-    if (p.P.dim < 1 || p.P.dim > kGenMaxDim || p.P.ncomp < 1 || p.P.ncomp > kMaxComp)
+    if (!p.P || p.dim < 1 || p.dim > kGenMaxDim || p.ncomp < 1 || p.ncomp > kMaxComp)
         return set_error(SPEO_ERR_UNSUPPORTED, "generic evaluation: dim must be in [1, 1024]");
-    for (int c = 0; c < p.P.ncomp; ++c) {
-        const GenComp &C = p.P.comp[c];
-        int total = 0;
-        for (int q = 0; q < C.nseg; ++q) total += C.seg[q].len;
-        if (C.nseg < 1 || C.nseg > kGenMaxSeg || total != p.P.dim)
-            return set_error(SPEO_ERR_ARG, "generic evaluation: segments do not cover the dimension");
-        if (!C.o64 && !C.o32) return set_error(SPEO_ERR_ARG, "generic evaluation: missing shift");
-        if (C.rotate && !C.M64 && !C.B32)
-            return set_error(SPEO_ERR_ARG, "generic evaluation: missing rotation");
-    }
-    const dim3 grid((p.n + kGenRows - 1) / kGenRows);
-    const size_t lds = generic_lds_bytes(p.P.dim);
-    if (p.P.dim <= 128) {
-        hipLaunchKernelGGL(k_eval_generic<2>, grid, dim3(256), lds, s, p);
-    } else if (p.P.dim <= 256) {
-        hipLaunchKernelGGL(k_eval_generic<4>, grid, dim3(256), lds, s, p);
-    } else {
-        static std::once_flag once;
-        std::call_once(once, [] {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval_generic<kGenMaxDim / 64>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)generic_lds_bytes(kGenMaxDim));
-        });
-        hipLaunchKernelGGL(k_eval_generic<kGenMaxDim / 64>, grid, dim3(256), lds, s, p);
-    }
-    return check_launch("k_eval_generic");
+    if (p.o32) return p.dim <= 256 ? launch_generic<1, true>(p, s) : launch_generic<4, true>(p, s);
+    return p.dim <= 256 ? launch_generic<1, false>(p, s) : launch_generic<4, false>(p, s);
 }
 
 // ------------------------------------------------------- function tables
+
+GenSeg gen_seg(int objective, int len, double rate) {
+    return GenSeg{objective, len, rate, objective == SPEO_OBJ_KATSUURA ? 10.0 / std::pow((double)len, 1.2) : 0.0};
+}
 
 bool generic_objective(int objective) {
     return objective > SPEO_OBJ_SCHWEFEL;
@@ -402,7 +373,7 @@ bool hybrid_segments(int objective, int dim, GenComp &c) {
     for (int s = 0; s < d.nseg; ++s) {
         // ceil(p D) in FP64, CEC2014.cc:961-967; the last segment takes the rest
         const int len = s + 1 < d.nseg ? (int)std::ceil(d.p[s] * dim) : dim - used;
-        c.seg[s] = GenSeg{d.obj[s], len, d.rate[s]};
+        c.seg[s] = gen_seg(d.obj[s], len, d.rate[s]);
         used += len;
     }
     return true;

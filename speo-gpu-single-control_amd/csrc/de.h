@@ -100,6 +100,52 @@ __host__ __device__ __forceinline__ void draw_donors(DonorStream &s, const float
     jr = (int)(s.next(inj, n_inj) * (float)D);
 }
 
+// (f ascending, row ascending, NaN last): whether (a, ia) comes before (b, ib).
+__device__ __forceinline__ bool before(float a, int ia, float b, int ib) {
+    const bool an = isnan(a), bn = isnan(b);
+    if (an != bn) return bn;
+    if (!an && a != b) return a < b;
+    return ia < ib;
+}
+
+// Block argmin of (f[slot], slot) over members t in [0, count): slot =
+// perm ? perm[base + t] : base + t.  Valid on thread 0; sf and si hold one
+// entry per wave.
+__device__ __forceinline__ int block_argmin(const float *f, const int *perm, int base, int count,
+                                            float *sf, int *si) {
+    float bf = NAN;
+    int bi = 0x7fffffff;
+    for (int t = threadIdx.x; t < count; t += blockDim.x) {
+        const int slot = perm ? perm[base + t] : base + t;
+        const float v = f[slot];
+        if (bi == 0x7fffffff || before(v, slot, bf, bi)) {
+            bf = v;
+            bi = slot;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const float of = __shfl_xor(bf, off, 64);
+        const int oi = __shfl_xor(bi, off, 64);
+        if (oi != 0x7fffffff && (bi == 0x7fffffff || before(of, oi, bf, bi))) {
+            bf = of;
+            bi = oi;
+        }
+    }
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (lane == 0) {
+        sf[wave] = bf;
+        si[wave] = bi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
+            if (si[w] != 0x7fffffff && (bi == 0x7fffffff || before(sf[w], si[w], bf, bi))) {
+                bf = sf[w];
+                bi = si[w];
+            }
+    return bi;
+}
+
 int init_population(float *X, int ld, int n, int dim, float lo, float hi, uint64_t seed,
                     uint32_t row_base, hipStream_t s);
 int de_generate(const GenArgs &a, hipStream_t s);

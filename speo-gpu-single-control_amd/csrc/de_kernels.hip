@@ -155,60 +155,19 @@ int de_select(float *X, float *fX, const float *U, float *fU, int ld, int n, int
 
 // ---------------------------------------------------------------- argmin
 
-__device__ __forceinline__ bool before(float a, int ia, float b, int ib) {
-    const bool an = isnan(a), bn = isnan(b);
-    if (an != bn) return bn;
-    if (!an && a != b) return a < b;
-    return ia < ib;
-}
-
-// Block argmin of (f[slot], slot) over members t in [0, count): slot =
-// perm ? perm[base + t] : base + t.
-__device__ void block_argmin(const float *f, const int *perm, int base, int count,
-                             int *best_out) {
+__global__ void k_segment_argmin(const float *f, const int *off, int *best_out) {
     __shared__ float sf[4];
     __shared__ int si[4];
-    float bf = NAN;
-    int bi = 0x7fffffff;
-    for (int t = threadIdx.x; t < count; t += blockDim.x) {
-        const int slot = perm ? perm[base + t] : base + t;
-        const float v = f[slot];
-        if (bi == 0x7fffffff || before(v, slot, bf, bi)) {
-            bf = v;
-            bi = slot;
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const float of = __shfl_xor(bf, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (oi != 0x7fffffff && (bi == 0x7fffffff || before(of, oi, bf, bi))) {
-            bf = of;
-            bi = oi;
-        }
-    }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) {
-        sf[wave] = bf;
-        si[wave] = bi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-            if (si[w] != 0x7fffffff && (bi == 0x7fffffff || before(sf[w], si[w], bf, bi))) {
-                bf = sf[w];
-                bi = si[w];
-            }
-        *best_out = bi;
-    }
-}
-
-__global__ void k_segment_argmin(const float *f, const int *off, int *best_out) {
     const int s = blockIdx.x;
-    block_argmin(f, nullptr, off[s], off[s + 1] - off[s], best_out + s);
+    const int b = block_argmin(f, nullptr, off[s], off[s + 1] - off[s], sf, si);
+    if (threadIdx.x == 0) best_out[s] = b;
 }
 
 __global__ void k_subisland_best(const float *f, const int *perm, int S, int *best_out) {
-    block_argmin(f, perm, blockIdx.x * S, S, best_out + blockIdx.x);
+    __shared__ float sf[4];
+    __shared__ int si[4];
+    const int b = block_argmin(f, perm, blockIdx.x * S, S, sf, si);
+    if (threadIdx.x == 0) best_out[blockIdx.x] = b;
 }
 
 int subisland_best(const float *f, const int *perm, int S, int subs, int *best_out, hipStream_t s) {

@@ -14,6 +14,32 @@ struct FusedProblem {
     CompDev comp[kMaxComp];
 };
 
+// One island's answer of Engine::best, written by the kernels into pinned host
+// memory (no copies back; the caller synchronises the stream).
+struct BestOut {
+    double f64;
+    float f32;
+    int row;
+};
+
+struct BestArgs {
+    const IslandDesc *isl;
+    const FusedProblem *probs;
+    const CompParams *const *comps;
+    const float *X, *fX;
+    int *best_row;   // [islands]
+    BestOut *out;    // [islands]
+    double *part;    // [islands][kMaxComp][chunks][3] when chunks > 1
+    int chunks;      // 128-column chunks of the widest island
+};
+constexpr int kBestCols = 128;
+
+// Best row of each island and its FP64 value into p.out (the f64 of generic
+// problems is left to the generic kernel); ncomp: the most components of any
+// island's problem.
+int best_rows(const BestArgs &p, int islands, int ncomp, int max_dim, hipStream_t s);
+
+
 // ------------------------------------------------------------ epoch kernel
 //
 // k_island_epoch: a workgroup runs a whole epoch (the generations between

@@ -34,7 +34,6 @@
 
 #include "engine.h"
 #include "eval.h"
-#include "eval_f64.h"
 #include "surrogate.h"
 
 namespace speo {
@@ -322,18 +321,6 @@ __global__ void k_fill(float *p, int n, float v) {
 __global__ void k_add_u32(uint32_t *p, uint32_t v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) p[0] += v;
 }
-__global__ void k_eval_f64_rows(const CompParams *const *comps, const int *ncomp, const int *dims,
-                                const IslandDesc *isl, const int *rows, const float *X,
-                                double *out) {
-    extern __shared__ __align__(16) char lds_raw[];
-    const IslandDesc I = isl[blockIdx.x];
-    const int li = rows[blockIdx.x] - I.row_off;
-    const double f = eval_row_f64(comps[I.problem], ncomp[I.problem], dims[I.problem],
-                                  X + I.elem_off + (size_t)li * I.ld,
-                                  reinterpret_cast<double *>(lds_raw));
-    if (threadIdx.x == 0) out[blockIdx.x] = f;
-}
-
 // ------------------------------------------------------------------ launch
 
 template <int RT, int PREC, int MODE>
@@ -469,10 +456,10 @@ struct Engine {
     IslandDesc *isl_dev = nullptr;
     int *row_off_dev = nullptr, *dst_dev = nullptr, *best_buf = nullptr, *worst_buf = nullptr;
     int *best_row_dev = nullptr;
-    double *best_f64_dev = nullptr;
+    BestOut *best_out = nullptr, *best_out_dev = nullptr;  // pinned host memory and its device address
+    double *best_part = nullptr;  // chunk sums of best() when an island is wider than kBestCols
     FusedProblem *probs_dev = nullptr;
     const CompParams **params_tab_dev = nullptr;
-    int *ncomp_dev = nullptr, *dims_dev = nullptr;
     std::map<int, TileDesc *> tiles_dev;  // per rows-per-block
     std::map<int, int> ntiles;
     uint32_t *gen_base = nullptr;
@@ -570,12 +557,13 @@ Engine::~Engine() {
     for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
     for (auto &kv : tiles_dev) (void)hipFree(kv.second);
     void *bufs[] = {isl_dev, row_off_dev, dst_dev, best_buf, worst_buf, best_row_dev,
-                    best_f64_dev, probs_dev, params_tab_dev, ncomp_dev, dims_dev, gen_base,
+                    best_part, probs_dev, params_tab_dev, gen_base,
                     blocks_dev, Xnext, donor_buf, row_island_dev,
                     X, fX[0], fX[1], U[0], U[1], fU[0], fU[1], srows_dev, cand, pred, rho_dev, scored_dev,
                     AX, Ay, Xb, tb, Xh, yh, predh, ranks_ws, heads_dev, round_dev, perm_dev,
                     best_sub_dev, info_dev};
     for (void *b : bufs) (void)hipFree(b);
+    (void)hipHostFree(best_out);
     if (own_stream && stream) (void)hipStreamDestroy(stream);
 }
 
@@ -612,7 +600,6 @@ int Engine::upload_tables() {
     SPEO_TRY(upload_vec(&dst_dev, dst));
     std::vector<FusedProblem> fp(problems.size());
     std::vector<const CompParams *> tab(problems.size());
-    std::vector<int> nc(problems.size()), dm(problems.size());
     for (size_t q = 0; q < problems.size(); ++q) {
         const ProblemHost &P = problems[q]->h;
         FusedProblem f{};
@@ -628,18 +615,18 @@ int Engine::upload_tables() {
         }
         fp[q] = f;
         tab[q] = P.params_dev;
-        nc[q] = P.ncomp;
-        dm[q] = P.dim;
     }
     SPEO_TRY(upload_vec(&probs_dev, fp));
     SPEO_TRY(upload_vec(&params_tab_dev, tab));
-    SPEO_TRY(upload_vec(&ncomp_dev, nc));
-    SPEO_TRY(upload_vec(&dims_dev, dm));
     const int k = std::max(cfg.migration_size, 1);
     SPEO_TRY_HIP(hipMalloc(&best_buf, sizeof(int) * (size_t)I * k));
     SPEO_TRY_HIP(hipMalloc(&worst_buf, sizeof(int) * (size_t)I * k));
     SPEO_TRY_HIP(hipMalloc(&best_row_dev, sizeof(int) * (size_t)I));
-    SPEO_TRY_HIP(hipMalloc(&best_f64_dev, sizeof(double) * (size_t)I));
+    SPEO_TRY_HIP(hipHostMalloc(reinterpret_cast<void **>(&best_out), sizeof(BestOut) * (size_t)I, hipHostMallocMapped));
+    SPEO_TRY_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&best_out_dev), best_out, 0));
+    if (max_dim > kBestCols)
+        SPEO_TRY_HIP(hipMalloc(&best_part, sizeof(double) * 3 * (size_t)I * kMaxComp *
+                                               ((size_t)(max_dim + kBestCols - 1) / kBestCols)));
     SPEO_TRY_HIP(hipMalloc(&gen_base, sizeof(uint32_t)));
     SPEO_TRY_HIP(hipMemset(gen_base, 0, sizeof(uint32_t)));
     return SPEO_OK;
@@ -1798,34 +1785,23 @@ int Engine::tune_epoch_parts() {
 int Engine::best(int *row_out, float *f32_out, double *f64_out) {
     SPEO_TRY(finalize_pending(stream));
     const int cur = cfg.mode == SPEO_MODE_FUSED ? p : 0;
-    SPEO_TRY(segment_argmin(fX[cur], row_off_dev, I, best_row_dev, stream));
-    const size_t lds = sizeof(double) * ((size_t)max_dim + 16);
-    if (lds > 48 * 1024)
-        SPEO_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval_f64_rows),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_eval_f64_rows, dim3(I), dim3(256), lds, stream, params_tab_dev,
-                       ncomp_dev, dims_dev, isl_dev, best_row_dev, X, best_f64_dev);
-    SPEO_TRY(check_launch("k_eval_f64_rows"));
+    const int chunks = (max_dim + kBestCols - 1) / kBestCols;
+    BestArgs a{isl_dev, probs_dev, params_tab_dev, X, fX[cur], best_row_dev, best_out_dev, best_part, chunks};
+    int nc = 1;
+    for (const auto *q : problems) nc = std::max(nc, q->h.ncomp);
+    SPEO_TRY(best_rows(a, I, nc, max_dim, stream));
     for (int i = 0; i < I && any_generic; ++i) {  // generic problems: the FP64 generic kernel
         const IslandDesc &d = isl[(size_t)i];
         const ProblemHost &P = problems[(size_t)d.problem]->h;
         if (P.generic)
-            SPEO_TRY(eval_problem_generic(P, X + d.elem_off, d.ld, 1, nullptr, best_f64_dev + i,
+            SPEO_TRY(eval_problem_generic(P, X + d.elem_off, d.ld, 1, nullptr, &best_out_dev[i].f64,
                                           best_row_dev + i, d.row_off, stream));
     }
-    std::vector<int> rows((size_t)I);
-    std::vector<double> f64((size_t)I);
-    std::vector<float> fall((size_t)total_rows);
-    SPEO_TRY_HIP(hipMemcpyAsync(rows.data(), best_row_dev, sizeof(int) * I, hipMemcpyDeviceToHost, stream));
-    SPEO_TRY_HIP(hipMemcpyAsync(f64.data(), best_f64_dev, sizeof(double) * I, hipMemcpyDeviceToHost, stream));
-    if (f32_out)
-        SPEO_TRY_HIP(hipMemcpyAsync(fall.data(), fX[cur], sizeof(float) * total_rows,
-                                    hipMemcpyDeviceToHost, stream));
     SPEO_TRY_HIP(hipStreamSynchronize(stream));
     for (int i = 0; i < I; ++i) {
-        if (row_out) row_out[i] = rows[(size_t)i];
-        if (f32_out) f32_out[i] = fall[(size_t)rows[(size_t)i]];
-        if (f64_out) f64_out[i] = f64[(size_t)i];
+        if (row_out) row_out[i] = best_out[i].row;
+        if (f32_out) f32_out[i] = best_out[i].f32;
+        if (f64_out) f64_out[i] = best_out[i].f64;
     }
     return SPEO_OK;
 }

@@ -29,7 +29,10 @@ size_t eval_scratch_floats(int ncomp, int dim, int n);
 int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out,
                  float *scratch, int precision, int rows_per_block, hipStream_t s);
 
-// FP64 evaluation, one block per row.
+// FP64 evaluation: the generic kernel up to its 1024 columns, else one block
+// per row (eval_rows_f64).
+int eval_rows_f64(const CompParams *comps, int ncomp, int dim, const float *X, int ld, int n,
+                  double *f_out, hipStream_t s);
 int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double *f_out,
                      hipStream_t s);
 

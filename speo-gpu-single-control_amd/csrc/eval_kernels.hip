@@ -6,12 +6,13 @@
 // CalW/CombineFitness for compositions) by one kernel per N chunk of Z.
 #include <algorithm>
 #include <atomic>
+#include <map>
 #include <mutex>
+#include <tuple>
 #include <unordered_map>
 
 #include "cec_generic.h"
 #include "eval.h"
-#include "eval_f64.h"
 
 namespace speo {
 
@@ -276,16 +277,6 @@ __global__ __launch_bounds__(256) void k_comp_combine_rows(const CompParams *com
     }
 }
 
-__global__ __launch_bounds__(256) void k_eval_f64(const CompParams *comps, int ncomp, int dim,
-                                                  const float *X, int ld, int n, double *f_out) {
-    extern __shared__ __align__(16) char lds_raw[];
-    const int row = blockIdx.x;
-    if (row >= n) return;
-    const double f = eval_row_f64(comps, ncomp, dim, X + (size_t)row * ld,
-                                  reinterpret_cast<double *>(lds_raw));
-    if (threadIdx.x == 0) f_out[row] = f;
-}
-
 // ------------------------------------------------------------------ launch
 
 // k_eval_wide for the 16-bit evaluations that k_eval<64> would run.
@@ -348,7 +339,9 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
 int eval_problem_generic(const ProblemHost &P, const float *X, int ld, int n, float *f32,
                          double *f64, const int *rows, int row_base, hipStream_t s) {
     GenLaunch g{};
-    g.P = *P.gen;
+    g.P = P.gen;
+    g.dim = P.dim;
+    g.ncomp = P.ncomp;
     g.X = X;
     g.ld = ld;
     g.n = n;
@@ -403,14 +396,8 @@ int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_o
 int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double *f_out,
                      hipStream_t s) {
     if (n <= 0) return SPEO_OK;
-    if (P.generic) return eval_problem_generic(P, X, ld, n, nullptr, f_out, nullptr, 0, s);
-    const size_t lds = sizeof(double) * ((size_t)P.dim + 16);
-    if (lds > 48 * 1024)
-        SPEO_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval_f64),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_eval_f64, dim3(n), dim3(256), lds, s, P.params_dev, P.ncomp, P.dim, X,
-                       ld, n, f_out);
-    return check_launch("k_eval_f64");
+    if (P.gen) return eval_problem_generic(P, X, ld, n, nullptr, f_out, nullptr, 0, s);
+    return eval_rows_f64(P.params_dev, P.ncomp, P.dim, X, ld, n, f_out, s);
 }
 
 int default_rows_per_block(int n, int dim, int precision) {
@@ -463,43 +450,78 @@ int dim_tables(int dim, DimTables &out) {
 // d_rotated_data [ncomp][next_pow2(dim)][dim] (B = M^T, row-padded),
 // d_shuffle_data [ncomp][next_pow2(dim)] (1-based), d_sigma [ncomp] and the
 // scratch rows d_rotated_elements [pop_size][next_pow2(dim)].
+//
+// The device description of function `fid` at `dim` (objectives, segments,
+// rates and composition parameters; the arrays come with each call), built at
+// the first call that needs it on a device and kept, as the dimension's tables
+// are: at most 30 of 2 KB per dimension.
+static int dropin_problem(int fid, int dim, const GenProblem **out, int *ncomp) {
+    static std::mutex mu;
+    static std::map<std::tuple<int, int, int>, std::pair<GenProblem *, int>> table;
+    int dev = 0;
+    SPEO_TRY_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(mu);
+    auto &e = table[std::make_tuple(dev, fid, dim)];
+    if (!e.first) {
+        int nc = 0;
+        CecComp cc[kMaxComp];
+        if (!cec_function(fid, &nc, cc)) return set_error(SPEO_ERR_UNSUPPORTED, "unknown function");
+        GenProblem g{};
+        g.dim = dim;
+        g.ncomp = nc;
+        for (int c = 0; c < nc; ++c) {
+            GenComp &G = g.comp[c];
+            if (cc[c].objective >= SPEO_OBJ_HYBRID_1) {
+                hybrid_segments(cc[c].objective, dim, G);
+            } else {
+                G.nseg = 1;
+                G.seg[0] = gen_seg(cc[c].objective, dim, 1.0);
+            }
+            G.rate = cc[c].rate;
+            G.rotate = cc[c].rotate;
+            G.lambda = cc[c].lambda;
+            G.bias = cc[c].bias;
+            G.sigma = cc[c].sigma;
+        }
+        SPEO_TRY(check_gen_problem(g, true));
+        GenProblem *d = nullptr;
+        SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&d), sizeof(g)));
+        SPEO_TRY_HIP(hipMemcpy(d, &g, sizeof(g), hipMemcpyHostToDevice));
+        e = {d, nc};
+    }
+    *out = e.first;
+    *ncomp = e.second;
+    return SPEO_OK;
+}
+
 static int dropin_generic(real *f, real *X, real *shift, real *B, int *shuffle, real *sigma,
                           int n, int dim, real bias, int fid) {
     int nc = 0;
     CecComp cc[kMaxComp];
     if (!cec_function(fid, &nc, cc)) return set_error(SPEO_ERR_UNSUPPORTED, "unknown function");
-    const int Dp = next_pow2_dim(dim);
-    GenLaunch g{};
-    g.P.dim = dim;
-    g.P.ncomp = nc;
-    g.P.sigma32 = nc > 1 ? sigma : nullptr;
+    if (dim > kGenMaxDim)
+        return set_error(SPEO_ERR_UNSUPPORTED, "generic evaluation: dim must be in [1, 1024]");
+    bool hybrid = false;
     for (int c = 0; c < nc; ++c) {
-        GenComp &G = g.P.comp[c];
-        if (cc[c].objective >= SPEO_OBJ_HYBRID_1) {
-            if (!shuffle) return set_error(SPEO_ERR_ARG, "missing shuffle data");
-            hybrid_segments(cc[c].objective, dim, G);
-            G.perm = shuffle + (size_t)c * Dp;
-        } else {
-            G.nseg = 1;
-            G.seg[0] = GenSeg{cc[c].objective, dim, 1.0};
-        }
+        hybrid = hybrid || cc[c].objective >= SPEO_OBJ_HYBRID_1;
         if (cc[c].rotate && !B) return set_error(SPEO_ERR_ARG, "missing rotation matrix");
-        G.rate = cc[c].rate;
-        G.rotate = cc[c].rotate;
-        G.o32 = shift + (size_t)c * Dp;
-        G.B32 = B ? B + (size_t)c * Dp * dim : nullptr;
-        G.ldb = dim;
-        G.lambda = cc[c].lambda;
-        G.bias = cc[c].bias;
-        G.sigma = cc[c].sigma;
     }
+    if (hybrid && !shuffle) return set_error(SPEO_ERR_ARG, "missing shuffle data");
+    GenLaunch g{};
+    SPEO_TRY(dropin_problem(fid, dim, &g.P, &g.ncomp));
+    g.dim = dim;
     g.X = X;
-    g.ld = Dp;
+    g.ld = next_pow2_dim(dim);
     g.n = n;
     g.f32 = f;
     // F1-F16 ignore the call's bias; the hybrid and composition chains add it
     // in CombineFitness (kernel_CEC2014_CUDA.cu:205, 1227, 1447).
     g.out_bias = fid >= 17 ? bias : 0.0;
+    g.o32 = shift;
+    g.B32 = B;
+    g.sigma32 = sigma;
+    g.perm = hybrid ? shuffle : nullptr;
+    g.stride = g.ld;
     return eval_generic(g, nullptr);
 }
 

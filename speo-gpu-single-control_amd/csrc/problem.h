@@ -33,6 +33,7 @@ struct CompHost {
     uint16_t *Mbf[3] = {nullptr, nullptr, nullptr};  // BF16 parts of M, [dim][ldm16]
     uint16_t *Mh[3] = {nullptr, nullptr, nullptr};   // FP16 parts of 2^14 M
     double *M64 = nullptr;      // [dim][dim]
+    double *M64f = nullptr;     // M64 in the FP64 kernel's fragment order (dim <= 1024, rotated)
     // dim <= 128 only: zero-padded layouts of the register-resident-B path
     float *B32s = nullptr;                                   // 128 x 128, fragment order
     uint16_t *Mbfs[3] = {nullptr, nullptr, nullptr};         // [128][round_up(dim,32)]
@@ -67,7 +68,7 @@ struct ProblemHost {
     // whole problem is evaluated by the FP64 generic kernel (cec_generic.h).
     bool generic = false;
     int *perm[kMaxComp] = {};       // hybrids: 1-based shuffle [dim] on the device
-    GenProblem *gen = nullptr;      // host description with device pointers
+    GenProblem *gen = nullptr;      // the FP64 kernel's description, on the device (dim <= 1024)
 };
 
 }  // namespace speo

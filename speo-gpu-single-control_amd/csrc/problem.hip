@@ -115,6 +115,7 @@ static void free_problem(ProblemHost &P) {
         (void)hipFree(h.shift64);
         (void)hipFree(h.B32);
         (void)hipFree(h.M64);
+        (void)hipFree(h.M64f);
         (void)hipFree(h.B32s);
         for (int p = 0; p < 3; ++p) {
             (void)hipFree(h.Mbf[p]);
@@ -129,7 +130,7 @@ static void free_problem(ProblemHost &P) {
         (void)hipFree(P.perm[c]);
         P.perm[c] = nullptr;
     }
-    delete P.gen;
+    (void)hipFree(P.gen);
     P.gen = nullptr;
     P.generic = false;
     (void)hipFree(P.colw);
@@ -262,15 +263,14 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                                        h.shift32, h.shift64, h.M64};
     }
     SPEO_TRY(upload(&P.params_dev, params));
-    if (generic) {
-        P.generic = true;
-        P.gen = new (std::nothrow) GenProblem{};
-        if (!P.gen) return set_error(SPEO_ERR_ALLOC, "speo_problem_create: out of host memory");
-        P.gen->dim = dim;
-        P.gen->ncomp = ncomp;
+    P.generic = generic;
+    if (dim <= kGenMaxDim) {  // the FP64 kernel's description of the problem
+        std::vector<GenProblem> gen(1);
+        gen[0].dim = dim;
+        gen[0].ncomp = ncomp;
         for (int c = 0; c < ncomp; ++c) {
             const CompHost &h = P.comp[c];
-            GenComp &g = P.gen->comp[c];
+            GenComp &g = gen[0].comp[c];
             if (objectives[c] >= SPEO_OBJ_HYBRID_1) {
                 std::vector<int> perm(shuffle + (size_t)c * dim, shuffle + (size_t)(c + 1) * dim);
                 SPEO_TRY(upload(&P.perm[c], perm));
@@ -278,16 +278,24 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                 g.perm = P.perm[c];
             } else {
                 g.nseg = 1;
-                g.seg[0] = GenSeg{objectives[c], dim, 1.0};
+                g.seg[0] = gen_seg(objectives[c], dim, 1.0);
             }
             g.rate = h.rate64;
             g.rotate = rotation && !is_identity(rotation + (size_t)c * D * D, dim) ? 1 : 0;
             g.o64 = h.shift64;
-            g.M64 = h.M64;
+            if (g.rotate) {
+                SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&P.comp[c].M64f),
+                                       sizeof(double) * gen_fragment_doubles(dim)));
+                SPEO_TRY(gen_fragments(h.M64, dim, P.comp[c].M64f, nullptr));
+                g.M64f = h.M64f;
+            }
             g.lambda = h.lambda;
             g.bias = h.bias;
             g.sigma = h.sigma;
         }
+        SPEO_TRY(check_gen_problem(gen[0], false));
+        SPEO_TRY(upload(&P.gen, gen));
+        SPEO_TRY_HIP(hipStreamSynchronize(nullptr));  // the fragments, for callers on other streams
     }
     return SPEO_OK;
 }
