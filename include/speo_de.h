@@ -281,10 +281,11 @@ SPEO_EXPORT int speo_problem_create_cec(const char *dir, int func_id, int dim, s
 SPEO_EXPORT int speo_evaluate(speo_problem p, const float *X, int ld, int n, float *f_out,
                               int precision, speo_stream_t stream);
 
-/* Kernel of speo_evaluate's 16-bit evaluations (BF16, FP16 and their
- * splits) of problems wider than 128 columns on at least 1024 rows, where the
- * arithmetic is that of 64-row tiles: enable 1 (default) a kernel with
- * 256-column tiles, 0 the 64-row-tile kernel, -1 leaves the setting.  Both
+/* Kernel of speo_evaluate's evaluations of problems wider than 128 columns
+ * where the arithmetic is that of 64-row tiles (the 16-bit precisions and
+ * their splits on at least 1024 rows, FP32 when the rows fill the chip):
+ * enable 1 (default) a kernel with 256-column tiles, 0 the 64-row-tile kernel,
+ * -1 leaves the setting.  Both
  * give the same bits; the switch is for tests and measurements.  Process-wide;
  * returns the previous setting, and *launches (optional) the number of
  * launches of the 256-column kernel so far. */

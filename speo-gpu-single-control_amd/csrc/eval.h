@@ -22,12 +22,15 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
                    float *part, float lambda, float bias, int raw, int precision,
                    int rows_per_block, hipStream_t s);
 
-// Scratch (floats) eval_problem needs for n rows.
+// Scratch (floats) eval_problem needs for n rows; with eval_scratch_batched
+// floats a wide composition's components run in one launch.
 size_t eval_scratch_floats(int ncomp, int dim, int n);
+size_t eval_scratch_batched(int ncomp, int dim, int n);
 
-// Whole problem (single component or composition) over n rows.
-int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out,
-                 float *scratch, int precision, int rows_per_block, hipStream_t s);
+// Whole problem (single component or composition) over n rows; scratch holds
+// scratch_floats floats.
+int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out, float *scratch,
+                 size_t scratch_floats, int precision, int rows_per_block, hipStream_t s);
 
 // FP64 evaluation: the generic kernel up to its 1024 columns, else one block
 // per row (eval_rows_f64).
@@ -38,13 +41,13 @@ int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double
 
 int default_rows_per_block(int n, int dim, int precision = SPEO_PREC_FP32);
 
-// k_eval_wide: the 16-bit evaluation of one component wider than 128 columns
-// with k_eval<64, precision>'s bits (partial sums into part, finalized by the
-// caller); applies when X, the shift and the 16-bit operand rows allow
-// 16-byte loads.
-bool eval_wide_applies(const CompDev &c, const float *X, int ld, int dim, int precision);
-int eval_wide(const CompDev &c, const float *X, int ld, int n, int dim, float *part, int precision,
-              hipStream_t s);
+// k_eval_wide: the evaluation of components wider than 128 columns with
+// k_eval<64, precision>'s bits: component k's partial sums into part + k
+// nchunks 2 n, finalized by the caller; applies when X and its stride allow
+// 16-byte loads and, in FP32, when the rows fill the chip.
+bool eval_wide_applies(const CompDev &c, const float *X, int ld, int n, int dim, int precision);
+int eval_wide(const CompDev *c, int ncomp, const float *X, int ld, int n, int dim, float *part,
+              int precision, hipStream_t s);
 
 // Problems with objectives outside the fused FP32 epilogues (ProblemHost::
 // generic): the FP64 generic kernel, FP32 and/or FP64 outputs; rows (device,

@@ -108,6 +108,9 @@ struct CompDev {
     const float *B32s;
     const uint16_t *M16s[3];    // [128][kp32]: 16-bit parts of M (FP16 scaled by 2^14)
     int kp32;                   // round_up(dim, 32)
+    // M in the wide kernels' fragment order (wide_core.h) for the view's
+    // precision: FP32, or the 16-bit parts one after another; null: not kept.
+    const void *wide;
     HeavyCol heavy;             // heavy.j < 0: none
 };
 

@@ -101,17 +101,22 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
     }
 }
 
-__global__ void k_eval_finalize(const float *part, int nchunks, int n, int dim, int objective,
+// The chunks' sums of component blockIdx.y (in chunk order) and its value.
+struct FinalizeObjectives {
+    int obj[kMaxComp];
+};
+__global__ void k_eval_finalize(const float *part, int nchunks, int n, int dim, FinalizeObjectives objectives,
                                 float lambda, float bias, int raw, float *f_out) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
+    const int row = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
     if (row >= n) return;
+    part += (size_t)k * nchunks * 2 * n;
     float a = 0.f, b = 0.f;
     for (int c = 0; c < nchunks; ++c) {
         a += part[((size_t)c * 2 + 0) * n + row];
         b += part[((size_t)c * 2 + 1) * n + row];
     }
-    const float g = finish_objective_ext(objective, a, b, dim);
-    f_out[row] = raw ? g : fmaf(lambda, g, bias);
+    const float g = finish_objective_ext(objectives.obj[k], a, b, dim);
+    f_out[(size_t)k * n + row] = raw ? g : fmaf(lambda, g, bias);
 }
 
 // Composition (cf_cal, CEC2014.cc:1481-1519) in FP32: one wave per row.
@@ -279,7 +284,7 @@ __global__ __launch_bounds__(256) void k_comp_combine_rows(const CompParams *com
 
 // ------------------------------------------------------------------ launch
 
-// k_eval_wide for the 16-bit evaluations that k_eval<64> would run.
+// k_eval_wide for the wide evaluations that k_eval<64> would run.
 static std::atomic<int> g_wide_eval{1};
 static std::atomic<long long> g_wide_launches{0};
 
@@ -310,6 +315,12 @@ static int launch_rt(const EvalLaunch &p, int precision, int n, int nchunks, hip
     }
 }
 
+static bool use_wide(const CompDev &comp, const float *X, int ld, int n, int dim, int precision,
+                     int rows_per_block) {
+    return rows_per_block == 64 && g_wide_eval.load(std::memory_order_relaxed) &&
+           eval_wide_applies(comp, X, ld, n, dim, precision);
+}
+
 int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, float *f_out,
                    float *part, float lambda, float bias, int raw, int precision,
                    int rows_per_block, hipStream_t s) {
@@ -319,10 +330,9 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
     const int small = (dim <= kSmallD && comp.B32s != nullptr) ? 1 : 0;
     EvalLaunch p{comp, X, ld, n, dim, f_out, part, nchunks, lambda, bias, raw, small};
     int rc;
-    if (!small && rows_per_block == 64 && g_wide_eval.load(std::memory_order_relaxed) &&
-        eval_wide_applies(comp, X, ld, dim, precision)) {
+    if (use_wide(comp, X, ld, n, dim, precision, rows_per_block)) {
         // the same bits as k_eval<64, precision>, on wider tiles
-        rc = eval_wide(comp, X, ld, n, dim, part, precision, s);
+        rc = eval_wide(&comp, 1, X, ld, n, dim, part, precision, s);
         g_wide_launches.fetch_add(1, std::memory_order_relaxed);
     } else switch (rows_per_block) {
     case 16: rc = launch_rt<16>(p, precision, n, nchunks, s); break;
@@ -331,8 +341,21 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
     default: return set_error(SPEO_ERR_ARG, "rows_per_block must be 16, 32 or 64");
     }
     if (rc != SPEO_OK || nchunks == 1) return rc;
-    hipLaunchKernelGGL(k_eval_finalize, dim3((n + 255) / 256), dim3(256), 0, s, part, nchunks, n,
-                       dim, comp.objective, lambda, bias, raw, f_out);
+    hipLaunchKernelGGL(k_eval_finalize, dim3((n + 255) / 256), dim3(256), 0, s, part, nchunks, n, dim,
+                       FinalizeObjectives{{comp.objective}}, lambda, bias, raw, f_out);
+    return check_launch("k_eval_finalize");
+}
+
+// All components of a wide composition in one launch (no drain and refill of
+// the chip between them), their chunk sums finalized in another.
+static int eval_components_wide(const CompDev *comp, int ncomp, const float *X, int ld, int n, int dim,
+                                float *gbuf, float *part, int precision, hipStream_t s) {
+    SPEO_TRY(eval_wide(comp, ncomp, X, ld, n, dim, part, precision, s));
+    g_wide_launches.fetch_add(ncomp, std::memory_order_relaxed);
+    FinalizeObjectives o{};
+    for (int c = 0; c < ncomp; ++c) o.obj[c] = comp[c].objective;
+    hipLaunchKernelGGL(k_eval_finalize, dim3((n + 255) / 256, ncomp), dim3(256), 0, s, part,
+                       (dim + kNC - 1) / kNC, n, dim, o, 1.f, 0.f, 1, gbuf);
     return check_launch("k_eval_finalize");
 }
 
@@ -359,8 +382,14 @@ size_t eval_scratch_floats(int ncomp, int dim, int n) {
     return part + comp;
 }
 
-int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out,
-                 float *scratch, int precision, int rows_per_block, hipStream_t s) {
+size_t eval_scratch_batched(int ncomp, int dim, int n) {
+    const int nchunks = (dim + kNC - 1) / kNC;
+    if (ncomp == 1 || nchunks == 1) return eval_scratch_floats(ncomp, dim, n);
+    return (size_t)ncomp * n * (2 * nchunks + 1);
+}
+
+int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out, float *scratch,
+                 size_t scratch_floats, int precision, int rows_per_block, hipStream_t s) {
     if (n <= 0) return SPEO_OK;
     if (P.generic) return eval_problem_generic(P, X, ld, n, f_out, nullptr, nullptr, 0, s);
     const int nchunks = (P.dim + kNC - 1) / kNC;
@@ -374,8 +403,19 @@ int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_o
         return eval_component(P.view(0, prec_of(0)), X, ld, n, P.dim, f_out, part,
                               (float)c.lambda, (float)c.bias, 0, prec_of(0), rows_per_block, s);
     }
-    for (int c = 0; c < P.ncomp; ++c)
-        SPEO_TRY(eval_component(P.view(c, prec_of(c)), X, ld, n, P.dim, gbuf + (size_t)c * n, part,
+    CompDev view[kMaxComp];
+    bool batched = nchunks > 1 && scratch_floats >= eval_scratch_batched(P.ncomp, P.dim, n);
+    for (int c = 0; c < P.ncomp; ++c) {
+        view[c] = P.view(c, prec_of(c));
+        batched = batched && prec_of(c) == prec_of(0) &&
+                  use_wide(view[c], X, ld, n, P.dim, prec_of(c), rows_per_block);
+    }
+    if (batched) {
+        gbuf = scratch + (size_t)P.ncomp * nchunks * 2 * n;
+        SPEO_TRY(eval_components_wide(view, P.ncomp, X, ld, n, P.dim, gbuf, scratch, prec_of(0), s));
+    }
+    for (int c = 0; c < P.ncomp && !batched; ++c)
+        SPEO_TRY(eval_component(view[c], X, ld, n, P.dim, gbuf + (size_t)c * n, part,
                                 1.f, 0.f, 1, prec_of(c), rows_per_block, s));
     bool rows = (P.dim & 3) == 0 && P.dim <= 1024 && (ld & 3) == 0 &&
                 (reinterpret_cast<uintptr_t>(X) & 15) == 0 && n >= 4096;

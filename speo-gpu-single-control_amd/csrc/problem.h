@@ -38,6 +38,8 @@ struct CompHost {
     float *B32s = nullptr;                                   // 128 x 128, fragment order
     uint16_t *Mbfs[3] = {nullptr, nullptr, nullptr};         // [128][round_up(dim,32)]
     uint16_t *Mhs[3] = {nullptr, nullptr, nullptr};
+    float *wide32 = nullptr;    // M in the wide kernels' fragment order (wide_core.h): FP32,
+    uint16_t *wide_bf = nullptr, *wide_h = nullptr;  // the three BF16 and the three FP16 parts
     float *colw = nullptr;      // [dim] bent cigar / discus weights (elliptic: ProblemHost::colw)
     bool unrotated = false;     // M = I: evaluated in FP32 whatever the requested precision,
                                 // where the identity GEMM is exact

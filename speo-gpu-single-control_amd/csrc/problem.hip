@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "cec_generic.h"
+#include "wide_core.h"
 #include "eval.h"
 
 namespace speo {
@@ -93,6 +94,7 @@ CompDev ProblemHost::view(int c, int precision) const {
     d.B32s = h.B32s;
     for (int p = 0; p < 3; ++p) d.M16s[p] = half ? h.Mhs[p] : h.Mbfs[p];
     d.kp32 = round_up(dim, 32);
+    d.wide = precision == SPEO_PREC_FP32 ? (const void *)h.wide32 : half ? (const void *)h.wide_h : (const void *)h.wide_bf;
     d.heavy.j = heavy_column(h.objective, dim, &d.heavy.w);
     d.heavy.m64 = d.heavy.j >= 0 ? h.M64 + (size_t)d.heavy.j * dim : nullptr;
     d.heavy.o64 = h.shift64;
@@ -123,6 +125,9 @@ static void free_problem(ProblemHost &P) {
             (void)hipFree(h.Mbfs[p]);
             (void)hipFree(h.Mhs[p]);
         }
+        (void)hipFree(h.wide32);
+        (void)hipFree(h.wide_bf);
+        (void)hipFree(h.wide_h);
         (void)hipFree(h.colw);
         h = CompHost{};
     }
@@ -236,6 +241,17 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
             SPEO_TRY(upload(&h.Mbf[p], pb[p]));
             SPEO_TRY(upload(&h.Mh[p], ph[p]));
         }
+        // (the kernels move through the three parts by 32-bit byte offsets)
+        const size_t fe = wide_frag_elems(dim);
+        if (3 * 2 * fe < 0x7fffffffull) {
+            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide32), sizeof(float) * fe));
+            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide_bf), sizeof(uint16_t) * 3 * fe));
+            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide_h), sizeof(uint16_t) * 3 * fe));
+            const uint16_t *src[6] = {h.Mbf[0], h.Mbf[1], h.Mbf[2], h.Mh[0], h.Mh[1], h.Mh[2]};
+            uint16_t *dst[6] = {h.wide_bf, h.wide_bf + fe, h.wide_bf + 2 * fe,
+                                h.wide_h, h.wide_h + fe, h.wide_h + 2 * fe};
+            SPEO_TRY(wide_fragments(h.B32, P.ldb32, src, P.ldm16, dim, h.wide32, dst, nullptr));
+        }
         if (dim <= kSmallD) {
             const size_t kp32 = (size_t)round_up(dim, 32);
             // B = M^T zero padded to 128 x 128, in MFMA fragment order (CompDev::B32s)
@@ -295,8 +311,8 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
         }
         SPEO_TRY(check_gen_problem(gen[0], false));
         SPEO_TRY(upload(&P.gen, gen));
-        SPEO_TRY_HIP(hipStreamSynchronize(nullptr));  // the fragments, for callers on other streams
     }
+    SPEO_TRY_HIP(hipStreamSynchronize(nullptr));  // the fragments, for callers on other streams
     return SPEO_OK;
 }
 
@@ -527,7 +543,7 @@ int speo_evaluate(speo_problem p, const float *X, int ld, int n, float *f_out, i
         return set_error(SPEO_ERR_ARG, "speo_evaluate: bad arguments");
     if (precision < SPEO_PREC_FP32 || precision > SPEO_PREC_BF16X6)
         return set_error(SPEO_ERR_ARG, "speo_evaluate: unknown precision");
-    const size_t need = eval_scratch_floats(p->h.ncomp, p->h.dim, n);
+    const size_t need = eval_scratch_batched(p->h.ncomp, p->h.dim, n);
     if (need > p->scratch_cap) {
         SPEO_TRY_HIP(hipStreamSynchronize(as_stream(stream)));
         (void)hipFree(p->scratch);
@@ -536,7 +552,7 @@ int speo_evaluate(speo_problem p, const float *X, int ld, int n, float *f_out, i
         SPEO_TRY_HIP(hipMalloc(&p->scratch, sizeof(float) * need));
         p->scratch_cap = need;
     }
-    return eval_problem(p->h, X, ld, n, f_out, p->scratch, precision,
+    return eval_problem(p->h, X, ld, n, f_out, p->scratch, p->scratch_cap, precision,
                         default_rows_per_block(n, p->h.dim, precision), as_stream(stream));
 }
 

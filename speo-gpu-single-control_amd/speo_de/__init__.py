@@ -198,8 +198,8 @@ def evaluate(problem: Problem, X, f_out, precision=PREC_FP32, ld=None, n=None, s
 
 
 def wide_eval(enable=-1):
-    """Selects the kernel of the 16-bit evaluations wider than 128 columns on
-    at least 1024 rows (1: 256-column tiles, 0: 64-row tiles, -1: unchanged;
+    """Selects the kernel of the evaluations wider than 128 columns with the
+    arithmetic of 64-row tiles (1: 256-column tiles, 0: 64-row tiles, -1: unchanged;
     the same bits either way).  Returns (previous setting, launches of the
     256-column kernel so far)."""
     n = ctypes.c_longlong(0)

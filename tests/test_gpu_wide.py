@@ -1,0 +1,65 @@
+"""The tile kernel of wide problems (more than 128 columns): its values equal the
+64-row kernel's bit for bit (same MFMA chains, same sums) at the edges of its
+row blocks, K stages and column chunks, with rows padded by NaN, and the
+components of a composition in one launch equal one launch each."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(speo, objs, D, seed, rate=None):
+    rng = np.random.default_rng(seed)
+    o = np.float32(rng.uniform(-80, 80, (len(objs), D))).astype(np.float64)
+    M = np.stack([np.linalg.qr(rng.standard_normal((D, D)))[0] for _ in objs])
+    sigma = [10.0 * (c + 1) for c in range(len(objs))]
+    return speo.Problem(objs, o, M, sigma=sigma, bias=[100.0 * c for c in range(len(objs))], rate=rate)
+
+
+def _rows(n, D, ld, cuda):
+    import torch
+    X = torch.full((n, ld), float("nan"), device=cuda)
+    X[:, :D] = torch.rand((n, D), device=cuda, generator=torch.Generator(cuda).manual_seed(n)) * 200 - 100
+    return X
+
+
+# FP32 takes the tile kernel from 160 blocks of 128 rows x 256 columns on
+@pytest.mark.parametrize("D,ld,n,prec", [(129, 132, 20481, 0), (160, 160, 21000, 0), (257, 260, 11009, 0),
+                                         (1000, 1000, 5249, 0), (1023, 1024, 5120, 0), (129, 132, 1025, 1),
+                                         (255, 256, 1151, 3), (257, 300, 1153, 2), (1001, 1004, 1024, 5),
+                                         (513, 516, 1279, 4)])
+@pytest.mark.parametrize("obj,rate", [(2, 1.0), (6, 0.05)])
+def test_tile_kernel_equals_64_row_kernel(cuda, speo, D, ld, n, prec, obj, rate):
+    import torch
+    prob = _problem(speo, [obj], D, D, rate=[rate])
+    X = _rows(n, D, ld, cuda)
+    got = {}
+    for on in (1, 0):
+        prev, before = speo.wide_eval(on)
+        f = torch.zeros(n, device=cuda)
+        print(f"D={D} n={n} prec={prec} obj={obj} tile kernel {on}", flush=True)
+        speo.evaluate(prob, X, f, precision=prec, ld=ld)
+        torch.cuda.synchronize()
+        assert speo.wide_eval(prev)[1] - before == on
+        got[on] = f.cpu().numpy()
+    assert np.isfinite(got[1]).all()
+    np.testing.assert_array_equal(got[1], got[0])
+    prob.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1, 3])
+def test_batched_components_equal_one_launch_each(cuda, speo, prec):
+    """speo_evaluate runs a composition's components in one launch;
+    speo_evaluate_noalloc's fixed workspace (2^20 floats) is too small for
+    that here and takes them one by one."""
+    import torch
+    D, n = 260, 22016
+    prob = _problem(speo, [1, 2, 3, 3, 2, 1, 7], D, 11)
+    X = _rows(n, D, D, cuda)
+    a, b = torch.zeros(n, device=cuda), torch.zeros(n, device=cuda)
+    chunks = -(-D // 128)
+    assert n * (2 * chunks + 7) <= 2 ** 20 < 7 * n * (2 * chunks + 1)
+    speo.evaluate(prob, X, a, precision=prec)
+    speo.evaluate_noalloc(prob, X, b, precision=prec)
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+    prob.close()
