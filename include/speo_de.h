@@ -285,7 +285,8 @@ SPEO_EXPORT int speo_evaluate(speo_problem p, const float *X, int ld, int n, flo
  * where the arithmetic is that of 64-row tiles (the 16-bit precisions and
  * their splits on at least 1024 rows, FP32 when the rows fill the chip):
  * enable 1 (default) a kernel with 256-column tiles, 0 the 64-row-tile kernel,
- * -1 leaves the setting.  Both
+ * -1 leaves the setting.  Engines with islands wider than 128 columns take the
+ * setting at their creation.  Both
  * give the same bits; the switch is for tests and measurements.  Process-wide;
  * returns the previous setting, and *launches (optional) the number of
  * launches of the 256-column kernel so far. */

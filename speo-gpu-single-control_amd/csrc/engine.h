@@ -14,6 +14,37 @@ struct FusedProblem {
     CompDev comp[kMaxComp];
 };
 
+// --------------------------------------------- evaluation of wide islands
+//
+// The rows of islands wider than 128 columns are evaluated by launches of
+// their own over (64-row tile, component) items, then combined where a problem
+// is a composition.  nsplit: the column classes of the rows-per-block arithmetic
+// (64 rows: 1, 32: 2, 16: 4; gemm_chunk's NSPLIT).
+
+// Rows [row0, row0 + nrows) of an island, and one component of its problem.
+struct WideItem {
+    int64_t elem;  // first element of row 0 of the item
+    int row;       // its index in the fitness arrays
+    int nrows, ld, dim, problem, comp;
+};
+struct WideRowsArgs {
+    const WideItem *items;
+    const FusedProblem *probs;
+    const float *src;  // rows (the population's layout)
+    float *f;          // [rows] values of single-component problems
+    float *gval;       // [component][rows] of compositions
+    int rows;
+};
+constexpr int kWideRows = 64;
+// Whether the tile kernel takes a component (its M in fragment order, LDS for
+// the shift); else rows_chunk does.
+bool rows_wide_applies(const CompDev &c, int dim, int precision);
+int rows_wide(const WideRowsArgs &a, int nitems, int max_dim, int precision, int nsplit, hipStream_t s);
+int rows_chunk(const WideRowsArgs &a, int nitems, int precision, int nsplit, hipStream_t s);
+// The compositions among the items (component 0's): cf_cal weights and the sum;
+// ncomp: the most components of any.
+int rows_combine(const WideRowsArgs &a, int nitems, int ncomp, hipStream_t s);
+
 // One island's answer of Engine::best, written by the kernels into pinned host
 // memory (no copies back; the caller synchronises the stream).
 struct BestOut {

@@ -12,6 +12,9 @@
 //   kModeEval    f(U) through the MFMA evaluation    (plain engine, launch 2)
 //   kModeSelect  X, fX <- U, fU where fU < fX        (plain engine, launch 3)
 //   kModeFused   select(g-1) + generate(g) + evaluate(g) in one launch.
+// Evaluation inside this kernel is for rows of at most 128 columns; when an
+// island is wider, kModeFusedGen makes the generation's trials and the launches
+// of engine_wide.hip evaluate them.
 // The fused mode needs no grid-wide barrier: the selection of generation g-1
 // is not applied before the donors are read; instead a donor row r is read as
 // U_prev[r] when fU_prev[r] < fX_prev[r] and as X[r] otherwise, and X[r] is
@@ -38,7 +41,7 @@
 
 namespace speo {
 
-enum GenMode { kModeGen = 0, kModeEval = 1, kModeSelect = 2, kModeFused = 3 };
+enum GenMode { kModeGen = 0, kModeEval = 1, kModeSelect = 2, kModeFused = 3, kModeFusedGen = 4 };
 
 // A block's work item: rows [row0, row0 + nrows) of an island, with a copy of
 // the island's descriptor (immutable after set-up), so a block reads its work
@@ -65,20 +68,16 @@ struct GenerationArgs {
     uint64_t seed;
     const uint32_t *gen_base;
     uint32_t gen_offset;
-    int trial_in_lds;
     int clear_trials;
 };
 
-constexpr int kTLD = kSmallD;  // widest dimension whose rows stay in LDS
+constexpr int kTLD = kSmallD;  // widest dimension this kernel evaluates
 
-// LDS of one block: [trial rows RT x kTS] [gval kMaxComp x RT] [GEMM region];
-// with rows in LDS the GEMM region is the small-D path's (scratch + row
-// reduction), otherwise the K-chunked path's.
+// LDS of one block: [trial rows RT x kTS] [gval kMaxComp x RT] [scratch of the
+// GEMM and the row reduction].
 template <int RT, int PREC>
-constexpr int generation_lds_bytes(bool trial_in_lds) {
-    return trial_in_lds ? RT * kTS * 4 + kMaxComp * RT * 4 +
-                              small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4
-                        : kMaxComp * RT * 4 + gemm_lds_bytes<RT, PREC>();
+constexpr int generation_lds_bytes() {
+    return RT * kTS * 4 + kMaxComp * RT * 4 + small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4;
 }
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -121,12 +120,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
         return;
     }
 
-    const bool lds_trial = (MODE == kModeFused || MODE == kModeEval) && a.trial_in_lds;
+    constexpr bool FUSED = MODE == kModeFused || MODE == kModeFusedGen;
+    constexpr bool lds_trial = MODE == kModeFused || MODE == kModeEval;
     float *trial = reinterpret_cast<float *>(lds);
-    float *gval = trial + (lds_trial ? RT * kTS : 0);
+    float *gval = trial + RT * kTS;
     char *gemm_lds = reinterpret_cast<char *>(gval + kMaxComp * RT);
 
-    if constexpr (MODE == kModeGen || MODE == kModeFused) {
+    if constexpr (MODE == kModeGen || FUSED) {
         const uint32_t gen = (a.gen_base ? *a.gen_base : 0u) + a.gen_offset;
         const int ngroups = (I.dim + 3) >> 2;
         const uint32_t crt = cr_threshold(I.CR);
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             // Row `k` of the island as the parent population of this generation.
             auto parent = [&](int k) -> const float * {
                 const int g = I.row_off + k;
-                if (MODE == kModeFused && a.fU_prev[g] < a.fX_prev[g])
+                if (FUSED && a.fU_prev[g] < a.fX_prev[g])
                     return a.U_prev + I.elem_off + (size_t)k * I.ld;
                 return a.X + I.elem_off + (size_t)k * I.ld;
             };
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             c.p2 = parent(r[2]);
             c.own_acc = false;
             c.fx_own = c.fu_own = 0.f;
-            if (MODE == kModeFused) {
+            if (FUSED) {
                 c.fx_own = a.fX_prev[c.gr];
                 c.fu_own = a.fU_prev[c.gr];
                 c.own_acc = c.fu_own < c.fx_own;
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             const float4 out{v[0], v[1], v[2], v[3]};
             st4(a.U_new + I.elem_off + (size_t)c.li * I.ld + 4 * g, out);
             if (lds_trial) st4(trial + c.lr * kTS + 4 * g, out);
-            if (MODE == kModeFused && c.own_acc) st4(a.X + I.elem_off + (size_t)c.li * I.ld + 4 * g, xo);
+            if (FUSED && c.own_acc) st4(a.X + I.elem_off + (size_t)c.li * I.ld + 4 * g, xo);
         };
         for (int pass = 0; pass < RT / 16; pass += 2) {
             const int lrA = pass * 16 + (tid >> 4), lrB = lrA + 16;
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
                 if (B.valid) make(B, g, b0, b1, b2, bo);
                 else if (hasB && lds_trial) st4(trial + lrB * kTS + 4 * g, float4{0.f, 0.f, 0.f, 0.f});
             }
-            if (MODE == kModeFused && l == 0) {
+            if (FUSED && l == 0) {
                 if (A.valid) a.fX_new[A.gr] = A.own_acc ? A.fu_own : A.fx_own;
                 if (B.valid) a.fX_new[B.gr] = B.own_acc ? B.fu_own : B.fx_own;
             }
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
         const FusedProblem *P = a.probs + I.problem;
         if (MODE == kModeEval && P->generic) return;  // the generic kernel evaluates this island
         const int ncomp = P->ncomp, dim = I.dim;
-        if (MODE == kModeEval && lds_trial) {
+        if (MODE == kModeEval) {
             // stage the rows to evaluate into the LDS tile (zero rows past nrows)
             const float *srcp = a.eval_src + I.elem_off + (size_t)t.row0 * I.ld;
             const int ngroups = (dim + 3) >> 2;
@@ -240,37 +240,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             }
         }
         __syncthreads();
-        RowSource src;
-        if (lds_trial)
-            src = RowSource{trial, kTS, t.nrows};
-        else if (MODE == kModeEval)
-            src = RowSource{a.eval_src + I.elem_off + (size_t)t.row0 * I.ld, I.ld, t.nrows};
-        else
-            src = RowSource{a.U_new + I.elem_off + (size_t)t.row0 * I.ld, I.ld, t.nrows};
         for (int c = 0; c < ncomp; ++c) {
             const CompDev comp = P->comp[c];
-            if (lds_trial) {
-                float *red = reinterpret_cast<float *>(gemm_lds + small_scratch_bytes<RT>(Prec<PREC>::parts));
-                float *o1 = red + 8 * RT, *o2 = o1 + RT;
-                float s1[RT / 16][4], s2[RT / 16][4];
-                gemm_small<RT, PREC>(comp, trial, dim, gemm_lds, s1, s2);
-                reduce_rows_small<RT>(s1, s2, red, o1, o2);
-                if (tid < t.nrows) gval[c * RT + tid] = finish_objective_ext(comp.objective, o1[tid], o2[tid], dim);
-            } else {
-                float *red = reinterpret_cast<float *>(gemm_lds);
-                float *o1 = red + 8 * RT, *o2 = o1 + RT;
-                float s1[4] = {0.f, 0.f, 0.f, 0.f}, s2[4] = {0.f, 0.f, 0.f, 0.f};
-                for (int n0 = 0; n0 < dim; n0 += kNC)
-                    gemm_chunk<RT, PREC, false>(comp, src, dim, n0, gemm_lds, s1, s2);
-                reduce_rows<RT>(s1, s2, red, o1, o2);
-                if (tid < t.nrows) gval[c * RT + tid] = finish_objective_ext(comp.objective, o1[tid], o2[tid], dim);
-            }
+            float *red = reinterpret_cast<float *>(gemm_lds + small_scratch_bytes<RT>(Prec<PREC>::parts));
+            float *o1 = red + 8 * RT, *o2 = o1 + RT;
+            float s1[RT / 16][4], s2[RT / 16][4];
+            gemm_small<RT, PREC>(comp, trial, dim, gemm_lds, s1, s2);
+            reduce_rows_small<RT>(s1, s2, red, o1, o2);
+            if (tid < t.nrows) gval[c * RT + tid] = finish_objective_ext(comp.objective, o1[tid], o2[tid], dim);
             if (comp.heavy.j >= 0) {
                 // the heavy column's FP64 term, one wave per row
                 __syncthreads();
                 const int wave = tid >> 6, lane = tid & 63;
                 for (int r = wave; r < t.nrows; r += 4) {
-                    const double h = heavy_term(comp.heavy, src.rows + (size_t)r * src.ld, dim, lane);
+                    const double h = heavy_term(comp.heavy, trial + r * kTS, dim, lane);
                     if (lane == 0) gval[c * RT + r] = with_heavy(gval[c * RT + r], (float)h);
                 }
                 __syncthreads();
@@ -282,7 +265,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
                 f = fmaf(P->lambda[0], gval[tid], P->bias[0]);
             } else {
                 // cf_cal weights (CEC2014.cc:1481-1519) in the log domain.
-                const float *x = src.rows + (size_t)tid * src.ld;
+                const float *x = trial + tid * kTS;
                 // (components at distance 0 share the weight equally, as
                 // cf_cal's w = 1e99 each)
                 float lw[kMaxComp], lwmax = -INFINITY;
@@ -325,15 +308,12 @@ __global__ void k_add_u32(uint32_t *p, uint32_t v) {
 
 template <int RT, int PREC, int MODE>
 static int launch_generation(const GenerationArgs &a, int ntiles, hipStream_t s) {
-    const int lds = (MODE == kModeSelect || MODE == kModeGen)
-                        ? 0
-                        : generation_lds_bytes<RT, PREC>(a.trial_in_lds != 0);
+    const int lds = MODE == kModeEval || MODE == kModeFused ? generation_lds_bytes<RT, PREC>() : 0;
     static std::once_flag once;
     std::call_once(once, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_generation<RT, PREC, MODE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  std::max(generation_lds_bytes<RT, PREC>(true),
-                                           generation_lds_bytes<RT, PREC>(false)));
+                                  generation_lds_bytes<RT, PREC>());
     });
     hipLaunchKernelGGL((k_generation<RT, PREC, MODE>), dim3(ntiles), dim3(256), lds, s, a);
     return check_launch("k_generation");
@@ -345,13 +325,15 @@ static int launch_mode(int mode, const GenerationArgs &a, int ntiles, hipStream_
     case kModeGen: return launch_generation<RT, PREC, kModeGen>(a, ntiles, s);
     case kModeEval: return launch_generation<RT, PREC, kModeEval>(a, ntiles, s);
     case kModeSelect: return launch_generation<RT, SPEO_PREC_FP32, kModeSelect>(a, ntiles, s);
+    case kModeFusedGen: return launch_generation<RT, SPEO_PREC_FP32, kModeFusedGen>(a, ntiles, s);
     default: return launch_generation<RT, PREC, kModeFused>(a, ntiles, s);
     }
 }
 
 template <int RT>
 static int launch_prec(int prec, int mode, const GenerationArgs &a, int ntiles, hipStream_t s) {
-    if (mode == kModeGen || mode == kModeSelect) return launch_mode<RT, SPEO_PREC_FP32>(mode, a, ntiles, s);
+    if (mode == kModeGen || mode == kModeSelect || mode == kModeFusedGen)
+        return launch_mode<RT, SPEO_PREC_FP32>(mode, a, ntiles, s);
     switch (prec) {
     case SPEO_PREC_FP32: return launch_mode<RT, SPEO_PREC_FP32>(mode, a, ntiles, s);
     case SPEO_PREC_BF16: return launch_mode<RT, SPEO_PREC_BF16>(mode, a, ntiles, s);
@@ -462,6 +444,13 @@ struct Engine {
     const CompParams **params_tab_dev = nullptr;
     std::map<int, TileDesc *> tiles_dev;  // per rows-per-block
     std::map<int, int> ntiles;
+    // islands wider than kTLD (any of them): the evaluation's items, those the
+    // tile kernel takes first, then those of rows_chunk; component values
+    WideItem *wide_items = nullptr;
+    int wide_tile = 0, wide_chunk = 0, wide_ncomp = 1;
+    float *gval = nullptr;
+    int build_wide_items();
+    int eval_wide_rows(const float *src, float *out, int rt_, hipStream_t s);
     uint32_t *gen_base = nullptr;
 
     float *X = nullptr, *fX[2] = {nullptr, nullptr}, *U[2] = {nullptr, nullptr};
@@ -558,7 +547,7 @@ Engine::~Engine() {
     for (auto &kv : tiles_dev) (void)hipFree(kv.second);
     void *bufs[] = {isl_dev, row_off_dev, dst_dev, best_buf, worst_buf, best_row_dev,
                     best_part, probs_dev, params_tab_dev, gen_base,
-                    blocks_dev, Xnext, donor_buf, row_island_dev,
+                    blocks_dev, Xnext, donor_buf, row_island_dev, wide_items, gval,
                     X, fX[0], fX[1], U[0], U[1], fU[0], fU[1], srows_dev, cand, pred, rho_dev, scored_dev,
                     AX, Ay, Xb, tb, Xh, yh, predh, ranks_ws, heads_dev, round_dev, perm_dev,
                     best_sub_dev, info_dev};
@@ -591,6 +580,50 @@ int Engine::build_tiles(int rt_) {
     SPEO_TRY(upload_vec(&d, tiles));
     tiles_dev[rt_] = d;
     ntiles[rt_] = (int)tiles.size();
+    return SPEO_OK;
+}
+
+// Items of the wide evaluation: 64-row tiles of every island the fused
+// kernels' arithmetic evaluates, each component an item.  Groups of eight tiles
+// are listed component by component: workgroup b runs on XCD b mod 8, so a
+// tile's components run on one XCD, close in time, and share its rows in that
+// L2.  Wider islands first.
+int Engine::build_wide_items() {
+    std::vector<WideItem> tile, chunk;
+    std::vector<int> order((size_t)I);
+    for (int i = 0; i < I; ++i) order[(size_t)i] = i;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return isl[(size_t)x].dim > isl[(size_t)y].dim; });
+    for (int i : order) {
+        const IslandDesc &d = isl[(size_t)i];
+        const ProblemHost &P = problems[(size_t)d.problem]->h;
+        if (P.generic) continue;
+        wide_ncomp = std::max(wide_ncomp, P.ncomp);
+        for (int g0 = 0; g0 < d.np; g0 += 8 * kWideRows)
+            for (int c = 0; c < P.ncomp; ++c) {
+                auto &list = rows_wide_applies(P.view(c, cfg.precision), d.dim, cfg.precision) ? tile : chunk;
+                for (int r0 = g0; r0 < std::min(d.np, g0 + 8 * kWideRows); r0 += kWideRows)
+                    list.push_back(WideItem{d.elem_off + (int64_t)r0 * d.ld, d.row_off + r0,
+                                            std::min(kWideRows, d.np - r0), d.ld, d.dim, d.problem, c});
+            }
+    }
+    wide_tile = (int)tile.size();
+    wide_chunk = (int)chunk.size();
+    tile.insert(tile.end(), chunk.begin(), chunk.end());
+    SPEO_TRY(upload_vec(&wide_items, tile));
+    if (wide_ncomp > 1)
+        SPEO_TRY_HIP(hipMalloc(&gval, sizeof(float) * (size_t)wide_ncomp * (size_t)total_rows));
+    return SPEO_OK;
+}
+
+int Engine::eval_wide_rows(const float *src, float *out, int rt_, hipStream_t s) {
+    const WideRowsArgs a{wide_items, probs_dev, src, out, gval, total_rows};
+    WideRowsArgs rest = a;
+    rest.items = wide_items + wide_tile;
+    const int nsplit = 64 / rt_;
+    SPEO_TRY(rows_wide(a, wide_tile, max_dim, cfg.precision, nsplit, s));
+    SPEO_TRY(rows_chunk(rest, wide_chunk, cfg.precision, nsplit, s));
+    if (wide_ncomp > 1) SPEO_TRY(rows_combine(a, wide_tile + wide_chunk, wide_ncomp, s));
     return SPEO_OK;
 }
 
@@ -708,6 +741,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
         own_stream = true;
     }
     SPEO_TRY(upload_tables());
+    if (!all_small) SPEO_TRY(build_wide_items());
     if (any_generic && (c.mode != SPEO_MODE_PLAIN || c.surrogate_candidates > 0))
         return set_error(SPEO_ERR_UNSUPPORTED,
                          "speo_engine_create: objectives 9-22 run in SPEO_MODE_PLAIN without the surrogate");
@@ -763,14 +797,17 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
     if (configured) SPEO_TRY(configure_setup());
     SPEO_TRY(build_tiles(rt));
     // Initial evaluation (island_EA.cc:81 counts it as island_size FEs).
-    GenerationArgs a{};
-    a.isl = isl_dev;
-    a.tiles = tiles_dev[rt];
-    a.probs = probs_dev;
-    a.eval_src = X;
-    a.eval_out = fX[0];
-    a.trial_in_lds = all_small ? 1 : 0;
-    SPEO_TRY(launch_any(rt, cfg.precision, kModeEval, a, ntiles[rt], stream));
+    if (all_small) {
+        GenerationArgs a{};
+        a.isl = isl_dev;
+        a.tiles = tiles_dev[rt];
+        a.probs = probs_dev;
+        a.eval_src = X;
+        a.eval_out = fX[0];
+        SPEO_TRY(launch_any(rt, cfg.precision, kModeEval, a, ntiles[rt], stream));
+    } else {
+        SPEO_TRY(eval_wide_rows(X, fX[0], rt, stream));
+    }
     SPEO_TRY(eval_generic_islands(X, fX[0], stream));
     hipLaunchKernelGGL(k_fill, dim3(256), dim3(256), 0, stream, fX[1], total_rows, INFINITY);
     SPEO_TRY(check_launch("k_fill"));
@@ -1110,9 +1147,9 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
         a.U_new = U[0];
         break;
     case kModeEval:
+        if (!all_small) return eval_wide_rows(U[0], fU[0], rt_, s);
         a.eval_src = U[0];
         a.eval_out = fU[0];
-        a.trial_in_lds = all_small ? 1 : 0;
         break;
     case kModeSelect:
         if (cfg.mode == SPEO_MODE_FUSED) {  // apply the pending selection
@@ -1132,7 +1169,10 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
         a.fX_new = fX[1 - p];
         a.U_new = U[1 - p];
         a.fU_new = fU[1 - p];
-        a.trial_in_lds = all_small ? 1 : 0;
+        if (!all_small) {
+            SPEO_TRY(launch_any(rt_, cfg.precision, kModeFusedGen, a, ntiles[rt_], s));
+            return eval_wide_rows(U[1 - p], fU[1 - p], rt_, s);
+        }
         break;
     }
     return launch_any(rt_, cfg.precision, mode, a, ntiles[rt_], s);

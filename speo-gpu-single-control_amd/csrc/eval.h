@@ -41,6 +41,9 @@ int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double
 
 int default_rows_per_block(int n, int dim, int precision = SPEO_PREC_FP32);
 
+// The tile kernels of wide problems are switched on (speo_wide_eval).
+bool wide_eval_enabled();
+
 // k_eval_wide: the evaluation of components wider than 128 columns with
 // k_eval<64, precision>'s bits: component k's partial sums into part + k
 // nchunks 2 n, finalized by the caller; applies when X and its stride allow

@@ -287,6 +287,7 @@ __global__ __launch_bounds__(256) void k_comp_combine_rows(const CompParams *com
 // k_eval_wide for the wide evaluations that k_eval<64> would run.
 static std::atomic<int> g_wide_eval{1};
 static std::atomic<long long> g_wide_launches{0};
+bool wide_eval_enabled() { return g_wide_eval.load(std::memory_order_relaxed) != 0; }
 
 template <int RT, int PREC>
 static int launch_rt_prec(const EvalLaunch &p, int n, int nchunks, hipStream_t s) {
@@ -317,7 +318,7 @@ static int launch_rt(const EvalLaunch &p, int precision, int n, int nchunks, hip
 
 static bool use_wide(const CompDev &comp, const float *X, int ld, int n, int dim, int precision,
                      int rows_per_block) {
-    return rows_per_block == 64 && g_wide_eval.load(std::memory_order_relaxed) &&
+    return rows_per_block == 64 && wide_eval_enabled() &&
            eval_wide_applies(comp, X, ld, n, dim, precision);
 }
 

@@ -7,7 +7,7 @@
 // parts formed and multiplied in the same order), per row the terms summed lane
 // by lane over column tiles in order and then across the 16 lanes by sum16, so
 // the sums are gemm_chunk's bit for bit.  What differs is the data path:
-//  * a block of 8 waves owns RG x RTW x 16 rows; a wave owns RTW 16-row tiles x
+//  * a block owns RG x RTW x 16 rows; a wave owns RTW 16-row tiles x
 //    TPW 16-column tiles of accumulators;
 //  * K in stages of 32 over NBUF LDS buffers, requested NBUF - 1 stages ahead
 //    by buffer loads straight into LDS (no registers on the way; the lane's
@@ -28,22 +28,22 @@ namespace speo {
 
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 
-// PREC: SPEO_PREC_*; RG row groups, CG column chunks and NSPLIT column classes
-// (tiles wn, wn + NSPLIT, ... of a chunk) of a block's 8 waves; NBUF stage buffers
-// (0: three where they fit).
+// PREC: SPEO_PREC_*; a block's waves are RG row groups x CG column chunks x
+// NSPLIT column classes (tiles wn, wn + NSPLIT, ... of a chunk); NBUF stage
+// buffers (0: three where they fit).
 template <int PREC, int RG_, int RTW_, int CG_, int NSPLIT_, int NBUF_ = 0> struct WideTile {
     static constexpr int P = Prec<PREC>::parts;
     static constexpr bool H = Prec<PREC>::half, F32 = P == 0;
-    static constexpr int NW = 8, NT = 64 * NW;
+    static constexpr int NW = RG_ * CG_ * NSPLIT_, NT = 64 * NW;
+    static_assert(NW % 2 == 0, "the waves' row pieces alternate their swizzle");
     static constexpr int RG = RG_, RTW = RTW_, CG = CG_, NSPLIT = NSPLIT_, TPW = 8 / NSPLIT;
-    static_assert(RG * CG * NSPLIT == NW, "waves of a block");
     static constexpr int WR = RTW * 16, RB = RG * WR;  // rows per wave, per block
     static constexpr int PIECES = F32 ? 2 : P;         // 1 KB pieces per column tile and stage
     static constexpr int A_BYTES = RB * 128, B_BYTES = 8 * CG * PIECES * 1024, STAGE = A_BYTES + B_BYTES;
     static constexpr int NBUF = NBUF_ ? NBUF_ : 3 * STAGE <= 144 * 1024 ? 3 : 2;
     static constexpr int LDS = NBUF * STAGE;
-    static constexpr int NA = RB / 64, NB = CG * PIECES, NLD = NA + NB;  // loads per wave and stage
-    static_assert(RB % 64 == 0, "row loads tile the waves");
+    static constexpr int NA = RB / 8 / NW, NB = 8 * CG * PIECES / NW, NLD = NA + NB;  // loads per wave and stage
+    static_assert(RB % (8 * NW) == 0 && 8 * CG % NW == 0, "loads tile the waves");
 };
 
 // s_waitcnt vmcnt(N), the other counters left alone (gfx9 encoding: vmcnt
@@ -98,22 +98,22 @@ __device__ __forceinline__ void wide_gemm(const WideOperands &o, int chunk0, int
         const_cast<float *>(o.rows), (short)0, o.nrows * o.ld * 4, kBufferWord3);
     const __amdgpu_buffer_rsrc_t mr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void *>(o.frag), (short)0, (int)0xffffffff, kBufferWord3);
-    // row piece f = wave + 8 j: rows 8 f .. 8 f + 7, lane l row 8 f + l / 8
+    // row piece f = wave + NW j: rows 8 f .. 8 f + 7, lane l row 8 f + l / 8
     // ((8 f + l / 8) / 2 mod 8 = 4 (f mod 2) + l / 16: f mod 2 = wave mod 2)
     const int agrp = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
     const int avoff = ((8 * wave + (lane >> 3)) * o.ld + 4 * agrp) * 4;
-    const int arow8 = 64 * o.ld * 4;  // bytes between the wave's row pieces
+    const int arow8 = 8 * W::NW * o.ld * 4;  // bytes between the wave's row pieces
 
     auto issue = [&](int chunk, int s, int buf) __attribute__((always_inline)) {
         char *st = lds + buf * W::STAGE;
 #pragma unroll
         for (int j = 0; j < W::NA; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(st + (wave + 8 * j) * 1024), 16, avoff,
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(st + (wave + W::NW * j) * 1024), 16, avoff,
                                                      j * arow8 + s * 128, 0, 0);
 #pragma unroll
         for (int j = 0; j < W::NB; ++j) {
-            // piece f = wave + 8 j of [column tile][piece]
-            const int f = wave + 8 * j, ct = f / W::PIECES, pc = f % W::PIECES;
+            // piece f = wave + NW j of [column tile][piece]
+            const int f = wave + W::NW * j, ct = f / W::PIECES, pc = f % W::PIECES;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 mr, (lds_ptr)(st + W::A_BYTES + f * 1024), 16, lane * 16,
                 F32 ? (((chunk * 8 + ct) * nst + s) * 2 + pc) * 1024
@@ -298,7 +298,7 @@ __device__ __forceinline__ void wide_gemm(const WideOperands &o, int chunk0, int
 // l (lr = l % 16, lk = l / 16), element e at (((ct nst + s) 2 + h) 64 + l) 4 +
 // e, holding M[16 ct + lr][32 s + 16 h + 4 e + lk]; 16-bit, per part: lane l's
 // eight values M[16 ct + lr][32 s + 8 lk ..] at ((ct nst + s) 64 + l) 8.
-inline size_t wide_frag_elems(int dim) { return (size_t)round_up((dim + 15) / 16, 16) * 16 * round_up(dim, 32); }
+__host__ __device__ inline size_t wide_frag_elems(int dim) { return (size_t)round_up((dim + 15) / 16, 16) * 16 * round_up(dim, 32); }
 int wide_fragments(const float *B32, int ldb32, const uint16_t *const M16[6], int ldm16, int dim, float *f32,
                    uint16_t *const f16[6], hipStream_t s);
 
