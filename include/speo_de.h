@@ -344,7 +344,9 @@ SPEO_EXPORT int speo_segment_argmin(const float *f, const int *off, int nseg, in
 /* ---- the island engine ---------------------------------------------- */
 
 enum {
-    SPEO_MODE_PLAIN = 0, /* generate, evaluate, select: three launches per generation */
+    SPEO_MODE_PLAIN = 0, /* generate, evaluate, select over one population; generations of one
+                          * run share launches (sub-islands, surrogate, objectives 9-22: three
+                          * launches each) */
     SPEO_MODE_FUSED = 1, /* one launch per generation: select(g-1)+generate(g)+evaluate(g) */
     SPEO_MODE_EPOCH = 2  /* one launch per epoch (the generations between migrations):
                           * one workgroup per island keeps its population on chip.

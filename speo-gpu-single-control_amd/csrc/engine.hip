@@ -8,10 +8,13 @@
 //
 // One kernel, k_generation, covers the four per-generation roles over a table
 // of (island, row tile) work items, so every launch spans all islands:
-//   kModeGen     trials U <- X                       (plain engine, launch 1)
-//   kModeEval    f(U) through the MFMA evaluation    (plain engine, launch 2)
-//   kModeSelect  X, fX <- U, fU where fU < fX        (plain engine, launch 3)
+//   kModeGen     trials U <- X
+//   kModeEval    f(U) through the MFMA evaluation
+//   kModeSelect  X, fX <- U, fU where fU < fX
 //   kModeFused   select(g-1) + generate(g) + evaluate(g) in one launch.
+// A plain engine runs its generations as fused launches and one selection
+// after the last; the three separate roles serve sub-islands, the surrogate,
+// problems of the generic kernel and the per-role profile.
 // Evaluation inside this kernel is for rows of at most 128 columns; when an
 // island is wider, kModeFusedGen makes the generation's trials and the launches
 // of engine_wide.hip evaluate them.
@@ -68,6 +71,8 @@ struct GenerationArgs {
     uint64_t seed;
     const uint32_t *gen_base;
     uint32_t gen_offset;
+    const int4 *donors;  // [row] {r0, r1, r2, j_rand} of the generation (epoch_donors)
+    int pending;         // fused modes: trials of the previous generation await selection
     int clear_trials;
 };
 
@@ -86,6 +91,8 @@ __device__ __forceinline__ float comp4(const float4 &v, int q) {
     return q == 0 ? v.x : (q == 1 ? v.y : (q == 2 ? v.z : v.w));
 }
 
+// A generation's donors are drawn ahead of it, one row per lane (k_epoch_donors);
+// drawn here, all 16 lanes of a row repeated two Philox blocks and the redraws.
 // Row tile 32: three waves per SIMD (at most 168 registers).  Held to four
 // waves (128 registers) the fused FP32 kernel spills 44 registers and runs
 // 9 % slower on an uneven batch of 256 islands, D 10..100 (with 13 spilled
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             const int lr = pass * 16 + (tid >> 4), l = tid & 15;
             if (lr >= t.nrows) continue;
             const int li = t.row0 + lr, gr = I.row_off + li;
-            const float fu = a.fU_prev[gr], fx = a.fX_new[gr];
+            const float fu = a.fU_prev[gr], fx = a.fX_prev[gr];
             const bool acc = fu < fx;
             if (acc) {
                 const float *u = a.U_prev + I.elem_off + (size_t)li * I.ld;
@@ -113,7 +120,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
                 for (int g = l; g < (I.ld >> 2); g += 16) st4(x + 4 * g, ld4(u + 4 * g));
             }
             if (l == 0) {
-                if (acc) a.fX_new[gr] = fu;
+                a.fX_new[gr] = acc ? fu : fx;
                 if (a.clear_trials) a.fU_prev[gr] = INFINITY;
             }
         }
@@ -148,25 +155,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             if (!c.valid) return c;
             c.li = t.row0 + lr;
             c.gr = (uint32_t)(I.row_off + c.li);
-            DonorStream ds(a.seed, c.gr, gen);
-            int r[kMaxR];
-            draw_donors(ds, nullptr, 0, I.np, I.dim, r, c.jr);
+            const int4 d = a.donors[c.gr];
+            c.jr = d.w;
             // Row `k` of the island as the parent population of this generation.
             auto parent = [&](int k) -> const float * {
                 const int g = I.row_off + k;
-                if (FUSED && a.fU_prev[g] < a.fX_prev[g])
+                if (FUSED && a.pending && a.fU_prev[g] < a.fX_prev[g])
                     return a.U_prev + I.elem_off + (size_t)k * I.ld;
                 return a.X + I.elem_off + (size_t)k * I.ld;
             };
-            c.p0 = parent(r[0]);
-            c.p1 = parent(r[1]);
-            c.p2 = parent(r[2]);
+            c.p0 = parent(d.x);
+            c.p1 = parent(d.y);
+            c.p2 = parent(d.z);
             c.own_acc = false;
             c.fx_own = c.fu_own = 0.f;
             if (FUSED) {
                 c.fx_own = a.fX_prev[c.gr];
                 c.fu_own = a.fU_prev[c.gr];
-                c.own_acc = c.fu_own < c.fx_own;
+                c.own_acc = a.pending && c.fu_own < c.fx_own;
             }
             c.own = c.own_acc ? a.U_prev + I.elem_off + (size_t)c.li * I.ld
                               : a.X + I.elem_off + (size_t)c.li * I.ld;
@@ -455,7 +461,8 @@ struct Engine {
 
     float *X = nullptr, *fX[2] = {nullptr, nullptr}, *U[2] = {nullptr, nullptr};
     float *fU[2] = {nullptr, nullptr};
-    int p = 0;
+    int p = 0;            // fused mode: the buffers of the current fitness and trials
+    int pf = 0, pu = 0;   // the same within a plain chunk, where they part (both 0 outside)
     bool pending = false;
 
     int rt = 32;
@@ -490,14 +497,18 @@ struct Engine {
     std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;
     bool graph_failed = false;
 
+    // donors drawn ahead of the generations (engines that are neither configured nor screened)
+    int4 *donor_buf = nullptr;  // [donor_gens][rows]
+    int *row_island_dev = nullptr;
+    int donor_gens = 1;
+    int donor_setup();
+    int draw_ahead(int gen_offset, int L, hipStream_t s);
+
     // epoch mode: per-island plans, block order, LDS of a launch
     EpochBlock *blocks_dev = nullptr;
     int epoch_lds = 0, epoch_parts = 1, epoch_blocks = 0;
     float *Xnext = nullptr;  // split islands: the population of the next generation
     int ep_par = 0;          // split islands: buffers swapped an odd number of times
-    int4 *donor_buf = nullptr;    // [donor_gens][rows] donors drawn ahead of the epoch launches
-    int *row_island_dev = nullptr;
-    int donor_gens = 0;
     int epoch_setup();
     int epoch_plan_all(int parts, std::vector<EpochPlan> *plans, int *lds);
     int launch_epoch_chunk(int L, hipStream_t s);
@@ -508,6 +519,7 @@ struct Engine {
     int upload_tables();
     int build_tiles(int rt_);
     int launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear = 0);
+    int enqueue_plain(int L, hipStream_t s);
     int enqueue_chunk(int L, bool migrate, hipStream_t s);
     int finalize_pending(hipStream_t s);
     int migrate(hipStream_t s);
@@ -785,6 +797,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
                                                "of 4 * 2^k rows");
         }
     }
+    if (c.surrogate_candidates == 0 && !configured) SPEO_TRY(donor_setup());
     if (c.surrogate_candidates > 0 && c.mode != SPEO_MODE_PLAIN)
         return set_error(SPEO_ERR_UNSUPPORTED, "speo_engine_create: the surrogate runs in "
                                                "SPEO_MODE_PLAIN");
@@ -899,16 +912,21 @@ int Engine::epoch_setup() {
         e.heavy = c.heavy;
     }
     SPEO_TRY(upload_vec(&blocks_dev, blocks));
+    if (parts > 1) {
+        SPEO_TRY_HIP(hipMalloc(&Xnext, sizeof(float) * (size_t)total_elems));
+        SPEO_TRY_HIP(hipMemcpy(Xnext, X, sizeof(float) * (size_t)total_elems, hipMemcpyDeviceToDevice));
+    }
+    return SPEO_OK;
+}
+
+// The buffer of donors drawn ahead: at most 64 generations and 2^26 rows of them.
+int Engine::donor_setup() {
     std::vector<int> row_island((size_t)total_rows);
     for (int i = 0; i < I; ++i)
         for (int r = 0; r < isl[(size_t)i].np; ++r) row_island[(size_t)(isl[(size_t)i].row_off + r)] = i;
     SPEO_TRY(upload_vec(&row_island_dev, row_island));
     donor_gens = (int)std::max<int64_t>(1, std::min<int64_t>(64, (int64_t(1) << 26) / total_rows));
     SPEO_TRY_HIP(hipMalloc(&donor_buf, sizeof(int4) * (size_t)donor_gens * (size_t)total_rows));
-    if (parts > 1) {
-        SPEO_TRY_HIP(hipMalloc(&Xnext, sizeof(float) * (size_t)total_elems));
-        SPEO_TRY_HIP(hipMemcpy(Xnext, X, sizeof(float) * (size_t)total_elems, hipMemcpyDeviceToDevice));
-    }
     return SPEO_OK;
 }
 
@@ -1141,6 +1159,7 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
     a.seed = cfg.seed;
     a.gen_base = gen_base;
     a.gen_offset = (uint32_t)gen_offset;
+    a.donors = donor_buf ? donor_buf + (size_t)(gen_offset % donor_gens) * (size_t)total_rows : nullptr;
     a.clear_trials = clear;
     switch (mode) {
     case kModeGen:
@@ -1155,27 +1174,61 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
         if (cfg.mode == SPEO_MODE_FUSED) {  // apply the pending selection
             a.U_prev = U[p];
             a.fU_prev = fU[p];
-            a.fX_new = fX[p];
+            a.fX_prev = a.fX_new = fX[p];
         } else {
             a.U_prev = U[0];
             a.fU_prev = fU[0];
+            a.fX_prev = fX[pf];
             a.fX_new = fX[0];
         }
         break;
-    default:
-        a.fX_prev = fX[p];
-        a.U_prev = U[p];
-        a.fU_prev = fU[p];
-        a.fX_new = fX[1 - p];
-        a.U_new = U[1 - p];
-        a.fU_new = fU[1 - p];
+    default: {
+        const bool fused = cfg.mode == SPEO_MODE_FUSED;
+        const int u = fused ? p : pu, f = fused ? p : pf;
+        a.pending = fused || pending;
+        a.fX_prev = fX[f];
+        a.U_prev = U[u];
+        a.fU_prev = fU[u];
+        a.fX_new = fX[1 - f];
+        a.U_new = U[1 - u];
+        a.fU_new = fU[1 - u];
         if (!all_small) {
             SPEO_TRY(launch_any(rt_, cfg.precision, kModeFusedGen, a, ntiles[rt_], s));
-            return eval_wide_rows(U[1 - p], fU[1 - p], rt_, s);
+            return eval_wide_rows(a.U_new, a.fU_new, rt_, s);
         }
         break;
     }
+    }
     return launch_any(rt_, cfg.precision, mode, a, ntiles[rt_], s);
+}
+
+// Donors and j_rand of generations [gen_offset, gen_offset + L), L <= donor_gens,
+// into donor_buf, where launch() reads generation g's at g % donor_gens.
+int Engine::draw_ahead(int gen_offset, int L, hipStream_t s) {
+    return epoch_donors(isl_dev, row_island_dev, total_rows, L, cfg.seed, gen_base, (uint32_t)gen_offset,
+                        donor_buf, s);
+}
+
+// L generations of a plain engine as L fused launches and one selection: L + 1
+// launches instead of 3 L (100 rows, D = 10, ten generations and the best:
+// 144 us as separate launches, 100 us so).  The parities are chosen so that the
+// last trials end in U[0], fU[0] and the last selection writes fX[0]: the
+// buffers the three separate launches leave.
+int Engine::enqueue_plain(int L, hipStream_t s) {
+    pf = 0;
+    pu = L & 1;
+    pending = false;
+    for (int g = 0; g < L; ++g) {
+        if (g % donor_gens == 0) SPEO_TRY(draw_ahead(g, std::min(donor_gens, L - g), s));
+        SPEO_TRY(launch(kModeFused, g, rt, s));
+        pf = 1 - pf;
+        pu = 1 - pu;
+        pending = true;
+    }
+    if (L > 0) SPEO_TRY(launch(kModeSelect, 0, rt, s));
+    pf = pu = 0;
+    pending = false;
+    return SPEO_OK;
 }
 
 // ------------------------------------------------- sub-islands (plain mode)
@@ -1302,8 +1355,11 @@ int Engine::migrate(hipStream_t s) {
 int Engine::enqueue_chunk(int L, bool do_migrate, hipStream_t s) {
     if (cfg.mode == SPEO_MODE_EPOCH) {
         SPEO_TRY(launch_epoch_chunk(L, s));
+    } else if (cfg.mode == SPEO_MODE_PLAIN && C == 0 && !configured && !any_generic) {
+        SPEO_TRY(enqueue_plain(L, s));
     } else {
         for (int g = 0; g < L; ++g) {
+            if (donor_buf && g % donor_gens == 0) SPEO_TRY(draw_ahead(g, std::min(donor_gens, L - g), s));
             if (C > 0) {
                 SPEO_TRY(surrogate_generation(g, s));
             } else if (cfg.mode == SPEO_MODE_FUSED) {
@@ -1560,6 +1616,7 @@ int Engine::profile(int generations, double *avg_ms) {
         return SPEO_OK;
     };
     for (int g = 0; g < generations; ++g) {
+        if (donor_buf) SPEO_TRY(draw_ahead(0, 1, stream));
         const int64_t gi = gens;
         const int modes[3] = {kModeGen, kModeEval, kModeSelect};
         if (cfg.mode == SPEO_MODE_FUSED) {
@@ -1715,6 +1772,7 @@ int Engine::autotune() {
     for (int cand : {16, 32, 64}) {
         SPEO_TRY(build_tiles(cand));
         const int mode = cfg.mode == SPEO_MODE_FUSED ? kModeFused : kModeEval;
+        if (donor_buf) SPEO_TRY(draw_ahead(0, std::min(6, donor_gens), stream));
         for (int rep = 0; rep < 2; ++rep) SPEO_TRY(launch(mode, rep, cand, stream));
         SPEO_TRY_HIP(hipEventRecord(e0, stream));
         const int reps = 6;

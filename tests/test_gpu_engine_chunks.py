@@ -1,0 +1,46 @@
+"""A plain engine's run of several generations (one launch a generation, the last
+selection after it, donors drawn ahead) leaves what its separate generate,
+evaluate and select launches leave: population, fitness, the last trials and
+their fitness, bit for bit.  Odd and even lengths, the 64-generation limit of the
+donors drawn at once, migrations inside a run, eager and replayed."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _problems(speo, dims):
+    rng = np.random.default_rng(5)
+    out = []
+    for D, objs in dims:
+        o = np.float32(rng.uniform(-80, 80, (len(objs), D))).astype(np.float64)
+        M = np.stack([np.linalg.qr(rng.standard_normal((D, D)))[0] for _ in objs])
+        out.append(speo.Problem(objs, o, M, sigma=[10.0 * (c + 1) for c in range(len(objs))],
+                                bias=[100.0 * c for c in range(len(objs))]))
+    return out
+
+
+@pytest.mark.parametrize("lengths,interval,graph,dims", [
+    ((1, 2, 3), 0, 0, [(10, [2]), (7, [3])]),
+    ((1, 1, 4), 2, 0, [(10, [2]), (128, [1])]),
+    ((64, 1), 0, 1, [(9, [3]), (30, [1, 2])]),
+    ((65, 65), 0, 0, [(9, [3]), (30, [1, 2])]),
+    ((130, 130), 50, 1, [(5, [2]), (33, [5])]),
+    ((2, 3), 2, 0, [(129, [2]), (40, [3])]),
+])
+def test_run_equals_separate_launches(cuda, speo, lengths, interval, graph, dims):
+    probs = _problems(speo, dims)
+    kw = dict(seed=3, interval=interval, migration_size=2 if interval else 0, mode=speo.MODE_PLAIN,
+              rows_per_block=32)
+    sizes, which = [31, 64, 100, 8], [0, 1, 0, 1]
+    a = speo.Engine(probs, sizes, which, use_graph=bool(graph), **kw)
+    b = speo.Engine(probs, sizes, which, use_graph=False, **kw)
+    for L in lengths:
+        print(f"generations {L} interval {interval} graph {graph} dims {dims}", flush=True)
+        a.run(L)
+        b.profile(L)
+        for x, y in zip(a.read() + a.read_trials(), b.read() + b.read_trials()):
+            np.testing.assert_array_equal(x, y)
+    assert a.best()[1].tolist() == b.best()[1].tolist()
+    for o in [a, b] + probs:
+        o.close()
