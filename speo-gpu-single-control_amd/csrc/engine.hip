@@ -74,6 +74,7 @@ struct GenerationArgs {
     const int4 *donors;  // [row] {r0, r1, r2, j_rand} of the generation (epoch_donors)
     int pending;         // fused modes: trials of the previous generation await selection
     int clear_trials;
+    int composed;        // an island's problem has more than one component
 };
 
 constexpr int kTLD = kSmallD;  // widest dimension this kernel evaluates
@@ -98,8 +99,8 @@ __device__ __forceinline__ float comp4(const float4 &v, int q) {
 // 9 % slower on an uneven batch of 256 islands, D 10..100 (with 13 spilled
 // values, before the FP64 heavy-column step was added, four waves were 7 %
 // faster).  The other row tiles keep the compiler's allocation.
-template <int RT, int PREC, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 3 : 1))) void k_generation(
+template <int RT, int PREC, int MODE, bool COMP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? (COMP ? 3 : 4) : 1))) void k_generation(
     GenerationArgs a) {
     extern __shared__ __align__(16) char lds[];
     const TileDesc t = a.tiles[blockIdx.x];
@@ -133,6 +134,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
     float *gval = trial + RT * kTS;
     char *gemm_lds = reinterpret_cast<char *>(gval + kMaxComp * RT);
 
+    // The first component's rotation does not depend on the rows: its operands
+    // are requested before them.
+    constexpr bool EVAL = MODE == kModeEval || MODE == kModeFused;
+    constexpr bool AHEAD = EVAL && Prec<PREC>::parts == 0;
+    const FusedProblem *P = a.probs + I.problem;
+    if (MODE == kModeEval && P->generic) return;  // the generic kernel evaluates this island
+    SmallB B;
+
     if constexpr (MODE == kModeGen || FUSED) {
         const uint32_t gen = (a.gen_base ? *a.gen_base : 0u) + a.gen_offset;
         const int ngroups = (I.dim + 3) >> 2;
@@ -148,14 +157,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             const float *p0, *p1, *p2, *own;
         };
         const int l = tid & 15;
-        auto prep = [&](int lr) {
+        auto prep = [&](int lr, const int4 &d) {
             RowCtx c{};
             c.lr = lr;
             c.valid = lr < t.nrows;
             if (!c.valid) return c;
             c.li = t.row0 + lr;
             c.gr = (uint32_t)(I.row_off + c.li);
-            const int4 d = a.donors[c.gr];
             c.jr = d.w;
             // Row `k` of the island as the parent population of this generation.
             auto parent = [&](int k) -> const float * {
@@ -203,8 +211,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
         for (int pass = 0; pass < RT / 16; pass += 2) {
             const int lrA = pass * 16 + (tid >> 4), lrB = lrA + 16;
             const bool hasB = pass + 1 < RT / 16;
-            const RowCtx A = prep(lrA);
-            const RowCtx B = hasB ? prep(lrB) : RowCtx{};
+            const int4 *dn = a.donors + I.row_off + t.row0;
+            const int4 dA = dn[min(lrA, t.nrows - 1)], dB = dn[min(lrB, t.nrows - 1)];
+            const RowCtx A = prep(lrA, dA);
+            const RowCtx Bq = hasB ? prep(lrB, dB) : RowCtx{};
             for (int g = l; g < ngroups; g += 16) {
                 float4 a0, a1, a2, ao, b0, b1, b2, bo;
                 if (A.valid) {
@@ -213,28 +223,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
                     a2 = ld4(A.p2 + 4 * g);
                     ao = ld4(A.own + 4 * g);
                 }
-                if (B.valid) {
-                    b0 = ld4(B.p0 + 4 * g);
-                    b1 = ld4(B.p1 + 4 * g);
-                    b2 = ld4(B.p2 + 4 * g);
-                    bo = ld4(B.own + 4 * g);
+                if (Bq.valid) {
+                    b0 = ld4(Bq.p0 + 4 * g);
+                    b1 = ld4(Bq.p1 + 4 * g);
+                    b2 = ld4(Bq.p2 + 4 * g);
+                    bo = ld4(Bq.own + 4 * g);
                 }
                 if (A.valid) make(A, g, a0, a1, a2, ao);
                 else if (lds_trial) st4(trial + lrA * kTS + 4 * g, float4{0.f, 0.f, 0.f, 0.f});
-                if (B.valid) make(B, g, b0, b1, b2, bo);
+                if (Bq.valid) make(Bq, g, b0, b1, b2, bo);
                 else if (hasB && lds_trial) st4(trial + lrB * kTS + 4 * g, float4{0.f, 0.f, 0.f, 0.f});
             }
             if (FUSED && l == 0) {
                 if (A.valid) a.fX_new[A.gr] = A.own_acc ? A.fu_own : A.fx_own;
-                if (B.valid) a.fX_new[B.gr] = B.own_acc ? B.fu_own : B.fx_own;
+                if (Bq.valid) a.fX_new[Bq.gr] = Bq.own_acc ? Bq.fu_own : Bq.fx_own;
             }
         }
     }
 
     if constexpr (MODE == kModeEval || MODE == kModeFused) {
-        const FusedProblem *P = a.probs + I.problem;
-        if (MODE == kModeEval && P->generic) return;  // the generic kernel evaluates this island
-        const int ncomp = P->ncomp, dim = I.dim;
+        const int ncomp = COMP ? P->ncomp : 1, dim = I.dim;
         if (MODE == kModeEval) {
             // stage the rows to evaluate into the LDS tile (zero rows past nrows)
             const float *srcp = a.eval_src + I.elem_off + (size_t)t.row0 * I.ld;
@@ -245,13 +253,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
                     r < t.nrows ? ld4(srcp + (size_t)r * I.ld + 4 * g) : float4{0.f, 0.f, 0.f, 0.f});
             }
         }
+        if constexpr (AHEAD) {
+            B.load(P->comp[0], dim);
+            B.stage(gemm_lds);
+        }
         __syncthreads();
         for (int c = 0; c < ncomp; ++c) {
             const CompDev comp = P->comp[c];
             float *red = reinterpret_cast<float *>(gemm_lds + small_scratch_bytes<RT>(Prec<PREC>::parts));
             float *o1 = red + 8 * RT, *o2 = o1 + RT;
             float s1[RT / 16][4], s2[RT / 16][4];
-            gemm_small<RT, PREC>(comp, trial, dim, gemm_lds, s1, s2);
+            if constexpr (AHEAD) {
+                if (c > 0) {  // (the reduction's barriers lie between this and the last K loop)
+                    B.load(comp, dim);
+                    B.stage(gemm_lds);
+                    __syncthreads();
+                }
+                gemm_small_f32<RT>(comp, B, trial, dim, gemm_lds, s1, s2);
+            } else {
+                gemm_small<RT, PREC>(comp, trial, dim, gemm_lds, s1, s2);
+            }
             reduce_rows_small<RT>(s1, s2, red, o1, o2);
             if (tid < t.nrows) gval[c * RT + tid] = finish_objective_ext(comp.objective, o1[tid], o2[tid], dim);
             if (comp.heavy.j >= 0) {
@@ -267,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
         }
         if (tid < t.nrows) {
             float f;
-            if (ncomp == 1) {
+            if (!COMP || ncomp == 1) {
                 f = fmaf(P->lambda[0], gval[tid], P->bias[0]);
             } else {
                 // cf_cal weights (CEC2014.cc:1481-1519) in the log domain.
@@ -312,27 +333,33 @@ __global__ void k_add_u32(uint32_t *p, uint32_t v) {
 }
 // ------------------------------------------------------------------ launch
 
-template <int RT, int PREC, int MODE>
+template <int RT, int PREC, int MODE, bool COMP>
 static int launch_generation(const GenerationArgs &a, int ntiles, hipStream_t s) {
     const int lds = MODE == kModeEval || MODE == kModeFused ? generation_lds_bytes<RT, PREC>() : 0;
     static std::once_flag once;
     std::call_once(once, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_generation<RT, PREC, MODE>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_generation<RT, PREC, MODE, COMP>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                   generation_lds_bytes<RT, PREC>());
     });
-    hipLaunchKernelGGL((k_generation<RT, PREC, MODE>), dim3(ntiles), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((k_generation<RT, PREC, MODE, COMP>), dim3(ntiles), dim3(256), lds, s, a);
     return check_launch("k_generation");
+}
+
+template <int RT, int PREC, int MODE>
+static int launch_values(const GenerationArgs &a, int ntiles, hipStream_t s) {
+    return a.composed ? launch_generation<RT, PREC, MODE, true>(a, ntiles, s)
+                      : launch_generation<RT, PREC, MODE, false>(a, ntiles, s);
 }
 
 template <int RT, int PREC>
 static int launch_mode(int mode, const GenerationArgs &a, int ntiles, hipStream_t s) {
     switch (mode) {
-    case kModeGen: return launch_generation<RT, PREC, kModeGen>(a, ntiles, s);
-    case kModeEval: return launch_generation<RT, PREC, kModeEval>(a, ntiles, s);
-    case kModeSelect: return launch_generation<RT, SPEO_PREC_FP32, kModeSelect>(a, ntiles, s);
-    case kModeFusedGen: return launch_generation<RT, SPEO_PREC_FP32, kModeFusedGen>(a, ntiles, s);
-    default: return launch_generation<RT, PREC, kModeFused>(a, ntiles, s);
+    case kModeGen: return launch_generation<RT, PREC, kModeGen, false>(a, ntiles, s);
+    case kModeEval: return launch_values<RT, PREC, kModeEval>(a, ntiles, s);
+    case kModeSelect: return launch_generation<RT, SPEO_PREC_FP32, kModeSelect, false>(a, ntiles, s);
+    case kModeFusedGen: return launch_generation<RT, SPEO_PREC_FP32, kModeFusedGen, false>(a, ntiles, s);
+    default: return launch_values<RT, PREC, kModeFused>(a, ntiles, s);
     }
 }
 
@@ -461,6 +488,7 @@ struct Engine {
 
     float *X = nullptr, *fX[2] = {nullptr, nullptr}, *U[2] = {nullptr, nullptr};
     float *fU[2] = {nullptr, nullptr};
+    bool composed = false;  // a problem has more than one component
     int p = 0;            // fused mode: the buffers of the current fitness and trials
     int pf = 0, pu = 0;   // the same within a plain chunk, where they part (both 0 outside)
     bool pending = false;
@@ -652,6 +680,7 @@ int Engine::upload_tables() {
         f.dim = P.dim;
         f.generic = P.generic ? 1 : 0;
         any_generic = any_generic || P.generic;
+        composed = composed || P.ncomp > 1;
         for (int c = 0; c < P.ncomp; ++c) {
             f.lambda[c] = (float)P.comp[c].lambda;
             f.bias[c] = (float)P.comp[c].bias;
@@ -817,6 +846,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
         a.probs = probs_dev;
         a.eval_src = X;
         a.eval_out = fX[0];
+        a.composed = composed;
         SPEO_TRY(launch_any(rt, cfg.precision, kModeEval, a, ntiles[rt], stream));
     } else {
         SPEO_TRY(eval_wide_rows(X, fX[0], rt, stream));
@@ -1161,6 +1191,7 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
     a.gen_offset = (uint32_t)gen_offset;
     a.donors = donor_buf ? donor_buf + (size_t)(gen_offset % donor_gens) * (size_t)total_rows : nullptr;
     a.clear_trials = clear;
+    a.composed = composed;
     switch (mode) {
     case kModeGen:
         a.U_new = U[0];

@@ -635,46 +635,142 @@ template <int RT> constexpr int small_scratch_bytes(int parts) {
     return 128 * 4 + parts * RT * (kSmallD + 8) * 2;
 }
 
+// The terms of a wave's accumulators (column tiles wave and wave + 4).
 template <int RT, int PREC>
-__device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, int dim,
-                                           char *scratch, float (&s1)[RT / 16][4],
-                                           float (&s2)[RT / 16][4]) {
+__device__ __forceinline__ void small_terms(const CompDev &c, const floatx4 (&acc)[RT / 16][2], int dim,
+                                            float (&s1)[RT / 16][4], float (&s2)[RT / 16][4]) {
+    constexpr int NRT = RT / 16;
+    const int wave = threadIdx.x >> 6, lr = threadIdx.x & 15;
+    const int t0 = wave, t1 = wave + 4;
+    const float unscale = Prec<PREC>::half ? kF16Unscale : 1.0f;
+#pragma unroll
+    for (int i = 0; i < NRT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            s1[i][q] = 0.f;
+            s2[i][q] = 0.f;
+        }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int col = (t == 0 ? t0 : t1) * 16 + lr;
+        if (col < dim) {
+            const float w = (c.objective == SPEO_OBJ_ELLIPTIC) ? c.colw[col] : 1.0f;
+            with_objective(c.objective, [&](auto obj) {
+#pragma unroll
+                for (int i = 0; i < NRT; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        add_terms(decltype(obj)::value, acc[i][t][q] * unscale, w, s1[i][q], s2[i][q]);
+            });
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NRT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            s1[i][q] = sum16(s1[i][q]);
+            s2[i][q] = sum16(s2[i][q]);
+        }
+}
+
+// The FP32 operands of a component's rotation that do not depend on the rows:
+// both column tiles' B fragments and the shift, requested ahead of the rows.
+struct SmallB {
+    float b0[32], b1[32];
+    float o;  // the thread's shift value
+    __device__ __forceinline__ void load(const CompDev &c, int dim) {
+        const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+        const int KS = (dim + 3) >> 2;
+        load_b_frag(c.B32s, wave, wave * 16 < dim, KS, lane, b0);
+        load_b_frag(c.B32s, wave + 4, (wave + 4) * 16 < dim, KS, lane, b1);
+        o = tid < dim ? gld(c.shift + tid) : 0.f;
+    }
+    // into the scratch's shift (kSmallD floats); a barrier before gemm_small_f32
+    __device__ __forceinline__ void stage(char *scratch) const {
+        if (threadIdx.x < kSmallD) reinterpret_cast<float *>(scratch)[threadIdx.x] = o;
+    }
+};
+
+template <int RT>
+__device__ __forceinline__ void gemm_small_f32(const CompDev &c, const SmallB &B, const float *rows, int dim,
+                                               const char *scratch, float (&s1)[RT / 16][4],
+                                               float (&s2)[RT / 16][4]) {
     constexpr int NRT = RT / 16;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lk = lane >> 4;
-    float *sh = reinterpret_cast<float *>(scratch);  // shift, then rate-scaled in place
+    const float *sh = reinterpret_cast<const float *>(scratch);
     floatx4 acc[NRT][2];
 #pragma unroll
     for (int i = 0; i < NRT; ++i) {
         acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
         acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    const int t0 = wave, t1 = wave + 4;
-    const bool v0 = t0 * 16 < dim, v1 = t1 * 16 < dim;
-
-    if constexpr (Prec<PREC>::parts == 0) {
-        const int kp4 = (dim + 3) & ~3, KS = kp4 >> 2;
-        // B fragments into registers first (their latency overlaps the shift staging)
-        float b0[32], b1[32];
-        load_b_frag(c.B32s, t0, v0, KS, lane, b0);
-        load_b_frag(c.B32s, t1, v1, KS, lane, b1);
-        for (int k = tid; k < kSmallD; k += 256) sh[k] = k < dim ? gld(c.shift + k) : 0.f;
-        __syncthreads();
-        const float rate = c.rate;
+    const bool v0 = wave * 16 < dim, v1 = (wave + 4) * 16 < dim;
+    const int KS = (dim + 3) >> 2;
+    const float rate = c.rate;
+    // Blocks of four K steps: a block's rows and shift are read from LDS together
+    // (columns past the dimension are read but not multiplied: k < kSmallD < kTS).
+    auto steps = [&](auto both) {
 #pragma unroll
-        for (int ks = 0; ks < 32; ++ks) {
-            if (ks < KS) {
-                const int k = ks * 4 + lk;
-                const float o = sh[k];
+        for (int q = 0; q < 8; ++q) {
+            if (4 * q >= KS) break;
+            float x[NRT][4], o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 16 * q + 4 * e + lk;
+                o[e] = sh[k];
+#pragma unroll
+                for (int i = 0; i < NRT; ++i) x[i][e] = rows[(i * 16 + lr) * kTS + k];
+            }
+            auto step = [&](int e) {
 #pragma unroll
                 for (int i = 0; i < NRT; ++i) {
-                    const float a = (rows[(i * 16 + lr) * kTS + k] - o) * rate;
-                    if (v0) acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b0[ks], acc[i][0], 0, 0, 0);
-                    if (v1) acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b1[ks], acc[i][1], 0, 0, 0);
+                    const float a = (x[i][e] - o[e]) * rate;
+                    acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, B.b0[4 * q + e], acc[i][0], 0, 0, 0);
+                    if constexpr (decltype(both)::value)
+                        acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, B.b1[4 * q + e], acc[i][1], 0, 0, 0);
                 }
+            };
+            if (4 * q + 4 <= KS) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) step(e);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (4 * q + e < KS) step(e);
             }
         }
+    };
+    if (v1) steps(std::true_type{});
+    else if (v0) steps(std::false_type{});
+    small_terms<RT, SPEO_PREC_FP32>(c, acc, dim, s1, s2);
+}
+
+template <int RT, int PREC>
+__device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, int dim,
+                                           char *scratch, float (&s1)[RT / 16][4],
+                                           float (&s2)[RT / 16][4]) {
+    if constexpr (Prec<PREC>::parts == 0) {
+        SmallB B;
+        B.load(c, dim);
+        B.stage(scratch);
+        __syncthreads();
+        gemm_small_f32<RT>(c, B, rows, dim, scratch, s1, s2);
+        return;
     } else {
+        constexpr int NRT = RT / 16;
+        const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+        const int lr = lane & 15, lk = lane >> 4;
+        float *sh = reinterpret_cast<float *>(scratch);  // shift, then rate-scaled in place
+        floatx4 acc[NRT][2];
+#pragma unroll
+        for (int i = 0; i < NRT; ++i) {
+            acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+            acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int t0 = wave, t1 = wave + 4;
+        const bool v0 = t0 * 16 < dim, v1 = t1 * 16 < dim;
+
         constexpr int P = Prec<PREC>::parts;
         constexpr bool H = Prec<PREC>::half;
         typedef typename std::conditional<H, halfx8, bf16x8>::type vec8;
@@ -727,36 +823,8 @@ __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, 
                 }
             }
         }
+        small_terms<RT, PREC>(c, acc, dim, s1, s2);
     }
-    const float unscale = Prec<PREC>::half ? kF16Unscale : 1.0f;
-#pragma unroll
-    for (int i = 0; i < NRT; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            s1[i][q] = 0.f;
-            s2[i][q] = 0.f;
-        }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int col = (t == 0 ? t0 : t1) * 16 + lr;
-        if (col < dim) {
-            const float w = (c.objective == SPEO_OBJ_ELLIPTIC) ? c.colw[col] : 1.0f;
-            with_objective(c.objective, [&](auto obj) {
-#pragma unroll
-                for (int i = 0; i < NRT; ++i)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        add_terms(decltype(obj)::value, acc[i][t][q] * unscale, w, s1[i][q], s2[i][q]);
-            });
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NRT; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            s1[i][q] = sum16(s1[i][q]);
-            s2[i][q] = sum16(s2[i][q]);
-        }
 }
 
 // Per-row sums of gemm_small's per-wave partials (fixed order over waves).
