@@ -51,7 +51,8 @@ enum GenMode { kModeGen = 0, kModeEval = 1, kModeSelect = 2, kModeFused = 3, kMo
 // in one round trip instead of two dependent ones.
 struct TileDesc {
     IslandDesc I;
-    int island, row0, nrows, pad;
+    int island, row0, nrows;
+    uint32_t inv_ng;  // ceil(2^32 / ng), ng = ceil(dim / 4): exact for e < 64 ng (0: ng == 1 or >= 8192)
 };
 
 struct GenerationArgs {
@@ -77,13 +78,23 @@ struct GenerationArgs {
     int composed;        // an island's problem has more than one component
 };
 
+// TileDesc::inv_ng: with inv = ceil(2^32 / ng), e * inv / 2^32 exceeds e / ng by
+// less than e / 2^32, which reaches no next whole number while e * ng < 2^32.
+static uint32_t inverse_groups(int dim) {
+    const uint64_t ng = ((uint64_t)dim + 3) / 4;
+    return ng > 1 && 64 * ng * ng < (1ull << 32) ? (uint32_t)((0x100000000ull + ng - 1) / ng) : 0u;
+}
+
 constexpr int kTLD = kSmallD;  // widest dimension this kernel evaluates
 
 // LDS of one block: [trial rows RT x kTS] [gval kMaxComp x RT] [scratch of the
-// GEMM and the row reduction].
+// GEMM and the row reduction, before them the parents' table].  Generations
+// without evaluation hold the table alone.
+template <int RT> constexpr int parent_table_bytes() { return RT * (4 * 8 + 4); }
 template <int RT, int PREC>
 constexpr int generation_lds_bytes() {
-    return RT * kTS * 4 + kMaxComp * RT * 4 + small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4;
+    return RT * kTS * 4 + kMaxComp * RT * 4 +
+           std::max(small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4, parent_table_bytes<RT>());
 }
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -92,13 +103,18 @@ __device__ __forceinline__ float comp4(const float4 &v, int q) {
     return q == 0 ? v.x : (q == 1 ? v.y : (q == 2 ? v.z : v.w));
 }
 
-// A generation's donors are drawn ahead of it, one row per lane (k_epoch_donors);
-// drawn here, all 16 lanes of a row repeated two Philox blocks and the redraws.
-// Row tile 32: three waves per SIMD (at most 168 registers).  Held to four
-// waves (128 registers) the fused FP32 kernel spills 44 registers and runs
-// 9 % slower on an uneven batch of 256 islands, D 10..100 (with 13 spilled
-// values, before the FP64 heavy-column step was added, four waves were 7 %
-// faster).  The other row tiles keep the compiler's allocation.
+// What bounds the fused kernel: the crossover's Philox blocks (18 wide integer
+// multiplies per four coordinates) and, at D = 100, the FP32 matrix
+// instructions, about equally.  So every lane makes trials (items of a row and
+// four coordinates, where 16 lanes a row left 13 idle at D = 10), the parents of
+// a row are found once, not by 16 lanes, a generation's donors are drawn ahead
+// of it, one row per lane (k_epoch_donors), and blocks start at different
+// column classes.  256 uneven islands, D 10..100, one generation: 62 us with
+// donors drawn here, 49 without, 40 with the evaluation's registers at four
+// waves a SIMD unit, 33 with the items and classes.
+// Row tile 32 is held to four waves a SIMD unit (128 registers, no spills); with
+// the composition's code to three.  The other row tiles keep the compiler's
+// allocation.
 template <int RT, int PREC, int MODE, bool COMP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? (COMP ? 3 : 4) : 1))) void k_generation(
     GenerationArgs a) {
@@ -132,7 +148,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
     constexpr bool lds_trial = MODE == kModeFused || MODE == kModeEval;
     float *trial = reinterpret_cast<float *>(lds);
     float *gval = trial + RT * kTS;
-    char *gemm_lds = reinterpret_cast<char *>(gval + kMaxComp * RT);
+    char *gemm_lds = lds_trial ? reinterpret_cast<char *>(gval + kMaxComp * RT) : lds;
 
     // The first component's rotation does not depend on the rows: its operands
     // are requested before them.
@@ -142,119 +158,99 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
     if (MODE == kModeEval && P->generic) return;  // the generic kernel evaluates this island
     SmallB B;
 
+    const int ng = (I.dim + 3) >> 2;  // groups of four coordinates
+    // row and group of item e < RT * ng
+    auto item_row = [&](int e) { return t.inv_ng ? (int)__umulhi((uint32_t)e, t.inv_ng) : e / ng; };
+
     if constexpr (MODE == kModeGen || FUSED) {
         const uint32_t gen = (a.gen_base ? *a.gen_base : 0u) + a.gen_offset;
-        const int ngroups = (I.dim + 3) >> 2;
         const uint32_t crt = cr_threshold(I.CR);
-        // Two passes (rows lr and lr + 16 of the tile, 16 lanes per row) at a
-        // time: the parent-selection loads of both rows, then their row
-        // loads, are in flight together.
-        struct RowCtx {
-            bool valid, own_acc;
-            int lr, li, jr;
-            uint32_t gr;
-            float fx_own, fu_own;
-            const float *p0, *p1, *p2, *own;
-        };
-        const int l = tid & 15;
-        auto prep = [&](int lr, const int4 &d) {
-            RowCtx c{};
-            c.lr = lr;
-            c.valid = lr < t.nrows;
-            if (!c.valid) return c;
-            c.li = t.row0 + lr;
-            c.gr = (uint32_t)(I.row_off + c.li);
-            c.jr = d.w;
-            // Row `k` of the island as the parent population of this generation.
-            auto parent = [&](int k) -> const float * {
-                const int g = I.row_off + k;
-                if (FUSED && a.pending && a.fU_prev[g] < a.fX_prev[g])
-                    return a.U_prev + I.elem_off + (size_t)k * I.ld;
-                return a.X + I.elem_off + (size_t)k * I.ld;
-            };
-            c.p0 = parent(d.x);
-            c.p1 = parent(d.y);
-            c.p2 = parent(d.z);
-            c.own_acc = false;
-            c.fx_own = c.fu_own = 0.f;
+        // Four threads a row find its parents: the donors' rows and its own,
+        // each where the pending selection left it.
+        const float **src = reinterpret_cast<const float **>(gemm_lds);  // [RT][4]
+        int *own = reinterpret_cast<int *>(src + 4 * RT);                // [RT] j_rand, bit 31: own trial accepted
+        if (tid < 4 * t.nrows) {
+            const int lr = tid >> 2, j = tid & 3, li = t.row0 + lr, gr = I.row_off + li;
+            const int4 d = a.donors[gr];
+            const int r = j == 0 ? d.x : j == 1 ? d.y : j == 2 ? d.z : li;
+            bool acc = false;
             if (FUSED) {
-                c.fx_own = a.fX_prev[c.gr];
-                c.fu_own = a.fU_prev[c.gr];
-                c.own_acc = a.pending && c.fu_own < c.fx_own;
+                const float fx = a.fX_prev[I.row_off + r];
+                const float fu = a.pending ? a.fU_prev[I.row_off + r] : INFINITY;
+                acc = fu < fx;
+                if (j == 3) a.fX_new[gr] = acc ? fu : fx;
             }
-            c.own = c.own_acc ? a.U_prev + I.elem_off + (size_t)c.li * I.ld
-                              : a.X + I.elem_off + (size_t)c.li * I.ld;
+            src[tid] = (acc ? a.U_prev : a.X) + I.elem_off + (size_t)r * I.ld;
+            if (j == 3) own[lr] = d.w | (acc ? (int)0x80000000 : 0);
+        }
+        __syncthreads();
+        float *U_new = a.U_new + I.elem_off + (size_t)t.row0 * I.ld;
+        float *X = a.X + I.elem_off + (size_t)t.row0 * I.ld;
+        // Items of (row, group of four coordinates), two at a time: the loads
+        // of both are in flight together.
+        struct Item {
+            bool valid, acc;
+            int lr, g, jr;
+            float4 e0, e1, e2, xo;
+        };
+        auto load = [&](int e) {
+            Item c;
+            c.valid = e < t.nrows * ng;
+            if (!c.valid) return c;
+            c.lr = item_row(e);
+            c.g = e - c.lr * ng;
+            const int o = own[c.lr];
+            c.jr = o & 0x7fffffff;
+            c.acc = o < 0;
+            c.e0 = ld4(src[4 * c.lr + 0] + 4 * c.g);
+            c.e1 = ld4(src[4 * c.lr + 1] + 4 * c.g);
+            c.e2 = ld4(src[4 * c.lr + 2] + 4 * c.g);
+            c.xo = ld4(src[4 * c.lr + 3] + 4 * c.g);
             return c;
         };
-        // trial coordinates 4 g .. 4 g + 3 of a prepared row
-        auto make = [&](const RowCtx &c, int g, const float4 &e0, const float4 &e1, const float4 &e2,
-                        const float4 &xo) {
-            const U4 w = philox_block(a.seed, (uint32_t)g, c.gr, gen, kPurposeCross);
+        auto make = [&](const Item &c) {
+            const U4 w = philox_block(a.seed, (uint32_t)c.g, (uint32_t)(I.row_off + t.row0 + c.lr), gen,
+                                      kPurposeCross);
             float v[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int j = 4 * g + q;
-                if (j < I.dim) {
-                    const bool take = (j == c.jr) || cross_take(word(w, q), crt);
-                    const float m = take ? fmaf(I.F, comp4(e1, q) - comp4(e2, q), comp4(e0, q))
-                                         : comp4(xo, q);
-                    v[q] = check_bound(m, a.lo, a.hi);
-                } else {
-                    v[q] = 0.f;
-                }
+                const int j = 4 * c.g + q;
+                const bool take = (j == c.jr) || cross_take(word(w, q), crt);
+                const float m = take ? fmaf(I.F, comp4(c.e1, q) - comp4(c.e2, q), comp4(c.e0, q))
+                                     : comp4(c.xo, q);
+                v[q] = j < I.dim ? check_bound(m, a.lo, a.hi) : 0.f;
             }
             const float4 out{v[0], v[1], v[2], v[3]};
-            st4(a.U_new + I.elem_off + (size_t)c.li * I.ld + 4 * g, out);
-            if (lds_trial) st4(trial + c.lr * kTS + 4 * g, out);
-            if (FUSED && c.own_acc) st4(a.X + I.elem_off + (size_t)c.li * I.ld + 4 * g, xo);
+            st4(U_new + c.lr * I.ld + 4 * c.g, out);
+            if (lds_trial) st4(trial + c.lr * kTS + 4 * c.g, out);
+            if (FUSED && c.acc) st4(X + c.lr * I.ld + 4 * c.g, c.xo);
         };
-        for (int pass = 0; pass < RT / 16; pass += 2) {
-            const int lrA = pass * 16 + (tid >> 4), lrB = lrA + 16;
-            const bool hasB = pass + 1 < RT / 16;
-            const int4 *dn = a.donors + I.row_off + t.row0;
-            const int4 dA = dn[min(lrA, t.nrows - 1)], dB = dn[min(lrB, t.nrows - 1)];
-            const RowCtx A = prep(lrA, dA);
-            const RowCtx Bq = hasB ? prep(lrB, dB) : RowCtx{};
-            for (int g = l; g < ngroups; g += 16) {
-                float4 a0, a1, a2, ao, b0, b1, b2, bo;
-                if (A.valid) {
-                    a0 = ld4(A.p0 + 4 * g);
-                    a1 = ld4(A.p1 + 4 * g);
-                    a2 = ld4(A.p2 + 4 * g);
-                    ao = ld4(A.own + 4 * g);
-                }
-                if (Bq.valid) {
-                    b0 = ld4(Bq.p0 + 4 * g);
-                    b1 = ld4(Bq.p1 + 4 * g);
-                    b2 = ld4(Bq.p2 + 4 * g);
-                    bo = ld4(Bq.own + 4 * g);
-                }
-                if (A.valid) make(A, g, a0, a1, a2, ao);
-                else if (lds_trial) st4(trial + lrA * kTS + 4 * g, float4{0.f, 0.f, 0.f, 0.f});
-                if (Bq.valid) make(Bq, g, b0, b1, b2, bo);
-                else if (hasB && lds_trial) st4(trial + lrB * kTS + 4 * g, float4{0.f, 0.f, 0.f, 0.f});
-            }
-            if (FUSED && l == 0) {
-                if (A.valid) a.fX_new[A.gr] = A.own_acc ? A.fu_own : A.fx_own;
-                if (Bq.valid) a.fX_new[Bq.gr] = Bq.own_acc ? Bq.fu_own : Bq.fx_own;
-            }
+        for (int e = tid; e < t.nrows * ng; e += 512) {
+            const Item A = load(e), B = load(e + 256);
+            make(A);
+            if (B.valid) make(B);
         }
+        if (lds_trial)  // rows past the tile's
+            for (int e = t.nrows * ng + tid; e < RT * ng; e += 256) {
+                const int lr = item_row(e);
+                st4(trial + lr * kTS + 4 * (e - lr * ng), float4{0.f, 0.f, 0.f, 0.f});
+            }
+        if constexpr (EVAL) __syncthreads();  // the parents' table lies where the evaluation's scratch does
     }
 
     if constexpr (MODE == kModeEval || MODE == kModeFused) {
-        const int ncomp = COMP ? P->ncomp : 1, dim = I.dim;
+        const int ncomp = COMP ? P->ncomp : 1, dim = I.dim, cls = column_class();
         if (MODE == kModeEval) {
             // stage the rows to evaluate into the LDS tile (zero rows past nrows)
             const float *srcp = a.eval_src + I.elem_off + (size_t)t.row0 * I.ld;
-            const int ngroups = (dim + 3) >> 2;
-            for (int e = tid; e < RT * ngroups; e += 256) {
-                const int r = e / ngroups, g = e % ngroups;
+            for (int e = tid; e < RT * ng; e += 256) {
+                const int r = item_row(e), g = e - r * ng;
                 st4(trial + r * kTS + 4 * g,
                     r < t.nrows ? ld4(srcp + (size_t)r * I.ld + 4 * g) : float4{0.f, 0.f, 0.f, 0.f});
             }
         }
         if constexpr (AHEAD) {
-            B.load(P->comp[0], dim);
+            B.load(P->comp[0], dim, cls);
             B.stage(gemm_lds);
         }
         __syncthreads();
@@ -265,24 +261,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             float s1[RT / 16][4], s2[RT / 16][4];
             if constexpr (AHEAD) {
                 if (c > 0) {  // (the reduction's barriers lie between this and the last K loop)
-                    B.load(comp, dim);
+                    B.load(comp, dim, cls);
                     B.stage(gemm_lds);
                     __syncthreads();
                 }
-                gemm_small_f32<RT>(comp, B, trial, dim, gemm_lds, s1, s2);
+                gemm_small_f32<RT>(comp, B, trial, dim, cls, gemm_lds, s1, s2);
             } else {
-                gemm_small<RT, PREC>(comp, trial, dim, gemm_lds, s1, s2);
+                gemm_small<RT, PREC>(comp, trial, dim, cls, gemm_lds, s1, s2);
             }
-            reduce_rows_small<RT>(s1, s2, red, o1, o2);
+            reduce_rows_small<RT>(s1, s2, cls, red, o1, o2);
             if (tid < t.nrows) gval[c * RT + tid] = finish_objective_ext(comp.objective, o1[tid], o2[tid], dim);
             if (comp.heavy.j >= 0) {
                 // the heavy column's FP64 term, one wave per row
                 __syncthreads();
                 const int wave = tid >> 6, lane = tid & 63;
-                for (int r = wave; r < t.nrows; r += 4) {
-                    const double h = heavy_term(comp.heavy, trial + r * kTS, dim, lane);
-                    if (lane == 0) gval[c * RT + r] = with_heavy(gval[c * RT + r], (float)h);
-                }
+                heavy_rows(comp.heavy, dim, wave, 4, t.nrows, lane, [&](int r) { return trial + r * kTS; },
+                           [&](int r, double h) {
+                               if (lane == 0) gval[c * RT + r] = with_heavy(gval[c * RT + r], (float)h);
+                           });
                 __syncthreads();
             }
         }
@@ -335,7 +331,9 @@ __global__ void k_add_u32(uint32_t *p, uint32_t v) {
 
 template <int RT, int PREC, int MODE, bool COMP>
 static int launch_generation(const GenerationArgs &a, int ntiles, hipStream_t s) {
-    const int lds = MODE == kModeEval || MODE == kModeFused ? generation_lds_bytes<RT, PREC>() : 0;
+    const int lds = MODE == kModeEval || MODE == kModeFused ? generation_lds_bytes<RT, PREC>()
+                    : MODE == kModeSelect                     ? 0
+                                                              : parent_table_bytes<RT>();
     static std::once_flag once;
     std::call_once(once, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_generation<RT, PREC, MODE, COMP>),
@@ -609,7 +607,8 @@ int Engine::build_tiles(int rt_) {
     std::vector<TileDesc> tiles;
     for (int i = 0; i < I; ++i)
         for (int r0 = 0; r0 < isl[(size_t)i].np; r0 += rt_)
-            tiles.push_back(TileDesc{isl[(size_t)i], i, r0, std::min(rt_, isl[(size_t)i].np - r0), 0});
+            tiles.push_back(TileDesc{isl[(size_t)i], i, r0, std::min(rt_, isl[(size_t)i].np - r0),
+                                     inverse_groups(isl[(size_t)i].dim)});
     // Heaviest tiles first (rows x dim^2, ties in island order): blocks are
     // dispatched in this order, so with uneven islands the last wave of blocks
     // holds the cheap tiles.  Tiles are independent: the order changes no result.

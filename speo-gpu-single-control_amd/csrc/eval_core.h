@@ -291,6 +291,46 @@ __device__ __forceinline__ double heavy_term(const HeavyCol &c, const float *x, 
     return c.w * z * z;
 }
 
+// heavy_term of rows first, first + step, ... < nrows (x_of(r): the row), for
+// emit(r, term) on every lane.  Up to 128 columns the column of M and the shift
+// are read once and four rows' reductions run side by side: same terms, same
+// order.
+template <typename Row, typename Emit>
+__device__ __forceinline__ void heavy_rows(const HeavyCol &c, int dim, int first, int step, int nrows, int lane,
+                                           Row x_of, Emit emit) {
+    if (dim > 128) {
+        for (int r = first; r < nrows; r += step) emit(r, heavy_term(c, x_of(r), dim, lane));
+        return;
+    }
+    double m[2] = {0.0, 0.0}, o[2] = {0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = lane + 64 * h;
+        if (k < dim) {
+            m[h] = c.m64 ? c.m64[k] : (double)c.m32[(size_t)k * c.ld];
+            o[h] = c.o64 ? c.o64[k] : (double)c.o32[k];
+        }
+    }
+    for (int r0 = first; r0 < nrows; r0 += 4 * step) {
+        double z[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + i * step;
+            z[i] = 0.0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (r < nrows && lane + 64 * h < dim)
+                    z[i] = fma(m[h], ((double)x_of(r)[lane + 64 * h] - o[h]) * c.rate, z[i]);
+        }
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) z[i] += __shfl_xor(z[i], off, 64);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r0 + i * step < nrows) emit(r0 + i * step, c.w * z[i] * z[i]);
+    }
+}
+
 // The FP32 row sum with the heavy column's term added (the term rounded to
 // FP32 first, so that kernels that park it in an FP32 slot of LDS get the
 // same bits).
@@ -624,8 +664,9 @@ __device__ __forceinline__ void load_b_frag(const float *B32s, int t, bool valid
 // ------------------------------------------------------- small-D path
 //
 // dim <= 128.  The tile's RT rows are in LDS (rows[r * kTS + k], FP32,
-// unshifted; rows >= nrows and columns >= dim hold zeros).  Wave w owns the
-// 16-column tiles w and w + 4 for all RT rows; its B fragments come straight
+// unshifted; rows >= nrows and columns >= dim hold zeros).  The wave of column
+// class `cls` (0..3, one wave each) owns the 16-column tiles cls and cls + 4 for
+// all RT rows; its B fragments come straight
 // from the padded global layouts into registers (no LDS staging, no barrier
 // inside the K loop).  `scratch` holds the shifted rows' 16-bit parts for the
 // 16-bit precisions: P * RT * (kp32 + 8) uint16, and the shift: 128 floats.
@@ -637,11 +678,11 @@ template <int RT> constexpr int small_scratch_bytes(int parts) {
 
 // The terms of a wave's accumulators (column tiles wave and wave + 4).
 template <int RT, int PREC>
-__device__ __forceinline__ void small_terms(const CompDev &c, const floatx4 (&acc)[RT / 16][2], int dim,
+__device__ __forceinline__ void small_terms(const CompDev &c, const floatx4 (&acc)[RT / 16][2], int dim, int cls,
                                             float (&s1)[RT / 16][4], float (&s2)[RT / 16][4]) {
     constexpr int NRT = RT / 16;
-    const int wave = threadIdx.x >> 6, lr = threadIdx.x & 15;
-    const int t0 = wave, t1 = wave + 4;
+    const int lr = threadIdx.x & 15;
+    const int t0 = cls, t1 = cls + 4;
     const float unscale = Prec<PREC>::half ? kF16Unscale : 1.0f;
 #pragma unroll
     for (int i = 0; i < NRT; ++i)
@@ -678,11 +719,11 @@ __device__ __forceinline__ void small_terms(const CompDev &c, const floatx4 (&ac
 struct SmallB {
     float b0[32], b1[32];
     float o;  // the thread's shift value
-    __device__ __forceinline__ void load(const CompDev &c, int dim) {
-        const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    __device__ __forceinline__ void load(const CompDev &c, int dim, int cls) {
+        const int tid = threadIdx.x, lane = tid & 63;
         const int KS = (dim + 3) >> 2;
-        load_b_frag(c.B32s, wave, wave * 16 < dim, KS, lane, b0);
-        load_b_frag(c.B32s, wave + 4, (wave + 4) * 16 < dim, KS, lane, b1);
+        load_b_frag(c.B32s, cls, cls * 16 < dim, KS, lane, b0);
+        load_b_frag(c.B32s, cls + 4, (cls + 4) * 16 < dim, KS, lane, b1);
         o = tid < dim ? gld(c.shift + tid) : 0.f;
     }
     // into the scratch's shift (kSmallD floats); a barrier before gemm_small_f32
@@ -692,12 +733,11 @@ struct SmallB {
 };
 
 template <int RT>
-__device__ __forceinline__ void gemm_small_f32(const CompDev &c, const SmallB &B, const float *rows, int dim,
+__device__ __forceinline__ void gemm_small_f32(const CompDev &c, const SmallB &B, const float *rows, int dim, int cls,
                                                const char *scratch, float (&s1)[RT / 16][4],
                                                float (&s2)[RT / 16][4]) {
     constexpr int NRT = RT / 16;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int lr = lane & 15, lk = lane >> 4;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
     const float *sh = reinterpret_cast<const float *>(scratch);
     floatx4 acc[NRT][2];
 #pragma unroll
@@ -705,7 +745,7 @@ __device__ __forceinline__ void gemm_small_f32(const CompDev &c, const SmallB &B
         acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
         acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    const bool v0 = wave * 16 < dim, v1 = (wave + 4) * 16 < dim;
+    const bool v0 = cls * 16 < dim, v1 = (cls + 4) * 16 < dim;
     const int KS = (dim + 3) >> 2;
     const float rate = c.rate;
     // Blocks of four K steps: a block's rows and shift are read from LDS together
@@ -743,23 +783,23 @@ __device__ __forceinline__ void gemm_small_f32(const CompDev &c, const SmallB &B
     };
     if (v1) steps(std::true_type{});
     else if (v0) steps(std::false_type{});
-    small_terms<RT, SPEO_PREC_FP32>(c, acc, dim, s1, s2);
+    small_terms<RT, SPEO_PREC_FP32>(c, acc, dim, cls, s1, s2);
 }
 
 template <int RT, int PREC>
-__device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, int dim,
+__device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, int dim, int cls,
                                            char *scratch, float (&s1)[RT / 16][4],
                                            float (&s2)[RT / 16][4]) {
     if constexpr (Prec<PREC>::parts == 0) {
         SmallB B;
-        B.load(c, dim);
+        B.load(c, dim, cls);
         B.stage(scratch);
         __syncthreads();
-        gemm_small_f32<RT>(c, B, rows, dim, scratch, s1, s2);
+        gemm_small_f32<RT>(c, B, rows, dim, cls, scratch, s1, s2);
         return;
     } else {
         constexpr int NRT = RT / 16;
-        const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+        const int tid = threadIdx.x, lane = tid & 63;
         const int lr = lane & 15, lk = lane >> 4;
         float *sh = reinterpret_cast<float *>(scratch);  // shift, then rate-scaled in place
         floatx4 acc[NRT][2];
@@ -768,7 +808,7 @@ __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, 
             acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
             acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        const int t0 = wave, t1 = wave + 4;
+        const int t0 = cls, t1 = cls + 4;
         const bool v0 = t0 * 16 < dim, v1 = t1 * 16 < dim;
 
         constexpr int P = Prec<PREC>::parts;
@@ -823,17 +863,24 @@ __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, 
                 }
             }
         }
-        small_terms<RT, PREC>(c, acc, dim, s1, s2);
+        small_terms<RT, PREC>(c, acc, dim, cls, s1, s2);
     }
 }
 
-// Per-row sums of gemm_small's per-wave partials (fixed order over waves).
+// The column class of a wave: blocks start at different classes, since a
+// wave's place in its block fixes its SIMD unit and the first classes have the
+// most columns.
+__device__ __forceinline__ int column_class() {
+    return __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) + blockIdx.x) & 3;
+}
+
+// Per-row sums of gemm_small's per-class partials (fixed order over classes).
 // red: 2 * 4 * RT floats of LDS; out1/out2: RT floats each.
 template <int RT>
 __device__ __forceinline__ void reduce_rows_small(const float (&s1)[RT / 16][4],
-                                                  const float (&s2)[RT / 16][4], float *red,
+                                                  const float (&s2)[RT / 16][4], int cls, float *red,
                                                   float *out1, float *out2) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
     __syncthreads();
     if ((lane & 15) == 0) {
 #pragma unroll
@@ -841,8 +888,8 @@ __device__ __forceinline__ void reduce_rows_small(const float (&s1)[RT / 16][4],
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int r = i * 16 + (lane >> 4) * 4 + q;
-                red[(wave * RT + r) * 2 + 0] = s1[i][q];
-                red[(wave * RT + r) * 2 + 1] = s2[i][q];
+                red[(cls * RT + r) * 2 + 0] = s1[i][q];
+                red[(cls * RT + r) * 2 + 1] = s2[i][q];
             }
     }
     __syncthreads();

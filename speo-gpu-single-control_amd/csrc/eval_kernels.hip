@@ -67,8 +67,9 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
         }
         __syncthreads();
         float s1[RT / 16][4], s2[RT / 16][4];
-        gemm_small<RT, PREC>(p.comp, rows, p.dim, scratch, s1, s2);
-        reduce_rows_small<RT>(s1, s2, red, o1, o2);
+        const int cls = column_class();
+        gemm_small<RT, PREC>(p.comp, rows, p.dim, cls, scratch, s1, s2);
+        reduce_rows_small<RT>(s1, s2, cls, red, o1, o2);
     } else {
         RowSource src{p.X + (size_t)row0 * p.ld, p.ld, nrows};
         float s1[4] = {0.f, 0.f, 0.f, 0.f}, s2[4] = {0.f, 0.f, 0.f, 0.f};
@@ -82,10 +83,9 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
         // the heavy column's FP64 term, one wave per row, into the row sums
         // (the row staging area is free after the reductions' barriers)
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        for (int r = wave; r < nrows; r += 4) {
-            const double h = heavy_term(p.comp.heavy, p.X + (size_t)(row0 + r) * p.ld, p.dim, lane);
-            if (lane == 0) o1[r] = with_heavy(o1[r], (float)h);
-        }
+        heavy_rows(p.comp.heavy, p.dim, wave, 4, nrows, lane,
+                   [&](int r) { return p.X + (size_t)(row0 + r) * p.ld; },
+                   [&](int r, double h) { if (lane == 0) o1[r] = with_heavy(o1[r], (float)h); });
         __syncthreads();
     }
     const int t = threadIdx.x;

@@ -126,8 +126,6 @@ static void free_problem(ProblemHost &P) {
             (void)hipFree(h.Mhs[p]);
         }
         (void)hipFree(h.wide32);
-        (void)hipFree(h.wide_bf);
-        (void)hipFree(h.wide_h);
         (void)hipFree(h.colw);
         h = CompHost{};
     }
@@ -244,9 +242,10 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
         // (the kernels move through the three parts by 32-bit byte offsets)
         const size_t fe = wide_frag_elems(dim);
         if (3 * 2 * fe < 0x7fffffffull) {
-            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide32), sizeof(float) * fe));
-            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide_bf), sizeof(uint16_t) * 3 * fe));
-            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide_h), sizeof(uint16_t) * 3 * fe));
+            // one allocation: FP32, the BF16 parts, the FP16 parts
+            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide32), (sizeof(float) + 2 * 3 * sizeof(uint16_t)) * fe));
+            h.wide_bf = reinterpret_cast<uint16_t *>(h.wide32 + fe);
+            h.wide_h = h.wide_bf + 3 * fe;
             const uint16_t *src[6] = {h.Mbf[0], h.Mbf[1], h.Mbf[2], h.Mh[0], h.Mh[1], h.Mh[2]};
             uint16_t *dst[6] = {h.wide_bf, h.wide_bf + fe, h.wide_bf + 2 * fe,
                                 h.wide_h, h.wide_h + fe, h.wide_h + 2 * fe};
