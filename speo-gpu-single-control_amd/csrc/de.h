@@ -146,6 +146,15 @@ __device__ __forceinline__ int block_argmin(const float *f, const int *perm, int
     return bi;
 }
 
+// ceil(2^32 / ng), ng = ceil(dim / 4), for e / ng = mulhi(e, inverse): with it
+// e * inverse / 2^32 exceeds e / ng by less than e / 2^32, which reaches no next
+// whole number while e * ng < 2^32.  For e < 64 ng; 0 where that does not hold
+// or ng == 1.
+inline uint32_t group_inverse(int dim) {
+    const uint64_t ng = ((uint64_t)dim + 3) / 4;
+    return ng > 1 && 64 * ng * ng < (1ull << 32) ? (uint32_t)((0x100000000ull + ng - 1) / ng) : 0u;
+}
+
 int init_population(float *X, int ld, int n, int dim, float lo, float hi, uint64_t seed,
                     uint32_t row_base, hipStream_t s);
 int de_generate(const GenArgs &a, hipStream_t s);

@@ -52,7 +52,16 @@ enum GenMode { kModeGen = 0, kModeEval = 1, kModeSelect = 2, kModeFused = 3, kMo
 struct TileDesc {
     IslandDesc I;
     int island, row0, nrows;
-    uint32_t inv_ng;  // ceil(2^32 / ng), ng = ceil(dim / 4): exact for e < 64 ng (0: ng == 1 or >= 8192)
+    uint32_t inv_ng;  // group_inverse(I.dim)
+};
+
+// A screened generation's appends (C > 0): the evaluation writes the trials and
+// log(1 + f) to the archive and applies the selection itself.
+struct AppendArgs {
+    float *AX, *Ay;     // [problem][cap][Kp], [problem][cap]; AX null: evaluation only
+    const int *qrel;    // [island] first target's place among its problem's
+    const int *head;    // [problem] first slot of the generation
+    int cap, Kp;
 };
 
 struct GenerationArgs {
@@ -76,14 +85,8 @@ struct GenerationArgs {
     int pending;         // fused modes: trials of the previous generation await selection
     int clear_trials;
     int composed;        // an island's problem has more than one component
+    AppendArgs append;
 };
-
-// TileDesc::inv_ng: with inv = ceil(2^32 / ng), e * inv / 2^32 exceeds e / ng by
-// less than e / 2^32, which reaches no next whole number while e * ng < 2^32.
-static uint32_t inverse_groups(int dim) {
-    const uint64_t ng = ((uint64_t)dim + 3) / 4;
-    return ng > 1 && 64 * ng * ng < (1ull << 32) ? (uint32_t)((0x100000000ull + ng - 1) / ng) : 0u;
-}
 
 constexpr int kTLD = kSmallD;  // widest dimension this kernel evaluates
 
@@ -317,6 +320,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT == 32 ? 
             }
             float *out = MODE == kModeEval ? a.eval_out : a.fU_new;
             out[I.row_off + t.row0 + tid] = f;
+            if (MODE == kModeEval && a.append.AX) {
+                const int gr = I.row_off + t.row0 + tid;
+                const float fx = a.fX_new[gr];
+                const size_t slot = (size_t)I.problem * a.append.cap +
+                                    (size_t)(((int64_t)a.append.head[I.problem] + a.append.qrel[t.island] + t.row0 +
+                                              tid) % a.append.cap);
+                if (f < fx) a.fX_new[gr] = f;
+                a.append.Ay[slot] = log1pf(fmaxf(f, 0.f));
+                reinterpret_cast<int64_t *>(gemm_lds)[tid] = (int64_t)slot * 2 + (f < fx ? 1 : 0);
+            }
+        }
+        if (MODE == kModeEval && a.append.AX) {
+            // the rows to the archive (zeros past the dimension), accepted ones
+            // also to the population
+            __syncthreads();
+            const int64_t *slots = reinterpret_cast<const int64_t *>(gemm_lds);
+            float *X = a.X + I.elem_off + (size_t)t.row0 * I.ld;
+            const int kg = a.append.Kp >> 2;
+            for (int e = tid; e < t.nrows * kg; e += 256) {
+                const int r = e / kg, g = e - r * kg;
+                const int64_t sl = slots[r];
+                const float4 v = g < ng ? ld4(trial + r * kTS + 4 * g) : float4{0.f, 0.f, 0.f, 0.f};
+                st4(a.append.AX + (size_t)(sl >> 1) * a.append.Kp + 4 * g, v);
+                if ((sl & 1) && g < ng) st4(X + r * I.ld + 4 * g, v);
+            }
         }
     }
 }
@@ -508,7 +536,9 @@ struct Engine {
     long long *scored_dev = nullptr;  // candidates scored per problem by the one-kernel screening
     float *Xb = nullptr, *tb = nullptr, *Xh = nullptr, *yh = nullptr, *predh = nullptr;
     float2 *ranks_ws = nullptr;  // Spearman workspace
-    int *heads_dev = nullptr;         // next archive slot per problem (device)
+    int *heads_dev = nullptr;         // the generation's first archive slot per problem (device)
+    int *qrel_dev = nullptr;          // [island] first target's place among its problem's
+    int4 *drawn = nullptr;            // [target][candidate] donors and j_rand of scored candidates
     uint32_t *round_dev = nullptr;    // training rounds run (device; keys the minibatch draws)
     bool any_trained = false;
     int last_Ce = 1;  // candidates per target in the last surrogate generation
@@ -523,7 +553,7 @@ struct Engine {
     std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;
     bool graph_failed = false;
 
-    // donors drawn ahead of the generations (engines that are neither configured nor screened)
+    // donors drawn ahead of the generations (engines without sub-islands)
     int4 *donor_buf = nullptr;  // [donor_gens][rows]
     int *row_island_dev = nullptr;
     int donor_gens = 1;
@@ -544,7 +574,7 @@ struct Engine {
     int create(const speo_engine_config &c, hipStream_t s);
     int upload_tables();
     int build_tiles(int rt_);
-    int launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear = 0);
+    int launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear = 0, bool append = false);
     int enqueue_plain(int L, hipStream_t s);
     int enqueue_chunk(int L, bool migrate, hipStream_t s);
     int finalize_pending(hipStream_t s);
@@ -587,7 +617,7 @@ Engine::~Engine() {
                     best_part, probs_dev, params_tab_dev, gen_base,
                     blocks_dev, Xnext, donor_buf, row_island_dev, wide_items, gval,
                     X, fX[0], fX[1], U[0], U[1], fU[0], fU[1], srows_dev, cand, pred, rho_dev, scored_dev,
-                    AX, Ay, Xb, tb, Xh, yh, predh, ranks_ws, heads_dev, round_dev, perm_dev,
+                    AX, Ay, Xb, tb, Xh, yh, predh, ranks_ws, heads_dev, qrel_dev, drawn, round_dev, perm_dev,
                     best_sub_dev, info_dev};
     for (void *b : bufs) (void)hipFree(b);
     (void)hipHostFree(best_out);
@@ -608,7 +638,7 @@ int Engine::build_tiles(int rt_) {
     for (int i = 0; i < I; ++i)
         for (int r0 = 0; r0 < isl[(size_t)i].np; r0 += rt_)
             tiles.push_back(TileDesc{isl[(size_t)i], i, r0, std::min(rt_, isl[(size_t)i].np - r0),
-                                     inverse_groups(isl[(size_t)i].dim)});
+                                     group_inverse(isl[(size_t)i].dim)});
     // Heaviest tiles first (rows x dim^2, ties in island order): blocks are
     // dispatched in this order, so with uneven islands the last wave of blocks
     // holds the cheap tiles.  Tiles are independent: the order changes no result.
@@ -825,7 +855,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
                                                "of 4 * 2^k rows");
         }
     }
-    if (c.surrogate_candidates == 0 && !configured) SPEO_TRY(donor_setup());
+    if (!configured) SPEO_TRY(donor_setup());
     if (c.surrogate_candidates > 0 && c.mode != SPEO_MODE_PLAIN)
         return set_error(SPEO_ERR_UNSUPPORTED, "speo_engine_create: the surrogate runs in "
                                                "SPEO_MODE_PLAIN");
@@ -1031,13 +1061,16 @@ int Engine::surrogate_setup() {
                                        ">= 1024, batch >= 16, train interval >= 1, lr > 0");
     Kp = round_up(D, 32);
     std::vector<SurrRowDesc> rows;
+    std::vector<int> qrel((size_t)I, 0);
     for (int p = 0; p < cfg.num_problems; ++p) {
         auto sp = std::make_unique<SurrProblem>();
         sp->qoff = (int)rows.size();
         for (int i = 0; i < I; ++i)
-            if (isl[(size_t)i].problem == p)
+            if (isl[(size_t)i].problem == p) {
+                qrel[(size_t)i] = (int)rows.size() - sp->qoff;
                 for (int li = 0; li < isl[(size_t)i].np; ++li)
                     rows.push_back(SurrRowDesc{isl[(size_t)i].row_off + li, i, p, li});
+            }
         sp->rows = (int)rows.size() - sp->qoff;
         if (sp->rows > 0) {
             const int mb = std::max({cfg.surrogate_batch, sp->rows * C, 1024});
@@ -1062,7 +1095,13 @@ int Engine::surrogate_setup() {
     SPEO_TRY_HIP(hipMalloc(&predh, sizeof(float) * 1024));
     SPEO_TRY_HIP(hipMalloc(&ranks_ws, sizeof(float2) * 4096));
     SPEO_TRY_HIP(hipMalloc(&heads_dev, sizeof(int) * kMaxSurrProblems));
-    SPEO_TRY_HIP(hipMemset(heads_dev, 0, sizeof(int) * kMaxSurrProblems));
+    // (the first generation's pick advances the heads to slot 0)
+    std::vector<int> head0(kMaxSurrProblems, 0);
+    for (size_t p = 0; p < surr.size(); ++p)
+        head0[p] = (cfg.surrogate_archive - surr[p]->rows % cfg.surrogate_archive) % cfg.surrogate_archive;
+    SPEO_TRY_HIP(hipMemcpy(heads_dev, head0.data(), sizeof(int) * head0.size(), hipMemcpyHostToDevice));
+    SPEO_TRY(upload_vec(&qrel_dev, qrel));
+    SPEO_TRY_HIP(hipMalloc(&drawn, sizeof(int4) * (size_t)Q * C));
     SPEO_TRY_HIP(hipMalloc(&round_dev, sizeof(uint32_t)));
     SPEO_TRY_HIP(hipMemset(round_dev, 0, sizeof(uint32_t)));
     return SPEO_OK;
@@ -1076,6 +1115,14 @@ int Engine::surrogate_generation(int gen_offset, hipStream_t s) {
     last_Ce = Ce;
     const float rho_min = any_trained ? cfg.surrogate_rho_min : INFINITY;
     const float lo = cfg.min_bound, hi = cfg.max_bound;
+    SurrArchive ar{};
+    for (size_t p = 0; p < surr.size(); ++p) {
+        ar.heads.qoff[p] = surr[p]->qoff;
+        ar.heads.rows[p] = surr[p]->rows;
+    }
+    ar.problems = (int)surr.size();
+    ar.cap = cfg.surrogate_archive;
+    ar.head_dev = heads_dev;
     if (retain_cand || Kp > kFusedMaxKp) {
         // candidates written to memory, scored, the pick copied
         SPEO_TRY(gen_candidates(isl_dev, srows_dev, Q, Ce, X, lo, hi, cfg.seed, gen_base,
@@ -1087,7 +1134,7 @@ int Engine::surrogate_generation(int gen_offset, hipStream_t s) {
                                            pred + (size_t)sp->qoff * Ce, s));
             surr_pred += (int64_t)Q * Ce;
         }
-        SPEO_TRY(pick_candidates(isl_dev, srows_dev, Q, Ce, cand, Kp, pred, rho_dev, rho_min, U[0], s));
+        SPEO_TRY(pick_candidates(isl_dev, srows_dev, Q, Ce, cand, Kp, pred, rho_dev, rho_min, U[0], ar, s));
     } else {
         // candidates generated and scored in one kernel per problem, the pick
         // generated again into U: the same trials without the candidate buffer
@@ -1103,23 +1150,19 @@ int Engine::surrogate_generation(int gen_offset, hipStream_t s) {
                 }
             SPEO_TRY(cand_infer(nets.data(), qo.data(), nq.data(), pi.data(), (int)nets.size(), isl_dev,
                                 srows_dev, Ce, X, lo, hi, cfg.seed, gen_base, (uint32_t)gen_offset,
-                                rho_dev, rho_min, scored_dev, pred, s));
+                                rho_dev, rho_min, scored_dev, pred, drawn, s));
         }
-        SPEO_TRY(pick_regen(isl_dev, srows_dev, Q, Ce, pred, rho_dev, rho_min, X, lo, hi, cfg.seed,
-                            gen_base, (uint32_t)gen_offset, U[0], s));
+        SPEO_TRY(pick_regen(isl_dev, srows_dev, Q, Ce, pred, drawn, rho_dev, rho_min, X, lo, hi, cfg.seed,
+                            gen_base, (uint32_t)gen_offset, U[0], ar, s));
     }
-    SPEO_TRY(launch(kModeEval, gen_offset, rt, s));
-    SurrHeads h{};
-    for (size_t p = 0; p < surr.size(); ++p) {
-        h.qoff[p] = surr[p]->qoff;
-        h.rows[p] = surr[p]->rows;
-    }
-    SPEO_TRY(archive_append(isl_dev, srows_dev, Q, U[0], fU[0], AX, Ay, cfg.surrogate_archive, Kp,
-                            h, (int)surr.size(), heads_dev, s));
     for (auto &sp : surr) {  // host copies of the device heads
         sp->head = (int)(((int64_t)sp->head + sp->rows) % cfg.surrogate_archive);
         sp->appended += sp->rows;
     }
+    // up to 128 columns the evaluation appends and selects as well
+    if (all_small) return launch(kModeEval, gen_offset, rt, s, 0, true);
+    SPEO_TRY(launch(kModeEval, gen_offset, rt, s));
+    SPEO_TRY(archive_append(isl_dev, srows_dev, Q, U[0], fU[0], AX, Ay, Kp, ar, s));
     return launch(kModeSelect, gen_offset, rt, s);
 }
 
@@ -1177,7 +1220,7 @@ int Engine::surrogate_train(hipStream_t s) {
     return check_launch("k_add_u32");
 }
 
-int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) {
+int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear, bool append) {
     GenerationArgs a{};
     a.isl = isl_dev;
     a.tiles = tiles_dev[rt_];
@@ -1199,6 +1242,10 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear) 
         if (!all_small) return eval_wide_rows(U[0], fU[0], rt_, s);
         a.eval_src = U[0];
         a.eval_out = fU[0];
+        if (append) {
+            a.fX_new = fX[0];
+            a.append = AppendArgs{AX, Ay, qrel_dev, heads_dev, cfg.surrogate_archive, Kp};
+        }
         break;
     case kModeSelect:
         if (cfg.mode == SPEO_MODE_FUSED) {  // apply the pending selection
@@ -1389,7 +1436,7 @@ int Engine::enqueue_chunk(int L, bool do_migrate, hipStream_t s) {
         SPEO_TRY(enqueue_plain(L, s));
     } else {
         for (int g = 0; g < L; ++g) {
-            if (donor_buf && g % donor_gens == 0) SPEO_TRY(draw_ahead(g, std::min(donor_gens, L - g), s));
+            if (C == 0 && donor_buf && g % donor_gens == 0) SPEO_TRY(draw_ahead(g, std::min(donor_gens, L - g), s));
             if (C > 0) {
                 SPEO_TRY(surrogate_generation(g, s));
             } else if (cfg.mode == SPEO_MODE_FUSED) {

@@ -102,9 +102,17 @@ struct IslandDesc;
 int gen_candidates(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C, const float *X,
                    float lo, float hi, uint64_t seed, const uint32_t *gen_base,
                    uint32_t gen_offset, float *cand, int Kp, hipStream_t s);
+// The archive's next slots: the picks advance head_dev[p] past the slots of the
+// previous generation (by the problem's rows, modulo cap), the appends of the
+// same generation read it.
+struct SurrArchive {
+    SurrHeads heads;
+    int problems, cap;
+    int *head_dev;
+};
 int pick_candidates(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C,
                     const float *cand, int Kp, const float *pred, const float *rho,
-                    float rho_min, float *U, hipStream_t s);
+                    float rho_min, float *U, const SurrArchive &ar, hipStream_t s);
 // Per-problem networks of one fused screening launch.
 struct CandInferBatch {
     const uint16_t *W1b[kMaxSurrProblems], *W2b[kMaxSurrProblems];
@@ -117,26 +125,28 @@ struct CandInferBatch {
     float rho_min;
     long long *scored;  // candidates scored per problem (device, accumulated)
     int tiles;          // 64-candidate tiles of all problems
+    int dim, ng;        // D, ceil(D / 4)
+    uint32_t inv_ng;    // group_inverse(D)
+    int4 *drawn;        // [q C + c] donors and j_rand of the scored candidates
 };
 // gen_candidates for every problem's targets [qoff[k], qoff[k] + nq[k]) and
 // each problem's network on them, in one kernel that never stores the
 // candidates: pred[q C + c], Kp <= 128.  A problem whose rho (device) is not
 // at least rho_min is skipped on the device (its pick is candidate 0 without
-// scores); scored[problem] counts the candidates scored.
+// scores); scored[problem] counts the candidates scored.  drawn[q C + c]: the
+// scored candidates' donors and j_rand, for pick_regen.
 int cand_infer(Mlp *const *nets, const int *qoff, const int *nq, const int *prob, int nn,
                const IslandDesc *isl, const SurrRowDesc *rows, int C, const float *X, float lo,
                float hi, uint64_t seed, const uint32_t *gen_base, uint32_t gen_offset,
-               const float *rho, float rho_min, long long *scored, float *pred, hipStream_t s);
+               const float *rho, float rho_min, long long *scored, float *pred, int4 *drawn, hipStream_t s);
 // pick_candidates with the chosen candidate generated again into U.
-int pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C, const float *pred,
+int pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C, const float *pred, const int4 *drawn,
                const float *rho, float rho_min, const float *X, float lo, float hi, uint64_t seed,
-               const uint32_t *gen_base, uint32_t gen_offset, float *U, hipStream_t s);
-// Appends every target's trial and log(1 + f) at its problem's next archive
-// slots (head_dev[p] on the device), then advances head_dev[p] by the
-// problem's rows modulo cap.
+               const uint32_t *gen_base, uint32_t gen_offset, float *U, const SurrArchive &ar, hipStream_t s);
+// Appends every target's trial and log(1 + f) at its problem's archive slots
+// (head_dev[p] on the device).
 int archive_append(const IslandDesc *isl, const SurrRowDesc *rows, int Q, const float *U,
-                   const float *fU, float *AX, float *Ay, int cap, int Kp, SurrHeads heads,
-                   int nproblems, int *head_dev, hipStream_t s);
+                   const float *fU, float *AX, float *Ay, int Kp, const SurrArchive &ar, hipStream_t s);
 // *p += v (one thread; also inside captured graphs).
 int add_i32(int *p, int v, hipStream_t s);
 int gather_batch(const float *AX, const float *Ay, int n_valid, int Kp, uint64_t seed,

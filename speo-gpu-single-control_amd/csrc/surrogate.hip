@@ -15,6 +15,8 @@
 
 namespace speo {
 
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+
 enum { kEpiStore = 0, kEpiBiasSilu = 1, kEpiMulDsilu = 2 };
 
 struct GemmArgs {
@@ -159,8 +161,7 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) h[q] = to_bits((elem_ok(gr, gk, q) ? v[i][q] : 0.f) * scale, false);
             if (kfast) {
-                typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-                *reinterpret_cast<u16x4 *>(&dst[r * LDK + k]) = u16x4{h[0], h[1], h[2], h[3]};
+                            *reinterpret_cast<u16x4 *>(&dst[r * LDK + k]) = u16x4{h[0], h[1], h[2], h[3]};
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) dst[(r + q) * LDK + k] = h[q];
@@ -354,13 +355,17 @@ __global__ void k_sum(const float *v, int n, float *out) {
 // Adam with bias correction (Kingma & Ba, 2015) on parameter i with gradient
 // g; c1 = 1 - 0.9^t, c2 = 1 - 0.999^t.  Returns the new value.  Shared by
 // k_adam and the fused training step, so both give the same bits.
+__device__ __forceinline__ void adam_values(float &p, float &m, float &v, float g, float lr, float c1, float c2) {
+    m = fmaf(0.1f, g, 0.9f * m);  // (written out: the same contraction in every caller)
+    v = fmaf(0.001f * g, g, 0.999f * v);
+    p = p - lr * (m / c1) / (sqrtf(v / c2) + 1e-8f);
+}
 __device__ __forceinline__ float adam_update(float *P, float *m, float *v, size_t i, float g,
                                              float lr, float c1, float c2) {
-    const float mi = 0.9f * m[i] + 0.1f * g;
-    const float vi = 0.999f * v[i] + 0.001f * g * g;
+    float p = P[i], mi = m[i], vi = v[i];
+    adam_values(p, mi, vi, g, lr, c1, c2);
     m[i] = mi;
     v[i] = vi;
-    const float p = P[i] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
     P[i] = p;
     return p;
 }
@@ -672,7 +677,6 @@ __global__ __launch_bounds__(1024) void k_mlp_infer(const float *X, int ld, int 
     const int row0 = blockIdx.x * TM;
     MlpFrags<KP> f;
     mlp_prefetch<KP>(f, W1b, b1, W2b, b2, w3, b3);
-    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
     if ((ld & 3) == 0 && ld >= KP && (reinterpret_cast<uintptr_t>(X) & 15) == 0) {
         // 16-byte loads, all of the tile issued before the first is converted
         constexpr int G = (TM * KP / 4 + 1023) / 1024;
@@ -767,7 +771,10 @@ struct TrainRowsArgs {
 // tiles).  A wave's weight fragments (W1, W2 and W2^T for its columns, 20
 // 16-byte loads per lane) are all issued at the start, so the kernel waits
 // on one L2 round trip for them instead of one per K step.  Rows >= n are
-// zero inputs with dy = 0, so they add nothing to any gradient.
+// zero inputs with dy = 0, so they add nothing to any gradient.  Latency bound
+// (32 blocks a network): the rows' slots are drawn by every thread that gathers
+// them, and the transposed operands are stored from registers (15.3 us a step of
+// two networks with a shared draw and LDS transposes, 13.5 now).
 // Networks trained in one launch (one per problem), each a run of blocks.
 constexpr int kMaxTrainNets = 8;
 struct TrainRowsBatch {
@@ -783,10 +790,8 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
     __shared__ __align__(16) uint16_t Xs[TM * LX];
     __shared__ __align__(16) uint16_t Hs[TM * LH];  // H1
     __shared__ __align__(16) uint16_t Gs[TM * LH];  // dH2
-    __shared__ __align__(16) uint16_t Ds[TM * LH];  // dH1
     __shared__ float red[NW][TM];
     __shared__ float ts[TM], dys[TM], lts[TM];
-    __shared__ int slots[TM];
     const int tile = blockIdx.x % batch.tiles;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lk = lane >> 4;
@@ -804,10 +809,13 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
         w2t[ks] = *reinterpret_cast<const bf16x8 *>(&a.W2Tb[((size_t)(wave * K2 + ks) * 64 + lane) * 8]);
     }
     const float bias1 = a.b1[col], bias2 = a.b2[col], wout = a.w3[col], bias3 = a.b3[0];
-    if (tid < TM) {
-        const int b = row0 + tid;
+    {
+        // thread (row r, columns 4 c4 .. + 3): every thread of a row draws the
+        // row's slot, so the gather waits for no one; the row's first thread
+        // also fetches its target
+        const int r = tid >> 5, c4 = tid & 31, b = row0 + r;
         int slot = b;
-        float t = 0.f;
+        float t = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
         if (b < a.n) {
             if (a.AX) {  // the slot gather_batch draws for row b
                 const uint32_t round = a.round_dev ? *a.round_dev : a.round;
@@ -815,45 +823,28 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
                 slot = (int)(u01(word(w, (uint32_t)(b & 3))) * (float)a.n_valid);
                 slot = slot >= a.n_valid ? a.n_valid - 1 : slot;
                 if (slot % 8 == 7) slot -= 1;
-                t = a.Ay[slot];
-            } else {
-                t = a.t[b];
             }
-            t = (t - a.stats[1]) / a.stats[2];
+            if (c4 == 0) t = a.AX ? a.Ay[slot] : a.t[b];
+            if (4 * c4 < KP) {
+                const float *src = (a.AX ? a.AX + (size_t)slot * KP : a.X + (size_t)b * a.ld) + 4 * c4;
+                if (a.AX && (reinterpret_cast<uintptr_t>(a.AX) & 15) == 0) {
+                    const floatx4 v = *reinterpret_cast<const floatx4 *>(src);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = 4 * c4 + e < a.D ? v[e] : 0.f;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = 4 * c4 + e < a.D ? src[e] : 0.f;
+                }
+            }
+            if (c4 == 0) t = (t - a.stats[1]) / a.stats[2];
         }
-        slots[tid] = slot;
-        ts[tid] = t;
+        if (c4 == 0) ts[r] = t;
+        if (4 * c4 < KP)
+            *reinterpret_cast<u16x4 *>(&Xs[r * LX + 4 * c4]) =
+                u16x4{to_bits(x[0] * kXScale, false), to_bits(x[1] * kXScale, false),
+                      to_bits(x[2] * kXScale, false), to_bits(x[3] * kXScale, false)};
     }
     __syncthreads();
-    {
-        const float *src = a.AX ? a.AX : a.X;
-        const size_t ld = a.AX ? (size_t)KP : (size_t)a.ld;
-        constexpr int G = TM * KP / 1024;
-        float x[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int e = tid + g * 1024, r = e / KP, k = e % KP;
-            x[g] = (row0 + r < a.n && k < a.D) ? src[(size_t)slots[r] * ld + k] : 0.f;
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int e = tid + g * 1024, r = e / KP, k = e % KP;
-            Xs[r * LX + k] = to_bits(x[g] * kXScale, false);
-        }
-    }
-    __syncthreads();
-    // transposed copy of a [TM][stride] BF16 tile: element (c, row0 + r) of
-    // T, a [ncols][Bp] matrix as B-fragment operand (k = minibatch row), in
-    // fragment order (frag_index), 8 consecutive rows per 16-byte store
-    auto store_t = [&](const uint16_t *S, int stride, int ncols, uint16_t *T) __attribute__((always_inline)) {
-        for (int e = tid; e < ncols * (TM / 8); e += 1024) {
-            const int c = e / (TM / 8), r8 = (e % (TM / 8)) * 8;
-            u16x8 v;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = S[(r8 + u) * stride + c];
-            *reinterpret_cast<u16x8 *>(T + frag_index(c, row0 + r8, a.Bp / 32)) = v;
-        }
-    };
     floatx4 acc[2];
     // layer 1
     acc[0] = acc[1] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -865,6 +856,10 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 *reinterpret_cast<const bf16x8 *>(&Xs[(i * 16 + lr) * LX + kb]), w1[ks], acc[i], 0, 0, 0);
     }
+    // A lane holds four consecutive rows of its column: 8 bytes of the
+    // transposed operand's fragment, kept until the end (a barrier would wait
+    // for the stores).
+    u16x4 h1t[2], g2t[2], g1t[2];
     float d1[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -872,7 +867,8 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
         for (int q = 0; q < 4; ++q) {
             const float pre = acc[i][q] + bias1;
             d1[i][q] = dsiluf_(pre);
-            Hs[(i * 16 + lk * 4 + q) * LH + col] = to_bits(siluf_(pre), false);
+            h1t[i][q] = to_bits(siluf_(pre), false);
+            Hs[(i * 16 + lk * 4 + q) * LH + col] = h1t[i][q];
         }
     __syncthreads();
     // layer 2
@@ -923,7 +919,8 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
                 const int r = i * 16 + lk * 4 + q;
                 const float dy = dys[r];
                 const float g = dy * wout * d2[i][q];
-                Gs[r * LH + col] = to_bits(g, false);
+                g2t[i][q] = to_bits(g, false);
+                Gs[r * LH + col] = g2t[i][q];
                 pb2 += g;
                 pw3 = fmaf(h2[i][q], dy, pw3);
             }
@@ -965,20 +962,30 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float g = acc[i][q] * d1[i][q];
-                Ds[(i * 16 + lk * 4 + q) * LH + col] = to_bits(g, false);
+                g1t[i][q] = to_bits(g, false);
                 pb1 += g;
             }
         pb1 += __shfl_xor(pb1, 16, 64);
         pb1 += __shfl_xor(pb1, 32, 64);
         if (lk == 0) part[col] = pb1;
     }
-    __syncthreads();
-    // the four transposed activation tiles, stored last so that no barrier
-    // above waits for them
-    store_t(Xs, LX, KP, a.XT);
-    store_t(Hs, LH, kHidden, a.H1T);
-    store_t(Gs, LH, kHidden, a.dH2T);
-    store_t(Ds, LH, kHidden, a.dH1T);
+    // the transposed operands, element (c, row0 + r) of [ncols][Bp] matrices in
+    // fragment order (frag_index, k = minibatch row)
+    const int kbs = a.Bp / 32;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const size_t at = frag_index(col, row0 + i * 16 + lk * 4, kbs);
+        *reinterpret_cast<u16x4 *>(a.H1T + at) = h1t[i];
+        *reinterpret_cast<u16x4 *>(a.dH2T + at) = g2t[i];
+        *reinterpret_cast<u16x4 *>(a.dH1T + at) = g1t[i];
+    }
+    for (int e = tid; e < KP * (TM / 8); e += 1024) {
+        const int c = e / (TM / 8), r8 = (e % (TM / 8)) * 8;
+        u16x8 v;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = Xs[(r8 + u) * LX + c];
+        *reinterpret_cast<u16x8 *>(a.XT + frag_index(c, row0 + r8, kbs)) = v;
+    }
 }
 
 struct TrainUpdateArgs {
@@ -1002,7 +1009,9 @@ struct TrainUpdateArgs {
 // row tiles' partial sums (in tile order).  A GEMM block's four waves take
 // every fourth 32-row step of the minibatch, and their 32 x 32 results are
 // added in wave order.  Each block then writes the gradient and/or applies
-// Adam to its parameters and refreshes their BF16 copies.
+// Adam to its parameters, requested before the GEMM, and refreshes their BF16
+// copies (8.4 us for two networks of D = 100, 8.9 with the parameters read
+// after it).
 struct TrainUpdateBatch {
     TrainUpdateArgs net[kMaxTrainNets];
     int blocks;  // blocks per network
@@ -1011,7 +1020,6 @@ struct TrainUpdateBatch {
 __global__ __launch_bounds__(256) void k_train_update(TrainUpdateBatch batch) {
     const TrainUpdateArgs &a = batch.net[blockIdx.x / batch.blocks];
     float c1 = 1.f, c2 = 1.f;
-    if (a.adam) adam_corrections(*a.t_dev + a.t_off + 1, c1, c2);
     __shared__ float red[4][32][33];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lk = lane >> 4;
@@ -1039,6 +1047,7 @@ __global__ __launch_bounds__(256) void k_train_update(TrainUpdateBatch batch) {
                     g3 += v3[u];
                 }
         }
+        if (a.adam) adam_corrections(*a.t_dev + a.t_off + 1, c1, c2);
         const size_t o1 = a.L.ob1 + c, o2 = a.L.ob2 + c, o3 = a.L.ow3 + c;
         if (a.G) {
             a.G[o1] = g1;
@@ -1078,6 +1087,17 @@ __global__ __launch_bounds__(256) void k_train_update(TrainUpdateBatch batch) {
     const int i0 = (t / ncolt) * 32, j0 = (t % ncolt) * 32;
     const uint16_t *A = w2 ? a.dH2T : a.dH1T;
     const uint16_t *B = w2 ? a.H1T : a.XT;
+    // this thread's four parameters (16-byte aligned: Kp is a multiple of 32),
+    // requested before the GEMM that their update waits for
+    const int mr = tid >> 3, nc0 = (tid & 7) * 4, I = i0 + mr, J0 = j0 + nc0;
+    const size_t off = w2 ? a.L.oW2 + (size_t)I * kHidden + J0 : a.L.oW1 + (size_t)I * a.L.Kp + J0;
+    floatx4 pv{}, mv{}, vv{};
+    if (a.adam) {
+        pv = *reinterpret_cast<const floatx4 *>(a.P + off);
+        mv = *reinterpret_cast<const floatx4 *>(a.m + off);
+        vv = *reinterpret_cast<const floatx4 *>(a.v + off);
+        adam_corrections(*a.t_dev + a.t_off + 1, c1, c2);
+    }
     floatx4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -1115,23 +1135,32 @@ __global__ __launch_bounds__(256) void k_train_update(TrainUpdateBatch batch) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) red[wave][i * 16 + lk * 4 + q][j * 16 + lr] = acc[i][j][q];
     __syncthreads();
-    const int mr = tid >> 3;
+    floatx4 gv;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int nc = (tid & 7) * 4 + e;
-        const float g = ((red[0][mr][nc] + red[1][mr][nc]) + red[2][mr][nc]) + red[3][mr][nc];
-        const int I = i0 + mr, J = j0 + nc;
-        const size_t off = w2 ? a.L.oW2 + (size_t)I * kHidden + J : a.L.oW1 + (size_t)I * a.L.Kp + J;
-        if (a.G) a.G[off] = g;
-        if (a.adam) {
-            const float p = adam_update(a.P, a.m, a.v, off, g, a.lr, c1, c2);
-            const uint16_t h = to_bits(p, false);
-            if (w2) {
-                a.W2b[frag_index(I, J, kHidden / 32)] = h;
-                a.W2Tb[frag_index(J, I, kHidden / 32)] = h;
-            } else {
-                a.W1b[frag_index(I, J, a.L.Kp / 32)] = h;
-            }
+    for (int e = 0; e < 4; ++e)
+        gv[e] = ((red[0][mr][nc0 + e] + red[1][mr][nc0 + e]) + red[2][mr][nc0 + e]) + red[3][mr][nc0 + e];
+    if (a.G) *reinterpret_cast<floatx4 *>(a.G + off) = gv;
+    if (a.adam) {
+        u16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float p = pv[e], m = mv[e], v = vv[e];
+            adam_values(p, m, v, gv[e], a.lr, c1, c2);
+            pv[e] = p;
+            mv[e] = m;
+            vv[e] = v;
+            h[e] = to_bits(p, false);
+        }
+        *reinterpret_cast<floatx4 *>(a.P + off) = pv;
+        *reinterpret_cast<floatx4 *>(a.m + off) = mv;
+        *reinterpret_cast<floatx4 *>(a.v + off) = vv;
+        // four consecutive K of one row: 8 bytes of its fragment
+        if (w2) {
+            *reinterpret_cast<u16x4 *>(a.W2b + frag_index(I, J0, kHidden / 32)) = h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a.W2Tb[frag_index(J0 + e, I, kHidden / 32)] = h[e];
+        } else {
+            *reinterpret_cast<u16x4 *>(a.W1b + frag_index(I, J0, a.L.Kp / 32)) = h;
         }
     }
 }
@@ -1362,19 +1391,23 @@ struct CandSrc {
     uint32_t pc, gr, gen;
 };
 
-__device__ __forceinline__ CandSrc cand_src(const IslandDesc &I, const SurrRowDesc &rd, int c,
-                                            const float *X, uint64_t seed, uint32_t gen) {
+__device__ __forceinline__ int4 cand_draw(const IslandDesc &I, int gr, int c, uint64_t seed, uint32_t gen) {
     const uint32_t pd = c == 0 ? (uint32_t)kPurposeDonor : (uint32_t)(kPurposeCandidate + 2 * c);
-    DonorStream ds(seed, (uint32_t)rd.gr, gen, pd);
+    DonorStream ds(seed, (uint32_t)gr, gen, pd);
     int r[kMaxR], jr;
     draw_donors(ds, nullptr, 0, I.np, I.dim, r, jr);
+    return int4{r[0], r[1], r[2], jr};
+}
+
+__device__ __forceinline__ CandSrc cand_src(const IslandDesc &I, const SurrRowDesc &rd, int c, const int4 &d,
+                                            const float *X, uint32_t gen) {
     const float *base = X + I.elem_off;
     CandSrc cs;
-    cs.p0 = base + (size_t)r[0] * I.ld;
-    cs.p1 = base + (size_t)r[1] * I.ld;
-    cs.p2 = base + (size_t)r[2] * I.ld;
+    cs.p0 = base + (size_t)d.x * I.ld;
+    cs.p1 = base + (size_t)d.y * I.ld;
+    cs.p2 = base + (size_t)d.z * I.ld;
     cs.own = base + (size_t)rd.li * I.ld;
-    cs.jr = jr;
+    cs.jr = d.w;
     cs.dim = I.dim;
     cs.F = I.F;
     cs.CR = I.CR;
@@ -1385,13 +1418,17 @@ __device__ __forceinline__ CandSrc cand_src(const IslandDesc &I, const SurrRowDe
 }
 
 // Coordinates 4g .. 4g + 3 of the candidate (0 past the dimension).
-__device__ __forceinline__ float4 cand_group(const CandSrc &cs, int g, uint64_t seed, float lo,
-                                             float hi) {
+struct CandRows {
+    float4 e0, e1, e2, xo;
+};
+__device__ __forceinline__ CandRows cand_load(const CandSrc &cs, int g) {
+    return CandRows{ld4s(cs.p0 + 4 * g), ld4s(cs.p1 + 4 * g), ld4s(cs.p2 + 4 * g), ld4s(cs.own + 4 * g)};
+}
+__device__ __forceinline__ float4 cand_make(const CandSrc &cs, int g, const CandRows &x, uint64_t seed, float lo,
+                                            float hi) {
 #pragma clang fp contract(off)
-    if (4 * g >= cs.dim) return float4{0.f, 0.f, 0.f, 0.f};
     const U4 w = philox_block(seed, (uint32_t)g, cs.gr, cs.gen, cs.pc);
-    const float4 e0 = ld4s(cs.p0 + 4 * g), e1 = ld4s(cs.p1 + 4 * g), e2 = ld4s(cs.p2 + 4 * g);
-    const float4 xo = ld4s(cs.own + 4 * g);
+    const float4 &e0 = x.e0, &e1 = x.e1, &e2 = x.e2, &xo = x.xo;
     float v[4];
 #pragma unroll
     for (int qq = 0; qq < 4; ++qq) {
@@ -1405,6 +1442,10 @@ __device__ __forceinline__ float4 cand_group(const CandSrc &cs, int g, uint64_t 
         }
     }
     return float4{v[0], v[1], v[2], v[3]};
+}
+__device__ __forceinline__ float4 cand_group(const CandSrc &cs, int g, uint64_t seed, float lo, float hi) {
+    if (4 * g >= cs.dim) return float4{0.f, 0.f, 0.f, 0.f};
+    return cand_make(cs, g, cand_load(cs, g), seed, lo, hi);
 }
 
 // 16 lanes per (target q, candidate c): the candidate's Kp columns.
@@ -1420,22 +1461,34 @@ __global__ __launch_bounds__(256) void k_gen_candidates(const IslandDesc *isl,
     const SurrRowDesc rd = rows[q];
     const IslandDesc I = isl[rd.island];
     const uint32_t gen = (gen_base ? *gen_base : 0u) + gen_offset;
-    const CandSrc cs = cand_src(I, rd, c, X, seed, gen);
+    const CandSrc cs = cand_src(I, rd, c, cand_draw(I, rd.gr, c, seed, gen), X, gen);
     float *out = cand + (size_t)item * Kp;
     for (int g = l; g < (Kp >> 2); g += 16)
         *reinterpret_cast<float4 *>(out + 4 * g) = cand_group(cs, g, seed, lo, hi);
 }
 
 // The candidates of each problem's targets generated straight into LDS (64
-// per tile, 16 lanes per candidate) and scored by that problem's network
-// (mlp_tile64): the same predictions as k_gen_candidates followed by
-// k_mlp_infer, without writing the candidates to memory.  All problems in one
-// launch: problem k owns tiles [first[k], first[k + 1]).  One block per CU
-// walks the tiles (b, b + grid, ...), so a wave loads its weight fragments
-// once per problem instead of once per 64 candidates.  mlp_tile64 reads Xs
-// before its first barrier and Hs before its second, and the next tile's
-// candidates are written after both, so the tiles need no barrier between
-// them.
+// per tile) and scored by that problem's network (mlp_tile64): the same
+// predictions as k_gen_candidates followed by k_mlp_infer, without writing the
+// candidates to memory.  All problems in one launch: problem k owns tiles
+// [first[k], first[k + 1]).  One block per CU walks the tiles (b, b + grid,
+// ...), so a wave loads its weight fragments once per problem instead of once
+// per 64 candidates.  mlp_tile64 reads Xs before its first barrier and Hs
+// before its second, and the next tile's candidates are written after both, so
+// the tiles need no barrier between them.
+// The donors of up to 16 of the block's tiles are drawn at once, one candidate
+// per thread (16 lanes a candidate, each repeating the draw, spent a third of
+// the kernel on it), and the candidates are made as items of a candidate and
+// four coordinates spread over all lanes.  8,192 targets x 8 candidates,
+// D = 100: 61 us before, 49 us.
+struct CandLds {
+    const float *p[4];  // donor rows and the target's row
+    int jr, c;
+    uint32_t gr;
+    float F, CR;
+};
+constexpr int kCandChunk = 16;  // tiles drawn at once: one candidate per thread
+
 template <int KP>
 __global__ __launch_bounds__(1024) void k_cand_infer(CandInferBatch B, const IslandDesc *isl,
                                                      const SurrRowDesc *rows, int C, const float *X,
@@ -1446,40 +1499,70 @@ __global__ __launch_bounds__(1024) void k_cand_infer(CandInferBatch B, const Isl
     __shared__ __align__(16) uint16_t Xs[TM * LX];
     __shared__ __align__(16) uint16_t Hs[TM * LH];
     __shared__ float red[kHidden / 16][TM];
-    const int r = threadIdx.x >> 4, l = threadIdx.x & 15;  // candidate r of the tile, lane l
+    __shared__ CandLds cands[kCandChunk * TM];
+    const int tid = threadIdx.x, ng = B.ng;
     const uint32_t gen = (gen_base ? *gen_base : 0u) + gen_offset;
-    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-    MlpFrags<KP> f;
-    int kf = -1;  // the network whose fragments f holds
-    for (int tile = blockIdx.x; tile < B.tiles; tile += gridDim.x) {
+    auto net_of = [&](int tile) {
         int k = 0;
         while (k + 1 < B.nnets && tile >= B.first[k + 1]) ++k;
-        // a problem below the rho threshold picks candidate 0 without scores
-        // (every thread reads the same rho, so the whole block skips the tile)
-        if (!(B.rho[B.prob[k]] >= B.rho_min)) continue;
-        if (threadIdx.x == 0 && tile == B.first[k]) B.scored[B.prob[k]] += (long long)B.nq[k] * C;
-        const int qoff = B.qoff[k], n = B.nq[k] * C;
+        return k;
+    };
+    // a problem below the rho threshold picks candidate 0 without scores (every
+    // thread reads the same rho, so the whole block skips the tile)
+    auto scored = [&](int k) { return B.rho[B.prob[k]] >= B.rho_min; };
+    // columns past the dimension are zero in every tile
+    for (int e = tid; e < TM * (KP / 4 - ng); e += 1024) {
+        const int r = e / (KP / 4 - ng), g = ng + e - r * (KP / 4 - ng);
+        *reinterpret_cast<u16x4 *>(&Xs[r * LX + 4 * g]) = u16x4{0, 0, 0, 0};
+    }
+    MlpFrags<KP> f;
+    int kf = -1;  // the network whose fragments f holds
+    for (int i = 0, tile = blockIdx.x; tile < B.tiles; ++i, tile += gridDim.x) {
+        if (i % kCandChunk == 0) {
+            // wave w draws for the block's tile i + w
+            const int mine = tile + (tid >> 6) * (int)gridDim.x;
+            if (i > 0) __syncthreads();
+            if (mine < B.tiles) {
+                const int k = net_of(mine), item = (mine - B.first[k]) * TM + (tid & 63);
+                if (scored(k) && item < B.nq[k] * C) {
+                    const int q = B.qoff[k] + item / C, c = item % C;
+                    const SurrRowDesc rd = rows[q];
+                    const IslandDesc I = isl[rd.island];
+                    const int4 d = cand_draw(I, rd.gr, c, seed, gen);
+                    B.drawn[(size_t)q * C + c] = d;
+                    const CandSrc cs = cand_src(I, rd, c, d, X, gen);
+                    cands[tid] = CandLds{{cs.p0, cs.p1, cs.p2, cs.own}, cs.jr, c, cs.gr, cs.F, cs.CR};
+                }
+            }
+            __syncthreads();
+        }
+        const int k = net_of(tile);
+        if (!scored(k)) continue;
+        if (tid == 0 && tile == B.first[k]) B.scored[B.prob[k]] += (long long)B.nq[k] * C;
+        const int n = B.nq[k] * C;
         if (k != kf) {
             const float *P = B.P[k];
             mlp_prefetch<KP>(f, B.W1b[k], P + B.ob1, B.W2b[k], P + B.ob2, P + B.ow3, P + B.ob3);
             kf = k;
         }
-        const int item0 = (tile - B.first[k]) * TM, item = item0 + r;
-        if (item < n) {
-            const SurrRowDesc rd = rows[qoff + item / C];
-            const CandSrc cs = cand_src(isl[rd.island], rd, item % C, X, seed, gen);
-            for (int g = l; g < KP / 4; g += 16) {
-                const float4 v = cand_group(cs, g, seed, lo, hi);
-                *reinterpret_cast<u16x4 *>(&Xs[r * LX + 4 * g]) =
-                    u16x4{to_bits(v.x * kXScale, false), to_bits(v.y * kXScale, false),
-                          to_bits(v.z * kXScale, false), to_bits(v.w * kXScale, false)};
-            }
-        } else {
-            for (int g = l; g < KP / 4; g += 16)
-                *reinterpret_cast<u16x4 *>(&Xs[r * LX + 4 * g]) = u16x4{0, 0, 0, 0};
+        const int item0 = (tile - B.first[k]) * TM, items = min(TM, n - item0) * ng;
+        const CandLds *cl = cands + (i % kCandChunk) * TM;
+        // items of a candidate and four coordinates; rows past the tile's keep
+        // what they hold
+#pragma unroll 1
+        for (int e = tid; e < items; e += 1024) {
+            const int r = B.inv_ng ? (int)__umulhi((uint32_t)e, B.inv_ng) : e, g = e - r * ng;
+            const CandLds &c = cl[r];
+            const CandSrc cs{c.p[0], c.p[1], c.p[2], c.p[3], c.jr, B.dim, c.F, c.CR,
+                             c.c == 0 ? (uint32_t)kPurposeCross : (uint32_t)(kPurposeCandidate + 2 * c.c + 1),
+                             c.gr, gen};
+            const float4 v = cand_make(cs, g, cand_load(cs, g), seed, lo, hi);
+            *reinterpret_cast<u16x4 *>(&Xs[r * LX + 4 * g]) =
+                u16x4{to_bits(v.x * kXScale, false), to_bits(v.y * kXScale, false),
+                      to_bits(v.z * kXScale, false), to_bits(v.w * kXScale, false)};
         }
         __syncthreads();
-        mlp_tile64<KP>(Xs, Hs, red, f, n - item0, pred + (size_t)qoff * C + item0);
+        mlp_tile64<KP>(Xs, Hs, red, f, n - item0, pred + (size_t)B.qoff[k] * C + item0);
     }
 }
 
@@ -1502,7 +1585,7 @@ static int cand_infer_blocks() {
 int cand_infer(Mlp *const *nets, const int *qoff, const int *nq, const int *prob, int nn,
                const IslandDesc *isl, const SurrRowDesc *rows, int C, const float *X, float lo,
                float hi, uint64_t seed, const uint32_t *gen_base, uint32_t gen_offset,
-               const float *rho, float rho_min, long long *scored, float *pred, hipStream_t s) {
+               const float *rho, float rho_min, long long *scored, float *pred, int4 *drawn, hipStream_t s) {
     if (nn < 1 || nn > kMaxSurrProblems) return set_error(SPEO_ERR_ARG, "cand_infer: 1..16 problems");
     CandInferBatch B{};
     B.nnets = nn;
@@ -1531,6 +1614,10 @@ int cand_infer(Mlp *const *nets, const int *qoff, const int *nq, const int *prob
     B.scored = scored;
     if (blocks == 0) return SPEO_OK;
     B.tiles = blocks;
+    B.dim = L.D;
+    B.ng = (L.D + 3) / 4;
+    B.inv_ng = group_inverse(L.D);
+    B.drawn = drawn;
     const dim3 grid(std::min(blocks, cand_infer_blocks())), block(1024);
 #define SPEO_CAND_INFER(KP)                                                                          \
     hipLaunchKernelGGL(k_cand_infer<KP>, grid, block, 0, s, B, isl, rows, C, X, lo, hi, seed, gen_base, \
@@ -1560,7 +1647,9 @@ int gen_candidates(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C,
 // active, else candidate 0; copied into the target's trial row of U.
 __global__ void k_pick_candidates(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C,
                                   const float *cand, int Kp, const float *pred, const float *rho,
-                                  float rho_min, float *U) {
+                                  float rho_min, float *U, SurrArchive ar) {
+    if (blockIdx.x == 0 && threadIdx.x < ar.problems)
+        ar.head_dev[threadIdx.x] = (int)(((int64_t)ar.head_dev[threadIdx.x] + ar.heads.rows[threadIdx.x]) % ar.cap);
     const int q = blockIdx.x * 16 + (threadIdx.x >> 4);
     const int l = threadIdx.x & 15;
     if (q >= Q) return;
@@ -1586,16 +1675,19 @@ __global__ void k_pick_candidates(const IslandDesc *isl, const SurrRowDesc *rows
 // The same pick, the chosen candidate generated again into U instead of
 // copied (its coordinates are a function of the counters and X only).
 __global__ void k_pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C,
-                             const float *pred, const float *rho, float rho_min, const float *X,
-                             float lo, float hi, uint64_t seed, const uint32_t *gen_base,
-                             uint32_t gen_offset, float *U) {
+                             const float *pred, const int4 *drawn, const float *rho, float rho_min,
+                             const float *X, float lo, float hi, uint64_t seed, const uint32_t *gen_base,
+                             uint32_t gen_offset, float *U, SurrArchive ar) {
+    if (blockIdx.x == 0 && threadIdx.x < ar.problems)
+        ar.head_dev[threadIdx.x] = (int)(((int64_t)ar.head_dev[threadIdx.x] + ar.heads.rows[threadIdx.x]) % ar.cap);
     const int q = blockIdx.x * 16 + (threadIdx.x >> 4);
     const int l = threadIdx.x & 15;
     if (q >= Q) return;
     const SurrRowDesc rd = rows[q];
     const IslandDesc I = isl[rd.island];
     int best = 0;
-    if (rho[rd.problem] >= rho_min) {
+    const bool active = rho[rd.problem] >= rho_min;
+    if (active) {
         float bv = pred[(size_t)q * C];
         for (int c = 1; c < C; ++c) {
             const float v = pred[(size_t)q * C + c];
@@ -1606,63 +1698,55 @@ __global__ void k_pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int
         }
     }
     const uint32_t gen = (gen_base ? *gen_base : 0u) + gen_offset;
-    const CandSrc cs = cand_src(I, rd, best, X, seed, gen);
+    const int4 d = active ? drawn[(size_t)q * C + best] : cand_draw(I, rd.gr, 0, seed, gen);
+    const CandSrc cs = cand_src(I, rd, best, d, X, gen);
     float *dst = U + I.elem_off + (size_t)rd.li * I.ld;
     for (int g = l; g < (I.ld >> 2); g += 16)
         *reinterpret_cast<float4 *>(dst + 4 * g) = cand_group(cs, g, seed, lo, hi);
 }
 
-int pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C, const float *pred,
+int pick_regen(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C, const float *pred, const int4 *drawn,
                const float *rho, float rho_min, const float *X, float lo, float hi, uint64_t seed,
-               const uint32_t *gen_base, uint32_t gen_offset, float *U, hipStream_t s) {
+               const uint32_t *gen_base, uint32_t gen_offset, float *U, const SurrArchive &ar, hipStream_t s) {
     if (Q <= 0) return SPEO_OK;
-    hipLaunchKernelGGL(k_pick_regen, dim3((Q + 15) / 16), dim3(256), 0, s, isl, rows, Q, C, pred,
-                       rho, rho_min, X, lo, hi, seed, gen_base, gen_offset, U);
+    hipLaunchKernelGGL(k_pick_regen, dim3((Q + 15) / 16), dim3(256), 0, s, isl, rows, Q, C, pred, drawn,
+                       rho, rho_min, X, lo, hi, seed, gen_base, gen_offset, U, ar);
     return check_launch("k_pick_regen");
 }
 
 int pick_candidates(const IslandDesc *isl, const SurrRowDesc *rows, int Q, int C,
                     const float *cand, int Kp, const float *pred, const float *rho,
-                    float rho_min, float *U, hipStream_t s) {
+                    float rho_min, float *U, const SurrArchive &ar, hipStream_t s) {
     if (Q <= 0) return SPEO_OK;
     hipLaunchKernelGGL(k_pick_candidates, dim3((Q + 15) / 16), dim3(256), 0, s, isl, rows, Q, C,
-                       cand, Kp, pred, rho, rho_min, U);
+                       cand, Kp, pred, rho, rho_min, U, ar);
     return check_launch("k_pick_candidates");
 }
 
 // Archive slot of target q: (head[p] + q - qoff[p]) % cap of its problem p;
 // x is stored with Kp columns (zero padded) and y = log(1 + f).
 __global__ void k_archive_append(const IslandDesc *isl, const SurrRowDesc *rows, int Q,
-                                 const float *U, const float *fU, float *AX, float *Ay, int cap,
-                                 int Kp, SurrHeads heads, const int *head_dev) {
+                                 const float *U, const float *fU, float *AX, float *Ay, int Kp,
+                                 SurrArchive ar) {
     const int q = blockIdx.x * 16 + (threadIdx.x >> 4);
     const int l = threadIdx.x & 15;
     if (q >= Q) return;
     const SurrRowDesc rd = rows[q];
     const IslandDesc I = isl[rd.island];
     const int p = rd.problem;
-    const int slot = (int)(((int64_t)head_dev[p] + q - heads.qoff[p]) % cap);
+    const int cap = ar.cap, slot = (int)(((int64_t)ar.head_dev[p] + q - ar.heads.qoff[p]) % cap);
     float *dst = AX + ((size_t)p * cap + slot) * Kp;
     const float *src = U + I.elem_off + (size_t)rd.li * I.ld;
     for (int j = l; j < Kp; j += 16) dst[j] = j < I.dim ? src[j] : 0.f;
     if (l == 0) Ay[(size_t)p * cap + slot] = log1pf(fmaxf(fU[rd.gr], 0.f));
 }
 
-__global__ void k_archive_advance(int *head_dev, SurrHeads heads, int nproblems, int cap) {
-    const int p = threadIdx.x;
-    if (p < nproblems) head_dev[p] = (int)(((int64_t)head_dev[p] + heads.rows[p]) % cap);
-}
-
 int archive_append(const IslandDesc *isl, const SurrRowDesc *rows, int Q, const float *U,
-                   const float *fU, float *AX, float *Ay, int cap, int Kp, SurrHeads heads,
-                   int nproblems, int *head_dev, hipStream_t s) {
+                   const float *fU, float *AX, float *Ay, int Kp, const SurrArchive &ar, hipStream_t s) {
     if (Q <= 0) return SPEO_OK;
     hipLaunchKernelGGL(k_archive_append, dim3((Q + 15) / 16), dim3(256), 0, s, isl, rows, Q, U, fU,
-                       AX, Ay, cap, Kp, heads, head_dev);
-    SPEO_TRY(check_launch("k_archive_append"));
-    hipLaunchKernelGGL(k_archive_advance, dim3(1), dim3(kMaxSurrProblems), 0, s, head_dev, heads,
-                       nproblems, cap);
-    return check_launch("k_archive_advance");
+                       AX, Ay, Kp, ar);
+    return check_launch("k_archive_append");
 }
 
 // Minibatch of the valid archive slots [0, n_valid), skipping the held-out
