@@ -30,6 +30,10 @@ struct GenArgs {
     int n_inj;
     const float *inj_cr;
     int *r_out, *jrand_out;
+    // set: each sub-island's best member (fit [n] over rows) is found first and
+    // stored in best_out, `best` is not read
+    const float *fit = nullptr;
+    int *best_out = nullptr;
 };
 
 // Sequential donor-phase draws of one row: draw k is word k%4 of Philox block
@@ -46,9 +50,13 @@ struct DonorStream {
         w1 = philox_block(s, 1u, r, g, pur);
     }
     __host__ __device__ __forceinline__ float next(const float *inj, int n_inj) {
-        const uint32_t kk = k++;
+        // (the words move up by one a draw, so that none is picked by an index
+        // the compiler would put in memory)
+        const uint32_t kk = k++, head = w0.x;
+        w0 = U4{w0.y, w0.z, w0.w, w1.x};
+        w1 = U4{w1.y, w1.z, w1.w, 0u};
         if (inj && (int)kk < n_inj) return inj[kk];
-        if (kk < 8u) return u01(word(kk < 4u ? w0 : w1, kk & 3u));
+        if (kk < 8u) return u01(head);
         const uint32_t blk = kk >> 2;
         if (blk != cached) {
             cw = philox_block(seed, blk, row, gen, purpose);
@@ -73,8 +81,8 @@ __host__ __device__ __forceinline__ int scale_draw(float u, int S) {
 // on j, so the sequence of draws is that of the nested loops.
 __host__ __device__ __forceinline__ void draw_donors(DonorStream &s, const float *inj, int n_inj, int S,
                                             int D, int (&r)[kMaxR], int &jr) {
-#pragma unroll
-    for (int i = 0; i < kMaxR; ++i) {
+    // (the i-th donor, with the earlier ones by value: they stay in registers)
+    auto donor = [&](int i, int p0, int p1, int p2, int p3) {
         int v = 0, j = 0;
         bool draw = true, first = true;
         for (;;) {
@@ -85,18 +93,22 @@ __host__ __device__ __forceinline__ void draw_donors(DonorStream &s, const float
                 draw = false;
             }
             if (j >= i) break;
-            int rj = r[0];
-#pragma unroll
-            for (int q = 1; q < kMaxR - 1; ++q)
-                if (q == j) rj = r[q];
+            const int rj = j == 0 ? p0 : j == 1 ? p1 : j == 2 ? p2 : p3;
             if (v == rj && s.k < (uint32_t)kMaxDraws)
                 draw = true;
             else
                 ++j;
         }
-        if (v == S) v--;
-        r[i] = v;
-    }
+        return v == S ? v - 1 : v;
+    };
+    const int r0 = donor(0, 0, 0, 0, 0), r1 = donor(1, r0, 0, 0, 0), r2 = donor(2, r0, r1, 0, 0);
+    const int r3 = donor(3, r0, r1, r2, 0), r4 = donor(4, r0, r1, r2, r3);
+    r[0] = r0;
+    r[1] = r1;
+    r[2] = r2;
+    r[3] = r3;
+    r[4] = r4;
+    static_assert(kMaxR == 5, "five donors");
     jr = (int)(s.next(inj, n_inj) * (float)D);
 }
 

@@ -50,34 +50,80 @@ int init_population(float *X, int ld, int n, int dim, float lo, float hi, uint64
 
 // -------------------------------------------------------------- generate
 
-__device__ __forceinline__ float mutant(int st, float F, const float *X, int ld, int j, int sel,
-                                        const int *r, int best) {
-#define E(i) X[(size_t)(i) * ld + j]
-    switch (st) {
-    case 0: return fmaf(F, E(r[0]) - E(r[1]), E(sel));
-    case 1: return fmaf(F, E(r[2]) - E(r[3]), fmaf(F, E(r[0]) - E(r[1]), E(sel)));
-    case 2: return fmaf(F, E(r[0]) - E(r[1]), fmaf(F, E(best) - E(sel), E(sel)));
-    case 3:
-        return fmaf(F, E(r[1]) - E(r[2]),
-                    fmaf(F, E(r[0]) - E(r[1]), fmaf(F, E(best) - E(sel), E(sel))));
-    case 4: return fmaf(F, E(r[1]) - E(r[2]), E(r[0]));
-    case 5: return fmaf(F, E(r[3]) - E(r[4]), fmaf(F, E(r[1]) - E(r[2]), E(r[0])));
-    case 6: return fmaf(F, E(r[0]) - E(r[1]), E(best));
-    case 7: return fmaf(F, E(r[2]) - E(r[3]), fmaf(F, E(r[0]) - E(r[1]), E(best)));
-    case 8: return fmaf(F, E(r[1]) - E(r[2]), fmaf(F, E(r[0]) - E(sel), E(sel)));
-    default: return E(sel);
-    }
-#undef E
-}
+// Four consecutive coordinates of a row; those past the dimension are 0.
+struct Four {
+    float v[4];
+};
 
-// 16 lanes per row, 16 rows per 256-thread block.  The donor draw is uniform
-// within a row's lanes (each lane repeats it, as the reference's 32 lanes all
-// read lane 0's state, kernel_DE_CUDA.cu:184-185).
-template <bool INJ>
+// The mutant's coordinates (row(i): those of population row i).
+template <typename Row>
+__device__ __forceinline__ Four mutant(int st, float F, int sel, int r0, int r1, int r2, int r3, int r4, int best,
+                                       Row row) {
+    auto add = [F](Four x, const Four &a, const Four &b) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x.v[q] = fmaf(F, a.v[q] - b.v[q], x.v[q]);
+        return x;
+    };
+    switch (st) {
+    case 0: return add(row(sel), row(r0), row(r1));
+    case 1: return add(add(row(sel), row(r0), row(r1)), row(r2), row(r3));
+    case 2: {
+        const Four s = row(sel);
+        return add(add(s, row(best), s), row(r0), row(r1));
+    }
+    case 3: {
+        const Four s = row(sel), b = row(r1);
+        return add(add(add(s, row(best), s), row(r0), b), b, row(r2));
+    }
+    case 4: return add(row(r0), row(r1), row(r2));
+    case 5: return add(add(row(r0), row(r1), row(r2)), row(r3), row(r4));
+    case 6: return add(row(best), row(r0), row(r1));
+    case 7: return add(add(row(best), row(r0), row(r1)), row(r2), row(r3));
+    case 8: {
+        const Four s = row(sel);
+        return add(add(s, row(r0), s), row(r1), row(r2));
+    }
+    default: return row(sel);
+    }
+}
+__device__ __forceinline__ bool uses_best(int st) { return st == 2 || st == 3 || st == 6 || st == 7; }
+
+// LPR lanes per row, four coordinates each.  The call is bound by latency at
+// the drop-in sizes (donor draws, indices, rows, crossover draws, one after
+// another), so up to kWaveRows rows take a wave each: its draws diverge over no
+// other row and its rows' addresses are scalars.  Beyond, where the chip is
+// full, 16 lanes a row repeat the draws least.
+// a.fit: the sub-islands' best members are found here too, by blocks past the
+// rows' for the caller and, where the strategy reads it, by the rows' own blocks
+// (S a multiple of a block's rows, at most kBestMembers).
+// 1,024 rows, D = 100: best 5.1 us and generate 10.7 us as two launches of 16
+// lanes a row and scalar loads, 6.9 us now.
+constexpr int kWaveRows = 8192, kBestMembers = 4096;
+
+template <bool INJ, int LPR>
 __global__ __launch_bounds__(256) void k_de_generate(GenArgs a) {
-    const int tid = threadIdx.x;
-    const int i = blockIdx.x * 16 + (tid >> 4);
-    const int l = tid & 15;
+    constexpr int RB = 256 / LPR;
+    __shared__ float sf[4];
+    __shared__ int si[4], sbest;
+    const int tid = threadIdx.x, l = tid & (LPR - 1);
+    const int sub = LPR == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid / LPR;
+    const int rowblocks = (a.n + RB - 1) / RB;
+    int found = -1;
+    if (a.fit) {
+        const bool extra = (int)blockIdx.x >= rowblocks;
+        const int isl = extra ? (int)blockIdx.x - rowblocks : (int)blockIdx.x * RB / a.S;
+        if (extra || uses_best(a.de_info[isl].strategy_ID)) {
+            const int b = block_argmin(a.fit, a.perm, isl * a.S, a.S, sf, si);
+            if (tid == 0) {
+                sbest = b;
+                if (extra) a.best_out[isl] = b;
+            }
+            if (extra) return;
+            __syncthreads();
+            found = sbest;
+        }
+    }
+    const int i = blockIdx.x * RB + sub;
     if (i >= a.n) return;
     const uint32_t row = a.row_base + (uint32_t)i;
 
@@ -90,54 +136,104 @@ __global__ __launch_bounds__(256) void k_de_generate(GenArgs a) {
 
     const int isl = i / a.S;
     const int sel = a.perm ? a.perm[i] : i;
-#pragma unroll
-    for (int k = 0; k < kMaxR; ++k) r[k] = a.perm ? a.perm[r[k] + isl * a.S] : r[k] + isl * a.S;
+    auto member = [&](int k) { return a.perm ? a.perm[k + isl * a.S] : k + isl * a.S; };
+    const int r0 = member(r[0]), r1 = member(r[1]), r2 = member(r[2]), r3 = member(r[3]), r4 = member(r[4]);
     if (l == 0) {
-        if (a.r_out)
-            for (int k = 0; k < kMaxR; ++k) a.r_out[(size_t)i * kMaxR + k] = r[k];
+        if (a.r_out) {
+            int *out = a.r_out + (size_t)i * kMaxR;
+            out[0] = r0;
+            out[1] = r1;
+            out[2] = r2;
+            out[3] = r3;
+            out[4] = r4;
+        }
         if (a.jrand_out) a.jrand_out[i] = jr;
     }
     const DEInfo info = a.de_info[isl];
-    const int b = a.best ? a.best[isl] : sel;
+    const int b = a.fit ? found : a.best ? a.best[isl] : sel;
     const int ngroups = (a.dim + 3) >> 2;
-    for (int g = l; g < ngroups; g += 16) {
+    // 16-byte loads where the rows allow them (a group's last columns may be padding)
+    const bool vec = (a.ld & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.X) | reinterpret_cast<uintptr_t>(a.U)) & 15) == 0;
+    for (int g = l; g < ngroups; g += LPR) {
+        auto at = [&](int i_) {
+            const float *p = a.X + (size_t)i_ * a.ld + 4 * g;
+            Four x;
+            if (vec) {
+                const float4 v = *reinterpret_cast<const float4 *>(p);
+                x = Four{{v.x, v.y, v.z, v.w}};
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x.v[q] = 4 * g + q < a.dim ? p[q] : 0.f;
+            }
+            return x;
+        };
+        const Four own = at(sel);
+        const Four mut = mutant(info.strategy_ID, info.F, sel, r0, r1, r2, r3, r4, b, at);
         const U4 w = philox_block(a.seed, (uint32_t)g, row, a.gen, kPurposeCross);
+        Four out;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int j = g * 4 + q;
-            if (j < a.dim) {
-                const float u = (INJ && a.inj_cr) ? a.inj_cr[(size_t)i * a.dim + j] : u01(word(w, q));
-                const bool take = (j == jr) || (u < info.CR);
-                const float v = take ? mutant(info.strategy_ID, info.F, a.X, a.ld, j, sel, r, b)
-                                     : a.X[(size_t)sel * a.ld + j];
-                a.U[(size_t)sel * a.ld + j] = check_bound(v, a.lo, a.hi);
-            }
+            float u = u01(word(w, q));
+            if (INJ && a.inj_cr && j < a.dim) u = a.inj_cr[(size_t)i * a.dim + j];
+            const float v = (j == jr) || (u < info.CR) ? mut.v[q] : own.v[q];
+            out.v[q] = j < a.dim ? check_bound(v, a.lo, a.hi) : 0.f;
+        }
+        float *p = a.U + (size_t)sel * a.ld + 4 * g;
+        if (vec && 4 * g + 4 <= a.dim) {
+            *reinterpret_cast<float4 *>(p) = float4{out.v[0], out.v[1], out.v[2], out.v[3]};
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (4 * g + q < a.dim) p[q] = out.v[q];
         }
     }
 }
 
+template <bool INJ, int LPR>
+static int launch_generate(GenArgs a, hipStream_t s) {
+    constexpr int RB = 256 / LPR;
+    int blocks = (a.n + RB - 1) / RB;
+    if (a.fit) {
+        if (a.S % RB == 0 && a.S <= kBestMembers) {
+            blocks += a.n / a.S;
+        } else {
+            SPEO_TRY(subisland_best(a.fit, a.perm, a.S, a.n / a.S, a.best_out, s));
+            a.best = a.best_out;
+            a.fit = nullptr;
+        }
+    }
+    hipLaunchKernelGGL((k_de_generate<INJ, LPR>), dim3(blocks), dim3(256), 0, s, a);
+    return check_launch("k_de_generate");
+}
+
 int de_generate(const GenArgs &a, hipStream_t s) {
     if (a.n <= 0) return SPEO_OK;
-    const dim3 grid((a.n + 15) / 16), block(256);
-    if (a.inj_r || a.inj_cr)
-        hipLaunchKernelGGL(k_de_generate<true>, grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL(k_de_generate<false>, grid, block, 0, s, a);
-    return check_launch("k_de_generate");
+    const bool inj = a.inj_r || a.inj_cr;
+    if (a.n <= kWaveRows) return inj ? launch_generate<true, 64>(a, s) : launch_generate<false, 64>(a, s);
+    return inj ? launch_generate<true, 16>(a, s) : launch_generate<false, 16>(a, s);
 }
 
 // ---------------------------------------------------------------- select
 
-__global__ void k_de_select(float *X, float *fX, const float *U, float *fU, int ld, int n,
-                            int dim, uint8_t *accept_out, int clear_trials) {
+// 32 lanes per row, 16-byte copies where the rows allow them.
+__global__ __launch_bounds__(256) void k_de_select(float *X, float *fX, const float *U, float *fU, int ld, int n,
+                                                   int dim, uint8_t *accept_out, int clear_trials) {
     const int tid = threadIdx.x;
-    const int i = blockIdx.x * 16 + (tid >> 4);
-    const int l = tid & 15;
+    const int i = blockIdx.x * 8 + (tid >> 5);
+    const int l = tid & 31;
     if (i >= n) return;
     const float fu = fU[i], fx = fX[i];
     const bool acc = fu < fx;
-    if (acc)
-        for (int j = l; j < dim; j += 16) X[(size_t)i * ld + j] = U[(size_t)i * ld + j];
+    if (acc) {
+        float *x = X + (size_t)i * ld;
+        const float *u = U + (size_t)i * ld;
+        const bool vec = (ld & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(U)) & 15) == 0;
+        const int ng = vec ? dim >> 2 : 0;
+        for (int g = l; g < ng; g += 32)
+            reinterpret_cast<float4 *>(x)[g] = reinterpret_cast<const float4 *>(u)[g];
+        for (int j = 4 * ng + l; j < dim; j += 32) x[j] = u[j];
+    }
     if (l == 0) {
         if (acc) fX[i] = fu;
         if (accept_out) accept_out[i] = acc ? 1 : 0;
@@ -148,7 +244,7 @@ __global__ void k_de_select(float *X, float *fX, const float *U, float *fU, int 
 int de_select(float *X, float *fX, const float *U, float *fU, int ld, int n, int dim,
               uint8_t *accept_out, int clear_trials, hipStream_t s) {
     if (n <= 0) return SPEO_OK;
-    hipLaunchKernelGGL(k_de_select, dim3((n + 15) / 16), dim3(256), 0, s, X, fX, U, fU, ld, n,
+    hipLaunchKernelGGL(k_de_select, dim3((n + 7) / 8), dim3(256), 0, s, X, fX, U, fU, ld, n,
                        dim, accept_out, clear_trials);
     return check_launch("k_de_select");
 }
@@ -323,16 +419,14 @@ int API_DE_GenerateNewPopulation(GPU_Population d_candidate, GPU_Population d_po
     const int S = n / subs;
     // global_DE_FindBestIndividualInIsland (kernel_DE_CUDA.cu:120-158), with
     // each sub-island's own offset into permutated_index.
-    if (d_best_individual_ID) {
-        hipLaunchKernelGGL(k_subisland_best, dim3(subs), dim3(256), 0, nullptr,
-                           d_population.fitness_value, info.permutated_index, S,
-                           d_best_individual_ID);
-        SPEO_TRY(check_launch("k_subisland_best"));
-    }
     GenArgs a{d_candidate.elements, d_population.elements, next_pow2_dim(pi.dim), n, pi.dim, S,
-              info.permutated_index, d_DE_info, d_best_individual_ID, pi.min_bound,
+              info.permutated_index, d_DE_info, nullptr, pi.min_bound,
               pi.max_bound, rand_state->seed, rand_state->generation, rand_state->row_base,
               nullptr, 0, nullptr, nullptr, nullptr};
+    if (d_best_individual_ID) {
+        a.fit = d_population.fitness_value;
+        a.best_out = d_best_individual_ID;
+    }
     SPEO_TRY(de_generate(a, nullptr));
     rand_state->generation++;
     return SPEO_OK;

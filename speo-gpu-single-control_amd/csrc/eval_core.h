@@ -726,6 +726,28 @@ struct SmallB {
         load_b_frag(c.B32s, cls + 4, (cls + 4) * 16 < dim, KS, lane, b1);
         o = tid < dim ? gld(c.shift + tid) : 0.f;
     }
+    // The same from the row-major B32 (the drop-in call's matrix, which is not
+    // kept in another layout): elements past the dimension lie past the buffer's
+    // end, where loads return 0.
+    __device__ __forceinline__ void load_rows(const CompDev &c, int dim, int cls) {
+        const int tid = threadIdx.x, lr = tid & 15, lk = (tid & 63) >> 4;
+        const int KS = (dim + 3) >> 2;
+        const int bytes = ((dim - 1) * c.ldb32 + dim) * 4;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(c.B32), (short)0, bytes,
+                                                                           kBufferWord3);
+        auto tile = [&](int col, float (&b)[32]) {
+#pragma unroll
+            for (int ks = 0; ks < 32; ++ks)
+                if (ks < KS) {
+                    const int k = 4 * ks + lk;
+                    const int at = k < dim && col < dim ? (k * c.ldb32 + col) * 4 : 0x7ffffff0;
+                    b[ks] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
+                }
+        };
+        if (cls * 16 < dim) tile(cls * 16 + lr, b0);
+        if ((cls + 4) * 16 < dim) tile((cls + 4) * 16 + lr, b1);
+        o = tid < dim ? gld(c.shift + tid) : 0.f;
+    }
     // into the scratch's shift (kSmallD floats); a barrier before gemm_small_f32
     __device__ __forceinline__ void stage(char *scratch) const {
         if (threadIdx.x < kSmallD) reinterpret_cast<float *>(scratch)[threadIdx.x] = o;

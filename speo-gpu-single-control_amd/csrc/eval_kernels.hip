@@ -22,20 +22,22 @@ template <int RT, int PREC> constexpr int eval_small_lds_bytes() {
     return RT * kTS * 4 + small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4;
 }
 
-template <int RT, int PREC>
+template <int RT, int PREC, bool RAW>
 __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
     extern __shared__ __align__(16) char lds[];
     const int row0 = blockIdx.x * RT;
     const int chunk = blockIdx.y;
     const int nrows = min(RT, p.n - row0);
     float *o1, *o2;
-    if (p.small) {
+    if (RAW || p.small) {
         float *rows = reinterpret_cast<float *>(lds);
         char *scratch = lds + RT * kTS * 4;
         float *red = reinterpret_cast<float *>(scratch + small_scratch_bytes<RT>(Prec<PREC>::parts));
         o1 = red + 8 * RT;
         o2 = o1 + RT;
-        const int kp4 = (p.dim + 3) & ~3;
+        const int kp4 = (p.dim + 3) & ~3, cls = column_class();
+        SmallB B;
+        if constexpr (RAW) B.load_rows(p.comp, p.dim, cls);
         if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.X) & 15) == 0) {
             // 16-byte loads, all of the tile issued before the first is
             // stored; columns >= dim set to 0 (the row's padding may hold
@@ -65,10 +67,11 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
                 rows[r * kTS + k] = (r < nrows && k < p.dim) ? p.X[(size_t)(row0 + r) * p.ld + k] : 0.f;
             }
         }
+        if constexpr (RAW) B.stage(scratch);
         __syncthreads();
         float s1[RT / 16][4], s2[RT / 16][4];
-        const int cls = column_class();
-        gemm_small<RT, PREC>(p.comp, rows, p.dim, cls, scratch, s1, s2);
+        if constexpr (RAW) gemm_small_f32<RT>(p.comp, B, rows, p.dim, cls, scratch, s1, s2);
+        else gemm_small<RT, PREC>(p.comp, rows, p.dim, cls, scratch, s1, s2);
         reduce_rows_small<RT>(s1, s2, cls, red, o1, o2);
     } else {
         RowSource src{p.X + (size_t)row0 * p.ld, p.ld, nrows};
@@ -289,17 +292,17 @@ static std::atomic<int> g_wide_eval{1};
 static std::atomic<long long> g_wide_launches{0};
 bool wide_eval_enabled() { return g_wide_eval.load(std::memory_order_relaxed) != 0; }
 
-template <int RT, int PREC>
+template <int RT, int PREC, bool RAW = false>
 static int launch_rt_prec(const EvalLaunch &p, int n, int nchunks, hipStream_t s) {
     static std::once_flag once;
     constexpr int lds_max = std::max(gemm_lds_bytes<RT, PREC>(), eval_small_lds_bytes<RT, PREC>());
     std::call_once(once, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval<RT, PREC>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval<RT, PREC, RAW>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
     });
-    const int lds = p.small ? eval_small_lds_bytes<RT, PREC>() : gemm_lds_bytes<RT, PREC>();
+    const int lds = RAW || p.small ? eval_small_lds_bytes<RT, PREC>() : gemm_lds_bytes<RT, PREC>();
     dim3 grid((n + RT - 1) / RT, nchunks);
-    hipLaunchKernelGGL((k_eval<RT, PREC>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((k_eval<RT, PREC, RAW>), grid, dim3(256), lds, s, p);
     return check_launch("k_eval");
 }
 
@@ -335,6 +338,10 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
         // the same bits as k_eval<64, precision>, on wider tiles
         rc = eval_wide(&comp, 1, X, ld, n, dim, part, precision, s);
         g_wide_launches.fetch_add(1, std::memory_order_relaxed);
+    } else if (rows_per_block == 16 && precision == SPEO_PREC_FP32 && dim <= kSmallD && !small) {
+        // the row-major matrix straight into registers; the 16-row tile's sums
+        // are those of the staged path (four column classes in either)
+        rc = launch_rt_prec<16, SPEO_PREC_FP32, true>(p, n, nchunks, s);
     } else switch (rows_per_block) {
     case 16: rc = launch_rt<16>(p, precision, n, nchunks, s); break;
     case 32: rc = launch_rt<32>(p, precision, n, nchunks, s); break;
