@@ -177,7 +177,7 @@ int segment_argmin(const float *f, const int *off, int nseg, int *best_out, hipS
 // ties to the lower slot, NaN last.
 int subisland_best(const float *f, const int *perm, int S, int subs, int *best_out, hipStream_t s);
 int migrate_ring(float *X, float *fX, const IslandDesc *isl_desc_dev, const int *row_off_dev,
-                 const int *dst_dev, int *best_buf, int *worst_buf, int I, int k,
-                 hipStream_t s);
+                 const int *dst_dev, int *best_buf, int *worst_buf, int I, int max_np, int k,
+                 hipStream_t s);  // max_np: rows of the largest island
 
 }  // namespace speo

@@ -463,7 +463,7 @@ struct Engine {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     speo_engine_config cfg{};
-    int I = 0, total_rows = 0, max_dim = 0, max_ld = 0;
+    int I = 0, total_rows = 0, max_dim = 0, max_ld = 0, max_np = 0;
     int64_t total_elems = 0;
     std::vector<IslandDesc> isl;
     std::vector<int> row_off, dst;
@@ -788,6 +788,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
         eoff += (int64_t)np * d.ld;
         row_off[(size_t)i + 1] = row_off[(size_t)i] + np;
         max_dim = std::max(max_dim, d.dim);
+        max_np = std::max(max_np, np);
         max_ld = std::max(max_ld, d.ld);
     }
     total_rows = row_off[(size_t)I];
@@ -1423,7 +1424,7 @@ int Engine::migrate(hipStream_t s) {
     if (cfg.migration_size <= 0) return SPEO_OK;
     SPEO_TRY(finalize_pending(s));
     const int cur = cfg.mode == SPEO_MODE_FUSED ? p : 0;
-    return migrate_ring(X, fX[cur], isl_dev, row_off_dev, dst_dev, best_buf, worst_buf, I,
+    return migrate_ring(X, fX[cur], isl_dev, row_off_dev, dst_dev, best_buf, worst_buf, I, max_np,
                         cfg.migration_size, s);
 }
 

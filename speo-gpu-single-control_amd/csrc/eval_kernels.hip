@@ -37,7 +37,9 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
         o2 = o1 + RT;
         const int kp4 = (p.dim + 3) & ~3, cls = column_class();
         SmallB B;
+        constexpr bool F32 = Prec<PREC>::parts == 0;
         if constexpr (RAW) B.load_rows(p.comp, p.dim, cls);
+        else if constexpr (F32) B.load(p.comp, p.dim, cls);
         if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.X) & 15) == 0) {
             // 16-byte loads, all of the tile issued before the first is
             // stored; columns >= dim set to 0 (the row's padding may hold
@@ -67,10 +69,10 @@ __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
                 rows[r * kTS + k] = (r < nrows && k < p.dim) ? p.X[(size_t)(row0 + r) * p.ld + k] : 0.f;
             }
         }
-        if constexpr (RAW) B.stage(scratch);
+        if constexpr (F32) B.stage(scratch);
         __syncthreads();
         float s1[RT / 16][4], s2[RT / 16][4];
-        if constexpr (RAW) gemm_small_f32<RT>(p.comp, B, rows, p.dim, cls, scratch, s1, s2);
+        if constexpr (F32) gemm_small_f32<RT>(p.comp, B, rows, p.dim, cls, scratch, s1, s2);
         else gemm_small<RT, PREC>(p.comp, rows, p.dim, cls, scratch, s1, s2);
         reduce_rows_small<RT>(s1, s2, cls, red, o1, o2);
     } else {

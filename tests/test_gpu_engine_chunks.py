@@ -44,3 +44,36 @@ def test_run_equals_separate_launches(cuda, speo, lengths, interval, graph, dims
     assert a.best()[1].tolist() == b.best()[1].tolist()
     for o in [a, b] + probs:
         o.close()
+
+
+@pytest.mark.parametrize("sizes,k", [([4100, 8, 4097], 4), ([63, 64, 65, 130], 3), ([1000, 257], 128)])
+def test_migration_ranks(cuda, speo, oracle, sizes, k):
+    """Migration by rank against the oracle: more rows than one LDS pass, edges of a
+    block's rows, half an island moving; ties, both zeros, infinities and NaN."""
+    print(f"sizes {sizes} migrants {k}", flush=True)
+    probs = _problems(speo, [(6, [2])])
+    kw = dict(seed=3, mode=speo.MODE_PLAIN, rows_per_block=32)
+    which = [0] * len(sizes)
+    n = sum(sizes)
+    rng = np.random.default_rng(n)
+    f = rng.integers(-3, 3, n).astype(np.float32)  # trials never beat values this low; many ties
+    f[rng.random(n) < 0.1] = -0.0
+    f[rng.random(n) < 0.1] = np.nan
+    f[rng.random(n) < 0.05] = -np.inf
+    out = []
+    for interval in (0, 1):
+        e = speo.Engine(probs, sizes, which, interval=interval, migration_size=min(k, min(sizes) // 2), **kw)
+        X, _ = e.read()
+        e.write(X, f)
+        e.run(1)
+        out.append(e.read())
+        e.close()
+    X, f1 = out[0]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    dst = np.array([(i + 1) % len(sizes) for i in range(len(sizes))], np.int32)
+    Xo, fo = oracle.migrate_ring(X, f1, X.shape[1], off, np.full(len(sizes), 6, np.int32), dst,
+                                 min(k, min(sizes) // 2))
+    np.testing.assert_array_equal(out[1][1], fo)
+    np.testing.assert_array_equal(out[1][0], Xo)
+    for p in probs:
+        p.close()
