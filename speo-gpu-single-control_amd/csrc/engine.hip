@@ -88,6 +88,11 @@ struct GenerationArgs {
     AppendArgs append;
 };
 
+// Rows per block of the launches that only make trials or select: they depend on
+// no arithmetic of the evaluation's tile, and small tiles fill the chip (16,384
+// rows of D = 1000: trials 85 us at 64 rows a block, 55 us at 16).
+constexpr int kTrialRows = 16;
+
 constexpr int kTLD = kSmallD;  // widest dimension this kernel evaluates
 
 // LDS of one block: [trial rows RT x kTS] [gval kMaxComp x RT] [scratch of the
@@ -868,6 +873,7 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
     if (c.surrogate_candidates > 0) SPEO_TRY(surrogate_setup());
     if (configured) SPEO_TRY(configure_setup());
     SPEO_TRY(build_tiles(rt));
+    SPEO_TRY(build_tiles(kTrialRows));
     // Initial evaluation (island_EA.cc:81 counts it as island_size FEs).
     if (all_small) {
         GenerationArgs a{};
@@ -1271,11 +1277,16 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear, 
         a.U_new = U[1 - u];
         a.fU_new = fU[1 - u];
         if (!all_small) {
-            SPEO_TRY(launch_any(rt_, cfg.precision, kModeFusedGen, a, ntiles[rt_], s));
+            a.tiles = tiles_dev[kTrialRows];
+            SPEO_TRY(launch_any(kTrialRows, cfg.precision, kModeFusedGen, a, ntiles[kTrialRows], s));
             return eval_wide_rows(a.U_new, a.fU_new, rt_, s);
         }
         break;
     }
+    }
+    if (mode == kModeGen || mode == kModeSelect) {
+        a.tiles = tiles_dev[kTrialRows];
+        return launch_any(kTrialRows, cfg.precision, mode, a, ntiles[kTrialRows], s);
     }
     return launch_any(rt_, cfg.precision, mode, a, ntiles[rt_], s);
 }
@@ -1847,6 +1858,7 @@ int Engine::autotune() {
     float best_ms = 1e30f;
     int best_rt = 32;
     const int saved_p = p;
+    SPEO_TRY(build_tiles(kTrialRows));
     for (int cand : {16, 32, 64}) {
         SPEO_TRY(build_tiles(cand));
         const int mode = cfg.mode == SPEO_MODE_FUSED ? kModeFused : kModeEval;

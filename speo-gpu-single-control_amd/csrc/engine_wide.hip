@@ -172,9 +172,13 @@ __global__ __launch_bounds__(256) void k_rows_chunk(WideRowsArgs p) {
 // coordinates in order, here one lane per (row, component) over 64-column
 // pieces of the rows and shifts staged in LDS (a lane per row reading its row
 // and every shift from memory took milliseconds at D = 1000).
+// The next two pieces are in flight while this one is summed: with two barriers a
+// piece and its loads between them 16,384 rows of D = 1000 and three components
+// took 52 us, 26 us so.
 constexpr int kCombLd = 68;  // row stride (floats) in LDS: 16-byte reads of 16 rows in different banks
+constexpr int kCombGroups = kWideRows * 16 / 128;  // 16-byte groups of a piece per thread, two components or more
 __global__ __launch_bounds__(64 * kMaxComp) void k_rows_combine(WideRowsArgs p) {
-    __shared__ __align__(16) float xs[kWideRows * kCombLd], os[kMaxComp * 64];
+    __shared__ __align__(16) float xs[2][kWideRows * kCombLd], os[2][kMaxComp * 64];
     __shared__ float lws[kMaxComp][kWideRows], ds[kMaxComp][kWideRows];
     const WideItem it = p.items[blockIdx.x];
     const FusedProblem *P = p.probs + it.problem;
@@ -183,38 +187,71 @@ __global__ __launch_bounds__(64 * kMaxComp) void k_rows_combine(WideRowsArgs p) 
     const int tid = threadIdx.x, c = tid >> 6, r = tid & 63, nt = blockDim.x;
     const bool mine = c < nc && r < it.nrows;
     const float *rows = p.src + it.elem;
-    float d = 0.f;
-    for (int k0 = 0; k0 < dim; k0 += 64) {
+    struct Piece {
+        floatx4 x[kCombGroups];
+        float o;
+    };
+    const float *shift = P->comp[min(c, nc - 1)].shift;
+    // (addresses are clamped, not loads skipped: nothing waits on a merge)
+    auto load = [&](Piece &q, int k0) {
+        if (k0 >= dim) return;
         const int kc = min(64, dim - k0);
-        __syncthreads();
-        for (int e = tid; e < kWideRows * 16; e += nt) {
-            const int rr = e >> 4, k = (e & 15) * 4;  // (rows are padded to 32 floats: the group exists)
-            if (rr < it.nrows && k < kc)
-                *reinterpret_cast<float4 *>(xs + rr * kCombLd + k) =
-                    *reinterpret_cast<const float4 *>(rows + (size_t)rr * it.ld + k0 + k);
-        }
-        if (c < nc && r < kc) os[c * 64 + r] = P->comp[c].shift[k0 + r];
-        __syncthreads();
-        if (mine) {
-            const float *x = xs + r * kCombLd, *o = os + c * 64;
-            if (kc == 64) {
 #pragma unroll
-                for (int k = 0; k < 64; k += 4) {
-                    const float4 xv = *reinterpret_cast<const float4 *>(x + k);
-                    const float4 ov = *reinterpret_cast<const float4 *>(o + k);
-                    const float v0 = xv.x - ov.x, v1 = xv.y - ov.y, v2 = xv.z - ov.z, v3 = xv.w - ov.w;
-                    d = fmaf(v0, v0, d);
-                    d = fmaf(v1, v1, d);
-                    d = fmaf(v2, v2, d);
-                    d = fmaf(v3, v3, d);
-                }
-            } else {
-                for (int k = 0; k < kc; ++k) {
-                    const float v = x[k] - o[k];
-                    d = fmaf(v, v, d);
-                }
+        for (int i = 0; i < kCombGroups; ++i)
+            if (i * nt < kWideRows * 16) {
+                const int e = tid + i * nt, rr = min(e >> 4, it.nrows - 1), k = (e & 15) * 4;
+                q.x[i] = gld(reinterpret_cast<const floatx4 *>(rows + (size_t)rr * it.ld + k0 + (k < kc ? k : 0)));
+            }
+        q.o = shift[k0 + min(r, kc - 1)];
+    };
+    auto store = [&](const Piece &q, int b, int k0) {
+        if (k0 >= dim) return;
+#pragma unroll
+        for (int i = 0; i < kCombGroups; ++i)
+            if (i * nt < kWideRows * 16) {
+                const int e = tid + i * nt, rr = e >> 4, k = (e & 15) * 4;
+                if (rr < kWideRows) *reinterpret_cast<floatx4 *>(xs[b] + rr * kCombLd + k) = q.x[i];
+            }
+        os[b][c * 64 + r] = q.o;
+    };
+    float d = 0.f;
+    auto sum = [&](int b, int k0) {
+        const int kc = min(64, dim - k0);
+        if (!mine || kc <= 0) return;
+        const float *xr = xs[b] + r * kCombLd, *o = os[b] + c * 64;
+        if (kc == 64) {
+#pragma unroll
+            for (int k = 0; k < 64; k += 4) {
+                const float4 xv = *reinterpret_cast<const float4 *>(xr + k);
+                const float4 ov = *reinterpret_cast<const float4 *>(o + k);
+                const float v0 = xv.x - ov.x, v1 = xv.y - ov.y, v2 = xv.z - ov.z, v3 = xv.w - ov.w;
+                d = fmaf(v0, v0, d);
+                d = fmaf(v1, v1, d);
+                d = fmaf(v2, v2, d);
+                d = fmaf(v3, v3, d);
+            }
+        } else {
+            for (int k = 0; k < kc; ++k) {
+                const float v = xr[k] - o[k];
+                d = fmaf(v, v, d);
             }
         }
+    };
+    // each buffer is written after the barrier behind its last reads
+    Piece qa, qb;
+    load(qa, 0);
+    load(qb, 64);
+    store(qa, 0, 0);
+    __syncthreads();
+    for (int k0 = 0; k0 < dim; k0 += 128) {
+        load(qa, k0 + 128);
+        sum(0, k0);
+        store(qb, 1, k0 + 64);
+        __syncthreads();
+        load(qb, k0 + 192);
+        sum(1, k0 + 64);
+        store(qa, 0, k0 + 128);
+        __syncthreads();
     }
     if (mine) {
         const float s = P->sigma[c];
