@@ -836,30 +836,52 @@ __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, 
         constexpr int P = Prec<PREC>::parts;
         constexpr bool H = Prec<PREC>::half;
         typedef typename std::conditional<H, halfx8, bf16x8>::type vec8;
-        const int kp32 = c.kp32, KS = kp32 >> 5, LDA = kSmallD + 8;
+        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+        const int kp32 = c.kp32, KS = kp32 >> 5, LDA = kSmallD + 8;  // KS <= 4
         uint16_t *As = reinterpret_cast<uint16_t *>(sh + kSmallD);  // [P][RT][LDA]
+        // B's fragments ahead of the staging: all four K steps' (64 registers
+        // with two parts), with three parts two steps' at a time
+        constexpr int DEPTH = P <= 2 ? 4 : 2;
+        vec8 b[DEPTH][2][P];
+        auto fetch = [&](int ks) {
+            if (ks >= KS) return;
+            const int kb = ks * 32 + lk * 8;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                if (v0) b[ks % DEPTH][0][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t0 * 16 + lr) * kp32 + kb));
+                if (v1) b[ks % DEPTH][1][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t1 * 16 + lr) * kp32 + kb));
+            }
+        };
+#pragma unroll
+        for (int ks = 0; ks < DEPTH; ++ks) fetch(ks);
         for (int k = tid; k < kSmallD; k += 256) sh[k] = k < dim ? gld(c.shift + k) : 0.f;
         __syncthreads();
         const float scale = c.rate * (H ? kF16ScaleA : 1.0f);
-        for (int e = tid; e < RT * kp32; e += 256) {
-            const int r = e / kp32, k = e % kp32;
-            float rem = k < dim ? (rows[r * kTS + k] - sh[k]) * scale : 0.f;
+        // four columns a thread; e / ng = e ceil(2^16 / ng) / 2^16 for e < 64 ng <= 2048
+        const int ng = kp32 >> 2, inv = ng == 24 ? 2731 : 65536 / ng;
+        for (int e = tid; e < RT * ng; e += 256) {
+            const int r = (e * inv) >> 16, k = 4 * (e - r * ng);
+            const floatx4 x = *reinterpret_cast<const floatx4 *>(rows + r * kTS + k);
+            const floatx4 o = *reinterpret_cast<const floatx4 *>(sh + k);
+            u16x4 h[P];
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const uint16_t b = to_bits(rem, H);
-                As[(p * RT + r) * LDA + k] = b;
-                rem -= from_bits(b, H);
+            for (int q = 0; q < 4; ++q) {
+                float rem = k + q < dim ? (x[q] - o[q]) * scale : 0.f;
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    const uint16_t w = to_bits(rem, H);
+                    h[p][q] = w;
+                    rem -= from_bits(w, H);
+                }
             }
+#pragma unroll
+            for (int p = 0; p < P; ++p) *reinterpret_cast<u16x4 *>(As + (p * RT + r) * LDA + k) = h[p];
         }
         __syncthreads();
-        for (int ks = 0; ks < KS; ++ks) {
-            const int kb = ks * 32 + lk * 8;
-            vec8 b[2][P];
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                b[0][p] = v0 ? gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t0 * 16 + lr) * kp32 + kb)) : vec8{};
-                b[1][p] = v1 ? gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t1 * 16 + lr) * kp32 + kb)) : vec8{};
-            }
+        for (int ks = 0; ks < 4; ++ks) {
+            if (ks >= KS) break;
+            const int kb = ks * 32 + lk * 8;
 #pragma unroll
             for (int i = 0; i < NRT; ++i) {
                 vec8 a[P];
@@ -876,14 +898,15 @@ __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, 
                             const int pb = sum - pa;
                             if (pa < P && pb < P) {
                                 if constexpr (H)
-                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[pa], b[t][pb], acc[i][t], 0, 0, 0);
+                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
                                 else
-                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa], b[t][pb], acc[i][t], 0, 0, 0);
+                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
                             }
                         }
                     }
                 }
             }
+            if (DEPTH < 4 && ks + DEPTH < 4) fetch(ks + DEPTH);
         }
         small_terms<RT, PREC>(c, acc, dim, cls, s1, s2);
     }
