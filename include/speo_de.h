@@ -391,7 +391,9 @@ typedef struct {
      * there are fewer islands than compute units; 1, 2, 4 or 8 = fixed).  A
      * split island runs one launch per generation: every workgroup reads the
      * whole island from HBM, evolves its share of the rows and writes it back;
-     * the launch boundary is the only synchronisation (graph-capturable). */
+     * the launch boundary is the only synchronisation (graph-capturable).  An
+     * automatic plan may also run its generations as the fused mode's launches,
+     * where those measure faster (the same results). */
     int epoch_parts;
     /* The reference island's sub-islands and DE configuration (IslandInfo,
      * config.h:62-84; DE_CUDA::Initilize / ConfigureEA, DE_CUDA.cc:57-119;

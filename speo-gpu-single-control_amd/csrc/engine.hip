@@ -608,6 +608,10 @@ struct Engine {
     int tuned_from_cache = 0;  // bit 0: row tile, bit 1: epoch parts
     std::string tune_key(const char *what) const;
     int tune_epoch_parts();
+    // epoch mode: generations as fused launches instead of an epoch kernel
+    bool by_launches = false;
+    int tune_launches();
+    int time_plan(int parts, bool launches, double *seconds);
     int best(int *row_out, float *f32_out, double *f64_out);
     int read(float *Xo, float *fo);
     int read_rows(const float *src, const float *fsrc, float *Xo, float *fo);
@@ -865,8 +869,10 @@ int Engine::create(const speo_engine_config &c, hipStream_t s) {
     if (c.surrogate_candidates > 0 && c.mode != SPEO_MODE_PLAIN)
         return set_error(SPEO_ERR_UNSUPPORTED, "speo_engine_create: the surrogate runs in "
                                                "SPEO_MODE_PLAIN");
-    if (cfg.mode == SPEO_MODE_EPOCH && cfg.epoch_parts == 0 && !tuning_child)
+    if (cfg.mode == SPEO_MODE_EPOCH && cfg.epoch_parts == 0 && !tuning_child) {
         SPEO_TRY(tune_epoch_parts());
+        if (cfg.epoch_parts > 0) SPEO_TRY(tune_launches());
+    }
     if (cfg.mode == SPEO_MODE_EPOCH) SPEO_TRY(epoch_setup());
     rt = c.rows_per_block;
     if (rt == 0) SPEO_TRY(autotune());
@@ -1007,6 +1013,7 @@ void Engine::swap_epoch_buffers() {
 // launch per generation runs it (split islands, swapping the population
 // buffers).
 int Engine::launch_epoch_chunk(int L, hipStream_t s) {
+    if (by_launches) return enqueue_plain(L, s);
     EpochArgs a{};
     a.blocks = blocks_dev;
     a.Xalt = U[1];
@@ -1298,7 +1305,8 @@ int Engine::draw_ahead(int gen_offset, int L, hipStream_t s) {
                         donor_buf, s);
 }
 
-// L generations of a plain engine as L fused launches and one selection: L + 1
+// L generations of a plain engine (or of an epoch engine that runs by launches)
+// as L fused launches and one selection: L + 1
 // launches instead of 3 L (100 rows, D = 10, ten generations and the best:
 // 144 us as separate launches, 100 us so).  The parities are chosen so that the
 // last trials end in U[0], fU[0] and the last selection writes fX[0]: the
@@ -1308,13 +1316,23 @@ int Engine::enqueue_plain(int L, hipStream_t s) {
     pu = L & 1;
     pending = false;
     for (int g = 0; g < L; ++g) {
-        if (g % donor_gens == 0) SPEO_TRY(draw_ahead(g, std::min(donor_gens, L - g), s));
+        if (g % donor_gens == 0) {
+            const int Ls = std::min(donor_gens, L - g);
+            if (g > 0) SPEO_TRY(prof_end(s));
+            SPEO_TRY(prof_begin(5, Ls, s));
+            SPEO_TRY(draw_ahead(g, Ls, s));
+            SPEO_TRY(prof_end(s));
+            SPEO_TRY(prof_begin(4, Ls, s));
+        }
         SPEO_TRY(launch(kModeFused, g, rt, s));
         pf = 1 - pf;
         pu = 1 - pu;
         pending = true;
     }
-    if (L > 0) SPEO_TRY(launch(kModeSelect, 0, rt, s));
+    if (L > 0) {
+        SPEO_TRY(launch(kModeSelect, 0, rt, s));
+        SPEO_TRY(prof_end(s));
+    }
     pf = pu = 0;
     pending = false;
     return SPEO_OK;
@@ -1677,7 +1695,7 @@ int Engine::run(int generations, bool dry) {
                 pending = L > 0 ? true : pending;
                 if (mig && cfg.migration_size > 0) pending = false;
             }
-            if (cfg.mode == SPEO_MODE_EPOCH && epoch_parts > 1 && L % 2) swap_epoch_buffers();
+            if (cfg.mode == SPEO_MODE_EPOCH && epoch_parts > 1 && !by_launches && L % 2) swap_epoch_buffers();
         } else if (!dry) {
             SPEO_TRY(enqueue_chunk(L, mig, stream));
         }
@@ -1808,7 +1826,7 @@ int Engine::profile_epoch(int generations, double *avg_ms) {
 int Engine::autotune() {
     static std::mutex mu;
     static std::map<std::vector<int>, int> cache;
-    std::vector<int> key{cfg.precision, cfg.mode};
+    std::vector<int> key{cfg.precision, by_launches ? -1 : cfg.mode};
     for (const auto &d : isl) {
         key.push_back(d.np);
         key.push_back(d.dim);
@@ -1821,7 +1839,7 @@ int Engine::autotune() {
             return SPEO_OK;
         }
     }
-    const std::string pkey = tune_key("rt");
+    const std::string pkey = tune_key(by_launches ? "rt_launches" : "rt");
     int stored = 0;
     if (tune_lookup(pkey, &stored) && (stored == 16 || stored == 32 || stored == 64)) {
         rt = stored;
@@ -1861,7 +1879,7 @@ int Engine::autotune() {
     SPEO_TRY(build_tiles(kTrialRows));
     for (int cand : {16, 32, 64}) {
         SPEO_TRY(build_tiles(cand));
-        const int mode = cfg.mode == SPEO_MODE_FUSED ? kModeFused : kModeEval;
+        const int mode = cfg.mode == SPEO_MODE_FUSED || by_launches ? kModeFused : kModeEval;
         if (donor_buf) SPEO_TRY(draw_ahead(0, std::min(6, donor_gens), stream));
         for (int rep = 0; rep < 2; ++rep) SPEO_TRY(launch(mode, rep, cand, stream));
         SPEO_TRY_HIP(hipEventRecord(e0, stream));
@@ -1919,6 +1937,67 @@ std::string Engine::tune_key(const char *what) const {
     return k.str();
 }
 
+// Seconds of 24 generations of a throwaway engine of this configuration, after
+// a warm-up that captures the graphs.
+int Engine::time_plan(int parts, bool launches, double *seconds) {
+    speo_engine_config c2 = cfg;
+    c2.epoch_parts = parts;
+    c2.use_graph = 1;
+    c2.rows_per_block = cfg.rows_per_block ? cfg.rows_per_block : 32;
+    auto child = std::make_unique<Engine>();
+    child->tuning_child = true;
+    child->by_launches = launches;
+    SPEO_TRY(child->create(c2, stream));
+    SPEO_TRY(child->run(24));
+    SPEO_TRY_HIP(hipStreamSynchronize(stream));
+    const auto t0 = std::chrono::steady_clock::now();
+    SPEO_TRY(child->run(24));
+    SPEO_TRY_HIP(hipStreamSynchronize(stream));
+    *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    return SPEO_OK;
+}
+
+// Whether the generations of an epoch engine with an automatic plan run as
+// fused launches, which spread an island over as many workgroups as it has row
+// tiles: measured against the plan chosen (the same results either way).  An
+// epoch kernel's time grows with the rows of its largest island and, beyond two
+// islands a compute unit, in rounds; the launches' with all rows.  Us a generation,
+// epoch plan against launches of 32 rows: 16 x 512, D = 100: 85 / 14; 100 x 400,
+// D = 128: 79 / 38; 1024 x 64, D = 30: 27 / 17; 64 x 128, D = 100: 9.5 / 14.  Up
+// to 64 rows and two islands a unit the epoch kernel always was the faster one
+// or within 20 %, and nothing is measured.
+int Engine::tune_launches() {
+    static std::mutex mu;
+    static std::map<std::string, int> chosen;  // bounded by the workload shapes a program uses
+    int dev = 0, cus = 0;
+    SPEO_TRY_HIP(hipGetDevice(&dev));
+    SPEO_TRY_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (max_np <= 64 && I <= 2 * cus) return SPEO_OK;
+    std::vector<EpochPlan> plans;
+    int lds = 0;
+    if (epoch_plan_all(cfg.epoch_parts, &plans, &lds) != SPEO_OK) return SPEO_OK;  // epoch_setup reports it
+    const std::string key = tune_key(("launches" + std::to_string(cfg.epoch_parts)).c_str());
+    int stored = 0;
+    bool known = tune_lookup(key, &stored) && (stored == 0 || stored == 1);
+    if (!known) {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = chosen.find(key);
+        known = it != chosen.end();
+        if (known) stored = it->second;
+    }
+    if (!known) {
+        double plan = 0.0, launches = 0.0;
+        SPEO_TRY(time_plan(cfg.epoch_parts, false, &plan));
+        SPEO_TRY(time_plan(cfg.epoch_parts, true, &launches));
+        stored = launches < plan ? 1 : 0;
+        tune_store(key, stored);
+    }
+    by_launches = stored != 0;
+    std::lock_guard<std::mutex> lk(mu);
+    chosen[key] = stored;
+    return SPEO_OK;
+}
+
 // Workgroups per island for epoch mode: every feasible power of two up to 8
 // (islands x parts at most four per compute unit) timed on a throwaway
 // engine of this configuration over 24 generations after a warm-up that
@@ -1946,19 +2025,8 @@ int Engine::tune_epoch_parts() {
     if (cands.size() > 1) {
         double best_s = 1e30;
         for (int parts : cands) {
-            speo_engine_config c2 = cfg;
-            c2.epoch_parts = parts;
-            c2.use_graph = 1;
-            c2.rows_per_block = cfg.rows_per_block ? cfg.rows_per_block : 32;
-            auto child = std::make_unique<Engine>();
-            child->tuning_child = true;
-            SPEO_TRY(child->create(c2, stream));
-            SPEO_TRY(child->run(24));
-            SPEO_TRY_HIP(hipStreamSynchronize(stream));
-            const auto t0 = std::chrono::steady_clock::now();
-            SPEO_TRY(child->run(24));
-            SPEO_TRY_HIP(hipStreamSynchronize(stream));
-            const double dt = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+            double dt = 0.0;
+            SPEO_TRY(time_plan(parts, false, &dt));
             if (dt < best_s) {
                 best_s = dt;
                 best = parts;

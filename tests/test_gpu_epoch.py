@@ -182,3 +182,37 @@ def test_epoch_automatic_split(cuda, speo, oracle, tmp_path, monkeypatch):
     e.run(25)
     one.run(25)
     _assert_same(one, e)
+
+
+@pytest.mark.parametrize("sizes,dims,graph", [([300, 65, 512], [(100, 2), (30, 1), (128, 3)], 1),
+                                              ([128] * 8, [(100, 3)], 0), ([70, 90], [(5, 1), (20, 2)], 1)])
+def test_epoch_by_launches_equals_kernel(cuda, speo, oracle, tmp_path, monkeypatch, sizes, dims, graph):
+    # an automatic plan may run its generations as fused launches: the choice is
+    # measured, persisted, read back, and changes no result
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("SPEO_TUNE_CACHE", str(cache))
+    probs = _problems(speo, oracle, dims, base=3100)
+    pidx = [i % len(dims) for i in range(len(sizes))]
+    kw = dict(F=0.5, CR=0.9, seed=SEED, interval=6, migration_size=2, rows_per_block=32)
+    speo.Engine(probs, sizes, pidx, mode=speo.MODE_EPOCH, **kw).close()
+    lines = cache.read_text().splitlines()
+    key = [ln.split()[0] for ln in lines if ln.startswith("launches")]
+    assert len(key) == 1
+    plain = speo.Engine(probs, sizes, pidx, mode=speo.MODE_PLAIN, **kw)
+    engines = []
+    for choice in (0, 1):
+        cache.write_text("\n".join(lines) + f"\n{key[0]} {choice}\n")
+        engines.append(speo.Engine(probs, sizes, pidx, mode=speo.MODE_EPOCH, use_graph=bool(graph), **kw))
+    engines[1].prepare(20)
+    for chunk in (1, 2, 20, 70):
+        print(f"sizes {sizes} chunk {chunk}", flush=True)
+        plain.run(chunk)
+        for e in engines:
+            e.run(chunk)
+            _assert_same(plain, e)
+            for x, y in zip(plain.read_trials(), e.read_trials()):
+                np.testing.assert_array_equal(x, y)
+    kms = engines[1].profile(70)
+    assert kms["epoch"] > 0 and kms["donors"] > 0
+    plain.run(70)
+    _assert_same(plain, engines[1])
