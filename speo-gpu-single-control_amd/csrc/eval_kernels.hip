@@ -467,6 +467,8 @@ namespace {
 struct DimTables {
     float *colw[3] = {nullptr, nullptr, nullptr};  // elliptic, bent cigar, discus weights
     float *identity = nullptr;
+    int heavy_j[3] = {-1, -1, -1};  // their heavy columns
+    double heavy_w[3] = {0.0, 0.0, 0.0};
 };
 std::mutex g_tables_mu;
 std::unordered_map<int, DimTables> g_tables;
@@ -484,6 +486,7 @@ int dim_tables(int dim, DimTables &out) {
     const int kinds[3] = {SPEO_OBJ_ELLIPTIC, SPEO_OBJ_BENT_CIGAR, SPEO_OBJ_DISCUS};
     for (int k = 0; k < 3; ++k) {
         column_weights(kinds[k], dim, w.data());
+        t.heavy_j[k] = heavy_column(kinds[k], dim, &t.heavy_w[k]);
         SPEO_TRY_HIP(hipMalloc(&t.colw[k], sizeof(float) * dim));
         SPEO_TRY_HIP(hipMemcpy(t.colw[k], w.data(), sizeof(float) * dim, hipMemcpyHostToDevice));
     }
@@ -640,8 +643,8 @@ extern "C" void API_evaluateFitness(real *d_fitness_value, real *, real *d_rotat
     c.colw = t.colw[weights];
     c.heavy.j = -1;
     if (c.objective == SPEO_OBJ_ELLIPTIC) {
-        static const int kinds[3] = {SPEO_OBJ_ELLIPTIC, SPEO_OBJ_BENT_CIGAR, SPEO_OBJ_DISCUS};
-        c.heavy.j = heavy_column(kinds[weights], problem_dim, &c.heavy.w);
+        c.heavy.j = t.heavy_j[weights];
+        c.heavy.w = t.heavy_w[weights];
         c.heavy.m32 = c.B32 + (c.heavy.j >= 0 ? c.heavy.j : 0);  // column j of B = row j of M
         c.heavy.ld = problem_dim;
         c.heavy.o32 = d_shift_data;

@@ -41,6 +41,8 @@ struct CompHost {
     float *wide32 = nullptr;    // M in the wide kernels' fragment order (wide_core.h): FP32,
     uint16_t *wide_bf = nullptr, *wide_h = nullptr;  // the three BF16 and the three FP16 parts
     float *colw = nullptr;      // [dim] bent cigar / discus weights (elliptic: ProblemHost::colw)
+    int heavy_j = -1;           // heavy_column of the objective, found once (it takes dim
+    double heavy_w = 0.0;       // powers, more host time than the launch of a small evaluation)
     bool unrotated = false;     // M = I: evaluated in FP32 whatever the requested precision,
                                 // where the identity GEMM is exact
 };

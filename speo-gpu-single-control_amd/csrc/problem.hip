@@ -95,7 +95,8 @@ CompDev ProblemHost::view(int c, int precision) const {
     for (int p = 0; p < 3; ++p) d.M16s[p] = half ? h.Mhs[p] : h.Mbfs[p];
     d.kp32 = round_up(dim, 32);
     d.wide = precision == SPEO_PREC_FP32 ? (const void *)h.wide32 : half ? (const void *)h.wide_h : (const void *)h.wide_bf;
-    d.heavy.j = heavy_column(h.objective, dim, &d.heavy.w);
+    d.heavy.j = h.heavy_j;
+    d.heavy.w = h.heavy_w;
     d.heavy.m64 = d.heavy.j >= 0 ? h.M64 + (size_t)d.heavy.j * dim : nullptr;
     d.heavy.o64 = h.shift64;
     d.heavy.o32 = h.shift32;
@@ -193,6 +194,7 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
     for (int c = 0; c < ncomp; ++c) {
         CompHost &h = P.comp[c];
         h.objective = objectives[c];
+        h.heavy_j = heavy_column(h.objective, dim, &h.heavy_w);
         if (h.objective == SPEO_OBJ_BENT_CIGAR || h.objective == SPEO_OBJ_DISCUS) {
             column_weights(h.objective, dim, w.data());
             SPEO_TRY(upload(&h.colw, w));
