@@ -113,3 +113,38 @@ def test_dropin_evaluation_equals_problem(cuda, speo, n, D):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(f.cpu().numpy(), g.cpu().numpy())
         p.close()
+
+
+@pytest.mark.parametrize("prec", range(6))
+@pytest.mark.parametrize("n,D", [(1, 2), (33, 30), (100, 128), (5000, 17), (20000, 5), (40000, 64)])
+def test_composition_components_in_one_launch(cuda, speo, n, D, prec):
+    """A composition of up to 128 columns (its components in one launch) against the
+    same sum of its components evaluated as problems of their own: 16, 32 and 64-row
+    tiles."""
+    import torch
+    print(f"n {n} D {D} precision {prec}", flush=True)
+    rng = np.random.default_rng([n, D])
+    objs = [speo.OBJ_ELLIPTIC, speo.OBJ_RASTRIGIN, speo.OBJ_ACKLEY]
+    o = np.float32(rng.uniform(-80, 80, (3, D))).astype(np.float64)
+    M = np.stack([np.linalg.qr(rng.standard_normal((D, D)))[0] for _ in objs])
+    X = torch.from_numpy(rng.uniform(-100, 100, (n, D)).astype(np.float32)).to(cuda)
+    sigma, bias, lam = [10.0, 20.0, 30.0], [0.0, 100.0, 200.0], [1e-6, 1.0, 1.0]
+    comp = speo.Problem(objs, o, M, sigma=sigma, bias=bias, lam=lam)
+    f, g = torch.zeros(n, device=cuda), torch.zeros(3, n, device=cuda)
+    speo.evaluate(comp, X, f, precision=prec)
+    for c in range(3):
+        p = speo.Problem(objs[c:c + 1], o[c:c + 1], M[c:c + 1], bias=[bias[c]], lam=[lam[c]])
+        speo.evaluate(p, X, g[c], precision=prec)
+        torch.cuda.synchronize()
+        p.close()
+    x, g = X.cpu().numpy().astype(np.float64), g.cpu().numpy().astype(np.float64)
+    d = ((x[:, None, :] - o[None]) ** 2).sum(2)
+    lw = -0.5 * np.log(d) - d / (2.0 * D * np.array(sigma) ** 2)
+    w = np.exp(lw - lw.max(1, keepdims=True))
+    want = (w * g.T).sum(1) / w.sum(1)
+    # The weights' exponents are FP32 sums of D squares up to 4e4 each, so a weight
+    # is off by up to (D + 4) 2^-24 times |lw| <= 2e2 relative; the values are sums
+    # of non-negative terms and carry it as it is.
+    bound = (D + 4) * 2.0 ** -24 * (np.abs(lw).max() + 8)
+    np.testing.assert_allclose(f.cpu().numpy(), want, rtol=2 * bound)
+    comp.close()
