@@ -1978,7 +1978,8 @@ int Engine::tune_launches() {
     if (epoch_plan_all(cfg.epoch_parts, &plans, &lds) != SPEO_OK) return SPEO_OK;  // epoch_setup reports it
     const std::string key = tune_key(("launches" + std::to_string(cfg.epoch_parts)).c_str());
     int stored = 0;
-    bool known = tune_lookup(key, &stored) && (stored == 0 || stored == 1);
+    const bool on_file = tune_lookup(key, &stored) && (stored == 0 || stored == 1);
+    bool known = on_file;
     if (!known) {
         std::lock_guard<std::mutex> lk(mu);
         auto it = chosen.find(key);
@@ -1990,8 +1991,8 @@ int Engine::tune_launches() {
         SPEO_TRY(time_plan(cfg.epoch_parts, false, &plan));
         SPEO_TRY(time_plan(cfg.epoch_parts, true, &launches));
         stored = launches < plan ? 1 : 0;
-        tune_store(key, stored);
     }
+    if (!on_file) tune_store(key, stored);  // (also a choice measured while another file was in use)
     by_launches = stored != 0;
     std::lock_guard<std::mutex> lk(mu);
     chosen[key] = stored;
