@@ -73,6 +73,9 @@ struct ProblemHost {
     bool generic = false;
     int *perm[kMaxComp] = {};       // hybrids: 1-based shuffle [dim] on the device
     GenProblem *gen = nullptr;      // the FP64 kernel's description, on the device (dim <= 1024)
+    // Every array above lies in one of two device allocations: the data, and the
+    // tables that point into it (params_dev, gen).
+    void *data = nullptr, *tables = nullptr;
 };
 
 }  // namespace speo

@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -104,41 +105,59 @@ CompDev ProblemHost::view(int c, int precision) const {
     return d;
 }
 
-template <typename T>
-static int upload(T **dst, const std::vector<T> &src) {
-    SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(dst), sizeof(T) * src.size()));
-    SPEO_TRY_HIP(hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice));
-    return SPEO_OK;
-}
+// Arrays gathered on the host and placed in one device allocation (a problem of
+// D = 100 has some twenty; an allocation and a copy for each took most of the
+// millisecond of its creation).
+class DeviceArrays {
+  public:
+    template <typename T>
+    void add(T **dst, const std::vector<T> &src) {
+        const char *p = reinterpret_cast<const char *>(src.data());
+        reserve(dst, src.size());
+        items_.back().bytes.assign(p, p + sizeof(T) * src.size());
+    }
+    // room for n elements that the device fills itself
+    template <typename T>
+    void reserve(T **dst, size_t n) {
+        items_.push_back(Item{[dst](char *at) { *dst = reinterpret_cast<T *>(at); }, size_, {}});
+        size_ += (sizeof(T) * n + 255) / 256 * 256;
+    }
+    int commit(void **allocation) {
+        SPEO_TRY_HIP(hipMalloc(allocation, size_));
+        char *base = static_cast<char *>(*allocation);
+        constexpr size_t kStage = 4u << 20;  // up to here gathered into one copy
+        std::vector<char> stage;
+        if (size_ <= kStage) stage.resize(size_);
+        for (Item &i : items_) {
+            i.place(base + i.at);
+            if (i.bytes.empty()) continue;
+            if (size_ <= kStage)
+                std::memcpy(stage.data() + i.at, i.bytes.data(), i.bytes.size());
+            else
+                SPEO_TRY_HIP(hipMemcpy(base + i.at, i.bytes.data(), i.bytes.size(), hipMemcpyHostToDevice));
+        }
+        if (!stage.empty()) SPEO_TRY_HIP(hipMemcpy(base, stage.data(), size_, hipMemcpyHostToDevice));
+        return SPEO_OK;
+    }
+
+  private:
+    struct Item {
+        std::function<void(char *)> place;
+        size_t at;
+        std::vector<char> bytes;
+    };
+    std::vector<Item> items_;
+    size_t size_ = 0;
+};
 
 static void free_problem(ProblemHost &P) {
-    for (int c = 0; c < kMaxComp; ++c) {
-        CompHost &h = P.comp[c];
-        (void)hipFree(h.shift32);
-        (void)hipFree(h.shift64);
-        (void)hipFree(h.B32);
-        (void)hipFree(h.M64);
-        (void)hipFree(h.M64f);
-        (void)hipFree(h.B32s);
-        for (int p = 0; p < 3; ++p) {
-            (void)hipFree(h.Mbf[p]);
-            (void)hipFree(h.Mh[p]);
-            (void)hipFree(h.Mbfs[p]);
-            (void)hipFree(h.Mhs[p]);
-        }
-        (void)hipFree(h.wide32);
-        (void)hipFree(h.colw);
-        h = CompHost{};
-    }
-    for (int c = 0; c < kMaxComp; ++c) {
-        (void)hipFree(P.perm[c]);
-        P.perm[c] = nullptr;
-    }
-    (void)hipFree(P.gen);
+    (void)hipFree(P.data);
+    (void)hipFree(P.tables);
+    for (CompHost &h : P.comp) h = CompHost{};
+    for (int *&p : P.perm) p = nullptr;
+    P.data = P.tables = nullptr;
     P.gen = nullptr;
     P.generic = false;
-    (void)hipFree(P.colw);
-    (void)hipFree(P.params_dev);
     P.colw = nullptr;
     P.params_dev = nullptr;
 }
@@ -189,7 +208,8 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
     const size_t D = (size_t)dim;
     std::vector<float> w(D);
     column_weights(SPEO_OBJ_ELLIPTIC, dim, w.data());
-    SPEO_TRY(upload(&P.colw, w));
+    DeviceArrays data, tables;
+    data.add(&P.colw, w);
     std::vector<CompParams> params((size_t)ncomp);
     for (int c = 0; c < ncomp; ++c) {
         CompHost &h = P.comp[c];
@@ -197,7 +217,7 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
         h.heavy_j = heavy_column(h.objective, dim, &h.heavy_w);
         if (h.objective == SPEO_OBJ_BENT_CIGAR || h.objective == SPEO_OBJ_DISCUS) {
             column_weights(h.objective, dim, w.data());
-            SPEO_TRY(upload(&h.colw, w));
+            data.add(&h.colw, w);
         }
         h.rate = rate ? (float)rate[c] : 1.0f;
         h.rate64 = rate ? rate[c] : 1.0;
@@ -213,13 +233,13 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
         std::vector<double> o(shift + (size_t)c * D, shift + (size_t)(c + 1) * D);
         std::vector<float> o32(D);
         for (size_t j = 0; j < D; ++j) o32[j] = (float)o[j];
-        SPEO_TRY(upload(&h.shift32, o32));
-        SPEO_TRY(upload(&h.shift64, o));
-        SPEO_TRY(upload(&h.M64, M));
+        data.add(&h.shift32, o32);
+        data.add(&h.shift64, o);
+        data.add(&h.M64, M);
         std::vector<float> B((size_t)dim * P.ldb32, 0.f);
         for (size_t k = 0; k < D; ++k)
             for (size_t cc = 0; cc < D; ++cc) B[k * P.ldb32 + cc] = (float)M[cc * D + k];
-        SPEO_TRY(upload(&h.B32, B));
+        data.add(&h.B32, B);
         std::vector<uint16_t> pb[3], ph[3];
         for (int p = 0; p < 3; ++p) {
             pb[p].assign((size_t)dim * P.ldm16, 0);
@@ -238,20 +258,15 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                 }
             }
         for (int p = 0; p < 3; ++p) {
-            SPEO_TRY(upload(&h.Mbf[p], pb[p]));
-            SPEO_TRY(upload(&h.Mh[p], ph[p]));
+            data.add(&h.Mbf[p], pb[p]);
+            data.add(&h.Mh[p], ph[p]);
         }
         // (the kernels move through the three parts by 32-bit byte offsets)
         const size_t fe = wide_frag_elems(dim);
         if (3 * 2 * fe < 0x7fffffffull) {
-            // one allocation: FP32, the BF16 parts, the FP16 parts
-            SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&h.wide32), (sizeof(float) + 2 * 3 * sizeof(uint16_t)) * fe));
-            h.wide_bf = reinterpret_cast<uint16_t *>(h.wide32 + fe);
-            h.wide_h = h.wide_bf + 3 * fe;
-            const uint16_t *src[6] = {h.Mbf[0], h.Mbf[1], h.Mbf[2], h.Mh[0], h.Mh[1], h.Mh[2]};
-            uint16_t *dst[6] = {h.wide_bf, h.wide_bf + fe, h.wide_bf + 2 * fe,
-                                h.wide_h, h.wide_h + fe, h.wide_h + 2 * fe};
-            SPEO_TRY(wide_fragments(h.B32, P.ldb32, src, P.ldm16, dim, h.wide32, dst, nullptr));
+            data.reserve(&h.wide32, fe);
+            data.reserve(&h.wide_bf, 3 * fe);
+            data.reserve(&h.wide_h, 3 * fe);
         }
         if (dim <= kSmallD) {
             const size_t kp32 = (size_t)round_up(dim, 32);
@@ -264,7 +279,7 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                             const size_t k = 16 * q + 4 * e + l / 16, cc = 16 * t + l % 16;
                             if (k < D && cc < D) Bs[((t * 8 + q) * 64 + l) * 4 + e] = (float)M[cc * D + k];
                         }
-            SPEO_TRY(upload(&h.B32s, Bs));
+            data.add(&h.B32s, Bs);
             for (int p = 0; p < 3; ++p) {
                 std::vector<uint16_t> sb((size_t)kSmallD * kp32, 0), sh((size_t)kSmallD * kp32, 0);
                 for (size_t r = 0; r < D; ++r)
@@ -272,14 +287,31 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                         sb[r * kp32 + k] = pb[p][r * P.ldm16 + k];
                         sh[r * kp32 + k] = ph[p][r * P.ldm16 + k];
                     }
-                SPEO_TRY(upload(&h.Mbfs[p], sb));
-                SPEO_TRY(upload(&h.Mhs[p], sh));
+                data.add(&h.Mbfs[p], sb);
+                data.add(&h.Mhs[p], sh);
             }
         }
+        if (dim <= kGenMaxDim) {
+            if (rotation && !h.unrotated) data.reserve(&h.M64f, gen_fragment_doubles(dim));
+            if (objectives[c] >= SPEO_OBJ_HYBRID_1)
+                data.add(&P.perm[c], std::vector<int>(shuffle + (size_t)c * dim, shuffle + (size_t)(c + 1) * dim));
+        }
+    }
+    SPEO_TRY(data.commit(&P.data));
+    for (int c = 0; c < ncomp; ++c) {
+        CompHost &h = P.comp[c];
         params[(size_t)c] = CompParams{h.objective, h.rate64, h.sigma, h.bias, h.lambda,
                                        h.shift32, h.shift64, h.M64};
+        if (h.wide32) {
+            const size_t fe = wide_frag_elems(dim);
+            const uint16_t *src[6] = {h.Mbf[0], h.Mbf[1], h.Mbf[2], h.Mh[0], h.Mh[1], h.Mh[2]};
+            uint16_t *dst[6] = {h.wide_bf, h.wide_bf + fe, h.wide_bf + 2 * fe,
+                                h.wide_h, h.wide_h + fe, h.wide_h + 2 * fe};
+            SPEO_TRY(wide_fragments(h.B32, P.ldb32, src, P.ldm16, dim, h.wide32, dst, nullptr));
+        }
+        if (h.M64f) SPEO_TRY(gen_fragments(h.M64, dim, h.M64f, nullptr));
     }
-    SPEO_TRY(upload(&P.params_dev, params));
+    tables.add(&P.params_dev, params);
     P.generic = generic;
     if (dim <= kGenMaxDim) {  // the FP64 kernel's description of the problem
         std::vector<GenProblem> gen(1);
@@ -289,8 +321,6 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
             const CompHost &h = P.comp[c];
             GenComp &g = gen[0].comp[c];
             if (objectives[c] >= SPEO_OBJ_HYBRID_1) {
-                std::vector<int> perm(shuffle + (size_t)c * dim, shuffle + (size_t)(c + 1) * dim);
-                SPEO_TRY(upload(&P.perm[c], perm));
                 hybrid_segments(objectives[c], dim, g);
                 g.perm = P.perm[c];
             } else {
@@ -298,21 +328,17 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
                 g.seg[0] = gen_seg(objectives[c], dim, 1.0);
             }
             g.rate = h.rate64;
-            g.rotate = rotation && !is_identity(rotation + (size_t)c * D * D, dim) ? 1 : 0;
+            g.rotate = h.M64f ? 1 : 0;
             g.o64 = h.shift64;
-            if (g.rotate) {
-                SPEO_TRY_HIP(hipMalloc(reinterpret_cast<void **>(&P.comp[c].M64f),
-                                       sizeof(double) * gen_fragment_doubles(dim)));
-                SPEO_TRY(gen_fragments(h.M64, dim, P.comp[c].M64f, nullptr));
-                g.M64f = h.M64f;
-            }
+            g.M64f = h.M64f;
             g.lambda = h.lambda;
             g.bias = h.bias;
             g.sigma = h.sigma;
         }
         SPEO_TRY(check_gen_problem(gen[0], false));
-        SPEO_TRY(upload(&P.gen, gen));
+        tables.add(&P.gen, gen);
     }
+    SPEO_TRY(tables.commit(&P.tables));
     SPEO_TRY_HIP(hipStreamSynchronize(nullptr));  // the fragments, for callers on other streams
     return SPEO_OK;
 }
