@@ -462,7 +462,7 @@ def config1_gpu(S):
     _, f32, f64 = eng.best()
     eng.close()
     prob.close()
-    return {"seconds": dt, "best_f64": float(f64[0]), "mode": "plain (3 launches / generation)"}
+    return {"seconds": dt, "best_f64": float(f64[0]), "mode": "plain (1 launch / generation)"}
 
 
 def cpu_baseline(data, seconds, D, NP):
