@@ -6,10 +6,10 @@
 //
 // What bounds it: the tile kernel's matrix work and its stages' LDS reads
 // (BF16x3, 8 islands x 2048 rows x 1000, three components: 335 us, 45 % of the
-// matrix pipe), then the row traffic of the trials (102 us) and the distances'
-// serial sums (51 us).  Evaluated inside the generation kernel, one block per
+// matrix pipe), then the row traffic of the trials (55 us) and the distances'
+// serial sums (26 us).  Evaluated inside the generation kernel, one block per
 // 64 rows with its components one after another and one lane per row for the
-// distances, a generation took 8.5 ms; 0.5 ms now.
+// distances, a generation took 8.5 ms; 0.42 ms now.
 //
 // Reference counterpart: API_evaluateFitness on an island's population
 // (kernel_CEC2014_CUDA.cu:147-181, 1672-1797) and the composition chain

@@ -774,17 +774,41 @@ struct TrainRowsArgs {
 // zero inputs with dy = 0, so they add nothing to any gradient.  Latency bound
 // (32 blocks a network): the rows' slots are drawn by every thread that gathers
 // them, and the transposed operands are stored from registers (15.3 us a step of
-// two networks with a shared draw and LDS transposes, 13.5 now).
+// two networks with a shared draw and LDS transposes, 13.5 without, 12.5 with each
+// network on XCDs of its own).
 // Networks trained in one launch (one per problem), each a run of blocks.
 constexpr int kMaxTrainNets = 8;
+// The chip's eight XCDs (workgroup b runs on XCD b % 8) have an L2 each, and a
+// training kernel's inputs were just written by workgroups on all of them.  With
+// 1, 2, 4 or 8 networks each network is kept to 8 / nn XCDs, which then fetch its
+// matrices alone: a workgroup's network and its place there (place % groups:
+// its XCD of the network's).
+struct TrainPlace {
+    int net, place, groups;
+};
+__device__ __forceinline__ TrainPlace train_place(int nets, int per_net) {
+    const int b = blockIdx.x;
+    if (8 % nets) return TrainPlace{b / per_net, b % per_net, 1};
+    const int groups = 8 / nets, x = b & 7;
+    return TrainPlace{x / groups, (b >> 3) * groups + x % groups, groups};
+}
+// Workgroups of a launch that train_place spreads; places >= per_net have no work.
+static int train_blocks(int nets, int per_net) {
+    if (8 % nets) return nets * per_net;
+    const int groups = 8 / nets;
+    return 8 * ((per_net + groups - 1) / groups);
+}
+
 struct TrainRowsBatch {
     TrainRowsArgs net[kMaxTrainNets];
-    int tiles;  // row tiles per network
+    int nets, tiles;  // networks, row tiles per network
 };
 
 template <int KP>
 __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
-    const TrainRowsArgs &a = batch.net[blockIdx.x / batch.tiles];
+    const TrainPlace at = train_place(batch.nets, batch.tiles);
+    if (at.place >= batch.tiles) return;
+    const TrainRowsArgs &a = batch.net[at.net];
     constexpr int TM = kTrainRows, LX = KP + 8, LH = kHidden + 8, NW = kHidden / 16;
     constexpr int K1 = KP / 32, K2 = kHidden / 32;
     __shared__ __align__(16) uint16_t Xs[TM * LX];
@@ -792,7 +816,7 @@ __global__ __launch_bounds__(1024) void k_train_rows(TrainRowsBatch batch) {
     __shared__ __align__(16) uint16_t Gs[TM * LH];  // dH2
     __shared__ float red[NW][TM];
     __shared__ float ts[TM], dys[TM], lts[TM];
-    const int tile = blockIdx.x % batch.tiles;
+    const int tile = at.place;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lk = lane >> 4;
     const int row0 = tile * TM;
@@ -1014,18 +1038,30 @@ struct TrainUpdateArgs {
 // after it).
 struct TrainUpdateBatch {
     TrainUpdateArgs net[kMaxTrainNets];
-    int blocks;  // blocks per network
+    int nets, blocks;  // networks, blocks per network
 };
 
 __global__ __launch_bounds__(256) void k_train_update(TrainUpdateBatch batch) {
-    const TrainUpdateArgs &a = batch.net[blockIdx.x / batch.blocks];
+    const TrainPlace at = train_place(batch.nets, batch.blocks);
+    if (at.place >= batch.blocks) return;
+    const TrainUpdateArgs &a = batch.net[at.net];
     float c1 = 1.f, c2 = 1.f;
     __shared__ float red[4][32][33];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lk = lane >> 4;
     constexpr int nW2 = (kHidden / 32) * (kHidden / 32);
     const int kt = a.L.Kp / 32, nW1 = (kHidden / 32) * kt;
-    const int bid = blockIdx.x % batch.blocks;
+    int bid = at.place;
+    // tile rows i0 of either gradient are shared out over the network's XCDs, so
+    // that one reads only its rows' part of the left operand
+    {
+        const int G = at.groups, x = bid % G, k = bid / G, rowsx = (kHidden / 32) / G;
+        if (k < rowsx * (kHidden / 32)) {
+            bid = x * rowsx * (kHidden / 32) + k;
+        } else if (k - rowsx * (kHidden / 32) < rowsx * kt) {
+            bid = nW2 + x * rowsx * kt + k - rowsx * (kHidden / 32);
+        }
+    }
     if (bid == nW2 + nW1) {
         // tile partials in tile order, eight tiles' loads in flight at a time
         const int c = tid;
@@ -1176,6 +1212,7 @@ static int fused_steps(Mlp *const *nets, const TrainRowsArgs *r0, int nn, bool g
     const int blocks = (kHidden / 32) * (kHidden / 32) + (kHidden / 32) * (Kp / 32) + 1;
     TrainRowsBatch rb{};
     TrainUpdateBatch ub{};
+    rb.nets = ub.nets = nn;
     rb.tiles = tiles;
     ub.blocks = blocks;
     for (int k = 0; k < nn; ++k) {
@@ -1222,7 +1259,7 @@ static int fused_steps(Mlp *const *nets, const TrainRowsArgs *r0, int nn, bool g
         u.stats = N.stats;
         u.want_loss = want_loss ? 1 : 0;
     }
-    const dim3 grid(tiles * nn), block(1024);
+    const dim3 grid(train_blocks(nn, tiles)), block(1024);
     switch (Kp) {
     case 32: hipLaunchKernelGGL(k_train_rows<32>, grid, block, 0, s, rb); break;
     case 64: hipLaunchKernelGGL(k_train_rows<64>, grid, block, 0, s, rb); break;
@@ -1231,7 +1268,7 @@ static int fused_steps(Mlp *const *nets, const TrainRowsArgs *r0, int nn, bool g
     default: return set_error(SPEO_ERR_ARG, "mlp: fused step needs Kp <= 128");
     }
     SPEO_TRY(check_launch("k_train_rows"));
-    hipLaunchKernelGGL(k_train_update, dim3(blocks * nn), dim3(256), 0, s, ub);
+    hipLaunchKernelGGL(k_train_update, dim3(train_blocks(nn, blocks)), dim3(256), 0, s, ub);
     return check_launch("k_train_update");
 }
 
