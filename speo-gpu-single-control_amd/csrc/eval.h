@@ -39,7 +39,8 @@ int eval_rows_f64(const CompParams *comps, int ncomp, int dim, const float *X, i
 int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double *f_out,
                      hipStream_t s);
 
-int default_rows_per_block(int n, int dim, int precision = SPEO_PREC_FP32);
+// kept: the rotation is kept in a problem's layouts (the drop-in call's is not).
+int default_rows_per_block(int n, int dim, int precision, bool kept);
 
 // The tile kernels of wide problems are switched on (speo_wide_eval).
 bool wide_eval_enabled();

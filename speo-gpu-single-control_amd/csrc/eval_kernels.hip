@@ -408,8 +408,7 @@ static int eval_components_small(const CompDev *comp, int ncomp, const float *X,
     switch (rows_per_block) {
     case 16: return launch_comps_rt<16>(a, ncomp, precision, s);
     case 32: return launch_comps_rt<32>(a, ncomp, precision, s);
-    case 64: return launch_comps_rt<64>(a, ncomp, precision, s);
-    default: return set_error(SPEO_ERR_ARG, "rows_per_block must be 16, 32 or 64");
+    default: return set_error(SPEO_ERR_ARG, "eval_components_small: 16 or 32 rows per block");
     }
 }
 
@@ -511,7 +510,12 @@ int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double
     return eval_rows_f64(P.params_dev, P.ncomp, P.dim, X, ld, n, f_out, s);
 }
 
-int default_rows_per_block(int n, int dim, int precision) {
+int default_rows_per_block(int n, int dim, int precision, bool kept) {
+    // Up to 128 columns from a problem's layouts the tile changes no result: 32
+    // rows once they give a block a compute unit (Rastrigin, us at 16 / 32 / 64
+    // rows: 4,096 x 100 FP32 5.3 / 6.5 / 9.8, 65,536 x 100 BF16 19.5 / 15.6 /
+    // 17.3, 65,536 x 128 FP32 29.7 / 29.7 / 31.0).
+    if (kept && dim <= kSmallD) return (n + 31) / 32 >= 256 ? 32 : 16;
     // Enough blocks to cover the 256 CUs; larger tiles share B staging.
     const int nchunks = (dim + kNC - 1) / kNC;
     // 16-bit evaluations wider than one chunk: 64-row arithmetic from 1024
@@ -724,6 +728,7 @@ extern "C" void API_evaluateFitness(real *d_fitness_value, real *, real *d_rotat
     }
     const int rc = eval_component(c, d_original_elements, ld, pop_size, problem_dim,
                                   d_fitness_value, part, 1.f, 0.f, 0, SPEO_PREC_FP32,
-                                  default_rows_per_block(pop_size, problem_dim), nullptr);
+                                  default_rows_per_block(pop_size, problem_dim, SPEO_PREC_FP32, false),
+                                  nullptr);
     if (rc != SPEO_OK) defer_error(rc, speo_last_error());
 }
