@@ -39,6 +39,10 @@ int eval_rows_f64(const CompParams *comps, int ncomp, int dim, const float *X, i
 int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double *f_out,
                      hipStream_t s);
 
+// Floats that eval_problem can use beyond eval_scratch_batched (rounded up to
+// four): an aligned copy of rows wider than 128 columns that 16-byte accesses
+// cannot take as they are (0: they can, or the copy would pass 1 GiB).
+size_t eval_pack_floats(const ProblemHost &P, const float *X, int ld, int n);
 // kept: the rotation is kept in a problem's layouts (the drop-in call's is not).
 int default_rows_per_block(int n, int dim, int precision, bool kept);
 

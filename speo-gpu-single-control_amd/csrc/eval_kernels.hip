@@ -454,11 +454,45 @@ size_t eval_scratch_batched(int ncomp, int dim, int n) {
     return (size_t)ncomp * n * (2 * nchunks + 1);
 }
 
+// Rows copied to a stride of a multiple of four floats, the padding zero: a wave
+// a row, consecutive lanes consecutive floats.
+__global__ __launch_bounds__(256) void k_pack_rows(const float *X, int ld, int n, int dim, int ldp, float *out) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= n) return;
+    const float *x = X + (size_t)r * ld;
+    float *o = out + (size_t)r * ldp;
+#pragma unroll 4
+    for (int j = lane; j < ldp; j += 64) o[j] = j < dim ? x[j] : 0.f;
+}
+
+size_t eval_pack_floats(const ProblemHost &P, const float *X, int ld, int n) {
+    if (P.generic || P.dim <= kSmallD || n <= 0) return 0;
+    if ((ld & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0) return 0;
+    const size_t floats = (size_t)n * round_up(P.dim, 4);
+    return floats <= (size_t(1) << 28) ? floats : 0;
+}
+
 int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out, float *scratch,
                  size_t scratch_floats, int precision, int rows_per_block, hipStream_t s) {
     if (n <= 0) return SPEO_OK;
     if (P.generic) return eval_problem_generic(P, X, ld, n, f_out, nullptr, nullptr, 0, s);
     const int nchunks = (P.dim + kNC - 1) / kNC;
+    // Rows that 16-byte accesses cannot take (an odd stride, as torch's rows of
+    // an odd dimension have) are copied once where the scratch has room: staged
+    // element by element they kept the tile kernels out altogether (16,172 rows
+    // of D = 991 in BF16: 702 us, 73 us with the copy; 64 rows of D = 131 19 and
+    // 10 us; same bits).  The combination
+    // below reads the caller's rows, as its sums' order depends on the alignment.
+    const float *Xc = X;
+    const int ldc = ld;
+    const size_t pack = eval_pack_floats(P, X, ld, n), at = (eval_scratch_batched(P.ncomp, P.dim, n) + 3) / 4 * 4;
+    if (pack && scratch_floats >= at + pack && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0) {
+        const int ldp = round_up(P.dim, 4);
+        hipLaunchKernelGGL(k_pack_rows, dim3((n + 3) / 4), dim3(256), 0, s, X, ld, n, P.dim, ldp, scratch + at);
+        SPEO_TRY(check_launch("k_pack_rows"));
+        X = scratch + at;
+        ld = ldp;
+    }
     float *part = nchunks > 1 ? scratch : nullptr;
     float *gbuf = scratch + (nchunks > 1 ? (size_t)nchunks * 2 * n : 0);
     // an unrotated component's z = (x - o) rate is exact in FP32; a 16-bit
@@ -487,18 +521,18 @@ int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_o
     for (int c = 0; c < P.ncomp && !batched && !small; ++c)
         SPEO_TRY(eval_component(view[c], X, ld, n, P.dim, gbuf + (size_t)c * n, part,
                                 1.f, 0.f, 1, prec_of(c), rows_per_block, s));
-    bool rows = (P.dim & 3) == 0 && P.dim <= 1024 && (ld & 3) == 0 &&
-                (reinterpret_cast<uintptr_t>(X) & 15) == 0 && n >= 4096;
+    bool rows = (P.dim & 3) == 0 && P.dim <= 1024 && (ldc & 3) == 0 &&
+                (reinterpret_cast<uintptr_t>(Xc) & 15) == 0 && n >= 4096;
     for (int c = 0; c < P.ncomp; ++c) rows = rows && (reinterpret_cast<uintptr_t>(P.comp[c].shift32) & 15) == 0;
     if (rows) {
         hipLaunchKernelGGL(k_comp_combine_rows, dim3((n + 4 * kCombRows - 1) / (4 * kCombRows)), dim3(256),
-                           sizeof(float) * (size_t)P.ncomp * P.dim, s, P.params_dev, P.ncomp, P.dim, X, ld,
+                           sizeof(float) * (size_t)P.ncomp * P.dim, s, P.params_dev, P.ncomp, P.dim, Xc, ldc,
                            n, gbuf, f_out);
         return check_launch("k_comp_combine_rows");
     }
     const int waves_per_block = 4;
     hipLaunchKernelGGL(k_comp_combine, dim3((n + waves_per_block - 1) / waves_per_block),
-                       dim3(64 * waves_per_block), 0, s, P.params_dev, P.ncomp, P.dim, X, ld, n,
+                       dim3(64 * waves_per_block), 0, s, P.params_dev, P.ncomp, P.dim, Xc, ldc, n,
                        gbuf, f_out);
     return check_launch("k_comp_combine");
 }

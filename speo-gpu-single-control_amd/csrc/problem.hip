@@ -570,13 +570,20 @@ int speo_evaluate(speo_problem p, const float *X, int ld, int n, float *f_out, i
         return set_error(SPEO_ERR_ARG, "speo_evaluate: bad arguments");
     if (precision < SPEO_PREC_FP32 || precision > SPEO_PREC_BF16X6)
         return set_error(SPEO_ERR_ARG, "speo_evaluate: unknown precision");
-    const size_t need = eval_scratch_batched(p->h.ncomp, p->h.dim, n);
+    const size_t base = eval_scratch_batched(p->h.ncomp, p->h.dim, n), pack = eval_pack_floats(p->h, X, ld, n);
+    size_t need = pack ? (base + 3) / 4 * 4 + pack : base;
     if (need > p->scratch_cap) {
         SPEO_TRY_HIP(hipStreamSynchronize(as_stream(stream)));
         (void)hipFree(p->scratch);
         p->scratch = nullptr;
         p->scratch_cap = 0;
-        SPEO_TRY_HIP(hipMalloc(&p->scratch, sizeof(float) * need));
+        hipError_t e = hipMalloc(&p->scratch, sizeof(float) * need);
+        if (e == hipErrorOutOfMemory && pack && base) {  // without room for the copy, as the rows are
+            (void)hipGetLastError();
+            need = base;
+            e = hipMalloc(&p->scratch, sizeof(float) * need);
+        }
+        SPEO_TRY_HIP(e);
         p->scratch_cap = need;
     }
     return eval_problem(p->h, X, ld, n, f_out, p->scratch, p->scratch_cap, precision,

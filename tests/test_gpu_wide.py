@@ -63,3 +63,35 @@ def test_batched_components_equal_one_launch_each(cuda, speo, prec):
     speo.evaluate_noalloc(prob, X, b, precision=prec)
     np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
     prob.close()
+
+
+@pytest.mark.parametrize("prec", range(6))
+@pytest.mark.parametrize("n,D,extra,shift", [(5, 129, 0, 0), (700, 301, 0, 0), (3000, 515, 0, 0), (3000, 200, 1, 0),
+                                             (1500, 256, 0, 1), (9000, 131, 2, 3)])
+def test_unaligned_rows_equal_aligned(cuda, speo, n, D, extra, shift, prec):
+    """Rows with a stride or a start off 16 bytes, copied first, against the same rows
+    aligned (the components' values, single objectives: bit for bit) and against the
+    workspace without room for the copy."""
+    import torch
+    print(f"n {n} D {D} stride +{extra} start +{shift} precision {prec}", flush=True)
+    rng = np.random.default_rng([n, D])
+    ld, lda = D + extra, (D + 3) // 4 * 4
+    X = rng.uniform(-100, 100, (n, D)).astype(np.float32)
+    flat = torch.full((n * ld + 8,), float("nan"), device=cuda)
+    Xu = flat[shift:shift + n * ld].view(n, ld)
+    Xu[:, :D] = torch.from_numpy(X).to(cuda)
+    Xa = torch.zeros((n, lda), device=cuda)
+    Xa[:, :D] = torch.from_numpy(X).to(cuda)
+    for obj in (speo.OBJ_RASTRIGIN, speo.OBJ_DISCUS):
+        p = speo.Problem([obj], rng.uniform(-80, 80, (1, D)), np.linalg.qr(rng.standard_normal((D, D)))[0][None])
+        f, g, h = (torch.zeros(n, device=cuda) for _ in range(3))
+        speo.evaluate(p, Xu, f, precision=prec, ld=ld)
+        speo.evaluate(p, Xa, g, precision=prec, ld=lda)
+        m = min(n, 2 ** 20 // (2 * ((D + 127) // 128)))
+        speo.evaluate_noalloc(p, Xu, h, precision=prec, ld=ld, n=m)
+        torch.cuda.synchronize()
+        assert torch.isfinite(f).all()
+        np.testing.assert_array_equal(f.cpu().numpy(), g.cpu().numpy())
+        if m == n:  # (the same rows per block)
+            np.testing.assert_array_equal(h.cpu().numpy(), g.cpu().numpy())
+        p.close()
