@@ -64,10 +64,24 @@ __device__ __forceinline__ void eval_rows(const EvalLaunch &p, const CompDev &c,
                 *reinterpret_cast<floatx4 *>(rows + r * kTS + 4 * g) = v;
             }
         } else {
-            for (int e = threadIdx.x; e < RT * kp4; e += 256) {
-                const int r = e / kp4, k = e % kp4;
-                rows[r * kTS + k] = (r < nrows && k < p.dim) ? p.X[(size_t)(row0 + r) * p.ld + k] : 0.f;
-            }
+            // a wave per row, every fourth row; all loads of the tile issued
+            // before the first is stored
+            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+            float x[RT / 4][2];
+#pragma unroll
+            for (int i = 0; i < RT / 4; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int r = min(wave + 4 * i, nrows - 1), k = min(lane + 64 * h, p.dim - 1);
+                    x[i][h] = gld(p.X + (size_t)(row0 + r) * p.ld + k);
+                }
+#pragma unroll
+            for (int i = 0; i < RT / 4; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int r = wave + 4 * i, k = lane + 64 * h;
+                    if (k < kp4) rows[r * kTS + k] = r < nrows && k < p.dim ? x[i][h] : 0.f;
+                }
         }
         if constexpr (F32) B.stage(scratch);
         __syncthreads();
