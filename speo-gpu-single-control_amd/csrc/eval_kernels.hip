@@ -163,8 +163,10 @@ __global__ void k_eval_finalize(const float *part, int nchunks, int n, int dim, 
 // (per-lane partial sums, then a butterfly over the 64 lanes), the cf_cal
 // weights in the log domain and the weighted sum.  When the row stride, X and
 // every shift allow 16-byte loads and dim % 4 == 0, lane l takes coordinates
-// 4 (l + 64 i) .. + 3 and the row (dim <= 1024) is read once into registers
-// for all components; otherwise coordinates l + 64 i, one at a time.
+// 4 (l + 64 i) .. + 3; otherwise coordinates l + 64 i.  Up to 1024 coordinates
+// the row is read once into registers for all components (4,000 rows of D = 515
+// and three components in BF16: 46.2 us with the row read again for each, 41.8
+// so; compiled for at most four waves a SIMD unit it was slower than either).
 __global__ void k_comp_combine(const CompParams *comps, int ncomp, int dim, const float *X,
                                int ld, int n, const float *g, float *f_out) {
     constexpr int kGroups = 4;  // float4 groups per lane held in registers
@@ -184,6 +186,14 @@ __global__ void k_comp_combine(const CompParams *comps, int ncomp, int dim, cons
             xr[i] = q < ng ? *reinterpret_cast<const float4 *>(x + 4 * q) : float4{0.f, 0.f, 0.f, 0.f};
         }
     }
+    constexpr int kSingles = 16;  // coordinates per lane held where 16-byte loads cannot be used
+    const bool held = !vec && dim <= 64 * kSingles;
+    float xs[kSingles];
+    if (held) {
+#pragma unroll
+        for (int i = 0; i < kSingles; ++i)
+            if (64 * i < dim) xs[i] = gld(x + min(lane + 64 * i, dim - 1));
+    }
     float lw[kMaxComp];
     bool zero[kMaxComp];
     bool any_zero = false;
@@ -191,7 +201,18 @@ __global__ void k_comp_combine(const CompParams *comps, int ncomp, int dim, cons
     for (int c = 0; c < ncomp; ++c) {
         const float *o = comps[c].shift32;
         float d = 0.f;
-        if (vec) {
+        if (held) {
+            float os[kSingles];
+#pragma unroll
+            for (int i = 0; i < kSingles; ++i)
+                if (64 * i < dim) os[i] = gld(o + min(lane + 64 * i, dim - 1));
+#pragma unroll
+            for (int i = 0; i < kSingles; ++i)
+                if (lane + 64 * i < dim) {
+                    const float v = xs[i] - os[i];
+                    d = fmaf(v, v, d);
+                }
+        } else if (vec) {
 #pragma unroll
             for (int i = 0; i < kGroups; ++i) {
                 const int q = lane + 64 * i;
