@@ -213,7 +213,10 @@ bool eval_wide_applies(const CompDev &c, const float *X, int ld, int n, int dim,
     case SPEO_PREC_BF16X6: lds = EvalTile<SPEO_PREC_BF16X6>::LDS; break;
     default: return false;
     }
+    static_assert(EvalTile<SPEO_PREC_FP32>::RB == EvalTile<SPEO_PREC_BF16>::RB &&
+                  EvalTile<SPEO_PREC_FP32>::RB == EvalTile<SPEO_PREC_BF16X6>::RB, "one bound on the stride");
     return c.wide && dim > kNC && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 &&
+           wide_stride_fits(EvalTile<SPEO_PREC_FP32>::RB, ld) &&
            lds + 4 * round_up(dim, 32) <= kWideLdsMax;
 }
 

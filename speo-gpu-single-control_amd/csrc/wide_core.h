@@ -66,6 +66,26 @@ typedef __attribute__((address_space(3))) void *lds_ptr;
 
 constexpr int kWideLdsMax = 160 * 1024;  // LDS of one CU
 
+// Addresses of a block's rows, in bytes from its first row.  Row piece f holds
+// rows 8 f .. 8 f + 7; lane l of the wave that copies it starts at its row 8 f +
+// l / 8 with the 16-byte group that the swizzle stores there ((8 f + l / 8) / 2
+// mod 8 = 4 (f mod 2) + l / 16), and K stage s adds 128 s.
+__host__ __device__ inline int wide_row_offset(int f, int lane, int ld) {
+    const int group = (lane & 7) ^ ((4 * (f & 1) + (lane >> 4)) & 7);
+    return ((8 * f + (lane >> 3)) * ld + 4 * group) * 4;
+}
+// What of them may be read: the caller's rows end with the last row's last
+// column (rows of a wider matrix's column slice have nothing behind it), and the
+// last stage asks for the columns up to a multiple of 32.  The buffer's range
+// check, which counts the stage's scalar offset, returns 0 for the rest.
+__host__ __device__ inline int wide_row_bytes(int nrows, int ld, int dim) {
+    return ((nrows - 1) * ld + round_up(dim, 4)) * 4;
+}
+// Row strides whose offsets over a block's rows stay within 31 bits.
+__host__ __device__ inline bool wide_stride_fits(int rows_per_block, int ld) {
+    return (int64_t)rows_per_block * ld * 4 <= 0x7fffffff;
+}
+
 // A block's rows and operand.
 struct WideOperands {
     const float *rows;   // first row of the block
@@ -95,13 +115,11 @@ __device__ __forceinline__ void wide_gemm(const WideOperands &o, int chunk0, int
     const float sa = H ? kF16ScaleA : 1.0f;
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(o.rows), (short)0, o.nrows * o.ld * 4, kBufferWord3);
+        const_cast<float *>(o.rows), (short)0, wide_row_bytes(o.nrows, o.ld, dim), kBufferWord3);
     const __amdgpu_buffer_rsrc_t mr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void *>(o.frag), (short)0, (int)0xffffffff, kBufferWord3);
-    // row piece f = wave + NW j: rows 8 f .. 8 f + 7, lane l row 8 f + l / 8
-    // ((8 f + l / 8) / 2 mod 8 = 4 (f mod 2) + l / 16: f mod 2 = wave mod 2)
-    const int agrp = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
-    const int avoff = ((8 * wave + (lane >> 3)) * o.ld + 4 * agrp) * 4;
+    // row pieces f = wave + NW j (NW is even: one swizzle for all of a wave's)
+    const int avoff = wide_row_offset(wave, lane, o.ld);
     const int arow8 = 8 * W::NW * o.ld * 4;  // bytes between the wave's row pieces
 
     auto issue = [&](int chunk, int s, int buf) __attribute__((always_inline)) {

@@ -95,3 +95,43 @@ def test_unaligned_rows_equal_aligned(cuda, speo, n, D, extra, shift, prec):
         if m == n:  # (the same rows per block)
             np.testing.assert_array_equal(h.cpu().numpy(), g.cpu().numpy())
         p.close()
+
+
+@pytest.mark.parametrize("D,start,ld,n,prec", [(132, 64, 196, 20481, 0), (232, 280, 512, 1031, 3), (260, 4, 264, 1153, 1),
+                                               (131, 24, 156, 1025, 5)])
+def test_column_slices_equal_whole_rows(cuda, speo, D, start, ld, n, prec):
+    """Rows that are the last columns of a wider matrix: nothing of the caller's lies
+    behind the last row's last column (D = 131: one column of padding)."""
+    import torch
+    prob = _problem(speo, [2], D, D)
+    X = _rows(n, D, D + (-D) % 4, cuda)
+    parent = torch.full((n, ld), float("nan"), device=cuda)
+    parent[:, start:start + D] = X[:, :D]
+    f, g = torch.zeros(n, device=cuda), torch.zeros(n, device=cuda)
+    print(f"D={D} columns {start}.. of {ld} n={n} prec={prec}", flush=True)
+    before = speo.wide_eval(-1)[1]
+    speo.evaluate(prob, parent[:, start:], f, precision=prec, ld=ld, n=n)
+    speo.evaluate(prob, X, g, precision=prec, ld=X.shape[1])
+    torch.cuda.synchronize()
+    assert speo.wide_eval(-1)[1] == before + 2
+    assert torch.isfinite(f).all()
+    np.testing.assert_array_equal(f.cpu().numpy(), g.cpu().numpy())
+    prob.close()
+
+
+def test_stride_beyond_31_bit_offsets(cuda, speo):
+    """A tile of 128 rows 2^22 floats apart does not fit 31-bit byte offsets: the 64-row
+    kernel takes such rows, with the values of the same rows side by side."""
+    import torch
+    D, n, ld = 160, 1030, 2 ** 22
+    prob = _problem(speo, [2], D, D)
+    X = _rows(n, D, D, cuda)
+    far = torch.empty((n, ld), device=cuda)
+    far[:, :D] = X
+    f, g = torch.zeros(n, device=cuda), torch.zeros(n, device=cuda)
+    print(f"D={D} n={n} ld={ld}", flush=True)
+    speo.evaluate(prob, far, f, precision=speo.PREC_BF16, ld=ld)
+    speo.evaluate(prob, X, g, precision=speo.PREC_BF16)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(f.cpu().numpy(), g.cpu().numpy())
+    prob.close()
