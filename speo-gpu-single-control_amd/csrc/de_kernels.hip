@@ -91,14 +91,20 @@ __device__ __forceinline__ bool uses_best(int st) { return st == 2 || st == 3 ||
 // LPR lanes per row, four coordinates each.  The call is bound by latency at
 // the drop-in sizes (donor draws, indices, rows, crossover draws, one after
 // another), so up to kWaveRows rows take a wave each: its draws diverge over no
-// other row and its rows' addresses are scalars.  Beyond, where the chip is
-// full, 16 lanes a row repeat the draws least.
+// other row and its rows' addresses are scalars.  Beyond, 16 lanes a row repeat
+// the draws least (D = 100, rand/1, a wave / 16 lanes a row: 1,024 rows 5.0 / 6.1
+// us, 2,048 6.9 / 6.2, 4,096 11.5 / 8.7).
 // a.fit: the sub-islands' best members are found here too, by blocks past the
 // rows' for the caller and, where the strategy reads it, by the rows' own blocks
-// (S a multiple of a block's rows, at most kBestMembers).
+// (S a multiple of a block's rows): 4 to 5 us less than a launch of its own.  The
+// rows' searches are row blocks x S reads; up to kBestReads of them such a strategy
+// costs within 2 us of the two launches up to 16,384 rows (best/1, here / apart:
+// 8,192 as 1 island 20.5 / 20.9 us, 16,384 as 4 22.5 / 21.2) and the others gain;
+// at twice that (65,536 as 32: 55.6 / 32.6) it is slower than ever.
 // 1,024 rows, D = 100: best 5.1 us and generate 10.7 us as two launches of 16
-// lanes a row and scalar loads, 6.9 us now.
-constexpr int kWaveRows = 8192, kBestMembers = 4096;
+// lanes a row and scalar loads, 5.0 us now.
+constexpr int kWaveRows = 1024;
+constexpr int64_t kBestReads = 1 << 22;
 
 template <bool INJ, int LPR>
 __global__ __launch_bounds__(256) void k_de_generate(GenArgs a) {
@@ -195,7 +201,7 @@ static int launch_generate(GenArgs a, hipStream_t s) {
     constexpr int RB = 256 / LPR;
     int blocks = (a.n + RB - 1) / RB;
     if (a.fit) {
-        if (a.S % RB == 0 && a.S <= kBestMembers) {
+        if (a.S % RB == 0 && (int64_t)blocks * a.S <= kBestReads) {
             blocks += a.n / a.S;
         } else {
             SPEO_TRY(subisland_best(a.fit, a.perm, a.S, a.n / a.S, a.best_out, s));
@@ -210,7 +216,10 @@ static int launch_generate(GenArgs a, hipStream_t s) {
 int de_generate(const GenArgs &a, hipStream_t s) {
     if (a.n <= 0) return SPEO_OK;
     const bool inj = a.inj_r || a.inj_cr;
-    if (a.n <= kWaveRows) return inj ? launch_generate<true, 64>(a, s) : launch_generate<false, 64>(a, s);
+    // (sub-islands that only the smaller blocks divide keep them to 4,096 rows: 1,024 a
+    // sub-island 8.4 us, 10.5 with the search apart)
+    const bool wave = a.n <= kWaveRows || (a.fit && a.n <= 4 * kWaveRows && a.S % 16 && a.S % 4 == 0);
+    if (wave) return inj ? launch_generate<true, 64>(a, s) : launch_generate<false, 64>(a, s);
     return inj ? launch_generate<true, 16>(a, s) : launch_generate<false, 16>(a, s);
 }
 

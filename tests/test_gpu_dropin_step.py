@@ -148,3 +148,11 @@ def test_composition_components_in_one_launch(cuda, speo, n, D, prec):
     bound = (D + 4) * 2.0 ** -24 * (np.abs(lw).max() + 8)
     np.testing.assert_allclose(f.cpu().numpy(), want, rtol=2 * bound)
     comp.close()
+
+
+@pytest.mark.parametrize("n,subs,strategy", [(1024, 1, 2), (1040, 1, 3), (2000, 100, 6), (4100, 205, 7), (8192, 1, 2),
+                                             (16384, 2, 3), (16400, 1, 6), (32768, 16, 7)])
+def test_generation_at_the_lines(cuda, speo, oracle, n, subs, strategy):
+    """Either side of the lines between a wave and 16 lanes a row, and between the search
+    in the rows' own launch (row blocks x members <= 2^22) and a launch of its own."""
+    test_generation_finds_best(cuda, speo, oracle, n, subs, 13, strategy)
