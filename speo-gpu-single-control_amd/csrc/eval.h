@@ -28,9 +28,10 @@ size_t eval_scratch_floats(int ncomp, int dim, int n);
 size_t eval_scratch_batched(int ncomp, int dim, int n);
 
 // Whole problem (single component or composition) over n rows; scratch holds
-// scratch_floats floats.
+// scratch_floats floats; packed: null, or room for eval_pack_floats (16-byte
+// aligned), to which the rows are copied first.
 int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out, float *scratch,
-                 size_t scratch_floats, int precision, int rows_per_block, hipStream_t s);
+                 size_t scratch_floats, float *packed, int precision, int rows_per_block, hipStream_t s);
 
 // FP64 evaluation: the generic kernel up to its 1024 columns, else one block
 // per row (eval_rows_f64).
@@ -39,8 +40,7 @@ int eval_rows_f64(const CompParams *comps, int ncomp, int dim, const float *X, i
 int eval_problem_f64(const ProblemHost &P, const float *X, int ld, int n, double *f_out,
                      hipStream_t s);
 
-// Floats that eval_problem can use beyond eval_scratch_batched (rounded up to
-// four): an aligned copy of rows wider than 128 columns that 16-byte accesses
+// Floats of an aligned copy of rows wider than 128 columns that 16-byte accesses
 // cannot take as they are (0: they can, or the copy would pass 1 GiB).
 size_t eval_pack_floats(const ProblemHost &P, const float *X, int ld, int n);
 // kept: the rotation is kept in a problem's layouts (the drop-in call's is not).

@@ -508,24 +508,23 @@ size_t eval_pack_floats(const ProblemHost &P, const float *X, int ld, int n) {
 }
 
 int eval_problem(const ProblemHost &P, const float *X, int ld, int n, float *f_out, float *scratch,
-                 size_t scratch_floats, int precision, int rows_per_block, hipStream_t s) {
+                 size_t scratch_floats, float *packed, int precision, int rows_per_block, hipStream_t s) {
     if (n <= 0) return SPEO_OK;
     if (P.generic) return eval_problem_generic(P, X, ld, n, f_out, nullptr, nullptr, 0, s);
     const int nchunks = (P.dim + kNC - 1) / kNC;
     // Rows that 16-byte accesses cannot take (an odd stride, as torch's rows of
-    // an odd dimension have) are copied once where the scratch has room: staged
-    // element by element they kept the tile kernels out altogether (16,172 rows
-    // of D = 991 in BF16: 702 us, 73 us with the copy; 64 rows of D = 131 19 and
-    // 10 us; same bits).  The combination
-    // below reads the caller's rows, as its sums' order depends on the alignment.
+    // an odd dimension have) are copied once where there is room: staged element by
+    // element they kept the tile kernels out altogether (16,172 rows of D = 991 in
+    // BF16: 702 us, 73 us with the copy; 64 rows of D = 131 19 and 10 us; same
+    // bits).  The combination below reads the caller's rows, as its sums' order
+    // depends on the alignment.
     const float *Xc = X;
     const int ldc = ld;
-    const size_t pack = eval_pack_floats(P, X, ld, n), at = (eval_scratch_batched(P.ncomp, P.dim, n) + 3) / 4 * 4;
-    if (pack && scratch_floats >= at + pack && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0) {
+    if (packed) {
         const int ldp = round_up(P.dim, 4);
-        hipLaunchKernelGGL(k_pack_rows, dim3((n + 3) / 4), dim3(256), 0, s, X, ld, n, P.dim, ldp, scratch + at);
+        hipLaunchKernelGGL(k_pack_rows, dim3((n + 3) / 4), dim3(256), 0, s, X, ld, n, P.dim, ldp, packed);
         SPEO_TRY(check_launch("k_pack_rows"));
-        X = scratch + at;
+        X = packed;
         ld = ldp;
     }
     float *part = nchunks > 1 ? scratch : nullptr;

@@ -54,6 +54,9 @@ extern "C" int speo_evaluate_noalloc(speo_problem p, const float *X, int ld, int
                                            std::to_string(kNoAllocScratchFloats) + " it holds");
     float *ws = nullptr;
     SPEO_TRY(scratch_ptr(&ws));
-    return eval_problem(p->h, X, ld, n, f_out, ws, kNoAllocScratchFloats, precision, default_rows_per_block(n, p->h.dim, precision, true),
-                        as_stream(stream));
+    // (what the sums leave takes the copy of rows off 16 bytes, where it fits)
+    const size_t pack = eval_pack_floats(p->h, X, ld, n), at = (eval_scratch_batched(p->h.ncomp, p->h.dim, n) + 3) / 4 * 4;
+    const bool copy = pack && at + pack <= kNoAllocScratchFloats && (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    return eval_problem(p->h, X, ld, n, f_out, ws, kNoAllocScratchFloats, copy ? ws + at : nullptr, precision,
+                        default_rows_per_block(n, p->h.dim, precision, true), as_stream(stream));
 }

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "eval_core.h"
+#include "workspace.h"
 
 namespace speo {
 
@@ -82,6 +83,8 @@ struct ProblemHost {
 
 struct speo_problem_s {
     speo::ProblemHost h;
-    float *scratch = nullptr;  // eval_problem workspace of speo_evaluate
-    size_t scratch_cap = 0;
+    // speo_evaluate's: the sums of eval_problem, and rows copied to an aligned
+    // stride (a buffer of its own, so that a captured evaluation of aligned rows
+    // keeps its sums' addresses when rows of another stride come)
+    speo::Workspace scratch, packed;
 };

@@ -150,6 +150,29 @@ class DeviceArrays {
     size_t size_ = 0;
 };
 
+// A workspace's device memory, for calls on one stream.
+struct StreamMemory {
+    hipStream_t s;
+    hipError_t failed = hipSuccess;
+    bool may_allocate() {
+        hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &c) == hipSuccess) return c == hipStreamCaptureStatusNone;
+        (void)hipGetLastError();  // (the null stream beside a capture)
+        return false;
+    }
+    int settle() { return (failed = hipStreamSynchronize(s)) != hipSuccess; }
+    int allocate(float **out, size_t floats) {
+        failed = hipMalloc(reinterpret_cast<void **>(out), sizeof(float) * floats);
+        if (failed == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            return Workspace::kNoRoom;
+        }
+        return failed != hipSuccess;
+    }
+    void release(float *p) { (void)hipFree(p); }
+    int status(int rc) const { return rc ? check_hip(failed, "workspace") : SPEO_OK; }
+};
+
 static void free_problem(ProblemHost &P) {
     (void)hipFree(P.data);
     (void)hipFree(P.tables);
@@ -556,7 +579,8 @@ int speo_problem_destroy(speo_problem p) {
     if (!p) return SPEO_OK;
     (void)hipDeviceSynchronize();
     free_problem(p->h);
-    (void)hipFree(p->scratch);
+    (void)hipFree(p->scratch.p);
+    (void)hipFree(p->packed.p);
     delete p;
     return SPEO_OK;
 }
@@ -570,23 +594,15 @@ int speo_evaluate(speo_problem p, const float *X, int ld, int n, float *f_out, i
         return set_error(SPEO_ERR_ARG, "speo_evaluate: bad arguments");
     if (precision < SPEO_PREC_FP32 || precision > SPEO_PREC_BF16X6)
         return set_error(SPEO_ERR_ARG, "speo_evaluate: unknown precision");
-    const size_t base = eval_scratch_batched(p->h.ncomp, p->h.dim, n), pack = eval_pack_floats(p->h, X, ld, n);
-    size_t need = pack ? (base + 3) / 4 * 4 + pack : base;
-    if (need > p->scratch_cap) {
-        SPEO_TRY_HIP(hipStreamSynchronize(as_stream(stream)));
-        (void)hipFree(p->scratch);
-        p->scratch = nullptr;
-        p->scratch_cap = 0;
-        hipError_t e = hipMalloc(&p->scratch, sizeof(float) * need);
-        if (e == hipErrorOutOfMemory && pack && base) {  // without room for the copy, as the rows are
-            (void)hipGetLastError();
-            need = base;
-            e = hipMalloc(&p->scratch, sizeof(float) * need);
-        }
-        SPEO_TRY_HIP(e);
-        p->scratch_cap = need;
-    }
-    return eval_problem(p->h, X, ld, n, f_out, p->scratch, p->scratch_cap, precision,
+    if (n == 0) return SPEO_OK;
+    StreamMemory mem{as_stream(stream)};
+    if (!p->h.generic)
+        SPEO_TRY(mem.status(p->scratch.reserve(eval_scratch_floats(p->h.ncomp, p->h.dim, n),
+                                               eval_scratch_batched(p->h.ncomp, p->h.dim, n), mem)));
+    const size_t pack = eval_pack_floats(p->h, X, ld, n);
+    SPEO_TRY(mem.status(p->packed.reserve(0, pack, mem)));
+    return eval_problem(p->h, X, ld, n, f_out, p->scratch.p, p->scratch.cap,
+                        pack && p->packed.cap >= pack ? p->packed.p : nullptr, precision,
                         default_rows_per_block(n, p->h.dim, precision, true), as_stream(stream));
 }
 

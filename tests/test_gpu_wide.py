@@ -135,3 +135,43 @@ def test_stride_beyond_31_bit_offsets(cuda, speo):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(f.cpu().numpy(), g.cpu().numpy())
     prob.close()
+
+
+@pytest.mark.parametrize("objs", [[2], [1, 2, 3]])
+def test_odd_rows_under_capture_after_aligned_ones(cuda, speo, objs):
+    """An evaluation that a first call on aligned rows has prepared can be captured for
+    rows of an odd stride (they are not copied then), and a captured evaluation of
+    aligned rows outlives a later call on odd ones."""
+    import torch
+    D, n = 301, 700
+    prob = _problem(speo, objs, D, 5)
+    Xo = _rows(n, D, D, cuda)
+    Xa = torch.zeros((n, 304), device=cuda)
+    Xa[:, :D] = Xo
+    fo, fa, g, h = (torch.zeros(n, device=cuda) for _ in range(4))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        speo.evaluate(prob, Xa, h, stream=s)
+        s.synchronize()
+        graphs = []
+        for X, f in ((Xo, fo), (Xa, fa)):
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=s):
+                speo.evaluate(prob, X, f, stream=s)
+            graphs.append(graph)
+    torch.cuda.synchronize()
+    for rep in range(4):
+        print(f"replay {rep}", flush=True)
+        X = _rows(n, D, D, cuda) * (1.0 - 0.125 * rep)
+        Xo.copy_(X)
+        Xa[:, :D] = X
+        for graph in graphs:
+            graph.replay()
+        torch.cuda.synchronize()
+        speo.evaluate(prob, Xo, g)  # eager, with the copy
+        speo.evaluate(prob, Xa, h)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(fo.cpu().numpy(), g.cpu().numpy())
+        np.testing.assert_array_equal(fa.cpu().numpy(), h.cpu().numpy())
+    del graphs
+    prob.close()
