@@ -991,13 +991,22 @@ int Engine::epoch_setup() {
     return SPEO_OK;
 }
 
-// The buffer of donors drawn ahead: at most 64 generations and 2^26 rows of them.
+// The buffer of donors drawn ahead, 16 bytes a row and generation: at most 64
+// generations, none past a migration point (a chunk ends there), and outside
+// epoch mode, whose kernel runs a whole chunk from it, no more than the
+// population's own bytes or 64 MiB: by then one generation's draw fills the chip.
+// A surrogate engine draws its own donors and has one generation for profiles.
 int Engine::donor_setup() {
     std::vector<int> row_island((size_t)total_rows);
     for (int i = 0; i < I; ++i)
         for (int r = 0; r < isl[(size_t)i].np; ++r) row_island[(size_t)(isl[(size_t)i].row_off + r)] = i;
     SPEO_TRY(upload_vec(&row_island_dev, row_island));
-    donor_gens = (int)std::max<int64_t>(1, std::min<int64_t>(64, (int64_t(1) << 26) / total_rows));
+    int64_t ahead = std::min<int64_t>(64, (int64_t(1) << 26) / total_rows);
+    if (cfg.interval > 0 && cfg.migration_size > 0) ahead = std::min<int64_t>(ahead, cfg.interval);
+    if (cfg.mode != SPEO_MODE_EPOCH)
+        ahead = std::min(ahead, std::max<int64_t>(int64_t(64) << 20, 4 * total_elems) / (16 * (int64_t)total_rows));
+    if (cfg.surrogate_candidates > 0) ahead = 1;
+    donor_gens = (int)std::max<int64_t>(1, ahead);
     SPEO_TRY_HIP(hipMalloc(&donor_buf, sizeof(int4) * (size_t)donor_gens * (size_t)total_rows));
     return SPEO_OK;
 }

@@ -77,3 +77,29 @@ def test_migration_ranks(cuda, speo, oracle, sizes, k):
     np.testing.assert_array_equal(out[1][0], Xo)
     for p in probs:
         p.close()
+
+
+@pytest.mark.parametrize("mode", ["PLAIN", "FUSED"])
+@pytest.mark.parametrize("islands,rows,D,interval", [(1024, 1024, 10, 0), (512, 1024, 60, 2), (4, 100, 5, 0)])
+def test_donor_memory_in_proportion(cuda, speo, mode, islands, rows, D, interval):
+    """An engine's device memory beyond its three population arrays: at most one more of
+    them, or 64 MiB, for the donors drawn ahead, none past a migration point, and the
+    tables and fitness arrays."""
+    import torch
+    prob, = _problems(speo, [(D, [2])])
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    e = speo.Engine([prob], [rows] * islands, [0] * islands, mode=getattr(speo, "MODE_" + mode), seed=3,
+                    rows_per_block=32, interval=interval, migration_size=2 if interval else 0)
+    taken = free0 - torch.cuda.mem_get_info()[0]
+    print(f"{mode} {islands} x {rows} D {D}: {taken / 2 ** 20:.0f} MiB", flush=True)
+    R = islands * rows
+    population = 4 * R * ((D + 3) // 4 * 4)
+    donors = 16 * R * interval if interval else min(16 * R * 64, max(population, 64 << 20))
+    # per row: four fitness values, the row's island, a share of two tile tables (64 bytes
+    # a tile of at least 16 rows); 32 MiB for what the allocator rounds up
+    assert taken < 3 * population + donors + R * (16 + 4 + 8) + (32 << 20)
+    e.run(5)
+    e.sync()
+    e.close()
+    prob.close()
