@@ -41,6 +41,7 @@
 #include "engine.h"
 #include "eval.h"
 #include "surrogate.h"
+#include "wide_core.h"
 
 namespace speo {
 
@@ -511,6 +512,9 @@ struct Engine {
     // islands wider than kTLD (any of them): the evaluation's items, those the
     // tile kernel takes first, then those of rows_chunk; component values
     WideItem *wide_items = nullptr;
+    std::vector<FusedProblem> fused;    // probs_dev's contents
+    std::vector<void *> narrow_frags;   // M in the tile kernel's order, of problems up to kTLD
+    int narrow_fragments(const CompHost &h, const ProblemHost &P, CompDev &c);
     int wide_tile = 0, wide_chunk = 0, wide_ncomp = 1;
     float *gval = nullptr;
     int build_wide_items();
@@ -629,6 +633,7 @@ Engine::~Engine() {
                     AX, Ay, Xb, tb, Xh, yh, predh, ranks_ws, heads_dev, qrel_dev, drawn, round_dev, perm_dev,
                     best_sub_dev, info_dev};
     for (void *b : bufs) (void)hipFree(b);
+    for (void *b : narrow_frags) (void)hipFree(b);
     (void)hipHostFree(best_out);
     if (own_stream && stream) (void)hipStreamDestroy(stream);
 }
@@ -679,7 +684,7 @@ int Engine::build_wide_items() {
         wide_ncomp = std::max(wide_ncomp, P.ncomp);
         for (int g0 = 0; g0 < d.np; g0 += 8 * kWideRows)
             for (int c = 0; c < P.ncomp; ++c) {
-                auto &list = rows_wide_applies(P.view(c, cfg.precision), d.dim, cfg.precision) ? tile : chunk;
+                auto &list = rows_wide_applies(fused[(size_t)d.problem].comp[c], d.dim, cfg.precision) ? tile : chunk;
                 for (int r0 = g0; r0 < std::min(d.np, g0 + 8 * kWideRows); r0 += kWideRows)
                     list.push_back(WideItem{d.elem_off + (int64_t)r0 * d.ld, d.row_off + r0,
                                             std::min(kWideRows, d.np - r0), d.ld, d.dim, d.problem, c});
@@ -705,11 +710,30 @@ int Engine::eval_wide_rows(const float *src, float *out, int rt_, hipStream_t s)
     return SPEO_OK;
 }
 
+// A problem keeps its rotations in the tile kernel's order from 129 columns on;
+// those of narrower islands beside wider ones belong to the engine, in its precision.
+int Engine::narrow_fragments(const CompHost &h, const ProblemHost &P, CompDev &c) {
+    const int dim = P.dim;
+    const size_t fe = wide_frag_elems(dim);
+    const bool f32 = cfg.precision == SPEO_PREC_FP32;
+    const bool half = cfg.precision == SPEO_PREC_FP16 || cfg.precision == SPEO_PREC_FP16X3;
+    void *frag = nullptr;
+    SPEO_TRY_HIP(hipMalloc(&frag, f32 ? 4 * fe : 3 * 2 * fe));
+    narrow_frags.push_back(frag);
+    uint16_t *part = static_cast<uint16_t *>(frag);
+    const uint16_t *src[6] = {h.Mbf[0], h.Mbf[1], h.Mbf[2], h.Mh[0], h.Mh[1], h.Mh[2]};
+    uint16_t *dst[6] = {};
+    for (int q = 0; q < 3 && !f32; ++q) dst[(half ? 3 : 0) + q] = part + q * fe;
+    SPEO_TRY(wide_fragments(h.B32, P.ldb32, src, P.ldm16, dim, f32 ? static_cast<float *>(frag) : nullptr, dst, stream));
+    c.wide = frag;
+    return SPEO_OK;
+}
+
 int Engine::upload_tables() {
     SPEO_TRY(upload_vec(&isl_dev, isl));
     SPEO_TRY(upload_vec(&row_off_dev, row_off));
     SPEO_TRY(upload_vec(&dst_dev, dst));
-    std::vector<FusedProblem> fp(problems.size());
+    fused.resize(problems.size());
     std::vector<const CompParams *> tab(problems.size());
     for (size_t q = 0; q < problems.size(); ++q) {
         const ProblemHost &P = problems[q]->h;
@@ -724,11 +748,12 @@ int Engine::upload_tables() {
             f.bias[c] = (float)P.comp[c].bias;
             f.sigma[c] = (float)P.comp[c].sigma;
             f.comp[c] = P.view(c, cfg.precision);
+            if (!all_small && P.dim <= kTLD && !P.generic) SPEO_TRY(narrow_fragments(P.comp[c], P, f.comp[c]));
         }
-        fp[q] = f;
+        fused[q] = f;
         tab[q] = P.params_dev;
     }
-    SPEO_TRY(upload_vec(&probs_dev, fp));
+    SPEO_TRY(upload_vec(&probs_dev, fused));
     SPEO_TRY(upload_vec(&params_tab_dev, tab));
     const int k = std::max(cfg.migration_size, 1);
     SPEO_TRY_HIP(hipMalloc(&best_buf, sizeof(int) * (size_t)I * k));

@@ -172,14 +172,14 @@ __global__ void k_wide_fragments(const float *B32, int ldb32, const uint16_t *m0
     for (int e = threadIdx.x; e < nst * 64; e += blockDim.x) {
         const int s = e >> 6, l = e & 63, lr = l & 15, lk = l >> 4, col = 16 * ct + lr;
         const size_t at = (size_t)ct * nst + s;
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < 8 && f32; ++u) {
             const int k = 32 * s + 16 * (u >> 2) + 4 * (u & 3) + lk;
             f32[((at * 2 + (u >> 2)) * 64 + l) * 4 + (u & 3)] =
                 col < dim && k < dim ? B32[(size_t)k * ldb32 + col] : 0.f;
         }
 #pragma unroll
         for (int p = 0; p < 6; ++p)
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < 8 && f[p]; ++u) {
                 const int k = 32 * s + 8 * lk + u;
                 f[p][(at * 64 + l) * 8 + u] = col < dim && k < dim ? m[p][(size_t)col * ldm16 + k] : (uint16_t)0;
             }

@@ -39,7 +39,8 @@ struct CompHost {
     float *B32s = nullptr;                                   // 128 x 128, fragment order
     uint16_t *Mbfs[3] = {nullptr, nullptr, nullptr};         // [128][round_up(dim,32)]
     uint16_t *Mhs[3] = {nullptr, nullptr, nullptr};
-    float *wide32 = nullptr;    // M in the wide kernels' fragment order (wide_core.h): FP32,
+    // dim > 128, FP32 epilogues only: M in the wide kernels' fragment order (wide_core.h):
+    float *wide32 = nullptr;    // FP32,
     uint16_t *wide_bf = nullptr, *wide_h = nullptr;  // the three BF16 and the three FP16 parts
     float *colw = nullptr;      // [dim] bent cigar / discus weights (elliptic: ProblemHost::colw)
     int heavy_j = -1;           // heavy_column of the objective, found once (it takes dim

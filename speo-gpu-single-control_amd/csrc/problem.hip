@@ -284,9 +284,10 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
             data.add(&h.Mbf[p], pb[p]);
             data.add(&h.Mh[p], ph[p]);
         }
-        // (the kernels move through the three parts by 32-bit byte offsets)
+        // for the tile kernels of wide problems (an engine that also holds narrower
+        // ones makes theirs; the generic kernel reads none)
         const size_t fe = wide_frag_elems(dim);
-        if (3 * 2 * fe < 0x7fffffffull) {
+        if (dim > kSmallD && !generic && wide_frag_fits(dim)) {
             data.reserve(&h.wide32, fe);
             data.reserve(&h.wide_bf, 3 * fe);
             data.reserve(&h.wide_h, 3 * fe);

@@ -317,6 +317,9 @@ __device__ __forceinline__ void wide_gemm(const WideOperands &o, int chunk0, int
 // e, holding M[16 ct + lr][32 s + 16 h + 4 e + lk]; 16-bit, per part: lane l's
 // eight values M[16 ct + lr][32 s + 8 lk ..] at ((ct nst + s) 64 + l) 8.
 __host__ __device__ inline size_t wide_frag_elems(int dim) { return (size_t)round_up((dim + 15) / 16, 16) * 16 * round_up(dim, 32); }
+// The kernels move through the three 16-bit parts by 32-bit byte offsets.
+inline bool wide_frag_fits(int dim) { return 3 * 2 * wide_frag_elems(dim) < 0x7fffffffull; }
+// f32 and the six of f16 (BF16 parts, FP16 parts): any may be null.
 int wide_fragments(const float *B32, int ldb32, const uint16_t *const M16[6], int ldm16, int dim, float *f32,
                    uint16_t *const f16[6], hipStream_t s);
 
