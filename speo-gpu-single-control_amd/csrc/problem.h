@@ -75,9 +75,10 @@ struct ProblemHost {
     bool generic = false;
     int *perm[kMaxComp] = {};       // hybrids: 1-based shuffle [dim] on the device
     GenProblem *gen = nullptr;      // the FP64 kernel's description, on the device (dim <= 1024)
-    // Every array above lies in one of two device allocations: the data, and the
-    // tables that point into it (params_dev, gen).
-    void *data = nullptr, *tables = nullptr;
+    // Every array above lies in one of two device allocations, the data and the
+    // tables that point into it (params_dev, gen); the data of components of more
+    // than 4 MiB in one each.
+    void *data[kMaxComp + 1] = {}, *tables = nullptr;
 };
 
 }  // namespace speo

@@ -122,10 +122,13 @@ class DeviceArrays {
         items_.push_back(Item{[dst](char *at) { *dst = reinterpret_cast<T *>(at); }, size_, {}});
         size_ += (sizeof(T) * n + 255) / 256 * 256;
     }
+    static constexpr size_t kStage = 4u << 20;  // up to here gathered into one copy
+    bool large() const { return size_ > kStage; }
+    // The arrays placed in an allocation of their own, the host's copies gone.
     int commit(void **allocation) {
+        if (size_ == 0) return SPEO_OK;
         SPEO_TRY_HIP(hipMalloc(allocation, size_));
         char *base = static_cast<char *>(*allocation);
-        constexpr size_t kStage = 4u << 20;  // up to here gathered into one copy
         std::vector<char> stage;
         if (size_ <= kStage) stage.resize(size_);
         for (Item &i : items_) {
@@ -137,6 +140,8 @@ class DeviceArrays {
                 SPEO_TRY_HIP(hipMemcpy(base + i.at, i.bytes.data(), i.bytes.size(), hipMemcpyHostToDevice));
         }
         if (!stage.empty()) SPEO_TRY_HIP(hipMemcpy(base, stage.data(), size_, hipMemcpyHostToDevice));
+        items_.clear();
+        size_ = 0;
         return SPEO_OK;
     }
 
@@ -174,11 +179,14 @@ struct StreamMemory {
 };
 
 static void free_problem(ProblemHost &P) {
-    (void)hipFree(P.data);
+    for (void *&d : P.data) {
+        (void)hipFree(d);
+        d = nullptr;
+    }
     (void)hipFree(P.tables);
     for (CompHost &h : P.comp) h = CompHost{};
     for (int *&p : P.perm) p = nullptr;
-    P.data = P.tables = nullptr;
+    P.tables = nullptr;
     P.gen = nullptr;
     P.generic = false;
     P.colw = nullptr;
@@ -320,8 +328,10 @@ static int create_problem(int dim, int ncomp, const int *objectives, const doubl
             if (objectives[c] >= SPEO_OBJ_HYBRID_1)
                 data.add(&P.perm[c], std::vector<int>(shuffle + (size_t)c * dim, shuffle + (size_t)(c + 1) * dim));
         }
+        // (the host holds one component's arrays of a wide composition, not all)
+        if (data.large()) SPEO_TRY(data.commit(&P.data[c]));
     }
-    SPEO_TRY(data.commit(&P.data));
+    SPEO_TRY(data.commit(&P.data[ncomp]));
     for (int c = 0; c < ncomp; ++c) {
         CompHost &h = P.comp[c];
         params[(size_t)c] = CompParams{h.objective, h.rate64, h.sigma, h.bias, h.lambda,

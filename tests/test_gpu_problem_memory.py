@@ -65,3 +65,32 @@ def test_narrow_islands_beside_wide_ones(cuda, speo, prec):
         np.testing.assert_array_equal(a, b)
     for p in probs:
         p.close()
+
+
+_HOST = """
+import resource, sys
+import numpy as np, torch
+sys.path.insert(0, {pkg!r})
+import speo_de as S
+torch.zeros(1, device="cuda")
+rng = np.random.default_rng(1)
+D, nc = 1200, 8
+S.Problem([2], rng.random((1, D)), rng.random((1, D, D))).close()
+o, M = rng.random((nc, D)), rng.random((nc, D, D))
+before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+S.Problem([2] * nc, o, M)
+print("grown", resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before, flush=True)
+"""
+
+
+def test_host_memory_of_a_composition(cuda, speo):
+    """The host holds the arrays of one component of a wide composition at a time: 24
+    bytes an element twice (made and gathered), not of all eight."""
+    import subprocess
+    import sys
+    from conftest import REPO
+    res = subprocess.run([sys.executable, "-c", _HOST.format(pkg=str(REPO / "speo-gpu-single-control_amd"))],
+                         capture_output=True, text=True, timeout=100, check=True)
+    grown = int(res.stdout.split("grown")[1]) * 1024
+    print(f"{grown / 2 ** 20:.0f} MiB", flush=True)
+    assert grown < 3 * 24 * 1200 ** 2 + (32 << 20)
