@@ -516,6 +516,7 @@ struct Engine {
     std::vector<void *> narrow_frags;   // M in the tile kernel's order, of problems up to kTLD
     int narrow_fragments(const CompHost &h, const ProblemHost &P, CompDev &c);
     int wide_tile = 0, wide_chunk = 0, wide_ncomp = 1;
+    int wide_dim = 0;  // the widest of the tile kernel's items (their shift lies in LDS)
     float *gval = nullptr;
     int build_wide_items();
     int eval_wide_rows(const float *src, float *out, int rt_, hipStream_t s);
@@ -684,7 +685,9 @@ int Engine::build_wide_items() {
         wide_ncomp = std::max(wide_ncomp, P.ncomp);
         for (int g0 = 0; g0 < d.np; g0 += 8 * kWideRows)
             for (int c = 0; c < P.ncomp; ++c) {
-                auto &list = rows_wide_applies(fused[(size_t)d.problem].comp[c], d.dim, cfg.precision) ? tile : chunk;
+                const bool tiled = rows_wide_applies(fused[(size_t)d.problem].comp[c], d.dim, cfg.precision);
+                auto &list = tiled ? tile : chunk;
+                if (tiled) wide_dim = std::max(wide_dim, d.dim);
                 for (int r0 = g0; r0 < std::min(d.np, g0 + 8 * kWideRows); r0 += kWideRows)
                     list.push_back(WideItem{d.elem_off + (int64_t)r0 * d.ld, d.row_off + r0,
                                             std::min(kWideRows, d.np - r0), d.ld, d.dim, d.problem, c});
@@ -704,7 +707,7 @@ int Engine::eval_wide_rows(const float *src, float *out, int rt_, hipStream_t s)
     WideRowsArgs rest = a;
     rest.items = wide_items + wide_tile;
     const int nsplit = 64 / rt_;
-    SPEO_TRY(rows_wide(a, wide_tile, max_dim, cfg.precision, nsplit, s));
+    SPEO_TRY(rows_wide(a, wide_tile, wide_dim, cfg.precision, nsplit, s));
     SPEO_TRY(rows_chunk(rest, wide_chunk, cfg.precision, nsplit, s));
     if (wide_ncomp > 1) SPEO_TRY(rows_combine(a, wide_tile + wide_chunk, wide_ncomp, s));
     return SPEO_OK;
