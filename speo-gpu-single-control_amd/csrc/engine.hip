@@ -612,6 +612,7 @@ struct Engine {
     bool tuning_child = false;
     int tuned_from_cache = 0;  // bit 0: row tile, bit 1: epoch parts
     std::string tune_key(const char *what) const;
+    std::string plan_key(const char *what) const;
     int tune_epoch_parts();
     // epoch mode: generations as fused launches instead of an epoch kernel
     bool by_launches = false;
@@ -1974,23 +1975,42 @@ std::string Engine::tune_key(const char *what) const {
     return k.str();
 }
 
-// Seconds of 24 generations of a throwaway engine of this configuration, after
-// a warm-up that captures the graphs.
+// The key of a choice that was timed by whole runs: they have graphs or not, and
+// their launches end at the migration points.
+std::string Engine::plan_key(const char *what) const {
+    return tune_key(what) + ":g" + (cfg.use_graph ? '1' : '0') + ":i" +
+           std::to_string(cfg.migration_size > 0 ? cfg.interval : 0);
+}
+
+// Seconds a generation of a throwaway engine of this configuration, graphs or
+// not as it has them: the median of three runs of whole intervals (16 generations
+// where none are shorter), which are all of one launch sequence; the graphs that a
+// run needs are captured before its clock starts, and the first, cold one counts
+// no more than the others.
 int Engine::time_plan(int parts, bool launches, double *seconds) {
+    constexpr int kGens = 16;
     speo_engine_config c2 = cfg;
     c2.epoch_parts = parts;
-    c2.use_graph = 1;
     c2.rows_per_block = cfg.rows_per_block ? cfg.rows_per_block : 32;
+    const bool migrates = cfg.interval > 0 && cfg.migration_size > 0;
+    if (migrates) c2.interval = std::min(cfg.interval, kGens);
+    const int gens_timed = migrates ? kGens / c2.interval * c2.interval : kGens;
     auto child = std::make_unique<Engine>();
     child->tuning_child = true;
     child->by_launches = launches;
     SPEO_TRY(child->create(c2, stream));
-    SPEO_TRY(child->run(24));
-    SPEO_TRY_HIP(hipStreamSynchronize(stream));
-    const auto t0 = std::chrono::steady_clock::now();
-    SPEO_TRY(child->run(24));
-    SPEO_TRY_HIP(hipStreamSynchronize(stream));
-    *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    if (migrates) SPEO_TRY(child->run(1));  // up to the first migration point
+    double t[3];
+    for (double &dt : t) {
+        SPEO_TRY(child->prepare(gens_timed));
+        SPEO_TRY_HIP(hipStreamSynchronize(stream));
+        const auto t0 = std::chrono::steady_clock::now();
+        SPEO_TRY(child->run(gens_timed));
+        SPEO_TRY_HIP(hipStreamSynchronize(stream));
+        dt = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    }
+    std::sort(t, t + 3);
+    *seconds = t[1] / gens_timed;
     return SPEO_OK;
 }
 
@@ -2013,7 +2033,7 @@ int Engine::tune_launches() {
     std::vector<EpochPlan> plans;
     int lds = 0;
     if (epoch_plan_all(cfg.epoch_parts, &plans, &lds) != SPEO_OK) return SPEO_OK;  // epoch_setup reports it
-    const std::string key = tune_key(("launches" + std::to_string(cfg.epoch_parts)).c_str());
+    const std::string key = plan_key(("launches" + std::to_string(cfg.epoch_parts)).c_str());
     int stored = 0;
     const bool on_file = tune_lookup(key, &stored) && (stored == 0 || stored == 1);
     bool known = on_file;
@@ -2025,8 +2045,12 @@ int Engine::tune_launches() {
     }
     if (!known) {
         double plan = 0.0, launches = 0.0;
-        SPEO_TRY(time_plan(cfg.epoch_parts, false, &plan));
-        SPEO_TRY(time_plan(cfg.epoch_parts, true, &launches));
+        if (time_plan(cfg.epoch_parts, false, &plan) != SPEO_OK ||
+            time_plan(cfg.epoch_parts, true, &launches) != SPEO_OK) {
+            // no room beside this engine, say: it runs as planned, unmeasured
+            (void)hipGetLastError();
+            return SPEO_OK;
+        }
         stored = launches < plan ? 1 : 0;
     }
     if (!on_file) tune_store(key, stored);  // (also a choice measured while another file was in use)
@@ -2038,10 +2062,9 @@ int Engine::tune_launches() {
 
 // Workgroups per island for epoch mode: every feasible power of two up to 8
 // (islands x parts at most four per compute unit) timed on a throwaway
-// engine of this configuration over 24 generations after a warm-up that
-// captures the graphs; the fastest is kept and persisted.
+// engine of this configuration; the fastest is kept and persisted.
 int Engine::tune_epoch_parts() {
-    const std::string key = tune_key("epoch_parts");
+    const std::string key = plan_key("epoch_parts");
     int stored = 0;
     if (tune_lookup(key, &stored) && (stored == 1 || stored == 2 || stored == 4 || stored == 8)) {
         cfg.epoch_parts = stored;

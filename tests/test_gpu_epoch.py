@@ -216,3 +216,40 @@ def test_epoch_by_launches_equals_kernel(cuda, speo, oracle, tmp_path, monkeypat
     assert kms["epoch"] > 0 and kms["donors"] > 0
     plain.run(70)
     _assert_same(plain, engines[1])
+
+
+def test_epoch_choices_per_graph_and_interval(cuda, speo, oracle, tmp_path, monkeypatch):
+    # a choice is timed by runs with the engine's graphs (or none) and interval, and is
+    # read back by engines of the same; choices under the names of an earlier way of
+    # timing are not
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("SPEO_TUNE_CACHE", str(cache))
+    probs = _problems(speo, oracle, [(30, 2)], base=3200)
+    kw = dict(F=0.5, CR=0.9, seed=SEED, migration_size=2, rows_per_block=32, mode=speo.MODE_EPOCH)
+    cache.write_text("epoch_parts:m2:p0:n9:30/128*9 4\nlaunches4:m2:p0:n9:30/128*9 1\n"
+                     "launches1:m2:p0:n9:30/128*9 1\n")
+    old = len(cache.read_text().splitlines())
+    combos = [(False, 10), (True, 10), (True, 25), (False, 0)]
+    for graph, interval in combos:
+        print(f"graph {graph} interval {interval}", flush=True)
+        speo.Engine(probs, [100] * 9, [0] * 9, use_graph=graph, interval=interval, **kw).close()
+    lines = cache.read_text().splitlines()[old:]
+    for what in ("epoch_parts", "launches"):
+        keys = [ln.split()[0] for ln in lines if ln.startswith(what)]
+        assert len(set(keys)) == len(keys) == len(combos)
+    for graph, interval in combos:  # all known now
+        speo.Engine(probs, [100] * 9, [0] * 9, use_graph=graph, interval=interval, **kw).close()
+    assert cache.read_text().splitlines()[old:] == lines
+    # either way of running under graphs gives the plain engine's bits
+    keys = [ln.split()[0] for ln in lines]
+    for choice in (0, 1):
+        cache.write_text("".join(f"launches1{k[9:]} {choice}\n" if k.startswith("launches") else f"{k} 1\n"
+                                 for k in keys))
+        e = speo.Engine(probs, [100] * 9, [0] * 9, use_graph=True, interval=10, **kw)
+        plain = speo.Engine(probs, [100] * 9, [0] * 9, interval=10, **dict(kw, mode=speo.MODE_PLAIN))
+        for chunk in (1, 24, 11):
+            e.run(chunk)
+            plain.run(chunk)
+        _assert_same(plain, e)
+        e.close()
+        plain.close()
