@@ -613,6 +613,7 @@ struct Engine {
     int tuned_from_cache = 0;  // bit 0: row tile, bit 1: epoch parts
     std::string tune_key(const char *what) const;
     std::string plan_key(const char *what) const;
+    bool runs_fused() const;
     int tune_epoch_parts();
     // epoch mode: generations as fused launches instead of an epoch kernel
     bool by_launches = false;
@@ -1495,12 +1496,17 @@ int Engine::migrate(hipStream_t s) {
                         cfg.migration_size, s);
 }
 
+// Whether a plain engine's generations are fused launches (enqueue_plain).
+bool Engine::runs_fused() const {
+    return cfg.mode == SPEO_MODE_PLAIN && cfg.surrogate_candidates == 0 && !configured && !any_generic;
+}
+
 // L generations, then (optionally) migration, then gen_base += L.  The parity
 // `p` and `pending` advance on the host as the launches are enqueued.
 int Engine::enqueue_chunk(int L, bool do_migrate, hipStream_t s) {
     if (cfg.mode == SPEO_MODE_EPOCH) {
         SPEO_TRY(launch_epoch_chunk(L, s));
-    } else if (cfg.mode == SPEO_MODE_PLAIN && C == 0 && !configured && !any_generic) {
+    } else if (runs_fused()) {
         SPEO_TRY(enqueue_plain(L, s));
     } else {
         for (int g = 0; g < L; ++g) {
@@ -1864,7 +1870,10 @@ int Engine::profile_epoch(int generations, double *avg_ms) {
 int Engine::autotune() {
     static std::mutex mu;
     static std::map<std::vector<int>, int> cache;
-    std::vector<int> key{cfg.precision, by_launches ? -1 : cfg.mode};
+    // timed by the kernel that the engine's generations run
+    const bool plain = runs_fused();
+    const int mode = cfg.mode == SPEO_MODE_FUSED || by_launches || plain ? kModeFused : kModeEval;
+    std::vector<int> key{cfg.precision, by_launches ? -1 : plain ? -2 : cfg.mode};
     for (const auto &d : isl) {
         key.push_back(d.np);
         key.push_back(d.dim);
@@ -1877,7 +1886,7 @@ int Engine::autotune() {
             return SPEO_OK;
         }
     }
-    const std::string pkey = tune_key(by_launches ? "rt_launches" : "rt");
+    const std::string pkey = tune_key(by_launches ? "rt_launches" : plain ? "rt_plain" : "rt");
     int stored = 0;
     if (tune_lookup(pkey, &stored) && (stored == 16 || stored == 32 || stored == 64)) {
         rt = stored;
@@ -1914,10 +1923,11 @@ int Engine::autotune() {
     float best_ms = 1e30f;
     int best_rt = 32;
     const int saved_p = p;
+    const bool saved_pending = pending;
+    pending = true;  // as all generations of a run but its first
     SPEO_TRY(build_tiles(kTrialRows));
     for (int cand : {16, 32, 64}) {
         SPEO_TRY(build_tiles(cand));
-        const int mode = cfg.mode == SPEO_MODE_FUSED || by_launches ? kModeFused : kModeEval;
         if (donor_buf) SPEO_TRY(draw_ahead(0, std::min(6, donor_gens), stream));
         for (int rep = 0; rep < 2; ++rep) SPEO_TRY(launch(mode, rep, cand, stream));
         SPEO_TRY_HIP(hipEventRecord(e0, stream));
@@ -1936,6 +1946,7 @@ int Engine::autotune() {
         }
     }
     p = saved_p;
+    pending = saved_pending;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     X = saveX;

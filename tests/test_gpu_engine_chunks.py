@@ -103,3 +103,32 @@ def test_donor_memory_in_proportion(cuda, speo, mode, islands, rows, D, interval
     e.sync()
     e.close()
     prob.close()
+
+
+def test_row_tile_chosen_for_the_kernel_that_runs(cuda, speo, tmp_path, monkeypatch):
+    """rows_per_block = 0: a plain engine's tile is timed by the fused launches that its
+    runs consist of, under a name of its own; engines whose generations are separate
+    launches keep the other.  Stored choices are taken, and change no result."""
+    cache = tmp_path / "tune.txt"
+    monkeypatch.setenv("SPEO_TUNE_CACHE", str(cache))
+    probs = _problems(speo, [(21, [2])])
+    kw = dict(seed=3, mode=speo.MODE_PLAIN)
+    shape = "m0:p0:n3:21/64*3"
+    cache.write_text(f"rt:{shape} 64\n")  # timed by the evaluation kernel, under the earlier name
+    a = speo.Engine(probs, [50, 51, 52], [0] * 3, **kw)
+    b = speo.Engine(probs, [50, 51, 52], [0] * 3, **dict(kw, rows_per_block=16))
+    assert [ln.split()[0] for ln in cache.read_text().splitlines()] == [f"rt:{shape}", f"rt_plain:{shape}"]
+    speo.Engine(probs, [48, 44, 52], [0] * 3, strategy=6, **kw).close()
+    assert len(cache.read_text().splitlines()) == 2
+    for e in (a, b):
+        e.run(9)
+    for x, y in zip(a.read() + a.read_trials(), b.read() + b.read_trials()):
+        np.testing.assert_array_equal(x, y)
+    for o in [a, b] + probs:
+        o.close()
+    cache.write_text("rt_plain:m0:p0:n3:22/64*3 64\n")
+    p22 = _problems(speo, [(22, [2])])
+    e = speo.Engine(p22, [50, 51, 52], [0] * 3, **kw)
+    assert e.stats()["rows_per_block"] == 64
+    e.close()
+    p22[0].close()
