@@ -144,7 +144,7 @@ static size_t generic_lds_bytes(int dim) { return sizeof(double) * (size_t)kGenR
 // 16-column tiles of z (NQ per wave, dim <= 256 NQ) on v_mfma_f64_16x16x4f64
 // with the accumulators in registers, z replaces the rows in LDS, and wave r
 // evaluates row r.  K runs in steps of 8 as two MFMA steps whose lanes take
-// k = 8 s + 2 lk and + 1, so that a lane's part of M is one 16-byte load; eight
+// k = 8 s + 2 lk and + 1, so that a lane's part of M is one 16-byte load; four
 // of them are in flight before the first is used.
 //
 // What bounds it: at D = 100 the objective phase (FP64 vector work, one row

@@ -386,19 +386,12 @@ static int launch_values(const GenerationArgs &a, int ntiles, hipStream_t s) {
 
 template <int RT, int PREC>
 static int launch_mode(int mode, const GenerationArgs &a, int ntiles, hipStream_t s) {
-    switch (mode) {
-    case kModeGen: return launch_generation<RT, PREC, kModeGen, false>(a, ntiles, s);
-    case kModeEval: return launch_values<RT, PREC, kModeEval>(a, ntiles, s);
-    case kModeSelect: return launch_generation<RT, SPEO_PREC_FP32, kModeSelect, false>(a, ntiles, s);
-    case kModeFusedGen: return launch_generation<RT, SPEO_PREC_FP32, kModeFusedGen, false>(a, ntiles, s);
-    default: return launch_values<RT, PREC, kModeFused>(a, ntiles, s);
-    }
+    return mode == kModeEval ? launch_values<RT, PREC, kModeEval>(a, ntiles, s)
+                             : launch_values<RT, PREC, kModeFused>(a, ntiles, s);
 }
 
 template <int RT>
 static int launch_prec(int prec, int mode, const GenerationArgs &a, int ntiles, hipStream_t s) {
-    if (mode == kModeGen || mode == kModeSelect || mode == kModeFusedGen)
-        return launch_mode<RT, SPEO_PREC_FP32>(mode, a, ntiles, s);
     switch (prec) {
     case SPEO_PREC_FP32: return launch_mode<RT, SPEO_PREC_FP32>(mode, a, ntiles, s);
     case SPEO_PREC_BF16: return launch_mode<RT, SPEO_PREC_BF16>(mode, a, ntiles, s);
@@ -410,6 +403,7 @@ static int launch_prec(int prec, int mode, const GenerationArgs &a, int ntiles, 
     }
 }
 
+// kModeEval and kModeFused, tiles of rt rows.
 static int launch_any(int rt, int prec, int mode, const GenerationArgs &a, int ntiles,
                       hipStream_t s) {
     switch (rt) {
@@ -417,6 +411,16 @@ static int launch_any(int rt, int prec, int mode, const GenerationArgs &a, int n
     case 32: return launch_prec<32>(prec, mode, a, ntiles, s);
     case 64: return launch_prec<64>(prec, mode, a, ntiles, s);
     default: return set_error(SPEO_ERR_ARG, "rows_per_block must be 16, 32 or 64");
+    }
+}
+
+// The roles without evaluation, tiles of kTrialRows.
+static int launch_trials(int mode, const GenerationArgs &a, int ntiles, hipStream_t s) {
+    constexpr int RT = kTrialRows, FP32 = SPEO_PREC_FP32;
+    switch (mode) {
+    case kModeGen: return launch_generation<RT, FP32, kModeGen, false>(a, ntiles, s);
+    case kModeSelect: return launch_generation<RT, FP32, kModeSelect, false>(a, ntiles, s);
+    default: return launch_generation<RT, FP32, kModeFusedGen, false>(a, ntiles, s);
     }
 }
 
@@ -1324,7 +1328,7 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear, 
         a.fU_new = fU[1 - u];
         if (!all_small) {
             a.tiles = tiles_dev[kTrialRows];
-            SPEO_TRY(launch_any(kTrialRows, cfg.precision, kModeFusedGen, a, ntiles[kTrialRows], s));
+            SPEO_TRY(launch_trials(kModeFusedGen, a, ntiles[kTrialRows], s));
             return eval_wide_rows(a.U_new, a.fU_new, rt_, s);
         }
         break;
@@ -1332,7 +1336,7 @@ int Engine::launch(int mode, int gen_offset, int rt_, hipStream_t s, int clear, 
     }
     if (mode == kModeGen || mode == kModeSelect) {
         a.tiles = tiles_dev[kTrialRows];
-        return launch_any(kTrialRows, cfg.precision, mode, a, ntiles[kTrialRows], s);
+        return launch_trials(mode, a, ntiles[kTrialRows], s);
     }
     return launch_any(rt_, cfg.precision, mode, a, ntiles[rt_], s);
 }

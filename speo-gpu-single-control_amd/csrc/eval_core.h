@@ -474,11 +474,7 @@ __device__ __forceinline__ void stage_chunk_16(const CompDev &c, const RowSource
 // sum16, done by the caller).  All 256 threads of the block must call it.
 // src.rows is in global memory.
 // `lds` must hold gemm_lds_bytes<RT, PREC>() bytes.
-// VS: vector staging (ChunkF32 / stage_chunk_16) where the rows allow it.  Its registers
-// count in every kernel that contains the call, so a kernel whose other paths
-// need them (the generation kernel's small-D phases) keeps the element-wise
-// form.
-template <int RT, int PREC, bool VS = true>
+template <int RT, int PREC>
 __device__ __forceinline__ void gemm_chunk(const CompDev &c, RowSource src, int dim, int n0,
                                            char *lds, float (&s1)[4], float (&s2)[4]) {
     constexpr int NSPLIT = 4 / (RT / 16);  // waves sharing one 16-row tile
@@ -503,18 +499,18 @@ __device__ __forceinline__ void gemm_chunk(const CompDev &c, RowSource src, int 
                            : (c.ldm16 & 7) == 0 && (reinterpret_cast<uintptr_t>(c.M16[0]) & 15) == 0 &&
                                  (Prec<PREC>::parts < 2 || (reinterpret_cast<uintptr_t>(c.M16[1]) & 15) == 0) &&
                                  (Prec<PREC>::parts < 3 || (reinterpret_cast<uintptr_t>(c.M16[2]) & 15) == 0);
-    const bool vec = VS && b_vec && (src.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(src.rows) & 15) == 0;
+    const bool vec = b_vec && (src.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(src.rows) & 15) == 0;
 
     if constexpr (Prec<PREC>::parts == 0) {
         float *As = reinterpret_cast<float *>(lds);  // [RT][kKC+2]
         float *Bs = As + RT * (kKC + 2);             // [kKC][kNC+16]
         constexpr int LDA = kKC + 2, LDB = kNC + 16;
         ChunkF32<RT> stg;
-        if (VS && vec) stg.load(c, src, 0, min(kKC, dim), n0, ncols, tid);
+        if (vec) stg.load(c, src, 0, min(kKC, dim), n0, ncols, tid);
         for (int k0 = 0; k0 < dim; k0 += kKC) {
             const int kc = min(kKC, dim - k0);
             __syncthreads();
-            if (VS && vec) {
+            if (vec) {
                 stg.store(c, src, k0, kc, ncols, As, Bs, tid);
                 if (k0 + kKC < dim) stg.load(c, src, k0 + kKC, min(kKC, dim - k0 - kKC), n0, ncols, tid);
             } else {
@@ -556,7 +552,7 @@ __device__ __forceinline__ void gemm_chunk(const CompDev &c, RowSource src, int 
         for (int k0 = 0; k0 < dim; k0 += kKC) {
             const int kc = min(kKC, dim - k0);
             __syncthreads();
-            if (VS && vec) {
+            if (vec) {
                 stage_chunk_16<RT, P, H>(c, src, k0, kc, n0, ncols, As, Bs, tid);
             } else {
                 for (int e = tid; e < RT * kKC; e += 256) {
@@ -812,104 +808,96 @@ template <int RT, int PREC>
 __device__ __forceinline__ void gemm_small(const CompDev &c, const float *rows, int dim, int cls,
                                            char *scratch, float (&s1)[RT / 16][4],
                                            float (&s2)[RT / 16][4]) {
-    if constexpr (Prec<PREC>::parts == 0) {
-        SmallB B;
-        B.load(c, dim, cls);
-        B.stage(scratch);
-        __syncthreads();
-        gemm_small_f32<RT>(c, B, rows, dim, cls, scratch, s1, s2);
-        return;
-    } else {
-        constexpr int NRT = RT / 16;
-        const int tid = threadIdx.x, lane = tid & 63;
-        const int lr = lane & 15, lk = lane >> 4;
-        float *sh = reinterpret_cast<float *>(scratch);  // shift, then rate-scaled in place
-        floatx4 acc[NRT][2];
+    static_assert(Prec<PREC>::parts > 0, "FP32: gemm_small_f32");
+    constexpr int NRT = RT / 16;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int lr = lane & 15, lk = lane >> 4;
+    float *sh = reinterpret_cast<float *>(scratch);  // shift, then rate-scaled in place
+    floatx4 acc[NRT][2];
 #pragma unroll
-        for (int i = 0; i < NRT; ++i) {
-            acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
-            acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-        const int t0 = cls, t1 = cls + 4;
-        const bool v0 = t0 * 16 < dim, v1 = t1 * 16 < dim;
+    for (int i = 0; i < NRT; ++i) {
+        acc[i][0] = floatx4{0.f, 0.f, 0.f, 0.f};
+        acc[i][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int t0 = cls, t1 = cls + 4;
+    const bool v0 = t0 * 16 < dim, v1 = t1 * 16 < dim;
 
-        constexpr int P = Prec<PREC>::parts;
-        constexpr bool H = Prec<PREC>::half;
-        typedef typename std::conditional<H, halfx8, bf16x8>::type vec8;
-        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-        const int kp32 = c.kp32, KS = kp32 >> 5, LDA = kSmallD + 8;  // KS <= 4
-        uint16_t *As = reinterpret_cast<uint16_t *>(sh + kSmallD);  // [P][RT][LDA]
-        // B's fragments ahead of the staging: all four K steps' (64 registers
-        // with two parts), with three parts two steps' at a time
-        constexpr int DEPTH = P <= 2 ? 4 : 2;
-        vec8 b[DEPTH][2][P];
-        auto fetch = [&](int ks) {
-            if (ks >= KS) return;
-            const int kb = ks * 32 + lk * 8;
+    constexpr int P = Prec<PREC>::parts;
+    constexpr bool H = Prec<PREC>::half;
+    typedef typename std::conditional<H, halfx8, bf16x8>::type vec8;
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    const int kp32 = c.kp32, KS = kp32 >> 5, LDA = kSmallD + 8;  // KS <= 4
+    uint16_t *As = reinterpret_cast<uint16_t *>(sh + kSmallD);  // [P][RT][LDA]
+    // B's fragments ahead of the staging: all four K steps' (64 registers
+    // with two parts), with three parts two steps' at a time
+    constexpr int DEPTH = P <= 2 ? 4 : 2;
+    vec8 b[DEPTH][2][P];
+    auto fetch = [&](int ks) {
+        if (ks >= KS) return;
+        const int kb = ks * 32 + lk * 8;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            if (v0) b[ks % DEPTH][0][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t0 * 16 + lr) * kp32 + kb));
+            if (v1) b[ks % DEPTH][1][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t1 * 16 + lr) * kp32 + kb));
+        }
+    };
+#pragma unroll
+    for (int ks = 0; ks < DEPTH; ++ks) fetch(ks);
+    for (int k = tid; k < kSmallD; k += 256) sh[k] = k < dim ? gld(c.shift + k) : 0.f;
+    __syncthreads();
+    const float scale = c.rate * (H ? kF16ScaleA : 1.0f);
+    // four columns a thread; e / ng = e ceil(2^16 / ng) / 2^16 for e < 64 ng <= 2048
+    const int ng = kp32 >> 2, inv = ng == 24 ? 2731 : 65536 / ng;
+    for (int e = tid; e < RT * ng; e += 256) {
+        const int r = (e * inv) >> 16, k = 4 * (e - r * ng);
+        const floatx4 x = *reinterpret_cast<const floatx4 *>(rows + r * kTS + k);
+        const floatx4 o = *reinterpret_cast<const floatx4 *>(sh + k);
+        u16x4 h[P];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float rem = k + q < dim ? (x[q] - o[q]) * scale : 0.f;
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                if (v0) b[ks % DEPTH][0][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t0 * 16 + lr) * kp32 + kb));
-                if (v1) b[ks % DEPTH][1][p] = gld(reinterpret_cast<const vec8 *>(c.M16s[p] + (size_t)(t1 * 16 + lr) * kp32 + kb));
+                const uint16_t w = to_bits(rem, H);
+                h[p][q] = w;
+                rem -= from_bits(w, H);
             }
-        };
-#pragma unroll
-        for (int ks = 0; ks < DEPTH; ++ks) fetch(ks);
-        for (int k = tid; k < kSmallD; k += 256) sh[k] = k < dim ? gld(c.shift + k) : 0.f;
-        __syncthreads();
-        const float scale = c.rate * (H ? kF16ScaleA : 1.0f);
-        // four columns a thread; e / ng = e ceil(2^16 / ng) / 2^16 for e < 64 ng <= 2048
-        const int ng = kp32 >> 2, inv = ng == 24 ? 2731 : 65536 / ng;
-        for (int e = tid; e < RT * ng; e += 256) {
-            const int r = (e * inv) >> 16, k = 4 * (e - r * ng);
-            const floatx4 x = *reinterpret_cast<const floatx4 *>(rows + r * kTS + k);
-            const floatx4 o = *reinterpret_cast<const floatx4 *>(sh + k);
-            u16x4 h[P];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float rem = k + q < dim ? (x[q] - o[q]) * scale : 0.f;
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const uint16_t w = to_bits(rem, H);
-                    h[p][q] = w;
-                    rem -= from_bits(w, H);
-                }
-            }
-#pragma unroll
-            for (int p = 0; p < P; ++p) *reinterpret_cast<u16x4 *>(As + (p * RT + r) * LDA + k) = h[p];
         }
-        __syncthreads();
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if (ks >= KS) break;
-            const int kb = ks * 32 + lk * 8;
+        for (int p = 0; p < P; ++p) *reinterpret_cast<u16x4 *>(As + (p * RT + r) * LDA + k) = h[p];
+    }
+    __syncthreads();
 #pragma unroll
-            for (int i = 0; i < NRT; ++i) {
-                vec8 a[P];
+    for (int ks = 0; ks < 4; ++ks) {
+        if (ks >= KS) break;
+        const int kb = ks * 32 + lk * 8;
 #pragma unroll
-                for (int p = 0; p < P; ++p)
-                    a[p] = *reinterpret_cast<const vec8 *>(&As[(p * RT + i * 16 + lr) * LDA + kb]);
+        for (int i = 0; i < NRT; ++i) {
+            vec8 a[P];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (t == 0 ? !v0 : !v1) continue;
+            for (int p = 0; p < P; ++p)
+                a[p] = *reinterpret_cast<const vec8 *>(&As[(p * RT + i * 16 + lr) * LDA + kb]);
 #pragma unroll
-                    for (int sum = P - 1; sum >= 0; --sum) {
+            for (int t = 0; t < 2; ++t) {
+                if (t == 0 ? !v0 : !v1) continue;
 #pragma unroll
-                        for (int pa = 0; pa <= sum; ++pa) {
-                            const int pb = sum - pa;
-                            if (pa < P && pb < P) {
-                                if constexpr (H)
-                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
-                                else
-                                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
-                            }
+                for (int sum = P - 1; sum >= 0; --sum) {
+#pragma unroll
+                    for (int pa = 0; pa <= sum; ++pa) {
+                        const int pb = sum - pa;
+                        if (pa < P && pb < P) {
+                            if constexpr (H)
+                                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
+                            else
+                                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa], b[ks % DEPTH][t][pb], acc[i][t], 0, 0, 0);
                         }
                     }
                 }
             }
-            if (DEPTH < 4 && ks + DEPTH < 4) fetch(ks + DEPTH);
         }
-        small_terms<RT, PREC>(c, acc, dim, cls, s1, s2);
+        if (DEPTH < 4 && ks + DEPTH < 4) fetch(ks + DEPTH);
     }
+    small_terms<RT, PREC>(c, acc, dim, cls, s1, s2);
 }
 
 // The column class of a wave: blocks start at different classes, since a

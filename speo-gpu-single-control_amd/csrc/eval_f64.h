@@ -24,7 +24,8 @@ constexpr double kE64 = 2.7182818284590452353602874713526625;
 // Beyond 2^45: the fraction of x / (2 pi) from the bits of 1 / (2 pi) that the
 // integer part does not swallow (Payne and Hanek, 1983).  x = m 2^e with a
 // 53-bit m, so the bits of weight 2^-e and above only add whole turns; the next
-// 128 bits times m, modulo one turn, are the fraction to 2^-75.
+// 128 bits times m, modulo one turn, are the fraction, of which 64 bits are kept
+// (to 2^-63 of a turn).
 constexpr int kTurnWords = 20;
 __device__ inline double large_turns(double x) {
     static const __constant__ uint64_t kTurnBits[kTurnWords + 1] = {  // 1 / (2 pi), after 64 zero bits

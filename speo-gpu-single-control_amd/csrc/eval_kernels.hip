@@ -22,14 +22,15 @@ template <int RT, int PREC> constexpr int eval_small_lds_bytes() {
     return RT * kTS * 4 + small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4;
 }
 
-// RAW: the rotation in c.B32's rows alone (dim <= 128); SMALL: dim <= 128 only.
+// RAW: the rotation in c.B32's rows alone (dim <= 128); SMALL: dim <= 128 only.  The
+// small path has tiles of 16 and 32 rows (default_rows_per_block).
 template <int RT, int PREC, bool RAW, bool SMALL>
 __device__ __forceinline__ void eval_rows(const EvalLaunch &p, const CompDev &c, int chunk, float *f_out) {
     extern __shared__ __align__(16) char lds[];
     const int row0 = blockIdx.x * RT;
     const int nrows = min(RT, p.n - row0);
     float *o1, *o2;
-    if (RAW || SMALL || p.small) {
+    if (RT < 64 && (RAW || SMALL || p.small)) {
         float *rows = reinterpret_cast<float *>(lds);
         char *scratch = lds + RT * kTS * 4;
         float *red = reinterpret_cast<float *>(scratch + small_scratch_bytes<RT>(Prec<PREC>::parts));
@@ -410,6 +411,8 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
     const int nchunks = (dim + kNC - 1) / kNC;
     if (nchunks > 1 && part == nullptr) return set_error(SPEO_ERR_ARG, "eval: missing partial buffer");
     const int small = (dim <= kSmallD && comp.B32s != nullptr) ? 1 : 0;
+    if (small && rows_per_block == 64)
+        return set_error(SPEO_ERR_ARG, "up to 128 columns: 16 or 32 rows per block");
     EvalLaunch p{comp, X, ld, n, dim, f_out, part, nchunks, lambda, bias, raw, small};
     int rc;
     if (use_wide(comp, X, ld, n, dim, precision, rows_per_block)) {
