@@ -112,9 +112,12 @@ __device__ __forceinline__ float comp4(const float4 &v, int q) {
     return q == 0 ? v.x : (q == 1 ? v.y : (q == 2 ? v.z : v.w));
 }
 
-// What bounds the fused kernel: the crossover's Philox blocks (18 wide integer
-// multiplies per four coordinates) and, at D = 100, the FP32 matrix
-// instructions, about equally.  So every lane makes trials (items of a row and
+// What bounds the fused kernel: the chain of a block's phases (a D = 100 block of
+// 32 rows takes about 19 us) and the last blocks behind it, not the chip's issue
+// rates: over a 34 us launch of the uneven islands vector instructions issue in 35 %
+// of the SIMD units' cycles (18 wide integer multiplies per four coordinates of
+// the crossover, at a quarter of the rate, among them), the matrix pipe is busy
+// for 11 %, and 2.9 of the four waves that fit a unit are there.  So every lane makes trials (items of a row and
 // four coordinates, where 16 lanes a row left 13 idle at D = 10), the parents of
 // a row are found once, not by 16 lanes, a generation's donors are drawn ahead
 // of it, one row per lane (k_epoch_donors), and blocks start at different
