@@ -22,15 +22,20 @@ template <int RT, int PREC> constexpr int eval_small_lds_bytes() {
     return RT * kTS * 4 + small_scratch_bytes<RT>(Prec<PREC>::parts) + 10 * RT * 4;
 }
 
-// RAW: the rotation in c.B32's rows alone (dim <= 128); SMALL: dim <= 128 only.  The
-// small path has tiles of 16 and 32 rows (default_rows_per_block).
-template <int RT, int PREC, bool RAW, bool SMALL>
+// How a kernel evaluates its rows: by K chunks (gemm_chunk), the rotation in a
+// problem's layouts for up to 128 columns, or in c.B32's rows alone (the same
+// columns, FP32).  A kernel holds one of them: with the small path's code beside
+// it the chunked form was 1 to 2 % slower (FP32, one component: a row of D = 1000
+// 45.3 us, 44.6 alone; 1,000 rows of D = 500 25.5 / 25.2).
+enum EvalForm { kEvalChunk, kEvalSmall, kEvalRaw };
+template <int RT, int PREC, EvalForm FORM>
 __device__ __forceinline__ void eval_rows(const EvalLaunch &p, const CompDev &c, int chunk, float *f_out) {
     extern __shared__ __align__(16) char lds[];
     const int row0 = blockIdx.x * RT;
     const int nrows = min(RT, p.n - row0);
     float *o1, *o2;
-    if (RT < 64 && (RAW || SMALL || p.small)) {
+    if constexpr (FORM != kEvalChunk) {
+        constexpr bool RAW = FORM == kEvalRaw;
         float *rows = reinterpret_cast<float *>(lds);
         char *scratch = lds + RT * kTS * 4;
         float *red = reinterpret_cast<float *>(scratch + small_scratch_bytes<RT>(Prec<PREC>::parts));
@@ -90,7 +95,7 @@ __device__ __forceinline__ void eval_rows(const EvalLaunch &p, const CompDev &c,
         if constexpr (F32) gemm_small_f32<RT>(c, B, rows, p.dim, cls, scratch, s1, s2);
         else gemm_small<RT, PREC>(c, rows, p.dim, cls, scratch, s1, s2);
         reduce_rows_small<RT>(s1, s2, cls, red, o1, o2);
-    } else if constexpr (!RAW && !SMALL) {
+    } else {
         RowSource src{p.X + (size_t)row0 * p.ld, p.ld, nrows};
         float s1[4] = {0.f, 0.f, 0.f, 0.f}, s2[4] = {0.f, 0.f, 0.f, 0.f};
         gemm_chunk<RT, PREC>(c, src, p.dim, chunk * kNC, lds, s1, s2);
@@ -121,9 +126,9 @@ __device__ __forceinline__ void eval_rows(const EvalLaunch &p, const CompDev &c,
     }
 }
 
-template <int RT, int PREC, bool RAW>
+template <int RT, int PREC, EvalForm FORM>
 __global__ __launch_bounds__(256) void k_eval(EvalLaunch p) {
-    eval_rows<RT, PREC, RAW, false>(p, p.comp, blockIdx.y, p.f_out);
+    eval_rows<RT, PREC, FORM>(p, p.comp, blockIdx.y, p.f_out);
 }
 
 // The components of a composition of up to 128 columns in one launch: block row
@@ -134,7 +139,7 @@ struct EvalComps {
 };
 template <int RT, int PREC>
 __global__ __launch_bounds__(256) void k_eval_comps(EvalComps a) {
-    eval_rows<RT, PREC, false, true>(a.p, a.comp[blockIdx.y], 0, a.p.f_out + (size_t)blockIdx.y * a.p.n);
+    eval_rows<RT, PREC, kEvalSmall>(a.p, a.comp[blockIdx.y], 0, a.p.f_out + (size_t)blockIdx.y * a.p.n);
 }
 
 // The chunks' sums of component blockIdx.y (in chunk order) and its value.
@@ -346,18 +351,25 @@ static std::atomic<int> g_wide_eval{1};
 static std::atomic<long long> g_wide_launches{0};
 bool wide_eval_enabled() { return g_wide_eval.load(std::memory_order_relaxed) != 0; }
 
-template <int RT, int PREC, bool RAW = false>
-static int launch_rt_prec(const EvalLaunch &p, int n, int nchunks, hipStream_t s) {
+template <int RT, int PREC, EvalForm FORM>
+static int launch_form(const EvalLaunch &p, int n, int nchunks, hipStream_t s) {
     static std::once_flag once;
-    constexpr int lds_max = std::max(gemm_lds_bytes<RT, PREC>(), eval_small_lds_bytes<RT, PREC>());
+    constexpr int lds = FORM == kEvalChunk ? gemm_lds_bytes<RT, PREC>() : eval_small_lds_bytes<RT, PREC>();
     std::call_once(once, [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval<RT, PREC, RAW>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_eval<RT, PREC, FORM>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     });
-    const int lds = RAW || p.small ? eval_small_lds_bytes<RT, PREC>() : gemm_lds_bytes<RT, PREC>();
     dim3 grid((n + RT - 1) / RT, nchunks);
-    hipLaunchKernelGGL((k_eval<RT, PREC, RAW>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((k_eval<RT, PREC, FORM>), grid, dim3(256), lds, s, p);
     return check_launch("k_eval");
+}
+
+// (up to 128 columns: tiles of 16 and 32 rows, default_rows_per_block)
+template <int RT, int PREC>
+static int launch_rt_prec(const EvalLaunch &p, int n, int nchunks, hipStream_t s) {
+    if constexpr (RT < 64)
+        if (p.small) return launch_form<RT, PREC, kEvalSmall>(p, n, nchunks, s);
+    return launch_form<RT, PREC, kEvalChunk>(p, n, nchunks, s);
 }
 
 template <int RT, int PREC>
@@ -422,7 +434,7 @@ int eval_component(const CompDev &comp, const float *X, int ld, int n, int dim, 
     } else if (rows_per_block == 16 && precision == SPEO_PREC_FP32 && dim <= kSmallD && !small) {
         // the row-major matrix straight into registers; the 16-row tile's sums
         // are those of the staged path (four column classes in either)
-        rc = launch_rt_prec<16, SPEO_PREC_FP32, true>(p, n, nchunks, s);
+        rc = launch_form<16, SPEO_PREC_FP32, kEvalRaw>(p, n, nchunks, s);
     } else switch (rows_per_block) {
     case 16: rc = launch_rt<16>(p, precision, n, nchunks, s); break;
     case 32: rc = launch_rt<32>(p, precision, n, nchunks, s); break;
