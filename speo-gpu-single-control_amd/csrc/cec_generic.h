@@ -62,6 +62,7 @@ struct GenLaunch {
     float *f32;                // outputs (either may be null)
     double *f64;
     double out_bias;           // added to every output
+    int block_rows;            // set by eval_generic
     // The drop-in call's arrays, component c at c * stride (M^T: c * stride *
     // dim): used in place of the description's shift, rotation, shuffle and
     // sigma when o32 is set.

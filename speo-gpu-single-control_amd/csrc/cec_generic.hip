@@ -134,23 +134,24 @@ __device__ __forceinline__ double seg_value(int obj, const Seg &s, int lane) {
 }  // namespace
 
 // LDS: 16 rows of round_up(dim, 8) + 2 doubles, the shifted rows and then z in
-// the same place, and each row's component values.  (The stride is 4 banks past a multiple of 16, so the 16
-// rows of a 16-byte operand read start in different banks.)
+// the same place, and each row's component values.  (The stride is 4 banks past
+// a multiple of 16, so the 16 rows of a 16-byte operand read start in different
+// banks.)
 static int generic_ld(int dim) { return round_up(dim, 8) + 2; }
 static size_t generic_lds_bytes(int dim) { return sizeof(double) * (size_t)kGenRows * (generic_ld(dim) + 2 * kMaxComp); }
 
-// A block of 16 waves takes 16 rows through every component: wave r shifts
-// row r into LDS (and sums its squared distance), the waves share the
-// 16-column tiles of z (NQ per wave, dim <= 256 NQ) on v_mfma_f64_16x16x4f64
-// with the accumulators in registers, z replaces the rows in LDS, and wave r
-// evaluates row r.  K runs in steps of 8 as two MFMA steps whose lanes take
+// A block takes up to 16 rows (generic_block_rows), a wave each, through every
+// component: wave r shifts row r into LDS (and sums its squared distance), the
+// waves share the 16-column tiles of z (a wave each, up to sixteen waves; NQ per
+// wave, dim <= 256 NQ) on v_mfma_f64_16x16x4f64 with the accumulators in
+// registers, z replaces the rows in LDS, and wave r evaluates row r.  K runs in steps of 8 as two MFMA steps whose lanes take
 // k = 8 s + 2 lk and + 1, so that a lane's part of M is one 16-byte load; four
 // of them are in flight before the first is used.
 //
 // What bounds it: at D = 100 the objective phase (FP64 vector work, one row
 // per wave) and the latency of the phases, at D >= 250 the FP64 matrix pipe (64
 // cycles per step of 4).  Measured, FP64 values of 2048 rows x 250, three
-// components: 770 us with a block per row (M read again for every row), 45 us
+// components: 770 us with a block per row (M read again for every row), 39 us
 // here; a five-component CEC2014 composition on 4096 rows x 100: 164 us with
 // four waves per block (four rows per wave one after another, 8-byte strided
 // loads of M, library cosines), 41 us here.  Up to 256 columns two blocks fit a
@@ -164,10 +165,9 @@ __global__ __launch_bounds__(kGenThreads) __attribute__((amdgpu_waves_per_eu(NQ 
     double *As = reinterpret_cast<double *>(lds_raw);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lr = lane & 15, lk = lane >> 4;
-    const int row0 = blockIdx.x * kGenRows;
-    const int row = row0 + wave;           // this wave's row
-    const bool mine = row < p.n;
+    const int nw = blockDim.x >> 6, lr = lane & 15, lk = lane >> 4;
+    const int row = blockIdx.x * p.block_rows + wave;  // this wave's row
+    const bool mine = wave < p.block_rows && row < p.n;
     const float *x = p.X;
     if (mine) x += (size_t)(p.rows ? p.rows[row] - p.row_base : row) * p.ld;
     double *z = As + wave * ld;
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kGenThreads) __attribute__((amdgpu_waves_per_eu(NQ 
             for (int q = 0; q < NQ; ++q) {
                 acc[q] = doublex4{0.0, 0.0, 0.0, 0.0};
                 __builtin_amdgcn_sched_barrier(0);
-                const int t = wave + (kGenThreads / 64) * q;
+                const int t = wave + nw * q;
                 if (t >= T) continue;
                 const double *a = As + lr * ld + 2 * lk;
                 const int steps = ARRAYS ? dim >> 3 : (dim + 7) >> 3;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kGenThreads) __attribute__((amdgpu_waves_per_eu(NQ 
             // l / 16 + 4 i, column l % 16
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const int col = 16 * (wave + (kGenThreads / 64) * q) + lr;
+                const int col = 16 * (wave + nw * q) + lr;
                 if (col < dim)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) As[(lk + 4 * i) * ld + col] = acc[q][i];
@@ -299,8 +299,10 @@ static int launch_generic(const GenLaunch &p, hipStream_t s) {
                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)generic_lds_bytes(256 * NQ));
     });
-    const dim3 grid((p.n + kGenRows - 1) / kGenRows);
-    hipLaunchKernelGGL((k_eval_generic<NQ, ARRAYS>), grid, dim3(kGenThreads), generic_lds_bytes(p.dim), s, p);
+    const dim3 grid((p.n + p.block_rows - 1) / p.block_rows);
+    // a wave per row and, up to sixteen, per column tile
+    const int waves = std::min(kGenRows, std::max(p.block_rows, (p.dim + 15) / 16));
+    hipLaunchKernelGGL((k_eval_generic<NQ, ARRAYS>), grid, dim3(64 * waves), generic_lds_bytes(p.dim), s, p);
     return check_launch("k_eval_generic");
 }
 
@@ -320,10 +322,25 @@ int check_gen_problem(const GenProblem &g, bool arrays) {
     return SPEO_OK;
 }
 
-int eval_generic(const GenLaunch &p, hipStream_t s) {
+// Rows a block: as few as give no more than a block a compute unit.  A row's
+// objective is its wave's FP64 work, and sixteen rows on one unit while others had
+// none took longer than a block per row had (us, a block of four waves per row /
+// sixteen rows a block / now: 300 rows of D = 2, three components 9.7 / 13.3 / 8.9,
+// five 14.3 / 19.9 / 13.2; 2,048 of D = 250, three 689 / 42.0 / 38.8).  No result
+// depends on it.
+static int generic_block_rows(int n) {
+    constexpr int kUnits = 256;
+    int rows = 1;
+    while (rows < kGenRows && (n + rows - 1) / rows > kUnits) rows *= 2;
+    return rows;
+}
+
+int eval_generic(const GenLaunch &launch, hipStream_t s) {
+    GenLaunch p = launch;
     if (p.n <= 0) return SPEO_OK;
     if (!p.P || p.dim < 1 || p.dim > kGenMaxDim || p.ncomp < 1 || p.ncomp > kMaxComp)
         return set_error(SPEO_ERR_UNSUPPORTED, "generic evaluation: dim must be in [1, 1024]");
+    p.block_rows = generic_block_rows(p.n);
     if (p.o32) return p.dim <= 256 ? launch_generic<1, true>(p, s) : launch_generic<4, true>(p, s);
     return p.dim <= 256 ? launch_generic<1, false>(p, s) : launch_generic<4, false>(p, s);
 }

@@ -132,3 +132,29 @@ def test_best_rows(cuda, speo, oracle, dims):
     eng.close()
     for p in probs:
         p.close()
+
+
+@pytest.mark.parametrize("D,objs", [(3, [1, 2, 3]), (40, [10, 9]), (100, [2]), (300, [3, 6, 7])])
+def test_values_independent_of_the_batch(cuda, speo, D, objs):
+    """Blocks hold 1, 2, 4, 8 or 16 rows as the batch has more than 256, 512, ... of them:
+    a row's value is the same bits in all (FP64 values, and FP32 ones of objectives
+    that the FP64 kernel evaluates)."""
+    import torch
+    rng = np.random.default_rng(D)
+    o = np.float32(rng.uniform(-80, 80, (len(objs), D))).astype(np.float64)
+    prob = speo.Problem(objs, o, np.stack([_rotation(rng, D) for _ in objs]), sigma=[10.0 * (c + 1) for c in range(len(objs))])
+    X = _t(rng.uniform(-100, 100, (4101, D)).astype(np.float32), cuda)
+    whole = torch.zeros(4101, dtype=torch.float64, device=cuda)
+    speo.evaluate_f64(prob, X, whole)
+    w32 = torch.zeros(4101, device=cuda)
+    speo.evaluate(prob, X, w32)
+    for n in (1, 2, 255, 256, 257, 511, 513, 1025, 2048, 2049, 4096, 4097):
+        print(f"D={D} n={n}", flush=True)
+        f = torch.full((n,), -1.0, dtype=torch.float64, device=cuda)
+        speo.evaluate_f64(prob, X[4101 - n:], f)
+        np.testing.assert_array_equal(f.cpu().numpy(), whole[4101 - n:].cpu().numpy())
+        if max(objs) > 8:
+            g = torch.full((n,), -1.0, device=cuda)
+            speo.evaluate(prob, X[4101 - n:], g)
+            np.testing.assert_array_equal(g.cpu().numpy(), w32[4101 - n:].cpu().numpy())
+    prob.close()
